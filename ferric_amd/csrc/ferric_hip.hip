@@ -310,11 +310,191 @@ int i8_q_rot_ticks(State &s, int npanels, int ntp) {
     return (int)std::lround(s.wall_khz * 1.4e-3);
 }
 
+// Which calls run in residue arithmetic (residue.hip), and on what tiles. Measured
+// against the matrix kernel of the same precision (its time / residue time):
+// FP64    past 144 virtuals (one orbital a tile): 24/208/742 1.7, 70/208/889 2.1,
+//         100/200/2400 2.6, 60/450/1800 2.3, 100/900/3600 2.3; at small work the chip
+//         is not full: 14/160/556 1.3, 8/208/691 1.1, 4/340/1100 0.9. With 65 to 128
+//         virtuals two orbitals share a tile: 40/112/486 1.5, 70/128/633 1.6, but
+//         24/112/435 1.0. Fewer virtuals: 70/64/428 0.9.
+// MIXED   24/208/742 1.35, 70/208/889 2.0, 60/450/1800 1.8, 24/160/588 1.15, 40/112/486
+//         1.2, 24/112/435 0.9.
+// INT8X4 stays with its digit slices: ten moduli against their thirteen products gave
+//         70/208/889 1.2, but 70/340/1312 0.95 and 100/900/3600 0.98.
+bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, EnergyPlan *pl) {
+    if (s.arena || forced_tile() > 0 || naux > 4608) return false;
+    EnergyPlan p;
+    p.tile = 256;
+    p.nvir_pad = (int)((nvir + 15) / 16 * 16);
+    p.naux_pad = (int)((naux + 63) / 64 * 64);
+    p.ntile = (p.nvir_pad + p.tile - 1) / p.tile;
+    p.ntp = p.ntile * (p.ntile + 1) / 2;
+    p.group = nvir <= 128 ? 2 : 1;
+    const double work = (double)nocc * (nocc + 1) * (double)nvir * nvir * (double)naux;
+    if (nvir <= 64) return false;
+    switch (prec) {
+    case Prec::F64:
+        if (work < (nvir <= 143 ? 3.5e9 : nocc >= 11 ? 2.5e9 : 8e9)) return false;
+        break;
+    case Prec::MIXED:
+        if (work < 5e9) return false;
+        break;
+    default: return false;
+    }
+    const int64_t ngroup = ((int64_t)nocc + p.group - 1) / p.group;
+    p.nitems = ngroup * (ngroup + 1) / 2 * p.ntp;
+    if (p.nitems > 0x7fffff00LL) return false;
+    if (s.cus <= 0 &&
+        hipDeviceGetAttribute(&s.cus, hipDeviceAttributeMultiprocessorCount, s.device) !=
+            hipSuccess)
+        s.cus = 0;
+    if (s.cus < 8) return false;
+    *pl = p;
+    return true;
+}
+
+namespace {
+
+// Copies the device result (energies, then the row values) back.
+fh_status fetch_result(State &s, const double *dev, size_t nocc, hipStream_t stream,
+                       fh_spin_components *out, double *row_partials) {
+    std::vector<double> res(2 + 2 * nocc);
+    fh_status st = hip_check(hipMemcpyAsync(res.data(), dev, sizeof(double) * res.size(),
+                                            hipMemcpyDeviceToHost, stream),
+                             "D2H result");
+    if (st != FH_OK) return st;
+    st = hip_check(hipStreamSynchronize(stream), "stream sync");
+    if (st != FH_OK) return st;
+    s.pending.d2h_bytes += sizeof(double) * res.size();
+    out->e_os = res[0];
+    out->e_ss = res[1];
+    out->e_total = res[0] + res[1];
+    if (row_partials)
+        for (size_t i = 0; i < 2 * nocc; ++i) row_partials[i] = res[2 + i];
+    return FH_OK;
+}
+
+// Uploads [eps_occ, eps_vir] of the active orbitals.
+fh_status upload_eps(State &s, const double *eps, size_t first_occ, size_t nocc, size_t nocc_total,
+                     size_t nvir, hipStream_t stream) {
+    std::vector<double> e(nocc + nvir);
+    for (size_t i = 0; i < nocc; ++i) e[i] = eps[first_occ + i];
+    for (size_t a = 0; a < nvir; ++a) e[nocc + a] = eps[nocc_total + a];
+    fh_status st = hip_check(hipMemcpyAsync(s.slots[kSlotEps].ptr, e.data(),
+                                            sizeof(double) * e.size(), hipMemcpyHostToDevice,
+                                            stream),
+                             "H2D eps");
+    if (st == FH_OK) s.pending.h2d_bytes += sizeof(double) * e.size();
+    return st;
+}
+
+fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, size_t nocc,
+                         size_t nvir, const double *eps, size_t first_occ, size_t nocc_total,
+                         double kappa, Prec prec, hipStream_t stream, fh_spin_components *out,
+                         double *row_partials, const EnergyPlan &pl) {
+    const size_t rows = nocc * (size_t)pl.nvir_pad;
+    const size_t npairs = nocc * (nocc + 1) / 2;
+    const int blocks = s.cus / 8 * 8;  // whole rounds over the eight XCDs
+    const int words = residue_queue_words(blocks);
+    const size_t sets = (size_t)residue_scratch_sets(blocks);
+    const size_t stride = residue_scratch_stride(prec, pl.ntile > 1 ? 2 : 1);
+    fh_status st = reserve(s, {{kSlotOp0, rows * (size_t)pl.naux_pad * residue_moduli(prec)},
+                               {kSlotStage2, sizeof(double) * (size_t)(pl.naux_pad / 64) * nocc * nvir},
+                               {kSlotEps, sizeof(double) * (nocc + nvir)},
+                               {kSlotItems, sizeof(double) * 4 * npairs * (size_t)pl.ntp},
+                               {kSlotRows, sizeof(double) * 4 * nocc},
+                               {kSlotResult, sizeof(double) * (2 + 2 * nocc)},
+                               {kSlotScale, sizeof(int) * rows},
+                               {kSlotResidue,
+                                stride * sets + sizeof(int) * ((size_t)words + (size_t)pl.nitems)}});
+    if (st != FH_OK) return st;
+    if (prec == Prec::MIXED) {
+        st = reserve(s, {{kSlotScalar, 256}});
+        if (st == FH_OK)
+            st = range_check(s, b_dev, in_f32, naux * nocc * nvir,
+                             std::min(naux, (size_t)kMixedPanel), stream);
+        if (st != FH_OK) return st;
+    }
+    st = upload_eps(s, eps, first_occ, nocc, nocc_total, nvir, stream);
+    if (st != FH_OK) return st;
+    PackArgs pa{};
+    pa.b = b_dev;
+    pa.in_f32 = in_f32;
+    pa.naux = (int)naux;
+    pa.nocc = (int)nocc;
+    pa.nvir = (int)nvir;
+    pa.nvir_pad = pl.nvir_pad;
+    pa.naux_pad = pl.naux_pad;
+    pa.out0 = s.slots[kSlotOp0].ptr;
+    pa.rexp = (int *)s.slots[kSlotScale].ptr;
+    ResidueArgs ra;
+    ra.op = (const int8_t *)pa.out0;
+    ra.rexp = pa.rexp;
+    ra.np = pl.naux_pad / 64;
+    ra.beta = residue_beta(prec, pl.naux_pad);
+    ra.prec = prec;
+    ra.group = pl.group;
+    ra.ngroup = ((int)nocc + pl.group - 1) / pl.group;
+    ra.blocks = blocks;
+    ra.scratch = s.slots[kSlotResidue].ptr;
+    ra.scratch_stride = (int64_t)stride;
+    ra.queue = (int *)((char *)ra.scratch + stride * sets);
+    ResidueOrder ord;
+    ord.nocc = ra.ngroup;
+    ord.ntp = pl.ntp;
+    ord.queue = ra.queue;
+    ord.words = words;
+    ord.order = ra.queue + words;
+    ra.order = ord.order;
+    mark(s, 0, stream);
+    hipError_t he = launch_residue_pack(prec, pa, ord, (double *)s.slots[kSlotStage2].ptr, stream);
+    if (he != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(FH_KERNEL, "pack kernel: %s", hipGetErrorString(he));
+    }
+    ra.nocc = (int)nocc;
+    ra.nvir = (int)nvir;
+    ra.nvir_pad = pl.nvir_pad;
+    ra.ntile = pl.ntile;
+    ra.ntp = pl.ntp;
+    ra.nitems = pl.nitems;
+    ra.eps_occ = (const double *)s.slots[kSlotEps].ptr;
+    ra.eps_vir = ra.eps_occ + nocc;
+    ra.kappa = kappa;
+    ra.item_partials = (double *)s.slots[kSlotItems].ptr;
+    EnergyArgs ea{};  // what the reductions read
+    ea.nocc = ra.nocc;
+    ea.ntp = ra.ntp;
+    ea.item_partials = ra.item_partials;
+    ea.row_partials = (double *)s.slots[kSlotRows].ptr;
+    ea.result = (double *)s.slots[kSlotResult].ptr;
+    mark(s, 1, stream);
+    he = launch_residue_energy(ra, stream);
+    if (he != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(FH_KERNEL, "energy kernel: %s", hipGetErrorString(he));
+    }
+    mark(s, 2, stream);
+    he = launch_energy_reduce(ea, stream);
+    if (he != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(FH_KERNEL, "reduction kernels: %s", hipGetErrorString(he));
+    }
+    mark(s, 3, stream);
+    s.pending.kernel_launches += 5;
+    st = fetch_result(s, ea.result, nocc, stream, out, row_partials);
+    if (st == FH_OK) finish_timing(s, (uint64_t)pl.nitems, pl.tile);
+    return st;
+}
+
+}  // namespace
+
 fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux, size_t nocc,
                       size_t nvir, const double *eps, size_t first_occ, size_t nocc_total,
                       double kappa, Prec prec, hipStream_t stream, fh_spin_components *out,
                       double *row_partials, const EnergyPlan *forced, const void *neg_dev,
-                      size_t naux_neg, double *amp_out) {
+                      size_t naux_neg, double *amp_out, int *ntp_used,
+                      bool as_noalloc) {
     const bool in_f32 = b_dtype == FH_DT_F32;
     EnergyPlan pl = forced ? *forced : plan_energy(nocc, nvir, naux, prec);
     // A signed factor stacks B- after B+ along Q, each segment padded to the
@@ -361,6 +541,27 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
                         pl.naux_pad, kI8MaxNauxPad);
         req.push_back({kSlotScale, sizeof(int) * rows});
     }
+    // Residue arithmetic where it is faster. as_noalloc: the caller's results are
+    // also those of fh_rimp2_energy_dev_noalloc, bit for bit, so a call whose
+    // workspace would fit its array keeps the kernel that runs there.
+    size_t carved = 0;
+    for (const auto &r : req) carved = (carved + 255) / 256 * 256 + r.second;
+    EnergyPlan rpl;
+    if (!signed_k && !amp_out &&
+        !(as_noalloc && carved <= (size_t)FH_NOALLOC_SCRATCH_BYTES) &&
+        plan_residue(s, nocc, nvir, naux, prec, &rpl)) {
+        const uint64_t full = s.stats.fail_pool_full;
+        const fh_status rst =
+            residue_energy(s, b_dev, in_f32, naux, nocc, nvir, eps, first_occ, nocc_total, kappa,
+                           prec, stream, out, row_partials, rpl);
+        if (ntp_used) *ntp_used = rpl.ntp;
+        // Its larger workspace may be past the pool ceiling: then the matrix kernel
+        // below, which needs half the operand (or less) and no scratch.
+        if (rst != FH_POOL_FULL) return rst;
+        s.stats.fail_pool_full = full;
+        clear_error();
+    }
+    if (ntp_used) *ntp_used = pl.ntp;
     fh_status st = reserve(s, req);
     if (st != FH_OK) return st;
 
@@ -376,15 +577,9 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
             if (st != FH_OK) return st;
         }
     }
-    std::vector<double> e(nocc + nvir);
-    for (size_t i = 0; i < nocc; ++i) e[i] = eps[first_occ + i];
-    for (size_t a = 0; a < nvir; ++a) e[nocc + a] = eps[nocc_total + a];
-    double *deps = (double *)s.slots[kSlotEps].ptr;
-    st = hip_check(hipMemcpyAsync(deps, e.data(), sizeof(double) * e.size(),
-                                  hipMemcpyHostToDevice, stream),
-                   "H2D eps");
+    st = upload_eps(s, eps, first_occ, nocc, nocc_total, nvir, stream);
     if (st != FH_OK) return st;
-    s.pending.h2d_bytes += sizeof(double) * e.size();
+    double *deps = (double *)s.slots[kSlotEps].ptr;
 
     PackArgs pa;
     pa.b = b_dev;
@@ -465,21 +660,9 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
     }
     mark(s, 3, stream);
     s.pending.kernel_launches += 4;
-    std::vector<double> res(2 + 2 * nocc);
-    st = hip_check(hipMemcpyAsync(res.data(), ea.result, sizeof(double) * res.size(),
-                                  hipMemcpyDeviceToHost, stream),
-                   "D2H result");
-    if (st != FH_OK) return st;
-    st = hip_check(hipStreamSynchronize(stream), "stream sync");
-    if (st != FH_OK) return st;
-    s.pending.d2h_bytes += sizeof(double) * res.size();
-    finish_timing(s, (uint64_t)pl.nitems, pl.tile);
-    out->e_os = res[0];
-    out->e_ss = res[1];
-    out->e_total = res[0] + res[1];
-    if (row_partials)
-        for (size_t i = 0; i < 2 * nocc; ++i) row_partials[i] = res[2 + i];
-    return FH_OK;
+    st = fetch_result(s, ea.result, nocc, stream, out, row_partials);
+    if (st == FH_OK) finish_timing(s, (uint64_t)pl.nitems, pl.tile);
+    return st;
 }
 
 EnergyPlan plan_energy(size_t nocc, size_t nvir, size_t naux, Prec prec) {
@@ -671,7 +854,8 @@ fh_status fh_rimp2_energy_dev(const void *b_dev, fh_dtype b_dtype, size_t naux, 
     st = ensure_device(s);
     if (st != FH_OK) return st;
     st = energy_core(s, b_dev, b_dtype, naux, nocc, nvir, eps, first_occ, nocc_total, kappa, prec,
-                     (hipStream_t)stream, out, row_partials, nullptr);
+                     (hipStream_t)stream, out, row_partials, nullptr, nullptr, 0, nullptr, nullptr,
+                     true);
     if (st != FH_OK) return st;
     commit(s, prec, false, false);
     return FH_OK;
@@ -718,7 +902,8 @@ fh_status fh_rimp2_energy(const double *b_ov, size_t naux, size_t nocc, size_t n
     if (st != FH_OK) return st;
     s.pending.h2d_bytes += bbytes;
     st = energy_core(s, s.slots[kSlotStage].ptr, FH_DT_F64, naux, nocc, nvir, eps, first_occ,
-                     nocc_total, kappa, prec, stream, out, nullptr, &pl);
+                     nocc_total, kappa, prec, stream, out, nullptr, &pl, nullptr, 0, nullptr, nullptr,
+                     true);
     if (st != FH_OK) return st;
     commit(s, prec, false, false);
     return FH_OK;

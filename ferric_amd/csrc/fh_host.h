@@ -48,6 +48,7 @@ enum SlotId {
     kSlotDensAmp,    // MP2 densities: amplitude blocks of every ordered occupied pair
     kSlotDensPart,   // MP2 densities: split-K partial tiles
     kSlotDensOut,    // MP2 densities: P_vv (padded) then P_oo
+    kSlotResidue,    // FP64 in residue arithmetic: the workgroups' residue planes
     kNumSlots
 };
 
@@ -76,6 +77,7 @@ struct State {
     // Phase timing (FERRIC_TIMING): events on the call's stream.
     int timing = -1;  // -1: not yet read from the environment
     int wall_khz = -1;  // device wall-clock rate (kHz); -1: not yet queried
+    int cus = 0;        // compute units; 0: not yet queried
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     fh_timing last_timing{};
     // Fixed arena (fh_rimp2_energy_dev_noalloc): while set, reserve() carves
@@ -101,6 +103,7 @@ struct EnergyPlan {
     int ntile = 1;
     int ntp = 1;
     int64_t nitems = 0;
+    int group = 1;  // residue arithmetic: occupied orbitals side by side in a tile
 };
 
 State &state();
@@ -135,7 +138,10 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
                       double kappa, Prec prec, hipStream_t stream, fh_spin_components *out,
                       double *row_partials, const EnergyPlan *forced,
                       const void *neg_dev = nullptr, size_t naux_neg = 0,
-                      double *amp_out = nullptr);
+                      double *amp_out = nullptr, int *ntp_used = nullptr,
+                      bool as_noalloc = false);
+// Whether an energy of this shape runs in residue arithmetic, and its plan.
+bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, EnergyPlan *pl);
 void commit(State &s, Prec prec, bool adjoint, bool batched);
 bool to_prec(int p, Prec *out);
 void release_graphs(State &s);

@@ -180,6 +180,42 @@ struct EnergyArgs {
 };
 
 hipError_t launch_energy(const EnergyArgs &a, hipStream_t st);
+
+// The FP64 energy in residue arithmetic on the INT8 matrix cores (residue.hip).
+struct ResidueArgs {
+    Prec prec = Prec::F64;
+    const int8_t *op = nullptr;  // residues of the packed rows
+    const int *rexp = nullptr;   // per packed row, the exponent f: Y = x 2^(beta - 1 - f)
+    int np = 0, beta = 0;        // 64-deep Q panels; bits of Y
+    int nocc = 0, nvir = 0, nvir_pad = 0;
+    int ntile = 0, ntp = 0;      // tiles over the virtuals, tile pairs (tA <= tB)
+    int group = 1, ngroup = 0;   // occupied orbitals side by side in a tile; groups of them
+    int64_t nitems = 0;          // group pairs x ntp
+    const double *eps_occ = nullptr, *eps_vir = nullptr;
+    double kappa = 0.0;          // NaN = none
+    double *item_partials = nullptr;  // per occupied pair and tile pair
+    int blocks = 0;              // workgroups, one per CU (a multiple of kXcds)
+    void *scratch = nullptr;     // residue_scratch_sets(blocks) x scratch_stride bytes
+    int64_t scratch_stride = 0;
+    int *queue = nullptr;        // round counter and, per workgroup, parts done: zeroed by the packer
+    const int *order = nullptr;  // the items in the order they are taken
+};
+struct ResidueOrder {
+    int nocc = 0, ntp = 0;   // orbital groups, tile pairs
+    int words = 0;           // of the queue
+    int *queue = nullptr, *order = nullptr;
+};
+int residue_moduli(Prec prec);
+int residue_beta(Prec prec, int naux_pad);
+// Plane sets of a launch: one per workgroup, and one per item of a split round (two
+// or more workgroups to each).
+int residue_scratch_sets(int blocks);
+int residue_queue_words(int blocks);
+size_t residue_scratch_stride(Prec prec, int products);
+// pmax: (naux_pad / 64) x nocc nvir doubles of scratch.
+hipError_t launch_residue_pack(Prec prec, const PackArgs &a, const ResidueOrder &ord, double *pmax,
+                               hipStream_t st);
+hipError_t launch_residue_energy(const ResidueArgs &a, hipStream_t st);
 // Phase A of the adjoint: the pair kernel with the T~ / dE/deps epilogue.
 hipError_t launch_adjoint_pairs(const EnergyArgs &a, hipStream_t st);
 

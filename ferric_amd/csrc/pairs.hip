@@ -72,12 +72,13 @@ fh_status pair_energies_core(State &s, const void *b_dev, fh_dtype b_dtype, size
     fh_status st = reserve(s, {{kSlotPairs, sizeof(double) * 2 * npairs}});
     if (st != FH_OK) return st;
     fh_spin_components tot;
+    int ntp = pl.ntp;
     st = energy_core(s, b_dev, b_dtype, naux, nocc, nvir, eps, first_occ, nocc_total, NAN, prec,
-                     stream, &tot, nullptr, &pl);
+                     stream, &tot, nullptr, &pl, nullptr, 0, nullptr, &ntp);
     if (st != FH_OK) return st;
     double *dev = (double *)s.slots[kSlotPairs].ptr;
     hipLaunchKernelGGL(reduce_pairs_kernel, dim3((unsigned)npairs), dim3(256), 0, stream,
-                       (const double *)s.slots[kSlotItems].ptr, pl.ntp, dev);
+                       (const double *)s.slots[kSlotItems].ptr, ntp, dev);
     st = hip_check(hipGetLastError(), "pair reduction");
     if (st != FH_OK) return st;
     std::vector<double> h(2 * npairs);
