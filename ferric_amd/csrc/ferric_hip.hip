@@ -310,6 +310,56 @@ int i8_q_rot_ticks(State &s, int npanels, int ntp) {
     return (int)std::lround(s.wall_khz * 1.4e-3);
 }
 
+bool residue_tiles(State &s, size_t nvir, size_t naux, EnergyPlan *pl) {
+    // 4608: the most the int32 sums and byte remainders allow (residue.h).
+    if (s.arena || forced_tile() > 0 || naux > 4608) return false;
+    if (s.cus <= 0 &&
+        hipDeviceGetAttribute(&s.cus, hipDeviceAttributeMultiprocessorCount, s.device) !=
+            hipSuccess)
+        s.cus = 0;
+    if (s.cus < 8) return false;  // whole rounds over the eight XCDs
+    EnergyPlan p;
+    p.tile = 256;
+    p.nvir_pad = (int)((nvir + 15) / 16 * 16);
+    p.naux_pad = (int)((naux + 63) / 64 * 64);
+    p.ntile = (p.nvir_pad + p.tile - 1) / p.tile;
+    p.ntp = p.ntile * (p.ntile + 1) / 2;
+    *pl = p;
+    return true;
+}
+
+fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, size_t rows,
+                          int naux_pad, std::vector<std::pair<int, size_t>> more,
+                          ResidueSpace *out) {
+    const int blocks = s.cus / 8 * 8;
+    const int words = residue_queue_words(blocks);
+    const size_t stride = residue_scratch_stride(prec, products);
+    const size_t planes = stride * (size_t)residue_scratch_sets(blocks);
+    more.push_back({kSlotOp0, rows * (size_t)naux_pad * residue_moduli(prec)});
+    more.push_back({kSlotScale, sizeof(int) * rows});
+    more.push_back({kSlotResidue, planes + sizeof(int) * ((size_t)words + (size_t)nitems)});
+    const fh_status st = reserve(s, more);
+    if (st != FH_OK) return st;
+    out->op = (int8_t *)s.slots[kSlotOp0].ptr;
+    out->rexp = (int *)s.slots[kSlotScale].ptr;
+    ResidueArgs &ra = out->args;
+    ra.prec = prec;
+    ra.op = out->op;
+    ra.rexp = out->rexp;
+    ra.np = naux_pad / 64;
+    ra.beta = residue_beta(prec, naux_pad);
+    ra.nitems = nitems;
+    ra.blocks = blocks;
+    ra.scratch = s.slots[kSlotResidue].ptr;
+    ra.scratch_stride = (int64_t)stride;
+    ra.queue = (int *)((char *)ra.scratch + planes);
+    ra.order = ra.queue + words;
+    out->order.words = words;
+    out->order.queue = ra.queue;
+    out->order.order = ra.queue + words;
+    return FH_OK;
+}
+
 // Which calls run in residue arithmetic (residue.hip), and on what tiles. Measured
 // against the matrix kernel of the same precision (its time / residue time):
 // FP64    past 144 virtuals (one orbital a tile): 24/208/742 1.7, 70/208/889 2.1,
@@ -322,13 +372,8 @@ int i8_q_rot_ticks(State &s, int npanels, int ntp) {
 // INT8X4 stays with its digit slices: ten moduli against their thirteen products gave
 //         70/208/889 1.2, but 70/340/1312 0.95 and 100/900/3600 0.98.
 bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, EnergyPlan *pl) {
-    if (s.arena || forced_tile() > 0 || naux > 4608) return false;
     EnergyPlan p;
-    p.tile = 256;
-    p.nvir_pad = (int)((nvir + 15) / 16 * 16);
-    p.naux_pad = (int)((naux + 63) / 64 * 64);
-    p.ntile = (p.nvir_pad + p.tile - 1) / p.tile;
-    p.ntp = p.ntile * (p.ntile + 1) / 2;
+    if (!residue_tiles(s, nvir, naux, &p)) return false;
     p.group = nvir <= 128 ? 2 : 1;
     const double work = (double)nocc * (nocc + 1) * (double)nvir * nvir * (double)naux;
     if (nvir <= 64) return false;
@@ -344,18 +389,10 @@ bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, En
     const int64_t ngroup = ((int64_t)nocc + p.group - 1) / p.group;
     p.nitems = ngroup * (ngroup + 1) / 2 * p.ntp;
     if (p.nitems > 0x7fffff00LL) return false;
-    if (s.cus <= 0 &&
-        hipDeviceGetAttribute(&s.cus, hipDeviceAttributeMultiprocessorCount, s.device) !=
-            hipSuccess)
-        s.cus = 0;
-    if (s.cus < 8) return false;
     *pl = p;
     return true;
 }
 
-namespace {
-
-// Copies the device result (energies, then the row values) back.
 fh_status fetch_result(State &s, const double *dev, size_t nocc, hipStream_t stream,
                        fh_spin_components *out, double *row_partials) {
     std::vector<double> res(2 + 2 * nocc);
@@ -373,6 +410,8 @@ fh_status fetch_result(State &s, const double *dev, size_t nocc, hipStream_t str
         for (size_t i = 0; i < 2 * nocc; ++i) row_partials[i] = res[2 + i];
     return FH_OK;
 }
+
+namespace {
 
 // Uploads [eps_occ, eps_vir] of the active orbitals.
 fh_status upload_eps(State &s, const double *eps, size_t first_occ, size_t nocc, size_t nocc_total,
@@ -392,21 +431,16 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
                          size_t nvir, const double *eps, size_t first_occ, size_t nocc_total,
                          double kappa, Prec prec, hipStream_t stream, fh_spin_components *out,
                          double *row_partials, const EnergyPlan &pl) {
-    const size_t rows = nocc * (size_t)pl.nvir_pad;
     const size_t npairs = nocc * (nocc + 1) / 2;
-    const int blocks = s.cus / 8 * 8;  // whole rounds over the eight XCDs
-    const int words = residue_queue_words(blocks);
-    const size_t sets = (size_t)residue_scratch_sets(blocks);
-    const size_t stride = residue_scratch_stride(prec, pl.ntile > 1 ? 2 : 1);
-    fh_status st = reserve(s, {{kSlotOp0, rows * (size_t)pl.naux_pad * residue_moduli(prec)},
-                               {kSlotStage2, sizeof(double) * (size_t)(pl.naux_pad / 64) * nocc * nvir},
-                               {kSlotEps, sizeof(double) * (nocc + nvir)},
-                               {kSlotItems, sizeof(double) * 4 * npairs * (size_t)pl.ntp},
-                               {kSlotRows, sizeof(double) * 4 * nocc},
-                               {kSlotResult, sizeof(double) * (2 + 2 * nocc)},
-                               {kSlotScale, sizeof(int) * rows},
-                               {kSlotResidue,
-                                stride * sets + sizeof(int) * ((size_t)words + (size_t)pl.nitems)}});
+    ResidueSpace sp;
+    fh_status st = reserve_residue(
+        s, prec, pl.nitems, pl.ntile > 1 ? 2 : 1, nocc * (size_t)pl.nvir_pad, pl.naux_pad,
+        {{kSlotStage2, sizeof(double) * (size_t)(pl.naux_pad / 64) * nocc * nvir},
+         {kSlotEps, sizeof(double) * (nocc + nvir)},
+         {kSlotItems, sizeof(double) * 4 * npairs * (size_t)pl.ntp},
+         {kSlotRows, sizeof(double) * 4 * nocc},
+         {kSlotResult, sizeof(double) * (2 + 2 * nocc)}},
+        &sp);
     if (st != FH_OK) return st;
     if (prec == Prec::MIXED) {
         st = reserve(s, {{kSlotScalar, 256}});
@@ -425,27 +459,14 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     pa.nvir = (int)nvir;
     pa.nvir_pad = pl.nvir_pad;
     pa.naux_pad = pl.naux_pad;
-    pa.out0 = s.slots[kSlotOp0].ptr;
-    pa.rexp = (int *)s.slots[kSlotScale].ptr;
-    ResidueArgs ra;
-    ra.op = (const int8_t *)pa.out0;
-    ra.rexp = pa.rexp;
-    ra.np = pl.naux_pad / 64;
-    ra.beta = residue_beta(prec, pl.naux_pad);
-    ra.prec = prec;
+    pa.out0 = sp.op;
+    pa.rexp = sp.rexp;
+    ResidueArgs ra = sp.args;
     ra.group = pl.group;
     ra.ngroup = ((int)nocc + pl.group - 1) / pl.group;
-    ra.blocks = blocks;
-    ra.scratch = s.slots[kSlotResidue].ptr;
-    ra.scratch_stride = (int64_t)stride;
-    ra.queue = (int *)((char *)ra.scratch + stride * sets);
-    ResidueOrder ord;
+    ResidueOrder ord = sp.order;
     ord.nocc = ra.ngroup;
     ord.ntp = pl.ntp;
-    ord.queue = ra.queue;
-    ord.words = words;
-    ord.order = ra.queue + words;
-    ra.order = ord.order;
     mark(s, 0, stream);
     hipError_t he = launch_residue_pack(prec, pa, ord, (double *)s.slots[kSlotStage2].ptr, stream);
     if (he != hipSuccess) {
@@ -457,7 +478,6 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     ra.nvir_pad = pl.nvir_pad;
     ra.ntile = pl.ntile;
     ra.ntp = pl.ntp;
-    ra.nitems = pl.nitems;
     ra.eps_occ = (const double *)s.slots[kSlotEps].ptr;
     ra.eps_vir = ra.eps_occ + nocc;
     ra.kappa = kappa;

@@ -140,7 +140,22 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
                       const void *neg_dev = nullptr, size_t naux_neg = 0,
                       double *amp_out = nullptr, int *ntp_used = nullptr,
                       bool as_noalloc = false);
-// Whether an energy of this shape runs in residue arithmetic, and its plan.
+// Residue arithmetic (residue.hip). Tile sides and paddings of a shape, where it may
+// run at all (aux count, forced tiles, fixed arena); whether an energy of this
+// shape is faster so, and its plan; and the workspace of a launch.
+bool residue_tiles(State &s, size_t nvir, size_t naux, EnergyPlan *pl);
+struct ResidueSpace {
+    ResidueArgs args;    // prec, np, beta, op, rexp, nitems, blocks, scratch, queue, order
+    ResidueOrder order;  // words, queue, order
+    int8_t *op = nullptr;
+    int *rexp = nullptr;
+};
+fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, size_t rows,
+                          int naux_pad, std::vector<std::pair<int, size_t>> more,
+                          ResidueSpace *out);
+// Copies the device result (energies, then nocc rows' values) back and waits for it.
+fh_status fetch_result(State &s, const double *dev, size_t nocc, hipStream_t stream,
+                       fh_spin_components *out, double *row_partials);
 bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, EnergyPlan *pl);
 void commit(State &s, Prec prec, bool adjoint, bool batched);
 bool to_prec(int p, Prec *out);

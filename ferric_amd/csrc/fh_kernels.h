@@ -193,6 +193,10 @@ struct ResidueArgs {
     int64_t nitems = 0;          // group pairs x ntp
     const double *eps_occ = nullptr, *eps_vir = nullptr;
     double kappa = 0.0;          // NaN = none
+    // Opposite spin (nocc_b > 0): the beta side; its rows follow the alpha rows in op.
+    int nocc_b = 0, nvir_b = 0, nvir_pad_b = 0, ntile_b = 0;
+    const int *rexp_b = nullptr;
+    const double *eps_occ_b = nullptr, *eps_vir_b = nullptr;
     double *item_partials = nullptr;  // per occupied pair and tile pair
     int blocks = 0;              // workgroups, one per CU (a multiple of kXcds)
     void *scratch = nullptr;     // residue_scratch_sets(blocks) x scratch_stride bytes
@@ -202,6 +206,7 @@ struct ResidueArgs {
 };
 struct ResidueOrder {
     int nocc = 0, ntp = 0;   // orbital groups, tile pairs
+    int nocc_b = 0;          // > 0: every (i, J) instead of i <= j
     int words = 0;           // of the queue
     int *queue = nullptr, *order = nullptr;
 };
@@ -212,9 +217,10 @@ int residue_beta(Prec prec, int naux_pad);
 int residue_scratch_sets(int blocks);
 int residue_queue_words(int blocks);
 size_t residue_scratch_stride(Prec prec, int products);
-// pmax: (naux_pad / 64) x nocc nvir doubles of scratch.
+// pmax: (naux_pad / 64) x nocc nvir doubles of scratch. The rows go to row groups rg0
+// on, of nrg in all (0: only these). ord.order null: no order to be made.
 hipError_t launch_residue_pack(Prec prec, const PackArgs &a, const ResidueOrder &ord, double *pmax,
-                               hipStream_t st);
+                               hipStream_t st, int64_t nrg = 0, int64_t rg0 = 0);
 hipError_t launch_residue_energy(const ResidueArgs &a, hipStream_t st);
 // Phase A of the adjoint: the pair kernel with the T~ / dE/deps epilogue.
 hipError_t launch_adjoint_pairs(const EnergyArgs &a, hipStream_t st);

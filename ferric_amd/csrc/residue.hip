@@ -98,20 +98,29 @@ __global__ __launch_bounds__(256) void residue_colmax_kernel(const Tin *__restri
 // of 64, and all items of a round take the same time. order[position] = pair ntp + t.
 __device__ void order_items(const ResidueOrder &o) {
     constexpr int BI = 4, BJ = 8;
-    const int64_t n = o.nocc, npairs = n * (n + 1) / 2;
+    const int64_t n = o.nocc, npairs = o.nocc_b ? n * o.nocc_b : n * (n + 1) / 2;
     if (blockIdx.x == 0)
         for (int t = threadIdx.x; t < o.words; t += blockDim.x) o.queue[t] = 0;
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < npairs;
          p += (int64_t)gridDim.x * blockDim.x) {
         int i, j;
-        decode_pair(p, o.nocc, i, j);
-        const int i0 = i / BI * BI, i1 = min(i0 + BI, o.nocc);
-        const int j0 = j / BJ * BJ;
-        int64_t rank = i0 * n - (int64_t)i0 * (i0 - 1) / 2;  // pairs of the rows above
-        for (int r = i0; r < i1; ++r) {
-            rank += max(0, j0 - r);  // this band's pairs in the blocks to the left
-            if (r < i) rank += max(0, min(j0 + BJ, o.nocc) - max(j0, r));
-            if (r == i) rank += j - max(j0, r);
+        int64_t rank;
+        if (o.nocc_b) {  // opposite spin: every (i, J)
+            i = (int)(p / o.nocc_b);
+            j = (int)(p % o.nocc_b);
+            const int i0 = i / BI * BI, i1 = min(i0 + BI, o.nocc), j0 = j / BJ * BJ;
+            rank = (int64_t)i0 * o.nocc_b + (int64_t)(i1 - i0) * j0 +
+                   (i - i0) * min(BJ, o.nocc_b - j0) + j - j0;
+        } else {
+            decode_pair(p, o.nocc, i, j);
+            const int i0 = i / BI * BI, i1 = min(i0 + BI, o.nocc);
+            const int j0 = j / BJ * BJ;
+            rank = i0 * n - (int64_t)i0 * (i0 - 1) / 2;  // pairs of the rows above
+            for (int r = i0; r < i1; ++r) {
+                rank += max(0, j0 - r);  // this band's pairs in the blocks to the left
+                if (r < i) rank += max(0, min(j0 + BJ, o.nocc) - max(j0, r));
+                if (r == i) rank += j - max(j0, r);
+            }
         }
         int x = 0;
         while (x + 1 < kXcds && npairs * (x + 1) / kXcds <= rank) ++x;
@@ -123,11 +132,12 @@ __device__ void order_items(const ResidueOrder &o) {
 
 // One 64 x 64 tile (64 packed rows, one Q panel) to residues. The exponent f of a row
 // is that of the INT8X4 format: the least with max |x| <= (1 - 2^-7) 2^(f + 1); Y =
-// RN(x 2^(beta - 1 - f)). ROUND32: x is first rounded to FP32 (MIXED).
+// RN(x 2^(beta - 1 - f)). The rows go to row groups rg0 on, of nrg in all. ROUND32: x is first rounded to FP32 (MIXED).
 template <int N, bool ROUND32, typename Tin>
 __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict__ b, int64_t nov,
                                                            int naux, int nvir, int nvir_pad,
                                                            int64_t nrows, int np, int beta,
+                                                           int64_t nrg, int64_t rg0,
                                                            const double *__restrict__ pmax,
                                                            int *__restrict__ rexp,
                                                            int8_t *__restrict__ out,
@@ -136,7 +146,7 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
     __shared__ double part[4][64];
     __shared__ int exps[64];
     if ((int)blockIdx.y == np) {  // one more row of blocks: the item order and the queue words
-        order_items(ord);
+        if (ord.order) order_items(ord);
         return;
     }
     const int tx = threadIdx.x % 64, ty = threadIdx.x / 64;
@@ -212,8 +222,7 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
             w[k][q / 4] |= (x & 0xffu) << (8 * (q % 4));
         }
     }
-    const int64_t nrg = nrows / 16;
-    int8_t *o = out + ((int64_t)blockIdx.y * nrg + orow / 16) * 1024 + (t % 64) * 16;
+    int8_t *o = out + ((int64_t)blockIdx.y * nrg + rg0 + orow / 16) * 1024 + (t % 64) * 16;
 #pragma unroll
     for (int k = 0; k < N; ++k)
         *(uint4 *)(o + (int64_t)k * np * nrg * 1024) =
@@ -533,7 +542,55 @@ __device__ __forceinline__ void pair_energy(const ResidueArgs &a, const PairTile
     }
 }
 
+// Opposite spin: (ia|JB)^2 / D over one (i, J) and tile pair, weight 1.
 template <int N>
+__device__ __forceinline__ void rect_energy(const ResidueArgs &a, const PairTile &T,
+                                            const char *c1, char *lds, KSum &os) {
+    const int lane = threadIdx.x % kWave;
+    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int g = lane / 16, r = lane % 16;
+    const int nblk = T.nA * T.nB;
+    const double eij = a.eps_occ[T.i] + a.eps_occ_b[T.j];
+    PairTables &tab = *(PairTables *)(lds + kStage);  // as pair_energy
+    {
+        const int h = threadIdx.x / 256, c = threadIdx.x % 256;
+        const int v = 16 * (h ? T.b0 : T.a0) + c;
+        if (c < 16 * (h ? T.nB : T.nA)) {
+            tab.eps[h][c] = h ? (v < a.nvir_b ? a.eps_vir_b[v] : 0.0)
+                              : (v < a.nvir ? a.eps_vir[v] : 0.0);
+            tab.exp_i[h][c] = h ? a.rexp_b[(int64_t)T.j * a.nvir_pad_b + v]
+                                : a.rexp[(int64_t)T.i * a.nvir_pad + v];
+        }
+    }
+    __syncthreads();
+    const int esh = -2 * (a.beta - 1);
+    uint32_t n1[N];
+    if (wid < nblk) load_residues<N>(c1, wid / T.nB, wid % T.nB, lane, n1);
+#pragma unroll 1
+    for (int t = wid; t < nblk; t += 8) {
+        const int la = t / T.nB * 16, lb = t % T.nB * 16;
+        uint32_t d1[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) d1[k] = n1[k];
+        if (t + 8 < nblk) load_residues<N>(c1, (t + 8) / T.nB, (t + 8) % T.nB, lane, n1);
+        double g1[4];
+        res::crt4<N>(d1, g1);
+        const int xb = tab.exp_i[1][lb + r] + esh;
+        const bool okb = T.b0 * 16 + lb + r < a.nvir_b;
+        const double eb = tab.eps[1][lb + r];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const double x = res::scale_frac<N>(g1[v], tab.exp_i[0][la + 4 * g + v] + xb);
+            const bool ok = okb && T.a0 * 16 + la + 4 * g + v < a.nvir;
+            const double to = (x * x) / (eij - tab.eps[0][la + 4 * g + v] - eb);
+            os.add(ok ? to : 0.0);
+        }
+    }
+}
+
+// RECT: opposite spin, items (i, J, tA, tB) over every alpha i, beta J and tile of
+// each side, one product each; the beta rows follow the alpha rows in the operand.
+template <int N, bool RECT>
 __global__ __launch_bounds__(kThreads) void residue_energy_kernel(ResidueArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     __shared__ int turn;
@@ -584,15 +641,23 @@ __global__ __launch_bounds__(kThreads) void residue_energy_kernel(ResidueArgs a)
         const int id = a.order[lo + at];
         // Orbital groups I <= J (one orbital each unless several fit a tile).
         int I, J, ta, tb;
-        decode_pair(id / a.ntp, a.ngroup, I, J);
-        decode_tile_pair(id % a.ntp, a.ntile, ta, tb);
+        if (RECT) {
+            I = id / a.ntp / a.nocc_b;
+            J = id / a.ntp % a.nocc_b;
+            ta = id % a.ntp / a.ntile_b;
+            tb = id % a.ntp % a.ntile_b;
+        } else {
+            decode_pair(id / a.ntp, a.ngroup, I, J);
+            decode_tile_pair(id % a.ntp, a.ntile, ta, tb);
+        }
+        const int ngb = RECT ? a.nvir_pad_b / 16 : ng, ntb = RECT ? a.ntile_b : a.ntile;
         const int i0 = I * a.group, j0 = J * a.group;
-        const int ni = min(a.group, a.nocc - i0), nj = min(a.group, a.nocc - j0);
+        const int ni = min(a.group, a.nocc - i0), nj = RECT ? 1 : min(a.group, a.nocc - j0);
         const int a0 = ta * ng / a.ntile, wA = (ta + 1) * ng / a.ntile - a0;
-        const int b0 = tb * ng / a.ntile, wB = (tb + 1) * ng / a.ntile - b0;
+        const int b0 = tb * ngb / ntb, wB = (tb + 1) * ngb / ntb - b0;
         Product P;
         P.op = a.op;
-        P.step = (int64_t)a.nocc * ng * 1024;
+        P.step = ((int64_t)a.nocc * ng + (RECT ? (int64_t)a.nocc_b * ngb : 0)) * 1024;
         P.nA = ni * wA;
         P.nB = nj * wB;
         P.np = a.np;
@@ -602,11 +667,11 @@ __global__ __launch_bounds__(kThreads) void residue_energy_kernel(ResidueArgs a)
         P.nx = (wr ? P.nA : (P.nA + 1) / 2) - P.x0;
         P.y0 = wc * P.nB / 4;
         P.ny = (wc + 1) * P.nB / 4 - P.y0;
-        const int nprod = ta == tb || I == J ? 1 : 2;
+        const int nprod = RECT || ta == tb || I == J ? 1 : 2;
 #pragma unroll 1
         for (int c = 0; c < nprod; ++c) {
             P.rgA = (c ? j0 : i0) * ng + a0;
-            P.rgB = (c ? i0 : j0) * ng + b0;
+            P.rgB = RECT ? a.nocc * ng + j0 * ngb + b0 : (c ? i0 : j0) * ng + b0;
             P.planes = raw_rsrc(scr + (int64_t)c * planes_of(N), planes_of(N));
             if (P.ny > 3)
                 run_rows<N, 4>(P, lds);
@@ -628,6 +693,13 @@ __global__ __launch_bounds__(kThreads) void residue_energy_kernel(ResidueArgs a)
             if (turn != split - 1) return;  // split rounds are last rounds
         }
         __syncthreads();  // every wave's residues are in the scratch
+        if constexpr (RECT) {
+            const PairTile T{I, J, a0, b0, wA, wB, 0, 0, false};
+            KSum os;
+            rect_energy<N>(a, T, scr, lds, os);
+            pair::block_store(os, KSum{}, 1.0, a.item_partials + 4 * (int64_t)id);
+            continue;
+        }
         for (int u = 0; u < ni; ++u)
             for (int v = 0; v < nj; ++v) {
                 PairTile T;
@@ -653,7 +725,7 @@ __global__ __launch_bounds__(kThreads) void residue_energy_kernel(ResidueArgs a)
 
 template <int N, bool ROUND32>  // MIXED: ROUND32
 hipError_t launch_pack_n(const PackArgs &a, const ResidueOrder &ord, double *pmax, int beta,
-                         hipStream_t st) {
+                         int64_t nrg, int64_t rg0, hipStream_t st) {
     const int64_t nrows = (int64_t)a.nocc * a.nvir_pad, nov = (int64_t)a.nocc * a.nvir;
     const int np = a.naux_pad / 64;
     const dim3 mg((unsigned)((nov + 255) / 256), (unsigned)((a.naux + 63) / 64));
@@ -663,13 +735,13 @@ hipError_t launch_pack_n(const PackArgs &a, const ResidueOrder &ord, double *pma
                            nov, a.naux, pmax);
         hipLaunchKernelGGL((residue_pack_kernel<N, ROUND32, float>), grid, dim3(256), 0, st,
                            (const float *)a.b, nov, a.naux, a.nvir, a.nvir_pad, nrows, np, beta,
-                           (const double *)pmax, a.rexp, (int8_t *)a.out0, ord);
+                           nrg, rg0, (const double *)pmax, a.rexp, (int8_t *)a.out0, ord);
     } else {
         hipLaunchKernelGGL(residue_colmax_kernel<double>, mg, dim3(256), 0, st,
                            (const double *)a.b, nov, a.naux, pmax);
         hipLaunchKernelGGL((residue_pack_kernel<N, ROUND32, double>), grid, dim3(256), 0, st,
                            (const double *)a.b, nov, a.naux, a.nvir, a.nvir_pad, nrows, np, beta,
-                           (const double *)pmax, a.rexp, (int8_t *)a.out0, ord);
+                           nrg, rg0, (const double *)pmax, a.rexp, (int8_t *)a.out0, ord);
     }
     return hipGetLastError();
 }
@@ -691,35 +763,46 @@ size_t residue_scratch_stride(Prec prec, int products) {
 }
 
 hipError_t launch_residue_pack(Prec prec, const PackArgs &a, const ResidueOrder &ord, double *pmax,
-                               hipStream_t st) {
+                               hipStream_t st, int64_t nrg, int64_t rg0) {
+    const int64_t own = (int64_t)a.nocc * a.nvir_pad / 16;
+    if (nrg == 0) nrg = own;
+    if (rg0 < 0 || rg0 + own > nrg) return hipErrorInvalidValue;
     if (!a.rexp || !pmax || a.naux_pad % 64 != 0 || a.naux_pad < a.naux ||
         a.naux_pad - a.naux >= 64 || a.naux_pad > res::kMaxNauxPad || a.nvir_pad % 16 != 0)
         return hipErrorInvalidValue;
     const int beta = residue_beta(prec, a.naux_pad);
     switch (prec) {
-    case Prec::F64: return launch_pack_n<16, false>(a, ord, pmax, beta, st);
-    case Prec::MIXED: return launch_pack_n<10, true>(a, ord, pmax, beta, st);
+    case Prec::F64: return launch_pack_n<16, false>(a, ord, pmax, beta, nrg, rg0, st);
+    case Prec::MIXED: return launch_pack_n<10, true>(a, ord, pmax, beta, nrg, rg0, st);
     default: return hipErrorInvalidValue;
     }
 }
 
 hipError_t launch_residue_energy(const ResidueArgs &a, hipStream_t st) {
     const int ng = a.nvir_pad / 16;
+    const bool rect = a.nocc_b > 0;
     const int64_t groups = (a.nocc + a.group - 1) / a.group;
-    if (!a.op || !a.rexp || !a.scratch || !a.queue || !a.order || a.blocks <= 0 || a.nitems <= 0 ||
-        a.nitems > 0x7fffff00LL || a.np <= 0 || a.np * 64 > res::kMaxNauxPad ||
-        a.nvir_pad % 16 != 0 || a.group <= 0 || a.ngroup != groups ||
-        (a.group > 1 && (a.ntile != 1 || a.group * ng > kTB)) || a.ntile * kTB < ng ||
-        a.ntp != a.ntile * (a.ntile + 1) / 2 || a.nitems != groups * (groups + 1) / 2 * a.ntp ||
-        a.blocks % kXcds != 0 ||
-        a.scratch_stride < (int64_t)residue_scratch_stride(a.prec, a.ntile > 1 ? 2 : 1))
+    if (!a.op || !a.rexp || !a.scratch || !a.queue || !a.order || a.blocks <= 0 ||
+        a.blocks % kXcds != 0 || a.nitems <= 0 || a.nitems > 0x7fffff00LL || a.np <= 0 ||
+        a.np * 64 > res::kMaxNauxPad || a.nvir_pad % 16 != 0 || a.ntile * kTB < ng)
         return hipErrorInvalidValue;
-    if (residue_moduli(a.prec) == 16)
-        hipLaunchKernelGGL(residue_energy_kernel<16>, dim3((unsigned)a.blocks), dim3(kThreads),
-                           kBuf * kStage, st, a);
-    else
-        hipLaunchKernelGGL(residue_energy_kernel<10>, dim3((unsigned)a.blocks), dim3(kThreads),
-                           kBuf * kStage, st, a);
+    if (rect) {
+        if (a.prec != Prec::F64 || !a.rexp_b || a.nvir_pad_b % 16 != 0 || a.group != 1 ||
+            a.ntile_b * kTB < a.nvir_pad_b / 16 || a.ntp != a.ntile * a.ntile_b ||
+            a.nitems != (int64_t)a.nocc * a.nocc_b * a.ntp ||
+            a.scratch_stride < (int64_t)residue_scratch_stride(a.prec, 1))
+            return hipErrorInvalidValue;
+    } else if (a.group <= 0 || a.ngroup != groups ||
+               (a.group > 1 && (a.ntile != 1 || a.group * ng > kTB)) ||
+               a.ntp != a.ntile * (a.ntile + 1) / 2 ||
+               a.nitems != groups * (groups + 1) / 2 * a.ntp ||
+               a.scratch_stride < (int64_t)residue_scratch_stride(a.prec, a.ntile > 1 ? 2 : 1)) {
+        return hipErrorInvalidValue;
+    }
+    const auto kern = rect                             ? residue_energy_kernel<16, true>
+                      : residue_moduli(a.prec) == 16 ? residue_energy_kernel<16, false>
+                                                     : residue_energy_kernel<10, false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)a.blocks), dim3(kThreads), kBuf * kStage, st, a);
     return hipGetLastError();
 }
 

@@ -37,10 +37,147 @@ fh_status check_channel(const fh_spin_channel *ch, size_t naux, bool *empty) {
     return FH_OK;
 }
 
+// The FP64 opposite-spin block in residue arithmetic (residue.hip): alpha and beta
+// rows behind one another in one operand. *taken is false where the matrix kernel
+// is used instead. Sizes as for the closed shell (plan_residue): all three blocks of
+// 21/229, 20/230 over 960 aux 1.92 -> 1.43 ms; under 144 virtuals a side's tiles stay
+// half empty (one orbital a tile here).
+fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_channel &cb,
+                           const void *ba, const void *bb, bool in_f32, size_t naux,
+                           hipStream_t stream, double *energy, bool *taken) {
+    *taken = false;
+    const double work =
+        2.0 * ca.nocc * cb.nocc * (double)ca.nvir * (double)cb.nvir * (double)naux;
+    if (std::min(ca.nvir, cb.nvir) < 144 || work < (ca.nocc * cb.nocc >= 64 ? 2.5e9 : 8e9))
+        return FH_OK;
+    EnergyPlan pa, pb;
+    if (!residue_tiles(s, ca.nvir, naux, &pa) || !residue_tiles(s, cb.nvir, naux, &pb))
+        return FH_OK;
+    const int64_t npairs = (int64_t)ca.nocc * (int64_t)cb.nocc;
+    const int ntp = pa.ntile * pb.ntile;
+    if (npairs * ntp > 0x7fffff00LL) return FH_OK;
+    const size_t rows_a = ca.nocc * (size_t)pa.nvir_pad, rows_b = cb.nocc * (size_t)pb.nvir_pad;
+    const size_t neps = ca.nocc + ca.nvir + cb.nocc + cb.nvir;
+    const int np = pa.naux_pad / 64;
+    const size_t col_a = ca.nocc * ca.nvir, col_b = cb.nocc * cb.nvir;
+    const uint64_t full = s.stats.fail_pool_full;
+    ResidueSpace sp;
+    fh_status st = reserve_residue(
+        s, Prec::F64, npairs * ntp, 1, rows_a + rows_b, pa.naux_pad,
+        {{kSlotStage2, sizeof(double) * (size_t)np * (col_a + col_b)},
+         {kSlotEps, sizeof(double) * neps},
+         {kSlotItems, sizeof(double) * 4 * (size_t)(npairs * ntp)},
+         {kSlotRows, sizeof(double) * 4 * ca.nocc},
+         {kSlotResult, sizeof(double) * (2 + 2 * ca.nocc)}},
+        &sp);
+    if (st == FH_POOL_FULL) {  // the matrix kernel needs half of it
+        s.stats.fail_pool_full = full;
+        clear_error();
+        return FH_OK;
+    }
+    *taken = true;
+    if (st != FH_OK) return st;
+    std::vector<double> e;
+    e.reserve(neps);
+    for (size_t i = 0; i < ca.nocc; ++i) e.push_back(ca.eps[ca.first_occ + i]);
+    for (size_t a = 0; a < ca.nvir; ++a) e.push_back(ca.eps[ca.nocc_total + a]);
+    for (size_t i = 0; i < cb.nocc; ++i) e.push_back(cb.eps[cb.first_occ + i]);
+    for (size_t a = 0; a < cb.nvir; ++a) e.push_back(cb.eps[cb.nocc_total + a]);
+    double *deps = (double *)s.slots[kSlotEps].ptr;
+    st = hip_check(hipMemcpyAsync(deps, e.data(), sizeof(double) * e.size(),
+                                  hipMemcpyHostToDevice, stream),
+                   "H2D eps");
+    if (st != FH_OK) return st;
+    s.pending.h2d_bytes += sizeof(double) * e.size();
+    ResidueArgs ra = sp.args;
+    ra.nocc = (int)ca.nocc;
+    ra.nvir = (int)ca.nvir;
+    ra.nvir_pad = pa.nvir_pad;
+    ra.ntile = pa.ntile;
+    ra.nocc_b = (int)cb.nocc;
+    ra.nvir_b = (int)cb.nvir;
+    ra.nvir_pad_b = pb.nvir_pad;
+    ra.ntile_b = pb.ntile;
+    ra.ntp = ntp;
+    ra.ngroup = ra.nocc;
+    ra.rexp_b = ra.rexp + rows_a;
+    ra.eps_occ = deps;
+    ra.eps_vir = deps + ca.nocc;
+    ra.eps_occ_b = ra.eps_vir + ca.nvir;
+    ra.eps_vir_b = ra.eps_occ_b + cb.nocc;
+    ra.kappa = NAN;
+    ra.item_partials = (double *)s.slots[kSlotItems].ptr;
+    ResidueOrder ord = sp.order;
+    ord.nocc = ra.nocc;
+    ord.nocc_b = ra.nocc_b;
+    ord.ntp = ntp;
+    PackArgs pk{};
+    pk.in_f32 = in_f32;
+    pk.naux = (int)naux;
+    pk.naux_pad = pa.naux_pad;
+    pk.out0 = sp.op;
+    const int64_t nrg = (int64_t)(rows_a + rows_b) / 16;
+    double *pmax = (double *)s.slots[kSlotStage2].ptr;
+    mark(s, 0, stream);
+    pk.b = ba;
+    pk.nocc = ra.nocc;
+    pk.nvir = ra.nvir;
+    pk.nvir_pad = ra.nvir_pad;
+    pk.rexp = sp.rexp;
+    hipError_t he = launch_residue_pack(Prec::F64, pk, ord, pmax, stream, nrg, 0);
+    if (he == hipSuccess) {
+        pk.b = bb;
+        pk.nocc = ra.nocc_b;
+        pk.nvir = ra.nvir_b;
+        pk.nvir_pad = ra.nvir_pad_b;
+        pk.rexp = sp.rexp + rows_a;
+        he = launch_residue_pack(Prec::F64, pk, ResidueOrder{}, pmax + (size_t)np * col_a, stream,
+                                 nrg, (int64_t)rows_a / 16);
+    }
+    if (he != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(FH_KERNEL, "pack kernel: %s", hipGetErrorString(he));
+    }
+    mark(s, 1, stream);
+    he = launch_residue_energy(ra, stream);
+    if (he != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(FH_KERNEL, "opposite-spin kernel: %s", hipGetErrorString(he));
+    }
+    mark(s, 2, stream);
+    EnergyArgs ea{};  // what the reductions read
+    ea.nocc = ra.nocc;
+    ea.nocc_b = ra.nocc_b;
+    ea.ntile = ra.ntile;
+    ea.ntile_b = ra.ntile_b;
+    ea.item_partials = ra.item_partials;
+    ea.row_partials = (double *)s.slots[kSlotRows].ptr;
+    ea.result = (double *)s.slots[kSlotResult].ptr;
+    he = launch_rect_reduce(ea, stream);
+    if (he != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(FH_KERNEL, "reduction kernels: %s", hipGetErrorString(he));
+    }
+    mark(s, 3, stream);
+    s.pending.kernel_launches += 7;
+    fh_spin_components sc{};
+    st = fetch_result(s, ea.result, 0, stream, &sc, nullptr);
+    if (st != FH_OK) return st;
+    finish_timing(s, (uint64_t)(npairs * ntp), pa.tile);
+    *energy = sc.e_os;
+    return FH_OK;
+}
+
 fh_status opposite_core(State &s, const fh_spin_channel &ca, const fh_spin_channel &cb,
                         const void *ba, const void *bb, fh_dtype dt, size_t naux, Prec prec,
                         hipStream_t stream, double *energy) {
     const bool in_f32 = dt == FH_DT_F32;
+    if (prec == Prec::F64) {
+        bool taken = false;
+        const fh_status rst =
+            opposite_residue(s, ca, cb, ba, bb, in_f32, naux, stream, energy, &taken);
+        if (taken || rst != FH_OK) return rst;
+    }
     const EnergyPlan pa_plan = plan_energy(ca.nocc, std::max(ca.nvir, cb.nvir), naux, prec);
     const int tile = pa_plan.tile;
     const int vpa = (int)((ca.nvir + 15) / 16 * 16), vpb = (int)((cb.nvir + 15) / 16 * 16);

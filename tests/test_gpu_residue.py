@@ -138,3 +138,23 @@ def test_pool_ceiling_falls_back_to_the_matrix_kernel():
         lib.fh_set_pool_limit(0)
     assert _lib.stats()["fail_pool_full"] == before
     assert np.max(np.abs(pe.e - ref.e)) <= 1e-12 * np.max(np.abs(ref.e))
+
+
+@pytest.mark.parametrize("shape", [(9, 150, 8, 145, 1500), (12, 272, 7, 400, 900),
+                                   (3, 256, 4, 513, 4000)], ids=lambda s: "-".join(map(str, s)))
+def test_opposite_spin_rectangle(shape, oracle_mod, monkeypatch):
+    """Uneven channels: one tile a side, two, and one against three."""
+    from ferric_amd import unrestricted as un
+    na, va, nb, vb, naux = shape
+    print("residue rectangle", shape, flush=True)
+    ba, ea = _problem(na, va, naux, seed=3)
+    bb, eb = _problem(nb, vb, naux, seed=4)
+    g = torch.from_numpy
+    ca = un.SpinChannel(g(ba).cuda(), ea, na, va)
+    cb = un.SpinChannel(g(bb).cuda(), eb, nb, vb)
+    e = un.u_opposite_spin(ca, cb)
+    want = oracle_mod.u_opposite_spin((ba, ea, na, va, 0, na), (bb, eb, nb, vb, 0, nb),
+                                      nthreads=16)
+    assert abs(e - want) <= 1e-12 * abs(want)
+    monkeypatch.setenv("FERRIC_HIP_TILE", "64")
+    assert abs(e - un.u_opposite_spin(ca, cb)) <= 1e-12 * abs(want)
