@@ -7,7 +7,7 @@
 // (c_os, c_ss) = (1, 1) gives the MP2 density (T~ = 2t - t^T); otherwise
 // c_ss P_MP2 + (c_os - c_ss) P_OS.
 //
-// The fused FP64 energy kernel runs once with an epilogue that stores
+// The fused FP64 energy pass runs once with an epilogue that stores
 // t = g / D of every ordered occupied pair (both orientations of each unique
 // pair), the layout the reference's t2 has per (i, j) block. Both densities
 // are then one split-K FP64 MFMA product each over those blocks, every
@@ -15,9 +15,10 @@
 //   P_vv: K = (pair ij, c); A row a = t_ij[a][.], B row b = cd t_ij[b][.] - ce t_ji[b][.]
 //   P_oo: K = (k, ab);      A row i = t_ik,       B row j = cd t_jk - ce t_kj
 // (t_ij^ba = t_ji^ab makes the transposed reads of T~ plain reads of the
-// mirrored block). Each work item is one 64 x 64 output tile over one K slice;
-// a second kernel sums the slices of every tile in slice order, so the result
-// does not depend on scheduling.
+// mirrored block). Each work item is one 64 x 64 output tile over one K slice, of
+// the tiles on or above the diagonal only (both densities are symmetric; at 41/209
+// that took the two products from 1848 to 1484 us); a second kernel sums the slices
+// of every tile in a fixed order, so the result does not depend on scheduling.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -70,11 +71,11 @@ __device__ __forceinline__ DensRows dens_rows(const DensArgs &d, int64_t kp, int
 // barrier per panel.
 __global__ __launch_bounds__(256) void density_gemm_kernel(DensArgs d) {
     __shared__ __attribute__((aligned(16))) double lds[2][2][kDT][kDLdr];
-    const int64_t nt2 = (int64_t)d.ntile * d.ntile;
+    const int ntp = d.ntile * (d.ntile + 1) / 2;
     const int64_t item = blockIdx.x;
-    const int s = (int)(item / nt2);
-    const int t = (int)(item % nt2);
-    const int tm = t / d.ntile, tn = t % d.ntile;
+    const int s = (int)(item / ntp);
+    int tm, tn;  // both densities are symmetric: the tiles tm <= tn
+    decode_tile_pair((int)(item % ntp), d.ntile, tm, tn);
     const int64_t per = (d.kpanels + d.splits - 1) / d.splits;
     const int64_t p0 = (int64_t)s * per, p1 = min(d.kpanels, p0 + per);
     const int tid = threadIdx.x, lane = tid % kWave, wid = tid / kWave;
@@ -167,30 +168,42 @@ __global__ __launch_bounds__(256) void density_gemm_kernel(DensArgs d) {
             }
 }
 
-// out[m][n] = scale * sum over slices s = 0, 1, ... of the tile's partials.
-__global__ __launch_bounds__(256) void density_reduce_kernel(DensArgs d) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t total = (int64_t)d.mdim * d.mdim;
-    if (e >= total) return;
-    const int m = (int)(e / d.mdim), n = (int)(e % d.mdim);
-    const int tm = m / kDT, tn = n / kDT;
-    const int64_t nt2 = (int64_t)d.ntile * d.ntile;
-    const int64_t t = (int64_t)tm * d.ntile + tn;
-    const int off = (m % kDT) * kDT + (n % kDT);
+// out[m][n] = out[n][m] = scale * sum over slices s = 0, 1, ... of the tile's partials:
+// 64 elements of one tile a block, the slices dealt to sixteen groups of threads (group
+// w takes s = w, w + 16, ...) whose sums are added in group order. One thread per
+// element took 767 us for the 2048 slices of P_oo at 41/209, on the latency of its loads.
+constexpr int kRG = 16;
+__global__ __launch_bounds__(64 * kRG) void density_reduce_kernel(DensArgs d) {
+    const int ntp = d.ntile * (d.ntile + 1) / 2;
+    const int e = (int)(blockIdx.x % (kDT * kDT / 64)) * 64 + threadIdx.x % 64;
+    const int t = (int)(blockIdx.x / (kDT * kDT / 64)), w = threadIdx.x / 64;
+    int tm, tn;
+    decode_tile_pair(t, d.ntile, tm, tn);
+    const double *p = d.partial + (int64_t)t * kDT * kDT + e;
     double acc = 0.0;
-    for (int s = 0; s < d.splits; ++s) acc += d.partial[((int64_t)s * nt2 + t) * kDT * kDT + off];
-    d.out[e] = d.scale * acc;
+#pragma unroll 8
+    for (int s = w; s < d.splits; s += kRG) acc += p[(int64_t)s * ntp * kDT * kDT];
+    __shared__ double part[kRG][64];
+    part[w][threadIdx.x % 64] = acc;
+    __syncthreads();
+    if (w != 0) return;
+    for (int k = 1; k < kRG; ++k) acc += part[k][threadIdx.x];
+    const int m = tm * kDT + e / kDT, n = tn * kDT + e % kDT;
+    if (m >= d.mdim || n >= d.mdim) return;
+    // A diagonal tile holds both of (m, n) and (n, m): each writes its own.
+    d.out[(int64_t)m * d.mdim + n] = d.scale * acc;
+    if (tm != tn) d.out[(int64_t)n * d.mdim + m] = d.scale * acc;
 }
 
 }  // namespace
 
 hipError_t launch_density(const DensArgs &d, hipStream_t st) {
-    const int64_t nitems = (int64_t)d.ntile * d.ntile * d.splits;
+    const int ntp = d.ntile * (d.ntile + 1) / 2;
+    const int64_t nitems = (int64_t)ntp * d.splits;
     if (nitems <= 0 || nitems > 0x7fffffffLL || d.mdim <= 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(density_gemm_kernel, dim3((unsigned)nitems), dim3(256), 0, st, d);
-    const int64_t total = (int64_t)d.mdim * d.mdim;
-    hipLaunchKernelGGL(density_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
-                       st, d);
+    hipLaunchKernelGGL(density_reduce_kernel, dim3((unsigned)(ntp * (kDT * kDT / 64))),
+                       dim3(64 * kRG), 0, st, d);
     return hipGetLastError();
 }
 
@@ -199,7 +212,7 @@ namespace {
 // Slices per output tile: enough items to fill the chip (about 2048), each
 // slice at least 8 panels deep.
 int density_splits(int ntile, int64_t kpanels) {
-    const int64_t tiles = (int64_t)ntile * ntile;
+    const int64_t tiles = (int64_t)ntile * (ntile + 1) / 2;
     int64_t s = std::max<int64_t>(1, 2048 / tiles);
     s = std::min<int64_t>(s, std::max<int64_t>(1, kpanels / 8));
     return (int)s;
@@ -231,7 +244,8 @@ fh_status density_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t nau
     oo.splits = density_splits(oo.ntile, oo.kpanels);
     oo.scale = -1.0;
     const size_t part_elems =
-        std::max((size_t)vv.ntile * vv.ntile * vv.splits, (size_t)oo.ntile * oo.ntile * oo.splits) *
+        std::max((size_t)vv.ntile * (vv.ntile + 1) / 2 * vv.splits,
+                 (size_t)oo.ntile * (oo.ntile + 1) / 2 * oo.splits) *
         kDT * kDT;
     std::vector<std::pair<int, size_t>> req = {
         {kSlotDensAmp, amp_bytes},
