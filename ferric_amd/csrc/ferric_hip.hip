@@ -430,7 +430,7 @@ fh_status upload_eps(State &s, const double *eps, size_t first_occ, size_t nocc,
 fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, size_t nocc,
                          size_t nvir, const double *eps, size_t first_occ, size_t nocc_total,
                          double kappa, Prec prec, hipStream_t stream, fh_spin_components *out,
-                         double *row_partials, const EnergyPlan &pl) {
+                         double *row_partials, const EnergyPlan &pl, double *amp_out) {
     const size_t npairs = nocc * (nocc + 1) / 2;
     ResidueSpace sp;
     fh_status st = reserve_residue(
@@ -482,6 +482,7 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     ra.eps_vir = ra.eps_occ + nocc;
     ra.kappa = kappa;
     ra.item_partials = (double *)s.slots[kSlotItems].ptr;
+    ra.tamp = amp_out;
     EnergyArgs ea{};  // what the reductions read
     ea.nocc = ra.nocc;
     ea.ntp = ra.ntp;
@@ -567,13 +568,12 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
     size_t carved = 0;
     for (const auto &r : req) carved = (carved + 255) / 256 * 256 + r.second;
     EnergyPlan rpl;
-    if (!signed_k && !amp_out &&
-        !(as_noalloc && carved <= (size_t)FH_NOALLOC_SCRATCH_BYTES) &&
+    if (!signed_k && !(as_noalloc && carved <= (size_t)FH_NOALLOC_SCRATCH_BYTES) &&
         plan_residue(s, nocc, nvir, naux, prec, &rpl)) {
         const uint64_t full = s.stats.fail_pool_full;
         const fh_status rst =
             residue_energy(s, b_dev, in_f32, naux, nocc, nvir, eps, first_occ, nocc_total, kappa,
-                           prec, stream, out, row_partials, rpl);
+                           prec, stream, out, row_partials, rpl, amp_out);
         if (ntp_used) *ntp_used = rpl.ntp;
         // Its larger workspace may be past the pool ceiling: then the matrix kernel
         // below, which needs half the operand (or less) and no scratch.

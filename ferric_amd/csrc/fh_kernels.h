@@ -198,6 +198,7 @@ struct ResidueArgs {
     const int *rexp_b = nullptr;
     const double *eps_occ_b = nullptr, *eps_vir_b = nullptr;
     double *item_partials = nullptr;  // per occupied pair and tile pair
+    double *tamp = nullptr;      // amplitudes of every ordered pair (EnergyArgs::tamp), or null
     int blocks = 0;              // workgroups, one per CU (a multiple of kXcds)
     void *scratch = nullptr;     // residue_scratch_sets(blocks) x scratch_stride bytes
     int64_t scratch_stride = 0;

@@ -438,7 +438,13 @@ __device__ __forceinline__ void decode_upper(int t, int &x, int &y) {
 // waves; on a diagonal tile pair the unordered block pairs, g_ba from the mirror
 // block transposed through the LDS. The residues of the next block load while
 // this one is rebuilt.
-template <int N>
+// AMP: also stores t = g / D of both orderings of the pair,
+// a.tamp[((p nocc + q) nvir_pad + x) nvir_pad + y] for every x, y of the padded
+// block (0 past nvir), each element from exactly one lane: inside a diagonal block
+// (a, b) and (b, a) both come as t1, whose denominators need not agree to the last
+// bit, so t2 is left to the other lane. At 41/209/960 the pass takes 1119 us with the
+// 675 MB of amplitudes; the matrix kernel's took 2515 us.
+template <int N, bool AMP>
 __device__ __forceinline__ void pair_energy(const ResidueArgs &a, const PairTile &T,
                                             const char *c1, const char *c2, char *lds, KSum &os,
                                             KSum &ss) {
@@ -488,7 +494,8 @@ __device__ __forceinline__ void pair_energy(const ResidueArgs &a, const PairTile
 #pragma unroll 1
     for (int t = wid; t < nblk; t += 8) {
         const int la = bx * 16, lb = by * 16;  // in the tile
-        const double half = T.diag && bx == by ? 0.5 : 1.0;
+        const int bx0 = bx, by0 = by;
+        const double half = T.diag && bx0 == by0 ? 0.5 : 1.0;
         uint32_t d1[N], d2[N];
 #pragma unroll
         for (int k = 0; k < N; ++k) {
@@ -527,6 +534,30 @@ __device__ __forceinline__ void pair_energy(const ResidueArgs &a, const PairTile
         }
         const bool okb = T.b0 * 16 + lb + r < a.nvir;
         const double eb = tab.eps[1][lb + r];
+        if constexpr (AMP) {
+            const int64_t vp = a.nvir_pad;
+            double *bij = a.tamp + ((int64_t)T.i * a.nocc + T.j) * vp * vp;
+            double *bji = a.tamp + ((int64_t)T.j * a.nocc + T.i) * vp * vp;
+            const int64_t A = T.a0 * 16 + la + 4 * g, B = T.b0 * 16 + lb + r;
+            v4d t1, t2;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const double inv = 1.0 / (eij - tab.eps[0][la + 4 * g + v] - eb);
+                const bool ok = okb && A + v < a.nvir;
+                t1[v] = ok ? g1[v] * inv : 0.0;
+                t2[v] = ok ? g2[v] * inv : 0.0;
+            }
+            const bool other = !(T.diag && bx0 == by0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) bij[(A + v) * vp + B] = t1[v];
+            if (other) *(v4d *)(bij + B * vp + A) = t2;
+            if (T.i != T.j) {
+                *(v4d *)(bji + B * vp + A) = t1;
+                if (other)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) bji[(A + v) * vp + B] = t2[v];
+            }
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const bool ok = okb && T.a0 * 16 + la + 4 * g + v < a.nvir;
@@ -590,7 +621,8 @@ __device__ __forceinline__ void rect_energy(const ResidueArgs &a, const PairTile
 
 // RECT: opposite spin, items (i, J, tA, tB) over every alpha i, beta J and tile of
 // each side, one product each; the beta rows follow the alpha rows in the operand.
-template <int N, bool RECT>
+// AMP: the amplitudes are stored too.
+template <int N, bool RECT, bool AMP>
 __global__ __launch_bounds__(kThreads) void residue_energy_kernel(ResidueArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     __shared__ int turn;
@@ -714,7 +746,7 @@ __global__ __launch_bounds__(kThreads) void residue_energy_kernel(ResidueArgs a)
                 T.v0 = v * wB;
                 T.diag = ta == tb;
                 KSum os, ss;
-                pair_energy<N>(a, T, scr, nprod == 2 ? scr + planes_of(N) : nullptr, lds, os, ss);
+                pair_energy<N, AMP>(a, T, scr, nprod == 2 ? scr + planes_of(N) : nullptr, lds, os, ss);
                 const int64_t p = (int64_t)T.i * a.nocc - (int64_t)T.i * (T.i - 1) / 2 + T.j - T.i;
                 pair::block_store(os, ss, T.i == T.j ? 1.0 : 2.0,
                                   a.item_partials + 4 * (p * a.ntp + id % a.ntp));
@@ -799,9 +831,11 @@ hipError_t launch_residue_energy(const ResidueArgs &a, hipStream_t st) {
                a.scratch_stride < (int64_t)residue_scratch_stride(a.prec, a.ntile > 1 ? 2 : 1)) {
         return hipErrorInvalidValue;
     }
-    const auto kern = rect                             ? residue_energy_kernel<16, true>
-                      : residue_moduli(a.prec) == 16 ? residue_energy_kernel<16, false>
-                                                     : residue_energy_kernel<10, false>;
+    if (a.tamp && (rect || a.prec != Prec::F64)) return hipErrorInvalidValue;
+    const auto kern = rect                           ? residue_energy_kernel<16, true, false>
+                      : a.tamp                       ? residue_energy_kernel<16, false, true>
+                      : residue_moduli(a.prec) == 16 ? residue_energy_kernel<16, false, false>
+                                                     : residue_energy_kernel<10, false, false>;
     hipLaunchKernelGGL(kern, dim3((unsigned)a.blocks), dim3(kThreads), kBuf * kStage, st, a);
     return hipGetLastError();
 }
