@@ -8,7 +8,8 @@
 //   dE/deps_c = 2 P_cc =  2 sum_ijb t_ij^cb T~_ij^cb       (virtual)
 //     (oo_rimp2.rs:1192-1300, rimp2.rs:2026-2052).
 //
-// One batch per occupied row i, in ascending order:
+// FP64 up to kGammaBytes of amplitudes: all rows at once (adjoint_core_amp, gamma.hip).
+// Otherwise, and in BF16x3, one batch per occupied row i, in ascending order:
 //   A  pair kernel over (i, j >= i) (energy.hip, adjoint epilogue): recomputes
 //      K_ij, writes T~_ij for this row's pairs into row scratch (tbuf: a-major,
 //      ubuf: b-major per j > i) and per-item t*T~ sums;
@@ -1020,6 +1021,67 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
     return FH_OK;
 }
 
+// FP64 over whole amplitudes: the pair pass of the energy stores t, then the kernels of
+// gamma.hip. Refused with FH_POOL_FULL past kGammaBytes or the pool ceiling; the caller
+// then runs the rows one at a time. The bound is 1/16 of the card's memory: the largest
+// amplitudes it admits are 46341 (i, a) rows.
+constexpr size_t kGammaBytes = (size_t)16 << 30;
+
+static fh_status adjoint_core_amp(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux,
+                                  size_t nocc, size_t nvir, const double *eps, size_t n_eps,
+                                  size_t first_occ, size_t nocc_total, double c_os, double c_ss,
+                                  hipStream_t stream, fh_spin_components *out, double *gamma_dev,
+                                  double *deps) {
+    const size_t nov = nocc * nvir, ld = (size_t)gamma_ld((int64_t)nov);
+    GammaArgs g;
+    g.nocc = (int)nocc;
+    g.nvir = (int)nvir;
+    g.naux = (int)naux;
+    g.ld = (int64_t)ld;
+    g.cd = c_os + c_ss;
+    g.ce = c_ss;
+    g.splits = gamma_splits(g.naux, (int64_t)nov, compute_units(s));
+    g.gamma = gamma_dev;
+    fh_status st = reserve(
+        s, {{kSlotT, sizeof(double) * nov * ld},
+            {kSlotU, sizeof(double) * naux * ld},
+            {kSlotDeps, sizeof(double) * (nov * nocc + nocc + nvir)},
+            {kSlotSplit, g.splits > 1 ? sizeof(double) * (size_t)g.splits * naux * nov : 256}});
+    if (st != FH_OK) return st;
+    const AmpOut amp{(double *)s.slots[kSlotT].ptr, (int64_t)(nvir * ld), (int64_t)nvir,
+                     (int64_t)ld, (int)nvir};
+    st = energy_core(s, b_dev, b_dtype, naux, nocc, nvir, eps, first_occ, nocc_total, NAN,
+                     Prec::F64, stream, out, nullptr, nullptr, nullptr, 0, &amp);
+    if (st != FH_OK) return st;
+    g.t = amp.base;
+    g.b = (const double *)s.slots[kSlotU].ptr;
+    g.rsum = (double *)s.slots[kSlotDeps].ptr;
+    g.deps = g.rsum + nov * nocc;
+    g.partial = (double *)s.slots[kSlotSplit].ptr;
+    hipError_t he = launch_gamma_rows(b_dev, b_dtype == FH_DT_F32, g.naux, (int64_t)nov, g.ld,
+                                      (double *)s.slots[kSlotU].ptr, stream);
+    if (he == hipSuccess) he = launch_gamma(g, stream);
+    if (he != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(FH_KERNEL, "adjoint kernels: %s", hipGetErrorString(he));
+    }
+    s.pending.kernel_launches += g.splits > 1 ? 5 : 4;
+    std::vector<double> res(nocc + nvir);
+    st = hip_check(hipMemcpyAsync(res.data(), g.deps, sizeof(double) * res.size(),
+                                  hipMemcpyDeviceToHost, stream),
+                   "D2H adjoint result");
+    if (st != FH_OK) return st;
+    st = hip_check(hipStreamSynchronize(stream), "stream sync");
+    if (st != FH_OK) return st;
+    s.pending.d2h_bytes += sizeof(double) * res.size();
+    if (deps) {
+        for (size_t k = 0; k < n_eps; ++k) deps[k] = 0.0;
+        for (size_t i = 0; i < nocc; ++i) deps[first_occ + i] = res[i];
+        for (size_t a = 0; a < nvir; ++a) deps[nocc_total + a] = res[nocc + a];
+    }
+    return FH_OK;
+}
+
 static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux,
                               size_t nocc, size_t nvir, const double *eps, size_t n_eps,
                               size_t first_occ, size_t nocc_total, double c_os, double c_ss,
@@ -1030,6 +1092,15 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
     if (prec == Prec::I8X4)
         return adjoint_core_i8(s, b_dev, b_dtype, naux, nocc, nvir, eps, n_eps, first_occ,
                                nocc_total, c_os, c_ss, stream, out, gamma_dev, deps);
+    if (f64 && nocc * nvir <= kGammaBytes / sizeof(double) / (size_t)gamma_ld(nocc * nvir)) {
+        const uint64_t full = s.stats.fail_pool_full;
+        const fh_status ast =
+            adjoint_core_amp(s, b_dev, b_dtype, naux, nocc, nvir, eps, n_eps, first_occ,
+                             nocc_total, c_os, c_ss, stream, out, gamma_dev, deps);
+        if (ast != FH_POOL_FULL) return ast;
+        s.stats.fail_pool_full = full;
+        clear_error();
+    }
     const Prec gprec = f64 ? Prec::F64 : Prec::BF16X3;
     EnergyPlan pl = plan_energy(nocc, nvir, naux, prec);
     // The FP64 adjoint epilogue does not fit a 128-wide tile in the register

@@ -254,9 +254,11 @@ fh_status density_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t nau
     };
     fh_status st = reserve(s, req);
     if (st != FH_OK) return st;
+    const int64_t blk = (int64_t)(vp * vp);
     double *amp = (double *)s.slots[kSlotDensAmp].ptr;
+    const AmpOut amp_out{amp, (int64_t)nocc * blk, blk, (int64_t)vp, (int)vp, true};
     st = energy_core(s, b_dev, b_dtype, naux, nocc, nvir, eps, first_occ, nocc_total, NAN,
-                     Prec::F64, stream, out, nullptr, &pl, nullptr, 0, amp);
+                     Prec::F64, stream, out, nullptr, &pl, nullptr, 0, &amp_out);
     if (st != FH_OK) return st;
     double *dout = (double *)s.slots[kSlotDensOut].ptr;
     vv.tamp = oo.tamp = amp;

@@ -152,7 +152,7 @@ hipError_t launch_items(K kern, const EnergyArgs &a, hipStream_t st, int threads
 hipError_t launch_energy(const EnergyArgs &a, hipStream_t st) {
     if (a.nitems <= 0 || a.nitems > 0x7fffffffLL) return hipErrorInvalidValue;
     hipError_t e = hipErrorInvalidValue;
-    if (a.tamp) {  // MP2 densities: FP64 energy that also stores the amplitudes
+    if (a.amp.base) {  // FP64 energy that also stores the amplitudes
         if (a.prec != Prec::F64 || a.q_neg < a.naux_pad) return hipErrorInvalidValue;
         if (a.tile == 128) e = launch_items(pair_k4_kernel<double, 128, 16, false, false, false, true>, a, st);
         else if (a.tile == 64) e = launch_items(pair_k4_kernel<double, 64, 16, false, false, false, true>, a, st);

@@ -310,14 +310,21 @@ int i8_q_rot_ticks(State &s, int npanels, int ntp) {
     return (int)std::lround(s.wall_khz * 1.4e-3);
 }
 
+int compute_units(State &s) {
+    if (s.cus <= 0 &&
+        (hipDeviceGetAttribute(&s.cus, hipDeviceAttributeMultiprocessorCount, s.device) !=
+             hipSuccess ||
+         s.cus <= 0)) {
+        (void)hipGetLastError();
+        s.cus = 1;
+    }
+    return s.cus;
+}
+
 bool residue_tiles(State &s, size_t nvir, size_t naux, EnergyPlan *pl) {
     // 4608: the most the int32 sums and byte remainders allow (residue.h).
     if (s.arena || forced_tile() > 0 || naux > 4608) return false;
-    if (s.cus <= 0 &&
-        hipDeviceGetAttribute(&s.cus, hipDeviceAttributeMultiprocessorCount, s.device) !=
-            hipSuccess)
-        s.cus = 0;
-    if (s.cus < 8) return false;  // whole rounds over the eight XCDs
+    if (compute_units(s) < 8) return false;  // whole rounds over the eight XCDs
     EnergyPlan p;
     p.tile = 256;
     p.nvir_pad = (int)((nvir + 15) / 16 * 16);
@@ -430,7 +437,7 @@ fh_status upload_eps(State &s, const double *eps, size_t first_occ, size_t nocc,
 fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, size_t nocc,
                          size_t nvir, const double *eps, size_t first_occ, size_t nocc_total,
                          double kappa, Prec prec, hipStream_t stream, fh_spin_components *out,
-                         double *row_partials, const EnergyPlan &pl, double *amp_out) {
+                         double *row_partials, const EnergyPlan &pl, const AmpOut *amp_out) {
     const size_t npairs = nocc * (nocc + 1) / 2;
     ResidueSpace sp;
     fh_status st = reserve_residue(
@@ -482,7 +489,7 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     ra.eps_vir = ra.eps_occ + nocc;
     ra.kappa = kappa;
     ra.item_partials = (double *)s.slots[kSlotItems].ptr;
-    ra.tamp = amp_out;
+    if (amp_out) ra.amp = *amp_out;
     EnergyArgs ea{};  // what the reductions read
     ea.nocc = ra.nocc;
     ea.ntp = ra.ntp;
@@ -514,7 +521,7 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
                       size_t nvir, const double *eps, size_t first_occ, size_t nocc_total,
                       double kappa, Prec prec, hipStream_t stream, fh_spin_components *out,
                       double *row_partials, const EnergyPlan *forced, const void *neg_dev,
-                      size_t naux_neg, double *amp_out, int *ntp_used,
+                      size_t naux_neg, const AmpOut *amp_out, int *ntp_used,
                       bool as_noalloc) {
     const bool in_f32 = b_dtype == FH_DT_F32;
     EnergyPlan pl = forced ? *forced : plan_energy(nocc, nvir, naux, prec);
@@ -665,7 +672,7 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
     ea.row_partials = (double *)s.slots[kSlotRows].ptr;
     ea.result = (double *)s.slots[kSlotResult].ptr;
     ea.q_neg = q_neg;
-    ea.tamp = amp_out;
+    if (amp_out) ea.amp = *amp_out;
     mark(s, 1, stream);
     he = launch_energy(ea, stream);
     if (he != hipSuccess) {

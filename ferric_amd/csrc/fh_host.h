@@ -138,8 +138,9 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
                       double kappa, Prec prec, hipStream_t stream, fh_spin_components *out,
                       double *row_partials, const EnergyPlan *forced,
                       const void *neg_dev = nullptr, size_t naux_neg = 0,
-                      double *amp_out = nullptr, int *ntp_used = nullptr,
+                      const AmpOut *amp_out = nullptr, int *ntp_used = nullptr,
                       bool as_noalloc = false);
+int compute_units(State &s);  // of the device, asked once; at least 1
 // Residue arithmetic (residue.hip). Tile sides and paddings of a shape, where it may
 // run at all (aux count, forced tiles, fixed arena); whether an energy of this
 // shape is faster so, and its plan; and the workspace of a launch.

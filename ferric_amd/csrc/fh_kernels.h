@@ -123,6 +123,15 @@ inline int panel_depth(Prec p) {
     return 128;
 }
 
+// Where a pair pass stores the amplitudes t = g / D of every ordered occupied pair
+// (FP64): t_pq^xy at base[p sp + q sq + x sx + y] for x, y < n, zeros past nvir.
+struct AmpOut {
+    double *base = nullptr;
+    int64_t sp = 0, sq = 0, sx = 0;
+    int n = 0;
+    bool wide = false;  // n = nvir_pad and every stride a multiple of four
+};
+
 struct EnergyArgs {
     Prec prec;
     int tile;                 // 32, 64 or 128
@@ -174,9 +183,7 @@ struct EnergyArgs {
     int nocc_b = 0, nvir_b = 0, nvir_pad_b = 0, ntile_b = 0;
     const double *eps_occ_b = nullptr, *eps_vir_b = nullptr;
     const int *rexp_b = nullptr;  // I8X4: row exponents of the beta rows
-    // MP2 densities (FP64): the energy kernel also stores t = g / D of every
-    // ordered occupied pair, tamp[((i*nocc + j)*nvir_pad + a)*nvir_pad + b].
-    double *tamp = nullptr;
+    AmpOut amp;  // MP2 densities, FP64 adjoint: store the amplitudes too
 };
 
 hipError_t launch_energy(const EnergyArgs &a, hipStream_t st);
@@ -198,7 +205,7 @@ struct ResidueArgs {
     const int *rexp_b = nullptr;
     const double *eps_occ_b = nullptr, *eps_vir_b = nullptr;
     double *item_partials = nullptr;  // per occupied pair and tile pair
-    double *tamp = nullptr;      // amplitudes of every ordered pair (EnergyArgs::tamp), or null
+    AmpOut amp;                  // store the amplitudes too, unless base is null
     int blocks = 0;              // workgroups, one per CU (a multiple of kXcds)
     void *scratch = nullptr;     // residue_scratch_sets(blocks) x scratch_stride bytes
     int64_t scratch_stride = 0;
@@ -294,5 +301,24 @@ struct DensArgs {
     double *out;          // (mdim, mdim) row-major
 };
 hipError_t launch_density(const DensArgs &d, hipStream_t st);
+
+// FP64 adjoint over whole amplitudes (gamma.hip).
+struct GammaArgs {
+    int nocc, nvir, naux;
+    int64_t ld;           // row length of b and t, nocc nvir padded (gamma_ld)
+    const double *b;      // (naux, ld) B by Q, zeros past nocc nvir
+    double *t;            // (nocc nvir, ld): t on entry, then T~ = cd t - ce t^T
+    double cd, ce;
+    double *rsum;         // (nocc nvir, nocc): row sums of t T~ per partner
+    double *deps;         // (nocc + nvir): dE/deps
+    int splits;           // K slices of the product (gamma_splits)
+    double *partial;      // (splits, naux, nocc nvir) when splits > 1
+    double *gamma;        // (naux, nocc nvir)
+};
+int64_t gamma_ld(int64_t nov);
+int gamma_splits(int naux, int64_t nov, int cus);
+hipError_t launch_gamma_rows(const void *b, bool in_f32, int naux, int64_t nov, int64_t ld,
+                             double *out, hipStream_t st);
+hipError_t launch_gamma(const GammaArgs &g, hipStream_t st);
 
 }  // namespace fh

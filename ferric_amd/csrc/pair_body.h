@@ -350,13 +350,13 @@ __device__ __forceinline__ void adjoint_epilogue(const EnergyArgs &a, const Item
     }
 }
 
-// Amplitude store (the MP2 densities): t = g / D of the item's elements into
-// the ordered-pair amplitude blocks, a.tamp[((p*nocc + q)*nvir_pad + x)*nvir_pad + y]
-// = t_pq^xy for every ordered occupied pair (p, q). C1 gives t_ij^ab, stored as
+// Amplitude store (MP2 densities, FP64 adjoint): t = g / D of the item's elements,
+// t_pq^xy of every ordered occupied pair (p, q). C1 gives t_ij^ab, stored as
 // (i, j, a, b) and as its mirror (j, i, b, a); C2 gives t_ij^ba, stored as
 // (i, j, b, a) and (j, i, a, b) (on a diagonal tile pair C2 = C1^T, whose
-// elements other lanes store). Elements past nvir are stored as zeros, so the
-// padded blocks read back whole. Every element has exactly one writer.
+// elements other lanes store). Elements past nvir and inside the block's side are
+// stored as zeros, so padded blocks read back whole. Every element has exactly one
+// writer.
 template <int TILE, typename Acc, typename RowOfT>
 __device__ __forceinline__ void amp_store(const EnergyArgs &a, const Item &it, const Lane &L,
                                           Acc (&acc1)[TILE / 32][TILE / 32],
@@ -364,9 +364,9 @@ __device__ __forceinline__ void amp_store(const EnergyArgs &a, const Item &it, c
                                           const bool *cv, RowOfT row_of) {
     constexpr int TW = TILE / 2, NB = TW / 16;
     const double eij = a.eps_occ[it.i] + a.eps_occ[it.j];
-    const int64_t vp = a.nvir_pad;
-    double *bij = a.tamp + ((int64_t)it.i * a.nocc + it.j) * vp * vp;
-    double *bji = a.tamp + ((int64_t)it.j * a.nocc + it.i) * vp * vp;
+    const int64_t vp = a.amp.sx;
+    double *bij = a.amp.base + it.i * a.amp.sp + it.j * a.amp.sq;
+    double *bji = a.amp.base + it.j * a.amp.sp + it.i * a.amp.sq;
     const bool diag_tile = it.ta == it.tb;
 #pragma unroll
     for (int x = 0; x < NB; ++x)
@@ -385,6 +385,7 @@ __device__ __forceinline__ void amp_store(const EnergyArgs &a, const Item &it, c
                     t1 = acc1[x][y][v] * inv;
                     t2 = acc2[x][y][v] * inv;
                 }
+                if (aa >= a.amp.n || bb >= a.amp.n) continue;
                 bij[aa * vp + bb] = t1;
                 if (!diag_tile) bij[bb * vp + aa] = t2;
                 // For i == j the mirror block is the block itself: each of its
