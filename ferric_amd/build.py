@@ -67,7 +67,7 @@ def build(jobs: int | None = None, verbose: bool = False) -> str:
         list(ex.map(compile_one, zip(srcs, objs)))
     tmp = LIB + ".tmp"
     # rocBLAS carries the plain dense GEMMs of the dressing stage and the PNO
-    # transforms; rocSOLVER the PNO eigensolves and the domain fits' Cholesky.
+    # transforms; rocSOLVER the PNO eigensolves.
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs,
           "-L/opt/rocm/lib", "-lrocsolver", "-lrocblas", "-Wl,-rpath,/opt/rocm/lib"])
     os.replace(tmp, LIB)

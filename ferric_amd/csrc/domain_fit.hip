@@ -4,200 +4,417 @@
 //   J_ij = A_{i,D}^T V_DD^{-1} A_{j,D},   D = the aux functions within `radius`
 //                                          of the centre of i or of j,
 //
-// with A the unwhitened (P|ia) and V the aux metric. Pairs are batched at one
-// padded domain size dmax: a pair's V_DD sits in the leading d x d block with
-// the identity on the rest of the diagonal, and its A rows beyond d are zero,
-// so the padding leaves J unchanged. The Cholesky factorisation and the
-// inverse from it run on rocSOLVER (dpotrf, dpotri), the products on rocBLAS
-// (dsymm, dgemm); the gathers are the kernel below.
+// with A the unwhitened (P|ia) and V the aux metric: one workgroup per pair gathers,
+// factors, solves and multiplies.
 #include <hip/hip_runtime.h>
-#include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
+#include "fh_device.h"
 #include "fh_host.h"
 #include "fh_kernels.h"
 
 namespace fh {
 namespace {
 
-constexpr int kThreads = 256;
+// ---- One workgroup per pair --------------------------------------------------
+// With V_DD = U^T U and Y = U^-T [A_i | A_j], J = Y_i^T Y_j. The rows of
+// [V_DD | A_i | A_j] are eliminated 16 at a time, looking left: a 16 x 16 block of the
+// row takes the products with the rows above (v_mfma_f64_16x16x4f64, the block in the
+// accumulators), wave 0 factors the diagonal block and applies the same row operations
+// to the identity, and each wave multiplies its blocks by that U_kk^-T. An accumulator
+// element v of a lane is row 4 v + g, which is what the B operand of step v holds, so
+// the blocks stay in their registers. The finished rows lie in a slot of the workspace,
+// read from the caches. A row of blocks is a chain of two barriers and 16 dependent
+// pivots (about 4 us); the pairs of a call hide it, four workgroups to a CU.
+// 820 pairs of up to 120 aux functions and 100 virtuals: 276 us, 24% of it at the matrix
+// units, the rest the chain and the latency of the slots (530 MB past the L2); 2.5 ms
+// of rocSOLVER and rocBLAS launches (potf2, trtri, lauum, symm, gemm) before. Also
+// faster at 36 pairs of 41 (0.28 -> 0.09 ms a call), 820 of 480 (26 -> 4.7 ms) and 4 of
+// 1500 (20 -> 9.4 ms).
+struct FitArgs {
+    const int32_t *pairs;
+    const uint64_t *near;  // per occupied: words of aux bits inside the radius
+    int words;
+    const double *v, *a;
+    int64_t naux, nov;
+    int nvir, nv;          // nv: 16-wide blocks of virtuals
+    int cap;               // rows of a slot, a multiple of 16
+    int32_t *dom;          // cap per pair
+    double *u;             // cap (cap + 32 nv) per pair
+    int32_t *info;
+    double *j;
+};
 
-fh_status solver_ok(rocblas_status st, const char *what) {
-    if (st == rocblas_status_success) return FH_OK;
-    return fail(FH_KERNEL, "%s: rocBLAS/rocSOLVER status %d", what, (int)st);
+constexpr int kFitWaves = 4, kFitHeld = 5;  // blocks a wave keeps while the pivots are found
+constexpr int kFitThreads = kFitWaves * 64;
+
+__device__ __forceinline__ double lane_value(double x, int lane) {
+    const int64_t b = __builtin_bit_cast(int64_t, x);
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, lane);
+    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)b >> 32), lane);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
-// One workgroup per pair. vp (dmax x dmax, column-major): V[dom[r], dom[c]]
-// inside the domain, the identity on the padded diagonal, zero elsewhere.
-// x (dmax x 2 nvir, column-major): columns a < nvir hold A[dom[r], i nvir + a],
-// columns nvir + b hold A[dom[r], j nvir + b]; zero on padded rows.
-__global__ __launch_bounds__(kThreads) void fit_gather_kernel(
-    const int32_t *__restrict__ pairs, const int32_t *__restrict__ dom,
-    const int32_t *__restrict__ dsize, int dmax, const double *__restrict__ v, int64_t naux,
-    const double *__restrict__ a, int64_t nov, int nvir, double *__restrict__ vp,
-    double *__restrict__ x) {
-    const int p = blockIdx.x;
-    const int32_t *dp = dom + (int64_t)p * dmax;
-    const int d = dsize[p];
-    const int i = pairs[2 * p], j = pairs[2 * p + 1];
-    double *vq = vp + (int64_t)p * dmax * dmax;
-    for (int64_t e = threadIdx.x; e < (int64_t)dmax * dmax; e += kThreads) {
-        const int r = (int)(e % dmax), c = (int)(e / dmax);
-        double val;
-        if (r < d && c < d)
-            val = v[(int64_t)dp[r] * naux + dp[c]];
-        else
-            val = r == c ? 1.0 : 0.0;
-        vq[e] = val;
-    }
-    double *xq = x + (int64_t)p * dmax * 2 * nvir;
-    for (int64_t e = threadIdx.x; e < (int64_t)dmax * 2 * nvir; e += kThreads) {
-        const int r = (int)(e % dmax), col = (int)(e / dmax);
-        double val = 0.0;
-        if (r < d) {
-            const int occ = col < nvir ? i : j;
-            const int av = col < nvir ? col : col - nvir;
-            val = a[(int64_t)dp[r] * nov + (int64_t)occ * nvir + av];
+__global__ __launch_bounds__(kFitThreads, 4) void fit_pair_kernel(FitArgs g) {
+    __shared__ double diag[16][17];
+    __shared__ double linv[16][17];
+    __shared__ int wsum[kFitWaves];
+    __shared__ int bad;
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int wid = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int r = lane % 16, gg = lane / 16;
+    const int64_t p = blockIdx.x;
+    const int oi = g.pairs[2 * p], oj = g.pairs[2 * p + 1];
+    int32_t *dom = g.dom + p * g.cap;
+
+    // The domain: the aux functions near i or j, in aux order.
+    int d = 0;
+    for (int w0 = 0; w0 < g.words; w0 += kFitThreads) {
+        const int w = w0 + tid;
+        uint64_t m = 0;
+        if (w < g.words)
+            m = g.near[(int64_t)oi * g.words + w] | g.near[(int64_t)oj * g.words + w];
+        const int c = __popcll(m);
+        int at = c;
+        for (int k = 1; k < kWave; k *= 2) {
+            const int o = __shfl_up(at, k, kWave);
+            if (lane >= k) at += o;
         }
-        xq[e] = val;
+        if (lane == kWave - 1) wsum[wid] = at;
+        __syncthreads();
+        int total = 0;
+        for (int k = 0; k < kFitWaves; ++k) {
+            if (k < wid) at += wsum[k];
+            total += wsum[k];
+        }
+        for (at += d - c; m; m &= m - 1) dom[at++] = w * 64 + __ffsll((unsigned long long)m) - 1;
+        d += total;
+        __syncthreads();
+    }
+    if (tid == 0) bad = 0;
+    d = __builtin_amdgcn_readfirstlane(d);
+    const int nd = (d + 15) / 16;
+    const int64_t ldu = (int64_t)(nd + 2 * g.nv) * 16;
+    double *u = g.u + p * g.cap * (int64_t)(g.cap + 32 * g.nv);
+    const uint32_t off = (uint32_t)(gg * (int)ldu + r);
+
+    for (int k = 0; k < nd; ++k) {
+        const int nblk = nd - k + 2 * g.nv;  // block t: columns 16 (k + t) .. + 16
+        int row[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) row[v] = dom[min(16 * k + 4 * v + gg, d - 1)];
+        // Blocks t = t0 + wid, t0 + wid + 4, ..., H of them (one past the last stands for
+        // it and is not stored), as they stand before any elimination (the lower triangle
+        // of V, the identity past the domain, A past V), less the products with the rows
+        // above. All loads of a step are issued before the products of the last one.
+        v4d acc[kFitHeld];
+        auto update = [&](auto held, int t0) {
+            constexpr int H = decltype(held)::value;
+            int32_t first[H];  // of the column: V's row, A's column
+#pragma unroll
+            for (int q = 0; q < H; ++q) {
+                const int t = min(t0 + wid + q * kFitWaves, nblk - 1), x = t - (nd - k);
+                first[q] = x < 0 ? dom[min(16 * (k + t) + r, d - 1)]
+                                 : min((x < g.nv ? x : x - g.nv) * 16 + r, g.nvir - 1);
+            }
+#pragma unroll
+            for (int q = 0; q < H; ++q) {
+                const int t = min(t0 + wid + q * kFitWaves, nblk - 1), x = t - (nd - k);
+                const double *base = x < 0 ? g.v : g.a + (int64_t)(x < g.nv ? oi : oj) * g.nvir;
+                const int64_t sr = x < 0 ? 1 : g.nov, sc = x < 0 ? g.naux : 1;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[q][v] = base[row[v] * sr + first[q] * sc];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const double *um = u + 16 * k, *ut = um + 16 * (t0 + wid);
+            const int last = 16 * (min(t0 + wid + (H - 1) * kFitWaves, nblk - 1) - t0 - wid);
+            double fa[2][2], fb[2][2][H];
+            auto fetch = [&](int h) {  // half of the 16 rows at um
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const int64_t at = 4 * (2 * h + s) * ldu;
+                    fa[h][s] = (um + at)[off];
+#pragma unroll
+                    for (int q = 0; q < H; ++q)
+                        fb[h][s][q] = (ut + at + (q + 1 < H ? 16 * kFitWaves * q : last))[off];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto products = [&](int h) {
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int q = 0; q < H; ++q)
+                        acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(-fa[h][s], fb[h][s][q],
+                                                                      acc[q], 0, 0, 0);
+            };
+            if (k > 0) fetch(0);
+#pragma unroll
+            for (int q = 0; q < H; ++q) {
+                const int t = min(t0 + wid + q * kFitWaves, nblk - 1), x = t - (nd - k);
+                const int C = 16 * (k + t) + r, lim = (x < g.nv ? g.nvir : g.nvir + 16 * g.nv);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int R = 16 * k + 4 * v + gg;
+                    const bool in = R < d && (x < 0 ? C < d : 16 * x + r < lim);
+                    acc[q][v] = in ? acc[q][v] : (R == C ? 1.0 : 0.0);
+                }
+            }
+            for (int m = 0; m < k; ++m) {
+                fetch(1);
+                products(0);
+                if (m + 1 < k) {
+                    um += 16 * ldu;
+                    ut += 16 * ldu;
+                }
+                fetch(0);
+                products(1);
+            }
+        };
+        auto finish = [&](auto held, int t0) {
+            constexpr int H = decltype(held)::value;
+            double fa[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) fa[s] = linv[r][4 * s + gg];
+#pragma unroll
+            for (int q = 0; q < H; ++q) {
+                const int t = t0 + wid + q * kFitWaves;
+                v4d o = {0, 0, 0, 0};
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    o = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s], acc[q][s], o, 0, 0, 0);
+                if (t >= nblk || t == 0) continue;
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    (u + (16 * k + 4 * v) * ldu + 16 * (k + t))[off] = o[v];
+            }
+        };
+        auto with_held = [&](int t0, auto f) {
+            const int n = (nblk - t0 + kFitWaves - 1) / kFitWaves;
+            if (n >= kFitHeld) f(std::integral_constant<int, kFitHeld>{});
+            else if (n == 5) f(std::integral_constant<int, 5>{});
+            else if (n == 4) f(std::integral_constant<int, 4>{});
+            else if (n == 3) f(std::integral_constant<int, 3>{});
+            else if (n == 2) f(std::integral_constant<int, 2>{});
+            else f(std::integral_constant<int, 1>{});
+        };
+        with_held(0, [&](auto h) { update(h, 0); });
+        if (wid == 0)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) diag[4 * v + gg][r] = acc[0][v];
+        __syncthreads();
+        if (wid == 0) {
+            // Lanes 0 .. 15 hold the block's columns, 16 .. 31 the identity's; rows below
+            // the diagonal of a column are never read by another lane.
+            double c[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                c[i] = lane < 16 ? diag[i][r] : (lane < 32 && i == r ? 1.0 : 0.0);
+            int fault = 0;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const double piv = lane_value(c[i], i);
+                if (piv <= 0.0 && fault == 0) fault = 16 * k + i + 1;
+                c[i] *= 1.0 / sqrt(piv);
+#pragma unroll
+                for (int x = i + 1; x < 16; ++x) c[x] -= lane_value(c[i], x) * c[i];
+            }
+            if (lane >= 16 && lane < 32)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) linv[i][r] = c[i];
+            if (lane == 0) bad = fault;
+        }
+        __syncthreads();
+        if (bad) {
+            if (tid == 0) g.info[p] = bad;
+            return;
+        }
+        with_held(0, [&](auto h) { finish(h, 0); });
+        for (int t0 = kFitHeld * kFitWaves; t0 < nblk; t0 += kFitHeld * kFitWaves) {
+            with_held(t0, [&](auto h) { update(h, t0); });
+            with_held(t0, [&](auto h) { finish(h, t0); });
+        }
+        __syncthreads();
+    }
+    if (tid == 0) g.info[p] = 0;
+
+    // J = Y_i^T Y_j, 32 x 64 a wave and turn.
+    const int na = (g.nv + 1) / 2, nb = (g.nv + 3) / 4;
+    const double *yi = u + 16 * nd, *yj = yi + 16 * g.nv;
+    double *jp = g.j + p * (int64_t)g.nvir * g.nvir;
+    for (int t = wid; t < na * nb; t += kFitWaves) {
+        const int a0 = t / nb * 2, b0 = t % nb * 4;
+        int ca[2], cb[4];  // blocks past the end repeat the last one
+#pragma unroll
+        for (int x = 0; x < 2; ++x) ca[x] = 16 * min(a0 + x, g.nv - 1);
+#pragma unroll
+        for (int y = 0; y < 4; ++y) cb[y] = 16 * min(b0 + y, g.nv - 1);
+        v4d acc[2][4];
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) acc[x][y] = (v4d){0, 0, 0, 0};
+        double fa[2][2][2], fb[2][2][4];
+        const double *ri = yi, *rj = yj;
+        auto fetch = [&](int h) {  // eight rows
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                for (int x = 0; x < 2; ++x) fa[h][s][x] = (ri + 4 * s * ldu + ca[x])[off];
+#pragma unroll
+                for (int y = 0; y < 4; ++y) fb[h][s][y] = (rj + 4 * s * ldu + cb[y])[off];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            ri += 8 * ldu;
+            rj += 8 * ldu;
+        };
+        auto products = [&](int h) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+#pragma unroll
+                    for (int y = 0; y < 4; ++y)
+                        acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                            fa[h][s][x], fb[h][s][y], acc[x][y], 0, 0, 0);
+        };
+        fetch(0);
+        for (int k = 0; k < nd; ++k) {
+            fetch(1);
+            products(0);
+            if (k + 1 == nd) ri = yi, rj = yj;  // fetched again and not used
+            fetch(0);
+            products(1);
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+                const int b = 16 * (b0 + y) + r;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int av = 16 * (a0 + x) + 4 * v + gg;
+                    if (av < g.nvir && b < g.nvir) jp[(int64_t)av * g.nvir + b] = acc[x][y][v];
+                }
+            }
     }
 }
 
-size_t fit_batch(size_t npairs, size_t dmax, size_t nvir) {
+// Pairs of one batch, of `per` bytes each: 4 GiB of them.
+size_t fit_batch(size_t npairs, size_t per) {
     size_t nb = 0;
     if (const char *s = std::getenv("FERRIC_FIT_BATCH")) nb = (size_t)std::strtoull(s, nullptr, 10);
-    if (nb == 0) {
-        const size_t per = sizeof(double) * (dmax * dmax + 3 * dmax * nvir) + 64;
-        nb = std::max<size_t>(1, ((size_t)4 << 30) / per);
-    }
+    if (nb == 0) nb = std::max<size_t>(1, ((size_t)4 << 30) / (per + 64));
     return std::min(nb, npairs);
+}
+
+fh_status fit_pairs(State &s, const double *a, const double *v, size_t naux, size_t nocc,
+                    size_t nvir, const std::vector<uint64_t> &near, size_t words,
+                    const int32_t *pairs, size_t npairs, size_t dmax, hipStream_t stream,
+                    double *j_out) {
+    FitArgs g;
+    g.a = a;
+    g.v = v;
+    g.naux = (int64_t)naux;
+    g.nov = (int64_t)(nocc * nvir);
+    g.nvir = (int)nvir;
+    g.nv = (int)((nvir + 15) / 16);
+    g.cap = (int)((dmax + 15) / 16 * 16);
+    g.words = (int)words;
+    const size_t cap = (size_t)g.cap, slot = cap * (cap + 32 * (size_t)g.nv);
+    const size_t nb = fit_batch(npairs, sizeof(double) * slot);
+    const size_t near_bytes = sizeof(uint64_t) * near.size();
+    fh_status st = reserve(s, {{kSlotFitWork, sizeof(double) * nb * slot},
+                               {kSlotFitMeta, near_bytes + sizeof(int32_t) * (npairs * 2 +
+                                                                              nb * (cap + 1))}});
+    if (st != FH_OK) return st;
+    g.u = (double *)s.slots[kSlotFitWork].ptr;
+    uint64_t *dnear = (uint64_t *)s.slots[kSlotFitMeta].ptr;
+    int32_t *dpairs = (int32_t *)(dnear + near.size());
+    g.near = dnear;
+    g.dom = dpairs + 2 * npairs;
+    g.info = g.dom + nb * cap;
+    st = hip_check(hipMemcpyAsync(dnear, near.data(), near_bytes, hipMemcpyHostToDevice, stream),
+                   "H2D domains");
+    if (st != FH_OK) return st;
+    st = hip_check(hipMemcpyAsync(dpairs, pairs, sizeof(int32_t) * 2 * npairs,
+                                  hipMemcpyHostToDevice, stream),
+                   "H2D pairs");
+    if (st != FH_OK) return st;
+    s.pending.h2d_bytes += near_bytes + sizeof(int32_t) * 2 * npairs;
+    std::vector<int32_t> info(nb);
+    mark(s, 0, stream);
+    mark(s, 1, stream);
+    for (size_t p0 = 0; p0 < npairs; p0 += nb) {
+        const size_t n = std::min(nb, npairs - p0);
+        g.pairs = dpairs + 2 * p0;
+        g.j = j_out + p0 * nvir * nvir;
+        hipLaunchKernelGGL(fit_pair_kernel, dim3((unsigned)n), dim3(kFitThreads), 0, stream, g);
+        st = hip_check(hipGetLastError(), "domain fit kernel");
+        if (st != FH_OK) return st;
+        s.pending.kernel_launches += 1;
+        st = hip_check(hipMemcpyAsync(info.data(), g.info, sizeof(int32_t) * n,
+                                      hipMemcpyDeviceToHost, stream),
+                       "D2H Cholesky info");
+        if (st != FH_OK) return st;
+        st = hip_check(hipStreamSynchronize(stream), "stream sync");
+        if (st != FH_OK) return st;
+        for (size_t k = 0; k < n; ++k)
+            if (info[k] != 0)
+                return fail(FH_KERNEL,
+                            "domain metric of pair (%d, %d) is not positive definite (Cholesky "
+                            "info %d)",
+                            pairs[2 * (p0 + k)], pairs[2 * (p0 + k) + 1], info[k]);
+    }
+    mark(s, 2, stream);
+    mark(s, 3, stream);
+    finish_timing(s, (uint64_t)npairs, 0);
+    return FH_OK;
 }
 
 fh_status fit_core(State &s, const double *a, const double *v, size_t naux, size_t nocc,
                    size_t nvir, const double *aux_xyz, const double *centers, double radius,
                    const int32_t *pairs, size_t npairs, hipStream_t stream, double *j_out,
                    size_t *max_domain) {
-    // Domains on the host, in aux order (lmp2_amplitude.rs:1726-1735).
+    // Aux functions near each occupied (lmp2_amplitude.rs:1726-1735), one bit each; a
+    // pair's domain is the union of its two rows, in aux order.
     const double r2 = radius * radius;
-    std::vector<int32_t> sizes(npairs);
-    std::vector<std::vector<int32_t>> doms(npairs);
+    const size_t words = (naux + 63) / 64;
+    std::vector<uint64_t> near(nocc * words, 0);
+    std::vector<char> wanted(nocc, 0);
+    for (size_t k = 0; k < 2 * npairs; ++k) wanted[pairs[k]] = 1;
+    for (size_t i = 0; i < nocc; ++i) {
+        if (!wanted[i]) continue;
+        const double *c = centers + 3 * i;
+        for (size_t p = 0; p < naux; ++p) {
+            const double ux = aux_xyz[3 * p] - c[0], uy = aux_xyz[3 * p + 1] - c[1],
+                         uz = aux_xyz[3 * p + 2] - c[2];
+            double di = 0.0;
+            di += ux * ux;
+            di += uy * uy;
+            di += uz * uz;
+            if (di <= r2) near[i * words + p / 64] |= 1ull << (p % 64);
+        }
+    }
     size_t dmax = 0;
     for (size_t k = 0; k < npairs; ++k) {
         const int32_t i = pairs[2 * k], j = pairs[2 * k + 1];
-        for (size_t p = 0; p < naux; ++p) {
-            double di = 0.0, dj = 0.0;
-            for (int x = 0; x < 3; ++x) {
-                const double ui = aux_xyz[3 * p + x] - centers[3 * (size_t)i + x];
-                const double uj = aux_xyz[3 * p + x] - centers[3 * (size_t)j + x];
-                di += ui * ui;
-                dj += uj * uj;
-            }
-            if (di <= r2 || dj <= r2) doms[k].push_back((int32_t)p);
-        }
-        if (doms[k].empty())
+        size_t d = 0;
+        for (size_t w = 0; w < words; ++w)
+            d += (size_t)__builtin_popcountll(near[i * words + w] | near[j * words + w]);
+        if (d == 0)
             return fail(FH_LAYOUT, "empty aux domain for pair (%d, %d) at radius %g bohr", i, j,
                         radius);
-        sizes[k] = (int32_t)doms[k].size();
-        dmax = std::max(dmax, doms[k].size());
+        dmax = std::max(dmax, d);
     }
     if (max_domain) *max_domain = dmax;
-    std::vector<int32_t> flat(npairs * dmax, 0);
-    for (size_t k = 0; k < npairs; ++k)
-        std::copy(doms[k].begin(), doms[k].end(), flat.begin() + k * dmax);
-
-    const size_t nb = fit_batch(npairs, dmax, nvir);
-    const size_t vmat = dmax * dmax, xmat = dmax * 2 * nvir, wmat = dmax * nvir,
-                 jmat = nvir * nvir;
-    fh_status st = reserve(s, {{kSlotFitWork, sizeof(double) * nb * (vmat + xmat + wmat)},
-                               {kSlotFitMeta, sizeof(int32_t) * (npairs * (dmax + 3) + 2 * nb)}});
-    if (st != FH_OK) return st;
-    double *Vp = (double *)s.slots[kSlotFitWork].ptr;
-    double *X = Vp + nb * vmat;
-    double *W = X + nb * xmat;  // V_DD^-1 A_j
-    int32_t *ddom = (int32_t *)s.slots[kSlotFitMeta].ptr;
-    int32_t *dsz = ddom + npairs * dmax;
-    int32_t *dpairs = dsz + npairs;
-    int32_t *info = dpairs + 2 * npairs;  // Cholesky
-    int32_t *info2 = info + nb;           // inverse
-    st = hip_check(hipMemcpyAsync(ddom, flat.data(), sizeof(int32_t) * flat.size(),
-                                  hipMemcpyHostToDevice, stream),
-                   "H2D domains");
-    if (st != FH_OK) return st;
-    st = hip_check(hipMemcpyAsync(dsz, sizes.data(), sizeof(int32_t) * npairs,
-                                  hipMemcpyHostToDevice, stream),
-                   "H2D domain sizes");
-    if (st != FH_OK) return st;
-    st = hip_check(hipMemcpyAsync(dpairs, pairs, sizeof(int32_t) * 2 * npairs,
-                                  hipMemcpyHostToDevice, stream),
-                   "H2D pairs");
-    if (st != FH_OK) return st;
-    s.pending.h2d_bytes += sizeof(int32_t) * (flat.size() + 3 * npairs);
-
-    void *hv = nullptr;
-    st = blas_handle(s, stream, &hv);
-    if (st != FH_OK) return st;
-    rocblas_handle h = (rocblas_handle)hv;
-    const double one = 1.0, zero = 0.0;
-    const int D = (int)dmax, V = (int)nvir;
-    std::vector<int32_t> hinfo(2 * nb);
-    mark(s, 0, stream);
-    mark(s, 1, stream);
-    for (size_t p0 = 0; p0 < npairs; p0 += nb) {
-        const int n = (int)std::min(nb, npairs - p0);
-        hipLaunchKernelGGL(fit_gather_kernel, dim3(n), dim3(kThreads), 0, stream,
-                           dpairs + 2 * p0, ddom + p0 * dmax, dsz + p0, D, v, (int64_t)naux, a,
-                           (int64_t)(nocc * nvir), V, Vp, X);
-        st = hip_check(hipGetLastError(), "domain gather");
-        if (st != FH_OK) return st;
-        st = solver_ok(rocsolver_dpotrf_strided_batched(h, rocblas_fill_lower, D, Vp, D,
-                                                        (rocblas_stride)vmat, info, n),
-                       "domain metric Cholesky");
-        if (st != FH_OK) return st;
-        // V_DD^-1 from the factor (the reference inverts through the Cholesky
-        // factor too), W = V_DD^-1 A_j on the lower triangle, J = A_i^T W. One
-        // inverse per pair instead of triangular solves on its 2 nvir columns:
-        // 9x faster at dmax 120, nvir 100, the same to rounding.
-        st = solver_ok(rocsolver_dpotri_strided_batched(h, rocblas_fill_lower, D, Vp, D,
-                                                        (rocblas_stride)vmat, info2, n),
-                       "domain metric inverse");
-        if (st != FH_OK) return st;
-        st = solver_ok(rocblas_dsymm_strided_batched(
-                           h, rocblas_side_left, rocblas_fill_lower, D, V, &one, Vp, D,
-                           (rocblas_stride)vmat, X + (size_t)D * V, D, (rocblas_stride)xmat, &zero,
-                           W, D, (rocblas_stride)wmat, n),
-                       "domain inverse product");
-        if (st != FH_OK) return st;
-        // Row-major J[a][b] = sum_r A_i[r, a] W[r, b]: column-major J^T = W^T A_i.
-        st = solver_ok(rocblas_dgemm_strided_batched(
-                           h, rocblas_operation_transpose, rocblas_operation_none, V, V, D, &one,
-                           W, D, (rocblas_stride)wmat, X, D, (rocblas_stride)xmat, &zero,
-                           j_out + p0 * jmat, V, (rocblas_stride)jmat, n),
-                       "domain fit GEMM");
-        if (st != FH_OK) return st;
-        s.pending.kernel_launches += 4;
-        st = hip_check(hipMemcpyAsync(hinfo.data(), info, sizeof(int32_t) * 2 * nb,
-                                      hipMemcpyDeviceToHost, stream),
-                       "D2H Cholesky info");
-        if (st != FH_OK) return st;
-        st = hip_check(hipStreamSynchronize(stream), "stream sync");
-        if (st != FH_OK) return st;
-        for (int k = 0; k < n; ++k)
-            if (hinfo[k] != 0 || hinfo[nb + k] != 0)
-                return fail(FH_KERNEL,
-                            "domain metric of pair (%d, %d) is not positive definite (Cholesky "
-                            "info %d)",
-                            pairs[2 * (p0 + k)], pairs[2 * (p0 + k) + 1], hinfo[k]);
-    }
-    mark(s, 2, stream);
-    mark(s, 3, stream);
-    finish_timing(s, (uint64_t)npairs, 0);
-    return FH_OK;
+    return fit_pairs(s, a, v, naux, nocc, nvir, near, words, pairs, npairs, dmax, stream, j_out);
 }
 
 fh_status fit_checks(size_t naux, size_t nocc, size_t nvir, const double *aux_xyz,
