@@ -62,6 +62,162 @@ __global__ __launch_bounds__(256) void pair_k4_kernel(EnergyArgs a) {
     pair::pair_k4_body<T, TILE, KP, ADJ, false, SIGNED, FLUSH, AMP>(a, decode_item(a), lds);
 }
 
+// FP64 at tile 64, the energies and the amplitude passes: the items, operands and
+// epilogues of pair_k4_body, with 8-deep panels brought into three LDS stages by direct
+// loads two panels ahead, and a panel's fragments read while the products of the one
+// before it run. v_mfma_f64_16x16x4f64 holds a SIMD 64 cycles, so 16 products a wave and
+// panel cover its 8 KB of LDS reads and the barrier; 48 KB and 143 registers let three
+// workgroups share a CU, whose starts, ends and epilogues the other two fill. Where the
+// last tile of the virtuals holds at most two blocks, the four waves take 16 rows each
+// of it instead of leaving half of them idle (209 virtuals: 3 of 10 items).
+// 41/209/960: 1540 us (53 TFLOP/s of products issued, 70% of the issue slots at the
+// 2.09 GHz that the load leaves of 2.4) against 2330 us for the register-staged body
+// (45%, bank conflicts, an LDS write per operand byte, two workgroups); with 16-deep
+// panels in two stages, two workgroups, 1630 us.
+constexpr int kPK = 8, kPBuf = 3;      // panel depth, stages
+constexpr int kPS = 64 * kPK * 8;      // one operand's panel
+constexpr int kPStage = 4 * kPS;
+typedef const __attribute__((address_space(1))) void *GlobalPtr;
+typedef __attribute__((address_space(3))) void *LdsPtr;
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+// Where the chunks of rows 4 x .. 4 x + 3 begin: with slot g ^ spread(x), the 16 lanes of
+// any one pass of a fragment read fall on distinct banks (multiplication by 2 in GF(4)).
+__device__ __forceinline__ int spread(int x) { return ((x << 1) & 3) ^ ((x >> 1) * 3); }
+
+template <bool AMP>
+__global__ __launch_bounds__(256, 3) void pair_f64_kernel(EnergyArgs a) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    constexpr int TILE = 64, NB = 2, kRow = kPK * 8;
+    const pair::Item it = decode_item(a);
+    const int A0 = it.ta * TILE, B0 = it.tb * TILE;
+    const pair::SplitQ sq(it, a.naux_pad, kPK);
+    const int limA = min(TILE, a.nvir_pad - A0), limB = min(TILE, a.nvir_pad - B0);
+    const int lane = threadIdx.x % kWave;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const bool narrow = limB <= 32 && it.ta != it.tb;  // then limA = 64
+    const pair::Lane L{narrow ? A0 + 16 * wid : A0, B0, narrow ? 0 : wid / 2,
+                       narrow ? 0 : wid % 2, lane % 16, lane / 16};
+    bool rv[NB], cv[NB];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+        rv[k] = narrow ? k == 0 : L.wr * 32 + k * 16 < limA;
+        cv[k] = L.wc * 32 + k * 16 < limB;
+    }
+
+    // Operands as in pair_k4_body. A wave stages rows 16 wid .. 16 wid + 15 of each;
+    // rows past the tile's last repeat it, in blocks that no product reads.
+    const double *b = (const double *)a.op0;
+    const int64_t ld = a.naux_pad;
+    const double *src[4] = {
+        b + ((int64_t)it.i * a.nvir_pad + A0) * ld, b + ((int64_t)it.j * a.nvir_pad + B0) * ld,
+        b + ((int64_t)(sq.single ? it.i : it.j) * a.nvir_pad + A0) * ld,
+        b + ((int64_t)(sq.single ? it.j : it.i) * a.nvir_pad + B0) * ld};
+    const int row = 16 * wid + lane / 4;
+    const uint32_t chunk = ((lane % 4) ^ spread(lane / 16)) * 16;
+    const uint32_t offa = (uint32_t)min(row, limA - 1) * (uint32_t)(ld * 8) + chunk;
+    const uint32_t offb = (uint32_t)min(row, limB - 1) * (uint32_t)(ld * 8) + chunk;
+    // Past the last iteration its panels are loaded again and not read. (naux_pad is even
+    // in panels, so a single-product item has its two in every iteration.)
+    uint32_t to = 0;
+    int ahead = 0;
+    auto fetch = [&] {
+        const int q0 = min(ahead++, sq.iters - 1) * sq.step;
+#pragma unroll
+        for (int op = 0; op < 4; ++op) {
+            const char *p = (const char *)(src[op] + (op < 2 ? q0 : q0 + sq.off23));
+            __builtin_amdgcn_global_load_lds((GlobalPtr)(p + (op & 1 ? offb : offa)),
+                                             (LdsPtr)(lds + to + op * kPS + 16 * wid * kRow), 16,
+                                             0, 0);
+        }
+        to = to + kPStage == kPBuf * kPStage ? 0 : to + kPStage;
+    };
+    const uint32_t slot = (uint32_t)(L.g ^ spread(L.r / 4)) * 16;
+    const uint32_t ra = (uint32_t)((narrow ? 16 * wid : L.wr * 32) + L.r) * kRow + slot;
+    const uint32_t rb = (uint32_t)(L.wc * 32 + L.r) * kRow + slot;
+    v2d f0[2][NB], f1[2][NB], f2[2][NB], f3[2][NB];
+    uint32_t cur = 0;
+    auto read = [&](int h) {
+        const char *s = lds + cur;
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+            // the narrow layout's second row block is not used: any row in the stage
+            const uint32_t xa = narrow ? ra : ra + k * 16 * kRow, xb = rb + k * 16 * kRow;
+            f0[h][k] = *(const v2d *)(s + xa);
+            f1[h][k] = *(const v2d *)(s + kPS + xb);
+            f2[h][k] = *(const v2d *)(s + 2 * kPS + xa);
+            f3[h][k] = *(const v2d *)(s + 3 * kPS + xb);
+        }
+        cur = cur + kPStage == kPBuf * kPStage ? 0 : cur + kPStage;
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    v4d acc1[NB][NB], acc2[NB][NB];
+#pragma unroll
+    for (int x = 0; x < NB; ++x)
+#pragma unroll
+        for (int y = 0; y < NB; ++y) acc1[x][y] = acc2[x][y] = (v4d){0, 0, 0, 0};
+    auto products = [&](int h, auto nx, auto ny) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int x = 0; x < decltype(nx)::value; ++x)
+#pragma unroll
+                for (int y = 0; y < decltype(ny)::value; ++y) {
+                    acc1[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(f0[h][x][e], f1[h][y][e],
+                                                                      acc1[x][y], 0, 0, 0);
+                    acc2[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(f2[h][x][e], f3[h][y][e],
+                                                                      acc2[x][y], 0, 0, 0);
+                }
+    };
+    auto meet = [&] {  // the next panel is in, the last one is read by every wave
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto run = [&](auto nx, auto ny) {
+        int f = 0;
+        for (; f + 2 <= sq.iters; f += 2) {
+            meet();
+            fetch();
+            read(1);
+            products(0, nx, ny);
+            meet();
+            fetch();
+            read(0);
+            products(1, nx, ny);
+        }
+        if (f < sq.iters) products(0, nx, ny);
+    };
+    using std::integral_constant;
+    const int nx = rv[1] ? 2 : rv[0] ? 1 : 0, ny = cv[1] ? 2 : cv[0] ? 1 : 0;
+#pragma unroll
+    for (int k = 0; k < kPBuf; ++k) {
+        fetch();
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    read(0);
+    // The same barriers on every side.
+    if (nx == 2 && ny == 2)
+        run(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+    else if (nx == 1 && ny == 2)
+        run(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+    else if (nx == 2 && ny == 1)
+        run(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    else if (nx == 1 && ny == 1)
+        run(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    else
+        run(integral_constant<int, 0>{}, integral_constant<int, 0>{});
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (sq.single)
+        pair::derive_c2<TILE, double>(it, L, acc1, acc2, pair::RowOf<double>{}, (double *)lds);
+    if constexpr (AMP)
+        pair::amp_store<TILE>(a, it, L, acc1, acc2, rv, cv, pair::RowOf<double>{});
+    pair::energy_epilogue<TILE>(a, it, L, acc1, acc2, rv, cv, pair::RowOf<double>{},
+                                pair::NoCorr{});
+}
+
 // Opposite-spin rectangle: item (i, J, tA, tB), J and tB on the beta side;
 // the items of alpha row i are contiguous.
 template <typename T, int TILE, int KP, bool FLUSH = false>
@@ -147,6 +303,15 @@ hipError_t launch_items(K kern, const EnergyArgs &a, hipStream_t st, int threads
     return hipGetLastError();
 }
 
+template <typename K>
+hipError_t launch_f64(K kern, const EnergyArgs &a, hipStream_t st) {
+    if (a.naux_pad < 16 || a.naux_pad % 16 != 0 || a.nvir_pad % 16 != 0 ||
+        64LL * a.naux_pad * 8 > 0xffffffffLL)  // row offsets inside a tile are 32-bit
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kern, dim3((unsigned)a.nitems), dim3(256), kPBuf * kPStage, st, a);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t launch_energy(const EnergyArgs &a, hipStream_t st) {
@@ -155,7 +320,7 @@ hipError_t launch_energy(const EnergyArgs &a, hipStream_t st) {
     if (a.amp.base) {  // FP64 energy that also stores the amplitudes
         if (a.prec != Prec::F64 || a.q_neg < a.naux_pad) return hipErrorInvalidValue;
         if (a.tile == 128) e = launch_items(pair_k4_kernel<double, 128, 16, false, false, false, true>, a, st);
-        else if (a.tile == 64) e = launch_items(pair_k4_kernel<double, 64, 16, false, false, false, true>, a, st);
+        else if (a.tile == 64) e = launch_f64(pair_f64_kernel<true>, a, st);
         else if (a.tile == 32) e = launch_items(pair_k4_kernel<double, 32, 16, false, false, false, true>, a, st);
         return e;
     }
@@ -174,7 +339,7 @@ hipError_t launch_energy(const EnergyArgs &a, hipStream_t st) {
     switch (a.prec) {
     case Prec::F64:
         if (a.tile == 128) e = launch_items(pair_k4_kernel<double, 128, 16, false>, a, st);
-        else if (a.tile == 64) e = launch_items(pair_k4_kernel<double, 64, 16, false>, a, st);
+        else if (a.tile == 64) e = launch_f64(pair_f64_kernel<false>, a, st);
         else if (a.tile == 32) e = launch_items(pair_k4_kernel<double, 32, 16, false>, a, st);
         break;
     case Prec::F32:

@@ -369,11 +369,14 @@ fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, siz
 
 // Which calls run in residue arithmetic (residue.hip), and on what tiles. Measured
 // against the matrix kernel of the same precision (its time / residue time):
-// FP64    past 144 virtuals (one orbital a tile): 24/208/742 1.7, 70/208/889 2.1,
-//         100/200/2400 2.6, 60/450/1800 2.3, 100/900/3600 2.3; at small work the chip
-//         is not full: 14/160/556 1.3, 8/208/691 1.1, 4/340/1100 0.9. With 65 to 128
-//         virtuals two orbitals share a tile: 40/112/486 1.5, 70/128/633 1.6, but
-//         24/112/435 1.0. Fewer virtuals: 70/64/428 0.9.
+// FP64    the chip is full and the rebuild of a product (16 moduli, the same at any aux
+//         count) is small beside it: 24/208/742 1.15, 70/208/889 1.4, 100/200/2400 1.9,
+//         60/450/1800 1.8, 100/900/3600 1.8. Small work: 20/150/529 1.13, 12/160/1100
+//         1.0, 11/250/500 0.8; few pairs: 10/250/1500 1.3, 8/256/1059 below 1. With 65 to
+//         128 virtuals two orbitals share a tile: 60/66/627 1.1, 60/80/420 1.0, 40/112/486
+//         1.1, 20/128/726 0.8. Two tiles: 16/400/919 1.1, 9/400/1600 1.0, and up to 362
+//         virtuals, where a third of the tiles' area is used: 16/300/1633 1.07 but
+//         24/300/900 0.94, 30/280/700 0.9. Fewer than 65 virtuals: below 1.
 // MIXED   24/208/742 1.35, 70/208/889 2.0, 60/450/1800 1.8, 24/160/588 1.15, 40/112/486
 //         1.2, 24/112/435 0.9.
 // INT8X4 stays with its digit slices: ten moduli against their thirteen products gave
@@ -386,7 +389,8 @@ bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, En
     if (nvir <= 64) return false;
     switch (prec) {
     case Prec::F64:
-        if (work < (nvir <= 143 ? 3.5e9 : nocc >= 11 ? 2.5e9 : 8e9)) return false;
+        if (work < (nvir <= 128 || nocc < 11 ? 1e10 : nvir <= 256 ? 5e9 : 3e10)) return false;
+        if (nvir > 256 && nvir <= 362 && naux < 1500) return false;
         break;
     case Prec::MIXED:
         if (work < 5e9) return false;

@@ -289,10 +289,6 @@ hipError_t launch_gamma(const GammaArgs &g, hipStream_t st) {
                        dim3((unsigned)npair, (unsigned)((g.nvir + kTRows - 1) / kTRows)),
                        dim3(256), 0, st, g);
     hipLaunchKernelGGL(gamma_deps_kernel, dim3((unsigned)(g.nocc + g.nvir)), dim3(256), 0, st, g);
-    hipError_t e = hipFuncSetAttribute((const void *)gamma_gemm_kernel,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       kGBuf * kGStage);
-    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(gamma_gemm_kernel, dim3((unsigned)items), dim3(256), kGBuf * kGStage, st,
                        g);
     if (g.splits > 1)

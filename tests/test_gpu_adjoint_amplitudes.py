@@ -2,7 +2,7 @@
 
 Sizes at the edges of its tiles and panels, K slices, both pair kernels, against dense
 FP64 host arithmetic; the row-by-row path, which a pool ceiling selects, against the
-same. Tolerance: Gamma and dE/deps are sums of at most nov = 2665 and nocc^2 nvir
+same. Tolerance: Gamma and dE/deps are sums of at most nov = 3965 and nocc^2 nvir
 products of amplitudes exact to about 1e-13 of the largest; 1e-11 of the largest result
 is the bar of the other FP64 adjoint tests.
 """
@@ -21,8 +21,8 @@ SHAPES = [
     (8, 16, 64),     # one tile exactly, no padding
     (5, 26, 65),     # two (i, a) past a tile, one Q past a tile
     (16, 47, 200),   # K of 47 panels in two slices
-    (41, 65, 600),   # residue pass, two orbitals a tile
-    (12, 145, 900),  # residue pass, three flushes and a remainder
+    (61, 65, 700),   # residue pass, two orbitals a tile
+    (14, 145, 1200), # residue pass, three flushes and a remainder
 ]
 
 

@@ -2,8 +2,8 @@
 
 Against P from dense FP64 amplitudes on the host. Tolerance: the amplitudes are within
 1e-13 of their block's largest (an FP64 product of naux terms and one division), and the two
-sums of up to nocc^2 nvir = 5e5 like-signed terms on the diagonal differ by a few
-2^-53 sqrt(5e5) = 8e-14; 1e-11 of the largest element is the bar of the other density
+sums of up to nocc^2 nvir = 1.6e6 like-signed terms on the diagonal differ by a few
+2^-53 sqrt(1.6e6) = 1.4e-13; 1e-11 of the largest element is the bar of the other density
 tests.
 """
 import numpy as np
@@ -19,9 +19,9 @@ SHAPES = [
     (3, 17, 40),     # one tile each, fewer slices than the reducing groups
     (5, 64, 33),     # the tile exactly full
     (65, 66, 90),    # both densities two tiles, the second nearly empty
-    (41, 65, 600),   # amplitudes from the residue pass: two orbitals a tile
-    (12, 145, 900),  # one orbital a tile
-    (11, 257, 400),  # two tiles
+    (61, 65, 700),   # amplitudes from the residue pass: two orbitals a tile
+    (14, 145, 1200), # one orbital a tile
+    (18, 257, 1500), # two tiles
 ]
 
 

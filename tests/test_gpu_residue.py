@@ -20,14 +20,14 @@ from ferric_amd import Precision, _lib, rimp2, synthetic  # noqa: E402
 from ferric_amd.dlpno import estimate_pair_energies_from_b_ov  # noqa: E402
 
 SHAPES = [
-    (41, 65, 600, 0),    # two orbitals a tile, 5 blocks each, the last group alone
-    (33, 128, 200, 0),   # two orbitals fill a tile
-    (12, 145, 900, 2),   # one orbital a tile, frozen core
-    (12, 256, 300, 0),   # a full tile
-    (11, 257, 400, 0),   # two tiles, 9 and 8 blocks
-    (5, 300, 4608, 0),   # the largest aux count, several workgroups to an item
-    (14, 513, 65, 0),    # three tiles, one row in the second panel
-    (40, 200, 60, 1),    # one panel
+    (60, 65, 700, 0),    # two orbitals a tile, 5 blocks each
+    (41, 128, 400, 0),   # two orbitals fill a tile, the last group alone
+    (14, 145, 1200, 2),  # one orbital a tile, frozen core
+    (13, 256, 430, 0),   # a full tile
+    (18, 257, 1500, 0),  # two tiles, 9 and 8 blocks
+    (9, 300, 4608, 0),   # the largest aux count, several workgroups to an item
+    (43, 513, 65, 0),    # three tiles, one row in the second panel
+    (46, 200, 60, 1),    # one panel
 ]
 
 
@@ -111,7 +111,7 @@ def test_fp64_energy_kappa_rows_and_storage(oracle_mod):
 
 @pytest.mark.parametrize("bad", [np.nan, np.inf])
 def test_non_finite_row_marks_its_pairs_only(bad):
-    nocc, nvir, naux = 14, 209, 300
+    nocc, nvir, naux = 14, 209, 560
     print("residue non-finite", bad, flush=True)
     b, eps = _problem(nocc, nvir, naux, spread=False)
     good = estimate_pair_energies_from_b_ov(torch.from_numpy(b).cuda(), eps, nocc, nvir)
