@@ -256,8 +256,45 @@ __global__ __launch_bounds__(256) void pair_bf16x3_kernel(EnergyArgs a) {
 // pairs (i, j >= i) start at p0 = i*nocc - i(i-1)/2), then an ascending fold
 // over i (the reference's i-ordered serial sum, rimp2.rs:1533-1538).
 // ---------------------------------------------------------------------------
+// The fold is the last row's workgroup's: a launch of its own read the rows one after
+// another (11 us at 41 rows). 0 between launches; the calls that run these kernels hold
+// the library's lock and wait for them.
+__device__ unsigned int rows_done;
+
+__device__ __forceinline__ void fold_rows(const double *rows, int nocc, double *result) {
+    __shared__ double part[256][4];
+    __shared__ unsigned int before;
+    if (threadIdx.x == 0) {
+        __threadfence();  // this row, written by this thread
+        before = atomicAdd(&rows_done, 1u);
+    }
+    __syncthreads();
+    if (before != gridDim.x - 1) return;
+    __threadfence();
+    KSum sum;  // thread 0: e_os, thread 64: e_ss, in row order
+    const bool folds = threadIdx.x % kWave == 0 && threadIdx.x < 2 * kWave;
+    const int c = 2 * (threadIdx.x / kWave);
+    for (int i0 = 0; i0 < nocc; i0 += 256) {
+        const int n = min(256, nocc - i0);
+        if ((int)threadIdx.x < n) {
+            const int64_t i = i0 + threadIdx.x;
+            double v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) part[threadIdx.x][k] = v[k] = rows[4 * i + k];
+            result[2 + 2 * i] = v[0] + v[1];
+            result[3 + 2 * i] = v[2] + v[3];
+        }
+        __syncthreads();
+        if (folds)
+            for (int k = 0; k < n; ++k) sum.merge(part[k][c], part[k][c + 1]);
+        __syncthreads();
+    }
+    if (folds) result[threadIdx.x / kWave] = sum.value();
+    if (threadIdx.x == 0) rows_done = 0;
+}
+
 __global__ __launch_bounds__(256) void reduce_rows_kernel(const double *__restrict__ ip, int nocc,
-                                                          int ntp, double *__restrict__ rows) {
+                                                          int ntp, double *rows, double *result) {
     const int i = blockIdx.x;
     const int64_t p0 = (int64_t)i * nocc - (int64_t)i * (i - 1) / 2;
     const int64_t w0 = p0 * ntp, w1 = (p0 + (nocc - i)) * ntp;
@@ -267,12 +304,13 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const double *__restri
         ss.merge(ip[4 * w + 2], ip[4 * w + 3]);
     }
     pair::block_store(os, ss, 1.0, rows + 4 * i);
+    fold_rows(rows, nocc, result);
 }
 
 // Rectangle rows: items [i*per_row, (i+1)*per_row) belong to alpha row i.
 __global__ __launch_bounds__(256) void reduce_rect_rows_kernel(const double *__restrict__ ip,
-                                                               int64_t per_row,
-                                                               double *__restrict__ rows) {
+                                                               int64_t per_row, int nocc,
+                                                               double *rows, double *result) {
     const int i = blockIdx.x;
     KSum os, ss;
     for (int64_t w = (int64_t)i * per_row + threadIdx.x; w < (int64_t)(i + 1) * per_row;
@@ -281,20 +319,7 @@ __global__ __launch_bounds__(256) void reduce_rect_rows_kernel(const double *__r
         ss.merge(ip[4 * w + 2], ip[4 * w + 3]);
     }
     pair::block_store(os, ss, 1.0, rows + 4 * i);
-}
-
-__global__ void fold_rows_kernel(const double *__restrict__ rows, int nocc,
-                                 double *__restrict__ result) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    KSum os, ss;
-    for (int i = 0; i < nocc; ++i) {
-        os.merge(rows[4 * i], rows[4 * i + 1]);
-        ss.merge(rows[4 * i + 2], rows[4 * i + 3]);
-        result[2 + 2 * i] = rows[4 * i] + rows[4 * i + 1];
-        result[3 + 2 * i] = rows[4 * i + 2] + rows[4 * i + 3];
-    }
-    result[0] = os.value();
-    result[1] = ss.value();
+    fold_rows(rows, nocc, result);
 }
 
 template <typename K>
@@ -427,17 +452,13 @@ hipError_t launch_energy_rect(const EnergyArgs &a, hipStream_t st) {
 hipError_t launch_rect_reduce(const EnergyArgs &a, hipStream_t st) {
     const int64_t per_row = (int64_t)a.nocc_b * a.ntile * a.ntile_b;
     hipLaunchKernelGGL(reduce_rect_rows_kernel, dim3((unsigned)a.nocc), dim3(256), 0, st,
-                       a.item_partials, per_row, a.row_partials);
-    hipLaunchKernelGGL(fold_rows_kernel, dim3(1), dim3(64), 0, st, a.row_partials, a.nocc,
-                       a.result);
+                       a.item_partials, per_row, a.nocc, a.row_partials, a.result);
     return hipGetLastError();
 }
 
 hipError_t launch_energy_reduce(const EnergyArgs &a, hipStream_t st) {
     hipLaunchKernelGGL(reduce_rows_kernel, dim3((unsigned)a.nocc), dim3(256), 0, st,
-                       a.item_partials, a.nocc, a.ntp, a.row_partials);
-    hipLaunchKernelGGL(fold_rows_kernel, dim3(1), dim3(64), 0, st, a.row_partials, a.nocc,
-                       a.result);
+                       a.item_partials, a.nocc, a.ntp, a.row_partials, a.result);
     return hipGetLastError();
 }
 

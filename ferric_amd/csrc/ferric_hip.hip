@@ -183,6 +183,18 @@ void release_all(State &s) {
         b.ptr = nullptr;
         b.bytes = 0;
     }
+    if (s.host) (void)hipHostFree(s.host);
+    s.host = nullptr;
+}
+
+double *host_buffer(State &s, size_t doubles) {
+    if (s.arena || doubles > kHostDoubles) return nullptr;
+    if (!s.host && hipHostMalloc((void **)&s.host, sizeof(double) * kHostDoubles,
+                                 hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+        (void)hipGetLastError();
+        s.host = nullptr;
+    }
+    return s.host;
 }
 
 fh_status hip_check(hipError_t e, const char *what) {
@@ -406,14 +418,20 @@ bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, En
 
 fh_status fetch_result(State &s, const double *dev, size_t nocc, hipStream_t stream,
                        fh_spin_components *out, double *row_partials) {
-    std::vector<double> res(2 + 2 * nocc);
-    fh_status st = hip_check(hipMemcpyAsync(res.data(), dev, sizeof(double) * res.size(),
-                                            hipMemcpyDeviceToHost, stream),
-                             "D2H result");
+    std::vector<double> copy;
+    const double *res = dev;  // already on the host when it is the pinned buffer
+    if (dev != s.host) {
+        copy.resize(2 + 2 * nocc);
+        const fh_status st = hip_check(hipMemcpyAsync(copy.data(), dev,
+                                                      sizeof(double) * copy.size(),
+                                                      hipMemcpyDeviceToHost, stream),
+                                       "D2H result");
+        if (st != FH_OK) return st;
+        res = copy.data();
+    }
+    const fh_status st = hip_check(hipStreamSynchronize(stream), "stream sync");
     if (st != FH_OK) return st;
-    st = hip_check(hipStreamSynchronize(stream), "stream sync");
-    if (st != FH_OK) return st;
-    s.pending.d2h_bytes += sizeof(double) * res.size();
+    s.pending.d2h_bytes += sizeof(double) * (2 + 2 * nocc);
     out->e_os = res[0];
     out->e_ss = res[1];
     out->e_total = res[0] + res[1];
@@ -424,18 +442,36 @@ fh_status fetch_result(State &s, const double *dev, size_t nocc, hipStream_t str
 
 namespace {
 
-// Uploads [eps_occ, eps_vir] of the active orbitals.
+// Where a call's 2 + 2 nocc results go, then its energies: the pinned buffer if it holds
+// both, else null. (Pageable copies of either cost a call about 10 us.)
+double *call_buffer(State &s, size_t nocc, size_t nvir) {
+    return host_buffer(s, 2 + 3 * nocc + nvir);
+}
+
+// Uploads [eps_occ, eps_vir] of the active orbitals; `pack`: left to that kernel when
+// they pass through the pinned buffer.
 fh_status upload_eps(State &s, const double *eps, size_t first_occ, size_t nocc, size_t nocc_total,
-                     size_t nvir, hipStream_t stream) {
-    std::vector<double> e(nocc + nvir);
+                     size_t nvir, hipStream_t stream, PackArgs *pack = nullptr) {
+    std::vector<double> own;
+    double *e = call_buffer(s, nocc, nvir);
+    if (e) {
+        e += 2 + 2 * nocc;
+    } else {
+        own.resize(nocc + nvir);
+        e = own.data();
+    }
     for (size_t i = 0; i < nocc; ++i) e[i] = eps[first_occ + i];
     for (size_t a = 0; a < nvir; ++a) e[nocc + a] = eps[nocc_total + a];
-    fh_status st = hip_check(hipMemcpyAsync(s.slots[kSlotEps].ptr, e.data(),
-                                            sizeof(double) * e.size(), hipMemcpyHostToDevice,
-                                            stream),
-                             "H2D eps");
-    if (st == FH_OK) s.pending.h2d_bytes += sizeof(double) * e.size();
-    return st;
+    s.pending.h2d_bytes += sizeof(double) * (nocc + nvir);
+    if (pack && own.empty()) {
+        pack->eps_src = e;
+        pack->eps_out = (double *)s.slots[kSlotEps].ptr;
+        pack->n_eps = (int)(nocc + nvir);
+        return FH_OK;
+    }
+    return hip_check(hipMemcpyAsync(s.slots[kSlotEps].ptr, e, sizeof(double) * (nocc + nvir),
+                                    hipMemcpyHostToDevice, stream),
+                     "H2D eps");
 }
 
 fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, size_t nocc,
@@ -499,7 +535,8 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     ea.ntp = ra.ntp;
     ea.item_partials = ra.item_partials;
     ea.row_partials = (double *)s.slots[kSlotRows].ptr;
-    ea.result = (double *)s.slots[kSlotResult].ptr;
+    ea.result = call_buffer(s, nocc, nvir);
+    if (!ea.result) ea.result = (double *)s.slots[kSlotResult].ptr;
     mark(s, 1, stream);
     he = launch_residue_energy(ra, stream);
     if (he != hipSuccess) {
@@ -513,7 +550,7 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
         return fail(FH_KERNEL, "reduction kernels: %s", hipGetErrorString(he));
     }
     mark(s, 3, stream);
-    s.pending.kernel_launches += 5;
+    s.pending.kernel_launches += 4;
     st = fetch_result(s, ea.result, nocc, stream, out, row_partials);
     if (st == FH_OK) finish_timing(s, (uint64_t)pl.nitems, pl.tile);
     return st;
@@ -608,11 +645,12 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
             if (st != FH_OK) return st;
         }
     }
-    st = upload_eps(s, eps, first_occ, nocc, nocc_total, nvir, stream);
+    PackArgs pa;
+    st = upload_eps(s, eps, first_occ, nocc, nocc_total, nvir, stream,
+                    prec == Prec::F64 ? &pa : nullptr);
     if (st != FH_OK) return st;
     double *deps = (double *)s.slots[kSlotEps].ptr;
 
-    PackArgs pa;
     pa.b = b_dev;
     pa.in_f32 = in_f32;
     pa.naux = (int)naux;
@@ -640,6 +678,7 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
         pn.b = neg_dev;
         pn.naux = (int)naux_neg;
         pn.naux_pad = pl.naux_pad - q_neg;
+        pn.n_eps = 0;
         pn.out0 = (char *)pa.out0 + (size_t)q_neg * eb;
         he = launch_pack(pa, stream);
         if (he == hipSuccess) he = launch_pack(pn, stream);
@@ -674,7 +713,8 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
     ea.nitems = pl.nitems;
     ea.item_partials = (double *)s.slots[kSlotItems].ptr;
     ea.row_partials = (double *)s.slots[kSlotRows].ptr;
-    ea.result = (double *)s.slots[kSlotResult].ptr;
+    ea.result = call_buffer(s, nocc, nvir);
+    if (!ea.result) ea.result = (double *)s.slots[kSlotResult].ptr;
     ea.q_neg = q_neg;
     if (amp_out) ea.amp = *amp_out;
     mark(s, 1, stream);
@@ -690,7 +730,7 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
         return fail(FH_KERNEL, "reduction kernels: %s", hipGetErrorString(he));
     }
     mark(s, 3, stream);
-    s.pending.kernel_launches += 4;
+    s.pending.kernel_launches += 3;
     st = fetch_result(s, ea.result, nocc, stream, out, row_partials);
     if (st == FH_OK) finish_timing(s, (uint64_t)pl.nitems, pl.tile);
     return st;

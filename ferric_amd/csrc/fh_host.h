@@ -84,6 +84,11 @@ struct State {
     // the requested slots out of it in request order and never allocates.
     char *arena = nullptr;
     size_t arena_bytes = 0, arena_used = 0;
+    // Pinned host memory of kHostDoubles: results written by the reductions and
+    // orbital energies read by the packer, instead of pageable copies. Calls hold `mu`
+    // and end with a stream sync, so it serves one at a time; fh_release_workspace
+    // frees it.
+    double *host = nullptr;
     size_t held_bytes() const;
 };
 
@@ -140,6 +145,10 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
                       const void *neg_dev = nullptr, size_t naux_neg = 0,
                       const AmpOut *amp_out = nullptr, int *ntp_used = nullptr,
                       bool as_noalloc = false);
+constexpr size_t kHostDoubles = 8192;
+// The pinned buffer, or null: more than it holds, the fixed arena (no allocation), or none
+// to be had.
+double *host_buffer(State &s, size_t doubles);
 int compute_units(State &s);  // of the device, asked once; at least 1
 // Residue arithmetic (residue.hip). Tile sides and paddings of a shape, where it may
 // run at all (aux count, forced tiles, fixed arena); whether an energy of this

@@ -93,6 +93,10 @@ struct PackArgs {
     // segment of them (the two factors of a signed kernel); 0 = naux_pad. The
     // segment is naux_pad columns wide and out0 points at its first column.
     int64_t ld = 0;
+    // F64 only: doubles copied to eps_out by the first workgroup (pinned host memory).
+    const double *eps_src = nullptr;
+    double *eps_out = nullptr;
+    int n_eps = 0;
 };
 
 hipError_t launch_pack(const PackArgs &a, hipStream_t st);

@@ -79,7 +79,12 @@ template <typename Tin>
 __global__ __launch_bounds__(256) void pack_f64_kernel(const Tin *__restrict__ b, int64_t nov,
                                                        int naux, int nvir, int nvir_pad,
                                                        int64_t nrows, int naux_pad,
-                                                       double *__restrict__ out, int64_t ld) {
+                                                       double *__restrict__ out, int64_t ld,
+                                                       const double *eps, double *eps_out,
+                                                       int n_eps) {
+    // The orbital energies, by the first workgroup: no copy of their own.
+    if (blockIdx.x == 0 && blockIdx.y == 0)
+        for (int k = threadIdx.x; k < n_eps; k += 256) eps_out[k] = eps[k];
     __shared__ double tile[PT][PT + 1];
     const int tx = threadIdx.x % PT, ty = threadIdx.x / PT;
     const int64_t r0 = (int64_t)blockIdx.x * PT;
@@ -516,7 +521,7 @@ hipError_t launch_pack(const PackArgs &a, hipStream_t st) {
     } while (0)
     switch (a.fmt) {
     case PackFmt::F64:
-        FH_LAUNCH(pack_f64_kernel, (double *)a.out0, ld);
+        FH_LAUNCH(pack_f64_kernel, (double *)a.out0, ld, a.eps_src, a.eps_out, a.n_eps);
         break;
     case PackFmt::F32:
         FH_LAUNCH(pack_f32_kernel, (float *)a.out0, ld);

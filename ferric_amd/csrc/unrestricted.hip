@@ -159,7 +159,7 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
         return fail(FH_KERNEL, "reduction kernels: %s", hipGetErrorString(he));
     }
     mark(s, 3, stream);
-    s.pending.kernel_launches += 7;
+    s.pending.kernel_launches += 6;
     fh_spin_components sc{};
     st = fetch_result(s, ea.result, 0, stream, &sc, nullptr);
     if (st != FH_OK) return st;
