@@ -446,6 +446,79 @@ batched_fp64_kernel(BatchArgs a) {
     }
 }
 
+// ---- a small energy in one launch ----------------------------------------------------
+// The items of one problem, a workgroup each, straight from the caller's B (no packed
+// copy), and the reduction by the workgroup that ends last. Such a call is launches and
+// latencies, not work: water in cc-pVDZ (15 items) is a call of 40 us instead of 46 with
+// the packer and two more launches.
+__device__ unsigned int items_done;  // 0 between launches, which the callers serialise
+
+__global__ __launch_bounds__(256) void small_energy_kernel(SmallEnergyArgs a) {
+    __shared__ __attribute__((aligned(16))) BatchLds64 lds;
+    __shared__ double eps[kSmallOrbitals];
+    __shared__ unsigned int before;
+    for (int k = threadIdx.x; k < a.nocc + a.nvir; k += 256) eps[k] = a.eps[k];
+    BatchArgs ba{};
+    ba.b = a.b;
+    ba.eps = eps;
+    ba.item_partials = a.item_partials;
+    DomDev dm{};
+    dm.nocc = a.nocc;
+    dm.nvir = a.nvir;
+    dm.naux = a.naux;
+    dm.nvir_pad = a.nvir_pad;
+    dm.naux_pad = a.naux_pad;
+    dm.ntile = a.ntile;
+    dm.ntp = a.ntp;
+    EnergyArgs e;
+    energy_args_init(ba, Prec::F64, e);
+    e.kappa = a.kappa;
+    pair::Item it;
+    item_setup(ba, dm, blockIdx.x, it, e);
+    if (a.tile == 64)
+        fp64_item<64>(ba, dm, it, e, lds.t64);
+    else
+        fp64_item<32>(ba, dm, it, e, lds.t32);
+    if (threadIdx.x == 0) {
+        __threadfence();  // the item's partial, written by this thread
+        before = atomicAdd(&items_done, 1u);
+    }
+    __syncthreads();
+    if (before != gridDim.x - 1) return;
+    __threadfence();
+    // Row i's items are contiguous: a wave to a row, then the rows in order.
+    double(*rows)[4] = (double(*)[4]) & lds;
+    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+    for (int i = wid; i < a.nocc; i += 4) {
+        const int p0 = i * a.nocc - i * (i - 1) / 2;
+        const int w1 = (p0 + a.nocc - i) * a.ntp;
+        KSum os, ss;
+        for (int w = p0 * a.ntp + lane; w < w1; w += kWave) {
+            const double *q = a.item_partials + 4 * w;
+            os.merge(q[0], q[1]);
+            ss.merge(q[2], q[3]);
+        }
+        wave_merge(os);
+        wave_merge(ss);
+        if (lane == 0) {
+            rows[i][0] = os.s;
+            rows[i][1] = os.c;
+            rows[i][2] = ss.s;
+            rows[i][3] = ss.c;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 * (unsigned)a.nocc)
+        a.result[2 + threadIdx.x] = rows[threadIdx.x / 2][2 * (threadIdx.x % 2)] +
+                                    rows[threadIdx.x / 2][2 * (threadIdx.x % 2) + 1];
+    if (lane == 0 && wid < 2) {
+        KSum s;
+        for (int i = 0; i < a.nocc; ++i) s.merge(rows[i][2 * wid], rows[i][2 * wid + 1]);
+        a.result[wid] = s.value();
+    }
+    if (threadIdx.x == 0) items_done = 0;
+}
+
 union BatchLdsBf {
     pair::Bf16Lds<64> t64;
     pair::Bf16Lds<32> t32;
@@ -513,6 +586,16 @@ __global__ __launch_bounds__(256) void batched_reduce_kernel(BatchArgs a) {
 }
 
 }  // namespace
+
+hipError_t launch_small_energy(const SmallEnergyArgs &a, hipStream_t st) {
+    const int64_t npairs = (int64_t)a.nocc * (a.nocc + 1) / 2;
+    if (a.nocc < 1 || 2 * a.nocc > 256 || a.nocc + a.nvir > kSmallOrbitals ||
+        (int64_t)a.nocc * a.nvir >= 1 << 22 || (a.tile != 32 && a.tile != 64) ||
+        npairs * a.ntp > kSmallItems)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(small_energy_kernel, dim3((unsigned)(npairs * a.ntp)), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
 
 // ---- plan and graph cache ------------------------------------------------------------
 struct Plan {

@@ -558,6 +558,15 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
 
 }  // namespace
 
+// One launch from the caller's B, or a packed copy and the kernels that stream it. A call
+// in us, packed / one launch: 5/19/84 46/40, 4/24/100 47/36, 16/24/160 47/44, 8/60/250
+// 56/52, 16/60/300 59/59; but past an aux count that hides the packing, or a workgroup
+// per CU, the packed kernels are faster: 5/40/600 66/69, 30/24/200 56/58, 10/100/400
+// 77/82, 16/60/900 84/92.
+static bool small_energy(size_t nvir, size_t naux, const EnergyPlan &pl) {
+    return pl.nitems <= kSmallItems && pl.tile <= 64 && nvir <= 64 && naux <= 256;
+}
+
 fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux, size_t nocc,
                       size_t nvir, const double *eps, size_t first_occ, size_t nocc_total,
                       double kappa, Prec prec, hipStream_t stream, fh_spin_components *out,
@@ -630,6 +639,8 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
         clear_error();
     }
     if (ntp_used) *ntp_used = pl.ntp;
+    const bool small = prec == Prec::F64 && !in_f32 && !signed_k && !amp_out &&
+                       forced_tile() == 0 && small_energy(nvir, naux, pl);
     fh_status st = reserve(s, req);
     if (st != FH_OK) return st;
 
@@ -646,6 +657,38 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
         }
     }
     PackArgs pa;
+    if (small) {
+        st = upload_eps(s, eps, first_occ, nocc, nocc_total, nvir, stream, &pa);
+        if (st != FH_OK) return st;
+        SmallEnergyArgs sa;
+        sa.b = (const double *)b_dev;
+        sa.eps = pa.eps_src ? pa.eps_src : (const double *)s.slots[kSlotEps].ptr;
+        sa.nocc = (int)nocc;
+        sa.nvir = (int)nvir;
+        sa.naux = (int)naux;
+        sa.nvir_pad = pl.nvir_pad;
+        sa.naux_pad = pl.naux_pad;
+        sa.ntile = pl.ntile;
+        sa.ntp = pl.ntp;
+        sa.tile = pl.tile;
+        sa.kappa = kappa;
+        sa.item_partials = (double *)s.slots[kSlotItems].ptr;
+        sa.result = call_buffer(s, nocc, nvir);
+        if (!sa.result) sa.result = (double *)s.slots[kSlotResult].ptr;
+        mark(s, 0, stream);
+        mark(s, 1, stream);
+        const hipError_t he = launch_small_energy(sa, stream);
+        if (he != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(FH_KERNEL, "energy kernel: %s", hipGetErrorString(he));
+        }
+        mark(s, 2, stream);
+        mark(s, 3, stream);
+        s.pending.kernel_launches += 1;
+        st = fetch_result(s, sa.result, nocc, stream, out, row_partials);
+        if (st == FH_OK) finish_timing(s, (uint64_t)pl.nitems, pl.tile);
+        return st;
+    }
     st = upload_eps(s, eps, first_occ, nocc, nocc_total, nvir, stream,
                     prec == Prec::F64 ? &pa : nullptr);
     if (st != FH_OK) return st;

@@ -282,6 +282,17 @@ hipError_t launch_bf16x3_nt(const Bf16x3Gemm &g, hipStream_t st);
 hipError_t launch_energy_rect(const EnergyArgs &a, hipStream_t st);
 hipError_t launch_rect_reduce(const EnergyArgs &a, hipStream_t st);
 // Row reductions and the ascending fold into a.result.
+// A small FP64 energy from the caller's B in one launch (batched.hip).
+constexpr int kSmallItems = 256, kSmallOrbitals = 128;
+struct SmallEnergyArgs {
+    const double *b;    // (naux, nocc nvir) row-major
+    const double *eps;  // nocc occupied, then nvir virtual; device or pinned host
+    int nocc, nvir, naux, nvir_pad, naux_pad, ntile, ntp, tile;
+    double kappa;
+    double *item_partials;  // 4 per item, as EnergyArgs'
+    double *result;         // as EnergyArgs'; device or pinned host
+};
+hipError_t launch_small_energy(const SmallEnergyArgs &a, hipStream_t st);
 hipError_t launch_energy_reduce(const EnergyArgs &a, hipStream_t st);
 
 // Split-K FP64 MFMA product of the MP2 densities from stored amplitudes:
