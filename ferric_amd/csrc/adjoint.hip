@@ -13,7 +13,6 @@
 //   A  pair kernel over (i, j >= i) (energy.hip, adjoint epilogue): recomputes
 //      K_ij, writes T~_ij for this row's pairs into row scratch (tbuf: a-major,
 //      ubuf: b-major per j > i) and per-item t*T~ sums;
-//   R  reduction of this row's energy and dE/deps partials, in a fixed order;
 //   BC one grouped GEMM launch:
 //      B  Gamma_i[Q, a]   += 4 sum_{j >= i, b} B_j[Q, b] T~_ij^ab   (K = (nocc-i) nvir)
 //      C  Gamma_j[Q, b]   += 4 sum_a B_i[Q, a] T~_ij^ab, j > i      (K = nvir)
@@ -28,8 +27,7 @@
 // slabs over the padded (i, a) index space: S (the group's rows, every column
 // from the group on) and St (the transposed blocks of the columns past the
 // group), 2 x R vpg x nocc vpg x 4 bytes (5.5 GB at 100/900/3600 with R = 8,
-// against the 64.8 GB amplitudes the reference holds); the per-row reductions
-// follow; then two hand-written BF16x3 GEMMs (bf16x3_nt_kernel, FP32
+// against the 64.8 GB amplitudes the reference holds); then two BF16x3 GEMMs in one launch (bf16x3_nt_kernel, FP32
 // accumulation) add this group's part of Gamma = 4 B T~ into an FP32 gamma,
 // widened to FP64 at the end.
 #include <hip/hip_runtime.h>
@@ -404,7 +402,7 @@ __global__ __launch_bounds__(256) void gemm_bf16x3_kernel(GemmArgs g) {
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 template <int WN>
-__global__ __launch_bounds__(128 * WN) void bf16x3_nt_kernel(Bf16x3Gemm g) {
+__global__ __launch_bounds__(128 * WN) void bf16x3_nt_kernel(Bf16x3Gemm g0, Bf16x3Gemm g1) {
     constexpr int T = 256, KP = 32;
     constexpr int NT = 128 * WN;        // threads: 2 waves along M x WN along N
     constexpr int WNE = T / WN;         // N extent of one wave
@@ -412,8 +410,12 @@ __global__ __launch_bounds__(128 * WN) void bf16x3_nt_kernel(Bf16x3Gemm g) {
     constexpr int RP = NT / 4;          // tile rows one load instruction covers
     constexpr int LPO = 2 * (T / RP);   // loads per thread per operand (hi and lo)
     __shared__ __attribute__((aligned(16))) v4i lds[2][2][T][8];
+    // The tiles of g0 first, then those of g1.
+    const int64_t tiles0 = (int64_t)((g0.M + T - 1) / T) * ((g0.N + T - 1) / T);
+    const bool second = (int64_t)blockIdx.x >= tiles0;
+    const Bf16x3Gemm g = second ? g1 : g0;
     const int mt = (g.M + T - 1) / T, nt = (g.N + T - 1) / T;
-    const int64_t tile = xcd_remap((int64_t)blockIdx.x, (int64_t)mt * nt);
+    const int64_t tile = xcd_remap((int64_t)blockIdx.x - (second ? tiles0 : 0), (int64_t)mt * nt);
     const int m0 = (int)(tile % mt) * T, n0 = (int)(tile / mt) * T;
     const int tid = threadIdx.x, lane = tid % kWave, wid = tid / kWave;
     const int wm = wid / WN, wn = wid % WN, c = lane % 32, h = lane / 32;
@@ -516,50 +518,85 @@ __global__ __launch_bounds__(128 * WN) void bf16x3_nt_kernel(Bf16x3Gemm g) {
         }
 }
 
-// ---- Row reduction of one batch: energy and dE/deps -------------------------
+// ---- Energy and dE/deps from the items of every row -----------------------------------
 struct AdjRed {
-    int i, nocc, nvir, tile, ntile, ntp, vec_stride;
-    int nchunks, jc;              // pair chunks of the virtual sums (jc pairs each)
-    const double *item_vec;       // (nocc - i) * ntp items
+    int nocc, nvir, tile, ntile, ntp, vec_stride;
+    int jc, nchunks;              // pairs in a chunk of the virtual sums, most chunks of a row
+    const double *item_vec;       // per item, items by pair (i, j >= i) and tile pair
     const double *item_partials;  // 4 per item
-    double *vpart;                // (nchunks, nvir, 2) virtual partial sums of this row
-    double *ppart;                // (npair, 6) per-pair sums of this row
+    double *vpart;                // (nocc, nchunks, nvir, 2) virtual partial sums
+    double *ppart;                // (pairs, 6) per-pair sums
     double *rows;                 // 4 per occupied row
-    double *dvir_s, *dvir_c;      // dE/deps_vir, compensated, accumulated over batches
-    double *docc_s, *docc_c;      // dE/deps_occ
+    double *result;               // e_os, e_ss, dE/deps_occ, dE/deps_vir
 };
 
-// Reduction of one row batch, in two launches with a fixed order:
-//   adjoint_reduce_kernel: blocks [0, nvb*nchunks) sum, for 256 virtual
-//     indices each, the t*T~ row and column sums of one chunk of jc pairs
-//     (f = 1 for j = i, else 2) into vpart; blocks from nvb*nchunks on take one
-//     pair each and sum its items' energy partials and t*T~ totals into ppart
-//     (strided per thread, then a fixed tree);
-//   adjoint_fold_kernel: adds the chunks into dE/deps_vir in chunk order, and
-//     one thread folds the pairs in j order into the row's energy and the
-//     occupied derivatives (dE/deps_i and dE/deps_j: -2 sum_ab t T~ per pair).
+// Three compensated sums of the workgroup's threads -> six doubles at o (thread 0's).
+__device__ __forceinline__ void block_sums(KSum a, KSum b, KSum c, double *o) {
+    wave_merge(a);
+    wave_merge(b);
+    wave_merge(c);
+    __shared__ double red[4][6];
+    const int wid = threadIdx.x / kWave;
+    if (threadIdx.x % kWave == 0) {
+        red[wid][0] = a.s;
+        red[wid][1] = a.c;
+        red[wid][2] = b.s;
+        red[wid][3] = b.c;
+        red[wid][4] = c.s;
+        red[wid][5] = c.c;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < 4; ++w) {
+        a.merge(red[w][0], red[w][1]);
+        b.merge(red[w][2], red[w][3]);
+        c.merge(red[w][4], red[w][5]);
+    }
+    o[0] = a.s;
+    o[1] = a.c;
+    o[2] = b.s;
+    o[3] = b.c;
+    o[4] = c.s;
+    o[5] = c.c;
+}
+
+__device__ __forceinline__ int64_t pair_index(int i, int j, int nocc) {
+    return (int64_t)i * nocc - (int64_t)i * (i - 1) / 2 + (j - i);
+}
+
+// Three launches for all rows, each sum in a fixed order (per row, with one thread to
+// fold the pairs, they took 1.45 ms of the INT8X4 adjoint at 60/450/1800):
+//   adjoint_reduce_kernel, row i = blockIdx.y: blocks [0, nvb nchunks) sum, for 256
+//     virtuals each, the t*T~ row and column sums of one chunk of jc pairs (f = 1 for
+//     j = i, else 2) into vpart; the blocks after them take a pair each and sum its
+//     items' energy partials and t*T~ totals into ppart;
+//   adjoint_fold_kernel: blocks [0, nvb) add a virtual's chunks in row and chunk order;
+//     block nvb + k sums the pairs of occupied k (dE/deps_k: -2 sum t T~ of each) and
+//     the energies of its row;
+//   adjoint_finish_kernel adds the rows in order.
 __global__ __launch_bounds__(256) void adjoint_reduce_kernel(AdjRed r) {
-    const int npair = r.nocc - r.i;
+    const int i = blockIdx.y, npair = r.nocc - i;
     const int nvb = (r.nvir + 255) / 256;
     const int b = blockIdx.x;
+    const int64_t p0 = pair_index(i, i, r.nocc);
     if (b < nvb * r.nchunks) {
         const int ch = b / nvb;
         const int c = (b % nvb) * 256 + threadIdx.x;
-        if (c >= r.nvir) return;
+        if (c >= r.nvir || ch * r.jc >= npair) return;
         const int tc = c / r.tile, off = c % r.tile;
         auto tp_of = [&](int ta, int tb) { return encode_tile_pair(ta, tb, r.ntile); };
         KSum s;
         const int j1 = min(npair, (ch + 1) * r.jc);
         for (int jj = ch * r.jc; jj < j1; ++jj) {
             const double f = jj == 0 ? 1.0 : 2.0;
-            const double *base = r.item_vec + (int64_t)jj * r.ntp * r.vec_stride;
+            const double *base = r.item_vec + (p0 + jj) * r.ntp * r.vec_stride;
             // tile pairs touching tile tc: (tc, u >= tc) by rows, (u <= tc, tc) by columns
             for (int u = 0; u < r.ntile; ++u) {
                 if (u >= tc) s.add(f * base[(int64_t)tp_of(tc, u) * r.vec_stride + off]);
                 if (u <= tc) s.add(f * base[(int64_t)tp_of(u, tc) * r.vec_stride + r.tile + off]);
             }
         }
-        double *o = r.vpart + 2 * ((int64_t)ch * r.nvir + c);
+        double *o = r.vpart + 2 * (((int64_t)i * r.nchunks + ch) * r.nvir + c);
         o[0] = s.s;
         o[1] = s.c;
         return;
@@ -568,103 +605,63 @@ __global__ __launch_bounds__(256) void adjoint_reduce_kernel(AdjRed r) {
     if (jj >= npair) return;
     KSum eos, ess, sp;
     for (int t = threadIdx.x; t < r.ntp; t += 256) {
-        const int64_t item = (int64_t)jj * r.ntp + t;
+        const int64_t item = (p0 + jj) * r.ntp + t;
         const double *ip = r.item_partials + 4 * item;
         eos.merge(ip[0], ip[1]);
         ess.merge(ip[2], ip[3]);
         sp.add(r.item_vec[item * r.vec_stride + 2 * r.tile]);
     }
-    wave_merge(eos);
-    wave_merge(ess);
-    wave_merge(sp);
-    __shared__ double red[4][6];
-    const int wid = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    if (lane == 0) {
-        red[wid][0] = eos.s;
-        red[wid][1] = eos.c;
-        red[wid][2] = ess.s;
-        red[wid][3] = ess.c;
-        red[wid][4] = sp.s;
-        red[wid][5] = sp.c;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        KSum a, e, p;
-        for (int w = 0; w < 4; ++w) {
-            a.merge(red[w][0], red[w][1]);
-            e.merge(red[w][2], red[w][3]);
-            p.merge(red[w][4], red[w][5]);
-        }
-        double *o = r.ppart + 6 * (int64_t)jj;
-        o[0] = a.s;
-        o[1] = a.c;
-        o[2] = e.s;
-        o[3] = e.c;
-        o[4] = p.s;
-        o[5] = p.c;
-    }
+    block_sums(eos, ess, sp, r.ppart + 6 * (p0 + jj));
 }
 
 __global__ __launch_bounds__(256) void adjoint_fold_kernel(AdjRed r) {
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c < r.nvir) {
+    const int nvb = (r.nvir + 255) / 256;
+    if ((int)blockIdx.x < nvb) {
+        const int c = blockIdx.x * 256 + threadIdx.x;
+        if (c >= r.nvir) return;
         KSum s;
-        s.s = r.dvir_s[c];
-        s.c = r.dvir_c[c];
-        for (int ch = 0; ch < r.nchunks; ++ch) {
-            const double *o = r.vpart + 2 * ((int64_t)ch * r.nvir + c);
-            s.merge(o[0], o[1]);
+        for (int i = 0; i < r.nocc; ++i) {
+            const double *o = r.vpart + 2 * ((int64_t)i * r.nchunks * r.nvir + c);
+            const int n = (r.nocc - i + r.jc - 1) / r.jc;
+#pragma unroll 4
+            for (int ch = 0; ch < n; ++ch) s.merge(o[2 * ch * r.nvir], o[2 * ch * r.nvir + 1]);
         }
-        r.dvir_s[c] = s.s;
-        r.dvir_c[c] = s.c;
+        r.result[2 + r.nocc + c] = s.value();
+        return;
     }
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    const int npair = r.nocc - r.i;
-    KSum eos, ess, di;
-    di.s = r.docc_s[r.i];
-    di.c = r.docc_c[r.i];
-    for (int jj = 0; jj < npair; ++jj) {
-        const double *o = r.ppart + 6 * (int64_t)jj;
+    const int k = blockIdx.x - nvb;
+    KSum eos, ess, dk;
+    for (int j = threadIdx.x; j < r.nocc; j += 256) {
+        const double *o = r.ppart + 6 * pair_index(min(j, k), max(j, k), r.nocc);
+        dk.add(-2.0 * (o[4] + o[5]));
+        if (j < k) continue;
         eos.merge(o[0], o[1]);
         ess.merge(o[2], o[3]);
-        const double spair = o[4] + o[5];
-        di.add(-2.0 * spair);
-        if (jj > 0) {
-            const int j = r.i + jj;
-            KSum dj;
-            dj.s = r.docc_s[j];
-            dj.c = r.docc_c[j];
-            dj.add(-2.0 * spair);
-            r.docc_s[j] = dj.s;
-            r.docc_c[j] = dj.c;
-        }
     }
-    r.docc_s[r.i] = di.s;
-    r.docc_c[r.i] = di.c;
-    r.rows[4 * r.i + 0] = eos.s;
-    r.rows[4 * r.i + 1] = eos.c;
-    r.rows[4 * r.i + 2] = ess.s;
-    r.rows[4 * r.i + 3] = ess.c;
+    __shared__ double sums[6];
+    block_sums(eos, ess, dk, sums);
+    if (threadIdx.x == 0) {
+        for (int q = 0; q < 4; ++q) r.rows[4 * k + q] = sums[q];
+        r.result[2 + k] = sums[4] + sums[5];
+    }
 }
 
-__global__ void adjoint_finish_kernel(const double *__restrict__ rows, int nocc, int nvir,
-                                      const double *__restrict__ docc_s,
-                                      const double *__restrict__ docc_c,
-                                      const double *__restrict__ dvir_s,
-                                      const double *__restrict__ dvir_c,
-                                      double *__restrict__ result) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k == 0) {
-        KSum os, ss;
-        for (int i = 0; i < nocc; ++i) {
-            os.merge(rows[4 * i], rows[4 * i + 1]);
-            ss.merge(rows[4 * i + 2], rows[4 * i + 3]);
-        }
-        result[0] = os.value();
-        result[1] = ss.value();
+__global__ __launch_bounds__(256) void adjoint_finish_kernel(AdjRed r) {
+    __shared__ double part[256][4];
+    KSum sum;  // thread 0: e_os, thread 64: e_ss
+    const bool folds = threadIdx.x % kWave == 0 && threadIdx.x < 2 * kWave;
+    const int c = 2 * (threadIdx.x / kWave);
+    for (int i0 = 0; i0 < r.nocc; i0 += 256) {
+        const int n = min(256, r.nocc - i0);
+        if ((int)threadIdx.x < n)
+            for (int q = 0; q < 4; ++q)
+                part[threadIdx.x][q] = r.rows[4 * ((int64_t)i0 + threadIdx.x) + q];
+        __syncthreads();
+        if (folds)
+            for (int k = 0; k < n; ++k) sum.merge(part[k][c], part[k][c + 1]);
+        __syncthreads();
     }
-    if (k < nocc) result[2 + k] = docc_s[k] + docc_c[k];
-    if (k < nvir) result[2 + nocc + k] = dvir_s[k] + dvir_c[k];
+    if (folds) r.result[threadIdx.x / kWave] = sum.value();
 }
 
 // BF16 hi/lo split of FP32 values (hi = RN(x), lo = RN(x - hi), the split of
@@ -707,6 +704,15 @@ void launch_split(const float *x, int64_t nr, int64_t cols, int64_t ld, uint16_t
     hipLaunchKernelGGL(split_bf16_kernel, dim3(blocks), dim3(256), 0, st, x, nr, cols, ld, hi, lo);
 }
 
+// The last gap (16) elements of every run of vpg.
+__global__ __launch_bounds__(256) void clear_gaps_kernel(uint16_t *p, int64_t runs, int vpg,
+                                                         int gap) {
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= runs) return;
+    v4i *q = (v4i *)(p + (k + 1) * vpg - gap);
+    for (int e = 0; e < gap / 8; ++e) q[e] = (v4i){0, 0, 0, 0};
+}
+
 template <typename T>
 void launch_fill(T *p, int64_t n, T v, hipStream_t st) {
     int64_t blocks = std::min<int64_t>((n + 255) / 256, 8192);
@@ -716,13 +722,31 @@ void launch_fill(T *p, int64_t n, T v, hipStream_t st) {
 
 }  // namespace
 
-hipError_t launch_bf16x3_nt(const Bf16x3Gemm &g, hipStream_t st) {
-    if (g.M <= 0 || g.N <= 0 || g.K < 0 || g.K % 32 != 0) return hipErrorInvalidValue;
-    // Byte offsets inside a 256-row tile are 32-bit (raw buffer loads).
-    if ((int64_t)256 * std::max(g.lda, g.ldb) * 2 >= 0x7fffffffLL) return hipErrorInvalidValue;
-    const int64_t tiles = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256);
+// Pairs of a chunk of the virtual sums: at most 16 chunks to a row.
+int adjoint_chunk(size_t nocc) { return (int)std::max<size_t>(4, (nocc + 15) / 16); }
+
+void launch_adjoint_sums(const AdjRed &r, hipStream_t st) {
+    const int nvb = (r.nvir + 255) / 256;
+    hipLaunchKernelGGL(adjoint_reduce_kernel,
+                       dim3((unsigned)(nvb * r.nchunks + r.nocc), (unsigned)r.nocc), dim3(256), 0,
+                       st, r);
+    hipLaunchKernelGGL(adjoint_fold_kernel, dim3((unsigned)(nvb + r.nocc)), dim3(256), 0, st, r);
+    hipLaunchKernelGGL(adjoint_finish_kernel, dim3(1), dim3(256), 0, st, r);
+}
+
+// Two products with outputs apart, the deeper one first; an empty second one has N = 0.
+hipError_t launch_bf16x3_nt(const Bf16x3Gemm &g, const Bf16x3Gemm &h, hipStream_t st) {
+    int64_t tiles = 0;
+    for (const Bf16x3Gemm *p : {&g, &h}) {
+        if (p->M <= 0 || p->N < (p == &g) || p->K < 0 || p->K % 32 != 0)
+            return hipErrorInvalidValue;
+        // Byte offsets inside a 256-row tile are 32-bit (raw buffer loads).
+        if ((int64_t)256 * std::max(p->lda, p->ldb) * 2 >= 0x7fffffffLL)
+            return hipErrorInvalidValue;
+        tiles += (int64_t)((p->M + 255) / 256) * ((p->N + 255) / 256);
+    }
     if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(bf16x3_nt_kernel<4>, dim3((unsigned)tiles), dim3(512), 0, st, g);
+    hipLaunchKernelGGL(bf16x3_nt_kernel<4>, dim3((unsigned)tiles), dim3(512), 0, st, g, h);
     return hipGetLastError();
 }
 
@@ -799,8 +823,8 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
     const size_t rows8 = nocc * (size_t)pl.nvir_pad;
     const int vec_stride = 2 * pl.tile + 2;
     const size_t items = (size_t)pl.nitems;
-    const int nvb = (int)((nvir + 255) / 256);
-    const int nchunks_max = (int)std::min<size_t>(nocc, (size_t)std::max(1, (512 + nvb - 1) / nvb));
+    const int jc = adjoint_chunk(nocc), nchunks = ((int)nocc + jc - 1) / jc;
+    const size_t vpart = 2 * nocc * (size_t)nchunks * nvir;
     std::vector<std::pair<int, size_t>> req = {
         {kSlotOp0, packed_op_bytes(pl, nocc, prec)},
         {kSlotScale, sizeof(int) * rows8},
@@ -812,10 +836,9 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
         {kSlotItems, sizeof(double) * 4 * items},
         {kSlotDeps, sizeof(double) * vec_stride * items},
         {kSlotRows, sizeof(double) * 4 * nocc},
-        {kSlotAcc, sizeof(double) * 2 * (nocc + nvir)},
         {kSlotResult, sizeof(double) * (2 + nocc + nvir)},
         {kSlotScalar, 256},
-        {kSlotRed, sizeof(double) * (2 * (size_t)nchunks_max * nvir + 6 * nocc)},
+        {kSlotRed, sizeof(double) * (vpart + 6 * (nocc * (nocc + 1) / 2))},
     };
     fh_status st = reserve(s, req);
     if (st != FH_OK) return st;
@@ -867,12 +890,15 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
     uint16_t *sthi = slo + slab, *stlo = sthi + slab;
     float *x32 = (float *)s.slots[kSlotG32].ptr;
     launch_split(b2, (int64_t)naux, (int64_t)ncol, (int64_t)ncol, b2hi, b2lo, stream);
-    double *acc = (double *)s.slots[kSlotAcc].ptr;
-    launch_fill<double>(acc, (int64_t)(2 * (nocc + nvir)), 0.0, stream);
     launch_fill<float>(x32, (int64_t)(naux * ncol), 0.0f, stream);
-    // The slabs' padding columns (nvir_pad <= y < vpg) are never written by
-    // phase A and must read as zero: clear both slabs once.
-    launch_fill<uint64_t>((uint64_t *)shi, (int64_t)(slab), (uint64_t)0, stream);
+    // The slabs' padding columns (nvir_pad <= y < vpg) are never written by phase A and
+    // must read as zero. (Padding rows only reach padding columns of x32; the last
+    // group's St, whose rows are shorter, is not read.)
+    if (const int gap = vpg - pl.nvir_pad; gap > 0) {
+        const int64_t runs = (int64_t)(slab / (size_t)vpg) * 4;
+        hipLaunchKernelGGL(clear_gaps_kernel, dim3((unsigned)((runs + 255) / 256)), dim3(256), 0,
+                           stream, shi, runs, vpg, gap);
+    }
     he = hipGetLastError();
     if (he != hipSuccess) return fail(FH_KERNEL, "adjoint set-up kernels: %s", hipGetErrorString(he));
     mark(s, 1, stream);
@@ -918,23 +944,26 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
     rd.ntile = pl.ntile;
     rd.ntp = pl.ntp;
     rd.vec_stride = vec_stride;
+    rd.item_vec = ea.item_vec;
+    rd.item_partials = ea.item_partials;
+    rd.jc = jc;
+    rd.nchunks = nchunks;
     rd.rows = ea.row_partials;
-    rd.docc_s = acc;
-    rd.docc_c = acc + nocc;
-    rd.dvir_s = acc + 2 * nocc;
-    rd.dvir_c = acc + 2 * nocc + nvir;
+    rd.result = ea.result;
     rd.vpart = (double *)s.slots[kSlotRed].ptr;
-    rd.ppart = rd.vpart + 2 * (size_t)nchunks_max * nvir;
+    rd.ppart = rd.vpart + vpart;
     auto first_item = [&](int64_t i) {
         return (i * (int64_t)nocc - i * (i - 1) / 2) * pl.ntp;
     };
 
-    // One group of R occupied rows at a time: phase A writes its T~ slabs, the
-    // per-row reductions follow, then
+    // One group of R occupied rows at a time: phase A writes its T~ slabs, then
     //   GEMM 1: gamma[Q, (i, a)] += 4 sum_{(j, b), j >= g0} B[Q, (j, b)] S[(i, a), (j, b)]
     //   GEMM 2: gamma[Q, (j, b)] += 4 sum_{(i, a) in group} B[Q, (i, a)] St[(j, b), (i, a)],
     //           j >= g1
     // (T~ symmetric: every ordered occupied pair enters gamma once).
+    // Their columns of gamma are apart, so one launch runs both: at 60/450/1800 GEMM 1 has
+    // 120 tiles for 256 CUs but up to 7.5 times the depth, and GEMM 2 fills the rest
+    // (13.4 -> 9.8 ms, 1050 TFLOP/s of the three products).
     for (int g0 = 0; g0 < (int)nocc; g0 += R) {
         const int g1 = std::min<int>((int)nocc, g0 + R);
         ea.g0 = g0;
@@ -945,19 +974,6 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
         he = launch_adjoint_pairs(ea, stream);
         if (he != hipSuccess)
             return fail(FH_KERNEL, "adjoint pair kernel: %s", hipGetErrorString(he));
-        for (int i = g0; i < g1; ++i) {
-            const int64_t first = first_item(i);
-            rd.i = i;
-            rd.item_partials = ea.item_partials + 4 * first;
-            rd.item_vec = ea.item_vec + first * vec_stride;
-            const int npair = (int)nocc - i;
-            rd.nchunks = std::min(npair, nchunks_max);
-            rd.jc = (npair + rd.nchunks - 1) / rd.nchunks;
-            rd.nchunks = (npair + rd.jc - 1) / rd.jc;
-            hipLaunchKernelGGL(adjoint_reduce_kernel, dim3((unsigned)(nvb * rd.nchunks + npair)),
-                               dim3(256), 0, stream, rd);
-            hipLaunchKernelGGL(adjoint_fold_kernel, dim3((unsigned)nvb), dim3(256), 0, stream, rd);
-        }
         Bf16x3Gemm g;
         g.ahi = b2hi + (size_t)g0 * vpg;
         g.alo = b2lo + (size_t)g0 * vpg;
@@ -971,16 +987,14 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
         g.N = (g1 - g0) * vpg;
         g.K = ((int)nocc - g0) * vpg;
         g.alpha = 4.0f;
-        he = launch_bf16x3_nt(g, stream);
-        if (he == hipSuccess && g1 < (int)nocc) {
-            g.bhi = sthi + (size_t)g1 * vpg * ea.ld_st;
-            g.blo = stlo + (size_t)g1 * vpg * ea.ld_st;
-            g.ldb = ea.ld_st;
-            g.c = x32 + (size_t)g1 * vpg;
-            g.N = ((int)nocc - g1) * vpg;
-            g.K = (g1 - g0) * vpg;
-            he = launch_bf16x3_nt(g, stream);
-        }
+        Bf16x3Gemm h = g;
+        h.bhi = sthi + (size_t)g1 * vpg * ea.ld_st;
+        h.blo = stlo + (size_t)g1 * vpg * ea.ld_st;
+        h.ldb = ea.ld_st;
+        h.c = x32 + (size_t)g1 * vpg;
+        h.N = ((int)nocc - g1) * vpg;
+        h.K = (g1 - g0) * vpg;
+        he = launch_bf16x3_nt(g, h, stream);
         if (he != hipSuccess) return fail(FH_KERNEL, "adjoint GEMM: %s", hipGetErrorString(he));
     }
     {
@@ -990,17 +1004,12 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
                            (int)nocc, (int)nvir, vpg, gamma_dev);
     }
     mark(s, 2, stream);
-    {
-        const int n = (int)std::max(nocc, nvir);
-        hipLaunchKernelGGL(adjoint_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                           stream, ea.row_partials, (int)nocc, (int)nvir, rd.docc_s, rd.docc_c,
-                           rd.dvir_s, rd.dvir_c, ea.result);
-    }
+    launch_adjoint_sums(rd, stream);
     he = hipGetLastError();
     if (he != hipSuccess) return fail(FH_KERNEL, "adjoint finish: %s", hipGetErrorString(he));
     mark(s, 3, stream);
     const int ngroups = (int)((nocc + R - 1) / R);
-    s.pending.kernel_launches += 2 * nocc + 3 * ngroups + 8;
+    s.pending.kernel_launches += 2 * ngroups + 9;
     std::vector<double> res(2 + nocc + nvir);
     st = hip_check(hipMemcpyAsync(res.data(), ea.result, sizeof(double) * res.size(),
                                   hipMemcpyDeviceToHost, stream),
@@ -1137,25 +1146,22 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
     const int64_t k0 = (int64_t)nocc * pl.nvir_pad;
     int splits = (int)std::min<int64_t>((512 + nbB - 1) / nbB, std::max<int64_t>(1, k0 / 256));
     splits = std::max(1, splits);
-    const size_t items_max = nocc * (size_t)pl.ntp;
-    // Row reductions: virtual sums in chunks of pairs (enough blocks to spread
-    // over the CUs), one block per pair for the energy and occupied sums.
-    const int nvb = (int)((nvir + 255) / 256);
-    const int nchunks_max = (int)std::min<size_t>(nocc, (size_t)std::max(1, (512 + nvb - 1) / nvb));
+    const size_t items = nocc * (nocc + 1) / 2 * (size_t)pl.ntp;
+    const int jc = adjoint_chunk(nocc), nchunks = ((int)nocc + jc - 1) / jc;
+    const size_t vpart = 2 * nocc * (size_t)nchunks * nvir;
     std::vector<std::pair<int, size_t>> req = {
         {kSlotOp0, op_bytes},
         {kSlotStage2, b2_bytes},
         {kSlotT, t_bytes},
         {kSlotU, u_bytes},
         {kSlotEps, sizeof(double) * (nocc + nvir)},
-        {kSlotItems, sizeof(double) * 4 * items_max},
-        {kSlotDeps, sizeof(double) * (vec_stride * items_max)},
+        {kSlotItems, sizeof(double) * 4 * items},
+        {kSlotDeps, sizeof(double) * (vec_stride * items)},
         {kSlotRows, sizeof(double) * 4 * nocc},
-        {kSlotAcc, sizeof(double) * 2 * (nocc + nvir)},
         {kSlotResult, sizeof(double) * (2 + nocc + nvir)},
         {kSlotScalar, 256},
         {kSlotSplit, sizeof(double) * (size_t)splits * m_pad * pl.nvir_pad},
-        {kSlotRed, sizeof(double) * (2 * (size_t)nchunks_max * nvir + 6 * nocc)},
+        {kSlotRed, sizeof(double) * (vpart + 6 * (nocc * (nocc + 1) / 2))},
     };
     if (prec == Prec::BF16X3) {
         req.push_back({kSlotOp1, op_bytes});
@@ -1217,9 +1223,7 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
                                    pl.nvir_pad, m_pad, (float *)b2);
         }
     }
-    double *acc = (double *)s.slots[kSlotAcc].ptr;
     launch_fill<double>(gamma_dev, (int64_t)naux * (int64_t)(nocc * nvir), 0.0, stream);
-    launch_fill<double>(acc, (int64_t)(2 * (nocc + nvir)), 0.0, stream);
     he = hipGetLastError();
     if (he != hipSuccess) return fail(FH_KERNEL, "adjoint set-up kernels: %s", hipGetErrorString(he));
     mark(s, 1, stream);
@@ -1281,13 +1285,12 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
     rd.vec_stride = vec_stride;
     rd.item_vec = ea.item_vec;
     rd.item_partials = ea.item_partials;
+    rd.jc = jc;
+    rd.nchunks = nchunks;
     rd.rows = ea.row_partials;
-    rd.docc_s = acc;
-    rd.docc_c = acc + nocc;
-    rd.dvir_s = acc + 2 * nocc;
-    rd.dvir_c = acc + 2 * nocc + nvir;
+    rd.result = ea.result;
     rd.vpart = (double *)s.slots[kSlotRed].ptr;
-    rd.ppart = rd.vpart + 2 * (size_t)nchunks_max * nvir;
+    rd.ppart = rd.vpart + vpart;
 
     int64_t total_items = 0;
     for (size_t i = 0; i < nocc; ++i) {
@@ -1296,16 +1299,8 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
         total_items += ea.nitems;
         he = launch_adjoint_pairs(ea, stream);
         if (he != hipSuccess) return fail(FH_KERNEL, "adjoint pair kernel: %s", hipGetErrorString(he));
-        rd.i = (int)i;
-        {
-            const int npair = (int)(nocc - i);
-            rd.nchunks = std::min(npair, nchunks_max);
-            rd.jc = (npair + rd.nchunks - 1) / rd.nchunks;
-            rd.nchunks = (npair + rd.jc - 1) / rd.jc;
-            hipLaunchKernelGGL(adjoint_reduce_kernel, dim3((unsigned)(nvb * rd.nchunks + npair)),
-                               dim3(256), 0, stream, rd);
-            hipLaunchKernelGGL(adjoint_fold_kernel, dim3((unsigned)nvb), dim3(256), 0, stream, rd);
-        }
+        ea.item_partials += 4 * ea.nitems;
+        ea.item_vec += ea.nitems * vec_stride;
         ga.i = (int)i;
         {
             // Same split count for every row (fixed summation structure); the
@@ -1318,16 +1313,11 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
         if (he != hipSuccess) return fail(FH_KERNEL, "adjoint GEMM: %s", hipGetErrorString(he));
     }
     mark(s, 2, stream);
-    {
-        const int n = (int)std::max(nocc, nvir);
-        hipLaunchKernelGGL(adjoint_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                           stream, ea.row_partials, (int)nocc, (int)nvir, rd.docc_s, rd.docc_c,
-                           rd.dvir_s, rd.dvir_c, ea.result);
-    }
+    launch_adjoint_sums(rd, stream);
     he = hipGetLastError();
     if (he != hipSuccess) return fail(FH_KERNEL, "adjoint reduction: %s", hipGetErrorString(he));
     mark(s, 3, stream);
-    s.pending.kernel_launches += 5 * nocc + 6;
+    s.pending.kernel_launches += 3 * nocc + 7;
     std::vector<double> res(2 + nocc + nvir);
     st = hip_check(hipMemcpyAsync(res.data(), ea.result, sizeof(double) * res.size(),
                                   hipMemcpyDeviceToHost, stream),

@@ -30,7 +30,6 @@ enum SlotId {
     kSlotDiag,       // BF16: lo^2 row sums
     kSlotStage2,     // adjoint: Q-major padded copy of B
     kSlotU,          // adjoint: b-major T~ blocks of one row
-    kSlotAcc,        // adjoint: dE/deps accumulators
     kSlotSplit,      // adjoint: split-K partial tiles of phase B
     kSlotRed,        // adjoint: per-row reduction partials
     kSlotDressX,     // dressing: (Q|nu i) half-transformed rows

@@ -277,7 +277,7 @@ struct Bf16x3Gemm {
     int M, N, K;
     float alpha;
 };
-hipError_t launch_bf16x3_nt(const Bf16x3Gemm &g, hipStream_t st);
+hipError_t launch_bf16x3_nt(const Bf16x3Gemm &g, const Bf16x3Gemm &h, hipStream_t st);
 // Opposite-spin rectangle (F64 / F32) and its row reduction + fold.
 hipError_t launch_energy_rect(const EnergyArgs &a, hipStream_t st);
 hipError_t launch_rect_reduce(const EnergyArgs &a, hipStream_t st);
