@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/ferric_hip.h"
@@ -35,137 +36,161 @@ namespace fh {
 namespace {
 
 constexpr int kDT = 64;   // output tile side
-constexpr int kDKP = 16;  // K panel depth
-constexpr int kDLdr = kDKP + 2;  // LDS row stride (doubles): 16 B of padding
+constexpr int kDKP = 8;   // K panel depth
+constexpr int kDBuf = 3;  // LDS stages
+constexpr int kDPS = kDT * kDKP * 8, kDStage = 3 * kDPS;  // bytes of an operand's panel, of all
 
-// Row pointers of the three operands at panel kp (K = kp * 16 .. + 16).
-struct DensRows {
-    const double *a, *b1, *b2;
-};
-
-__device__ __forceinline__ DensRows dens_rows(const DensArgs &d, int64_t kp, int m, int n) {
-    const int64_t vp = d.nvir_pad;
-    const int64_t k0 = kp * kDKP;
-    DensRows r;
-    if (d.mode == DensMode::VV) {
-        const int64_t q = k0 / vp, c = k0 % vp;
-        const int i = (int)(q / d.nocc), j = (int)(q % d.nocc);
-        const int64_t qt = (int64_t)j * d.nocc + i;
-        r.a = d.tamp + (q * vp + m) * vp + c;
-        r.b1 = d.tamp + (q * vp + n) * vp + c;
-        r.b2 = d.tamp + (qt * vp + n) * vp + c;
-    } else {
-        const int64_t blk = vp * vp;
-        const int64_t kk = k0 / blk, f = k0 % blk;
-        r.a = d.tamp + ((int64_t)m * d.nocc + kk) * blk + f;
-        r.b1 = d.tamp + ((int64_t)n * d.nocc + kk) * blk + f;
-        r.b2 = d.tamp + (kk * d.nocc + n) * blk + f;
-    }
-    return r;
-}
-
-// One item = (output tile tm, tn; K slice s). 256 threads: four waves in a
-// 2 x 2 grid, each a 32 x 32 quadrant of 16 x 16 v_mfma_f64_16x16x4 blocks.
-// Per panel each thread stages two 16-byte chunks of A and two of B (each B
-// chunk formed as cd B1 - ce B2 while in registers); double-buffered LDS, one
-// barrier per panel.
-__global__ __launch_bounds__(256) void density_gemm_kernel(DensArgs d) {
-    __shared__ __attribute__((aligned(16))) double lds[2][2][kDT][kDLdr];
+// One 64 x 64 tile over one K slice. v_mfma_f64_16x16x4f64 bounds it (8 a wave and panel,
+// 512 cycles, against 12 KB of operands): A, B1 and B2 come as they are through three LDS
+// stages, loaded directly two panels ahead, and B = cd B1 - ce B2 is formed from the
+// fragments of the next panel while the products of this one run; 36 KB and at most 128
+// registers put four workgroups on a CU. LDS slots as in pair_f64_kernel. Where the last
+// tile's columns are two blocks at most, the four waves take 16 rows each.
+// 41/209: 886 us for both densities; 1384 when the panels went through registers, with
+// their addresses worked out anew for each.
+__global__ __launch_bounds__(256, 4) void density_gemm_kernel(DensArgs d) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    constexpr int kRow = kDKP * 8;
     const int ntp = d.ntile * (d.ntile + 1) / 2;
-    const int64_t item = blockIdx.x;
+    const int64_t item = xcd_remap(blockIdx.x, gridDim.x);
     const int s = (int)(item / ntp);
     int tm, tn;  // both densities are symmetric: the tiles tm <= tn
     decode_tile_pair((int)(item % ntp), d.ntile, tm, tn);
     const int64_t per = (d.kpanels + d.splits - 1) / d.splits;
-    const int64_t p0 = (int64_t)s * per, p1 = min(d.kpanels, p0 + per);
-    const int tid = threadIdx.x, lane = tid % kWave, wid = tid / kWave;
-    const int wr = wid / 2, wc = wid % 2, r = lane % 16, g = lane / 16;
+    const int64_t p0 = std::min(d.kpanels, (int64_t)s * per);
+    const int count = (int)(std::min(d.kpanels, p0 + per) - p0);
+    const int lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int limA = std::min(kDT, d.mdim - tm * kDT), limB = std::min(kDT, d.mdim - tn * kDT);
+    const bool narrow = limB <= 32 && tm != tn;
+    const int rowA = narrow ? 16 * wid : wid / 2 * 32, rowB = narrow ? 0 : wid % 2 * 32;
 
-    // Staging: chunk c in [0, 512) of an operand = (row c / 8, 16-byte piece c % 8).
-    v4d sa[2], sb[2];
-    auto gload = [&](int64_t kp) {
+    // K runs over outer blocks o (VV: the pair (i, j); OO: the shared occupied) of `inner`
+    // contiguous elements. Rows past the end repeat the last one, for elements that the
+    // reduction does not read.
+    const bool vv = d.mode == DensMode::VV;
+    const int64_t vp = d.nvir_pad, blk = vp * vp, inner = vv ? vp : blk;
+    const int row = 16 * wid + lane / 4;
+    const int64_t chunk = ((lane % 4) ^ lds_spread(lane / 16)) * 2;
+    const int64_t ra = tm * kDT + std::min(row, limA - 1), rb = tn * kDT + std::min(row, limB - 1);
+    const int64_t s1 = vv ? vp : d.nocc * blk, s2 = vv ? vp : blk;
+    const int64_t off[3] = {ra * s1 + chunk, rb * s1 + chunk, rb * s2 + chunk};
+    int64_t o = p0 * kDKP / inner, f = p0 * kDKP % inner;
+    int oi = (int)(o / d.nocc), oj = (int)(o % d.nocc);  // VV
+    int ahead = count;
+    uint32_t to = 0;
+    // Past the last panel it is loaded again and not read.
+    auto fetch = [&] {
+        const double *b1 = d.tamp + o * blk + f;
+        const double *b2 =
+            d.tamp + (vv ? (int64_t)oj * d.nocc + oi : o * d.nocc) * blk + f;
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int c = tid + 256 * u;
-            const int row = c / 8, piece = c % 8;
-            const int m = tm * kDT + row, n = tn * kDT + row;
-            v4d va = {0, 0, 0, 0}, vb = {0, 0, 0, 0};
-            if (kp < p1) {
-                const DensRows rr = dens_rows(d, kp, m < d.mdim ? m : 0, n < d.mdim ? n : 0);
-                if (m < d.mdim) {
-                    const double2 x = *(const double2 *)(rr.a + 2 * piece);
-                    va[0] = x.x;
-                    va[1] = x.y;
-                }
-                if (n < d.mdim) {
-                    const double2 y1 = *(const double2 *)(rr.b1 + 2 * piece);
-                    const double2 y2 = *(const double2 *)(rr.b2 + 2 * piece);
-                    vb[0] = d.cd * y1.x - d.ce * y2.x;
-                    vb[1] = d.cd * y1.y - d.ce * y2.y;
+        for (int op = 0; op < 3; ++op)
+            __builtin_amdgcn_global_load_lds((GlobalPtr)((op == 2 ? b2 : b1) + off[op]),
+                                             (LdsPtr)(lds + to + op * kDPS + 16 * wid * kRow), 16,
+                                             0, 0);
+        to = to + kDStage == kDBuf * kDStage ? 0 : to + kDStage;
+        if (--ahead > 0) {
+            f += kDKP;
+            if (f == inner) {
+                f = 0;
+                ++o;
+                if (++oj == d.nocc) {
+                    oj = 0;
+                    ++oi;
                 }
             }
-            sa[u] = va;
-            sb[u] = vb;
         }
     };
-    auto lstore = [&](int buf) {
+    const uint32_t slot = (uint32_t)(g ^ lds_spread(r / 4)) * 16;
+    const uint32_t xa = (uint32_t)(rowA + r) * kRow + slot, xb = (uint32_t)(rowB + r) * kRow + slot;
+    v2d fa[2][2], f1[2][2], f2[2][2];
+    uint32_t cur = 0;
+    auto read = [&](int h) {
+        const char *q = lds + cur;
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int c = tid + 256 * u;
-            const int row = c / 8, piece = c % 8;
-            double *pa = &lds[buf][0][row][2 * piece];
-            double *pb = &lds[buf][1][row][2 * piece];
-            pa[0] = sa[u][0];
-            pa[1] = sa[u][1];
-            pb[0] = sb[u][0];
-            pb[1] = sb[u][1];
+        for (int k = 0; k < 2; ++k) {
+            // the narrow layout's second row block is not used
+            fa[h][k] = *(const v2d *)(q + (narrow ? xa : xa + k * 16 * kRow));
+            f1[h][k] = *(const v2d *)(q + kDPS + xb + k * 16 * kRow);
+            f2[h][k] = *(const v2d *)(q + 2 * kDPS + xb + k * 16 * kRow);
         }
+        cur = cur + kDStage == kDBuf * kDStage ? 0 : cur + kDStage;
+        __builtin_amdgcn_sched_barrier(0);
     };
-
     v4d acc[2][2];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y) acc[x][y] = (v4d){0, 0, 0, 0};
-
-    if (p0 < p1) {
-        gload(p0);
-        lstore(0);
-        __syncthreads();
-        for (int64_t kp = p0; kp < p1; ++kp) {
-            const int cur = (int)((kp - p0) & 1);
-            if (kp + 1 < p1) gload(kp + 1);
-            // lane group g owns k = 4 g .. 4 g + 3 of the panel for A and B alike
+    auto products = [&](int h, auto nx, auto ny) {
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) {
-                double fa[2], fb[2];
+        for (int e = 0; e < 2; ++e)
 #pragma unroll
-                for (int x = 0; x < 2; ++x) fa[x] = lds[cur][0][wr * 32 + x * 16 + r][4 * g + kk];
+            for (int y = 0; y < decltype(ny)::value; ++y) {
+                const double fb = d.cd * f1[h][y][e] - d.ce * f2[h][y][e];
 #pragma unroll
-                for (int y = 0; y < 2; ++y) fb[y] = lds[cur][1][wc * 32 + y * 16 + r][4 * g + kk];
-#pragma unroll
-                for (int x = 0; x < 2; ++x)
-#pragma unroll
-                    for (int y = 0; y < 2; ++y)
-                        acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[x], fb[y], acc[x][y],
-                                                                         0, 0, 0);
+                for (int x = 0; x < decltype(nx)::value; ++x)
+                    acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[h][x][e], fb, acc[x][y], 0,
+                                                                     0, 0);
             }
-            if (kp + 1 < p1) lstore(cur ^ 1);
-            __syncthreads();
+    };
+    auto meet = [&] {  // the next panel is in, the last one is read by every wave
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto run = [&](auto nx, auto ny) {
+        int p = 0;
+        for (; p + 2 <= count; p += 2) {
+            meet();
+            fetch();
+            read(1);
+            products(0, nx, ny);
+            meet();
+            fetch();
+            read(0);
+            products(1, nx, ny);
         }
+        if (p < count) products(0, nx, ny);
+    };
+    using std::integral_constant;
+    const int nx = narrow ? 1 : std::min(2, std::max(0, (limA - rowA + 15) / 16));
+    const int ny = std::min(2, std::max(0, (limB - rowB + 15) / 16));
+    if (count > 0) {  // uniform; an empty slice stores zeros
+#pragma unroll
+        for (int k = 0; k < kDBuf; ++k) {
+            fetch();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        asm volatile("s_waitcnt vmcnt(6)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        read(0);
+        // The same barriers on every side.
+        if (nx == 2 && ny == 2)
+            run(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+        else if (nx == 1 && ny == 2)
+            run(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+        else if (nx == 2 && ny == 1)
+            run(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+        else if (nx == 1 && ny == 1)
+            run(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+        else
+            run(integral_constant<int, 0>{}, integral_constant<int, 0>{});
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     }
     // partial tile, row-major 64 x 64
     double *out = d.partial + item * (int64_t)(kDT * kDT);
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int x = 0; x < 2; ++x) {
+        if (narrow && x == 1) break;
 #pragma unroll
         for (int y = 0; y < 2; ++y)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = wr * 32 + x * 16 + out_row<double>(g, v);
-                const int col = wc * 32 + y * 16 + r;
-                out[row * kDT + col] = acc[x][y][v];
-            }
+            for (int v = 0; v < 4; ++v)
+                out[(rowA + x * 16 + out_row<double>(g, v)) * kDT + rowB + y * 16 + r] =
+                    acc[x][y][v];
+    }
 }
 
 // out[m][n] = out[n][m] = scale * sum over slices s = 0, 1, ... of the tile's partials:
@@ -200,8 +225,11 @@ __global__ __launch_bounds__(64 * kRG) void density_reduce_kernel(DensArgs d) {
 hipError_t launch_density(const DensArgs &d, hipStream_t st) {
     const int ntp = d.ntile * (d.ntile + 1) / 2;
     const int64_t nitems = (int64_t)ntp * d.splits;
-    if (nitems <= 0 || nitems > 0x7fffffffLL || d.mdim <= 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(density_gemm_kernel, dim3((unsigned)nitems), dim3(256), 0, st, d);
+    if (nitems <= 0 || nitems > 0x7fffffffLL || d.mdim <= 0 || d.nvir_pad % kDKP != 0 ||
+        d.kpanels / d.splits >= 0x7fffffffLL)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(density_gemm_kernel, dim3((unsigned)nitems), dim3(256), kDBuf * kDStage, st,
+                       d);
     hipLaunchKernelGGL(density_reduce_kernel, dim3((unsigned)(ntp * (kDT * kDT / 64))),
                        dim3(64 * kRG), 0, st, d);
     return hipGetLastError();
@@ -210,11 +238,11 @@ hipError_t launch_density(const DensArgs &d, hipStream_t st) {
 namespace {
 
 // Slices per output tile: enough items to fill the chip (about 2048), each
-// slice at least 8 panels deep.
+// slice at least 16 panels deep.
 int density_splits(int ntile, int64_t kpanels) {
     const int64_t tiles = (int64_t)ntile * (ntile + 1) / 2;
     int64_t s = std::max<int64_t>(1, 2048 / tiles);
-    s = std::min<int64_t>(s, std::max<int64_t>(1, kpanels / 8));
+    s = std::min<int64_t>(s, std::max<int64_t>(1, kpanels / 16));
     return (int)s;
 }
 

@@ -77,13 +77,6 @@ __global__ __launch_bounds__(256) void pair_k4_kernel(EnergyArgs a) {
 constexpr int kPK = 8, kPBuf = 3;      // panel depth, stages
 constexpr int kPS = 64 * kPK * 8;      // one operand's panel
 constexpr int kPStage = 4 * kPS;
-typedef const __attribute__((address_space(1))) void *GlobalPtr;
-typedef __attribute__((address_space(3))) void *LdsPtr;
-typedef double v2d __attribute__((ext_vector_type(2)));
-
-// Where the chunks of rows 4 x .. 4 x + 3 begin: with slot g ^ spread(x), the 16 lanes of
-// any one pass of a fragment read fall on distinct banks (multiplication by 2 in GF(4)).
-__device__ __forceinline__ int spread(int x) { return ((x << 1) & 3) ^ ((x >> 1) * 3); }
 
 template <bool AMP>
 __global__ __launch_bounds__(256, 3) void pair_f64_kernel(EnergyArgs a) {
@@ -114,7 +107,7 @@ __global__ __launch_bounds__(256, 3) void pair_f64_kernel(EnergyArgs a) {
         b + ((int64_t)(sq.single ? it.i : it.j) * a.nvir_pad + A0) * ld,
         b + ((int64_t)(sq.single ? it.j : it.i) * a.nvir_pad + B0) * ld};
     const int row = 16 * wid + lane / 4;
-    const uint32_t chunk = ((lane % 4) ^ spread(lane / 16)) * 16;
+    const uint32_t chunk = ((lane % 4) ^ lds_spread(lane / 16)) * 16;
     const uint32_t offa = (uint32_t)min(row, limA - 1) * (uint32_t)(ld * 8) + chunk;
     const uint32_t offb = (uint32_t)min(row, limB - 1) * (uint32_t)(ld * 8) + chunk;
     // Past the last iteration its panels are loaded again and not read. (naux_pad is even
@@ -132,7 +125,7 @@ __global__ __launch_bounds__(256, 3) void pair_f64_kernel(EnergyArgs a) {
         }
         to = to + kPStage == kPBuf * kPStage ? 0 : to + kPStage;
     };
-    const uint32_t slot = (uint32_t)(L.g ^ spread(L.r / 4)) * 16;
+    const uint32_t slot = (uint32_t)(L.g ^ lds_spread(L.r / 4)) * 16;
     const uint32_t ra = (uint32_t)((narrow ? 16 * wid : L.wr * 32) + L.r) * kRow + slot;
     const uint32_t rb = (uint32_t)(L.wc * 32 + L.r) * kRow + slot;
     v2d f0[2][NB], f1[2][NB], f2[2][NB], f3[2][NB];

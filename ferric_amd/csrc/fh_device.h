@@ -7,6 +7,10 @@
 namespace fh {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
+// Operands of __builtin_amdgcn_global_load_lds.
+typedef const __attribute__((address_space(1))) void *GlobalPtr;
+typedef __attribute__((address_space(3))) void *LdsPtr;
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef int v8i __attribute__((ext_vector_type(8)));
@@ -38,6 +42,11 @@ template <>
 __device__ __forceinline__ constexpr int out_row<double>(int g, int v) {
     return 4 * v + g;
 }
+
+// FP64 panels of 8 in the LDS, 64-byte rows of four 16-byte chunks: chunk c of row y at
+// slot c ^ lds_spread(y / 4 % 4). The 16 lanes of any one pass of a fragment read, rows
+// of two lane groups, then fall on distinct banks (multiplication by 2 in GF(4)).
+__device__ __forceinline__ int lds_spread(int x) { return ((x << 1) & 3) ^ ((x >> 1) * 3); }
 
 // Compensated (Neumaier) FP64 sum: value() = s + c.
 struct KSum {

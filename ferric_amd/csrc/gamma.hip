@@ -101,9 +101,6 @@ __global__ __launch_bounds__(256) void gamma_deps_kernel(GammaArgs g) {
 // chains of 64 products instead of K / 4.
 constexpr int kGM = 64, kGN = 128, kGK = 16, kGBuf = 3, kFlush = 16;
 constexpr int kGStage = (kGM + kGN) * kGK * 8;
-typedef const __attribute__((address_space(1))) void *GlobalPtr;
-typedef __attribute__((address_space(3))) void *LdsPtr;
-typedef double v2d __attribute__((ext_vector_type(2)));
 
 template <int N>
 __device__ __forceinline__ void gamma_wait() {

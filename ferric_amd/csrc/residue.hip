@@ -256,8 +256,6 @@ __device__ __forceinline__ void meet() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 }
-typedef const __attribute__((address_space(1))) void *GlobalPtr;
-typedef __attribute__((address_space(3))) void *LdsPtr;
 
 // NL: kilobytes each wave fetches per step.
 template <int N, int NX, int NY, int NL>
