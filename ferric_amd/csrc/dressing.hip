@@ -58,10 +58,22 @@ fh_status dress_core(State &s, const double *j3, size_t naux, size_t nao, const 
     const double one = 1.0, zero = 0.0;
     mark(s, 0, stream);
     // 1. X^T (nleft x naux*nao) = C_left^T (nleft x nao) . J^T (nao x naux*nao)
-    st = blas_check(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, (int)nleft,
-                                  (int)(naux * nao), (int)nao, &one, cl, (int)nleft, j3, (int)nao,
-                                  &zero, X, (int)nleft),
-                    "dress GEMM 1");
+    // As one product, rocBLAS takes 128-wide tiles and multiplies the rows past nleft too;
+    // as naux products of one Q each, narrower ones. us, one / many: 250 x 20 x 900 (nao,
+    // nleft, naux) 371/218, 300 x 60 x 1200 692/629, 510 x 60 x 1800 2207/1465, 1000 x 60 x
+    // 1200 4793/2941, but 510 x 65 x 1800 2448/2904, 1000 x 100 x 1200 5136/5482.
+    if (nleft <= 64)
+        st = blas_check(rocblas_dgemm_strided_batched(
+                            h, rocblas_operation_none, rocblas_operation_none, (int)nleft,
+                            (int)nao, (int)nao, &one, cl, (int)nleft, 0, j3, (int)nao,
+                            (rocblas_stride)(nao * nao), &zero, X, (int)nleft,
+                            (rocblas_stride)(nao * nleft), (int)naux),
+                        "dress GEMM 1");
+    else
+        st = blas_check(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, (int)nleft,
+                                      (int)(naux * nao), (int)nao, &one, cl, (int)nleft, j3, (int)nao,
+                                      &zero, X, (int)nleft),
+                        "dress GEMM 1");
     if (st != FH_OK) return st;
     mark(s, 1, stream);
     // 2. per Q: Y_Q^T (nright x nleft) = C_right^T (nright x nao) . X_Q (nao x nleft)
