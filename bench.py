@@ -30,10 +30,12 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 # Useful-FLOP peaks: BF16x3 issues 3 MFMA products per useful one, INT8X4 13
-# INT8 digit products (dense INT8 5.0 POP/s).
-PEAK_TFLOPS = {"FP64": 78.6, "FP32": 157.3, "BF16X3": 2500.0 / 3.0, "FP8_E4M3": 5000.0,
-               "INT8X4": 5000.0 / 13.0}
-ISSUED_PER_USEFUL = {"BF16X3": 3, "INT8X4": 13}
+# INT8 digit products (dense INT8 5.0 POP/s); FP64 and MIXED in residue
+# arithmetic (reported as tile 256) 16 and 10 INT8 products.
+PEAK_TFLOPS = {"FP64": 78.6, "FP32": 157.3, "MIXED": 157.3, "BF16X3": 2500.0 / 3.0,
+               "FP8_E4M3": 5000.0, "INT8X4": 5000.0 / 13.0,
+               "FP64 residue": 5000.0 / 16.0, "MIXED residue": 5000.0 / 10.0}
+ISSUED_PER_USEFUL = {"BF16X3": 3, "INT8X4": 13, "FP64 residue": 16, "MIXED residue": 10}
 HBM_GBS = 8000.0
 
 
@@ -56,7 +58,7 @@ PROBE_LIB = os.path.join(ROOT, "tests", "hip", "build", "libmfma_probe.so")
 # launch); FP64 uses 8 accumulators per wave (three waves per SIMD), the
 # fastest f64 MFMA issue pattern
 RATE_PROBE = {"FP64": (5, 16000), "BF16X3": (2, 30000), "FP8_E4M3": (3, 15000),
-              "INT8X4": (14, 30000)}
+              "INT8X4": (14, 30000), "FP64 residue": (14, 30000), "MIXED residue": (14, 30000)}
 # every probe kind of tests/hip/mfma_probe.hip: (kind, label, iterations)
 ALL_PROBES = [
     (0, "f64 MFMA 16x16x4, 16 acc (1 wave/SIMD)", 8000),
@@ -289,8 +291,9 @@ def main():
         r.update(ms_per_step=ms, contract_ms=c_ms, pack_ms=p_ms, reduce_ms=r_ms, tile=tile,
                  tflops=F / (ms * 1e-3) / 1e12, kernel_tflops=F / (c_ms * 1e-3) / 1e12,
                  dE_vs_fp64=r["E"] - e_ref)
-        if prec.name in ISSUED_PER_USEFUL:
-            r["kernel_tflops_mfma_issued"] = ISSUED_PER_USEFUL[prec.name] * F / (c_ms * 1e-3) / 1e12
+        r["arithmetic"] = arith = prec.name + (" residue" if tile == 256 else "")
+        if arith in ISSUED_PER_USEFUL:
+            r["kernel_tflops_mfma_issued"] = ISSUED_PER_USEFUL[arith] * F / (c_ms * 1e-3) / 1e12
         log(f"{prec.name}: {ms:.2f} ms/step (kernel {c_ms:.2f} ms, pack {p_ms:.2f}, reduce "
             f"{r_ms:.3f}) {r['tflops']:.1f} TFLOP/s  dE {r['dE_vs_fp64']:+.3e}")
 
@@ -595,10 +598,11 @@ def main():
     ok = [v for v in variants if v != Precision.FP64 and abs(res[v.name]["dE_vs_fp64"]) <= 1e-6]
     head = min(ok, key=lambda v: res[v.name]["ms_per_step"]) if ok else Precision.FP64
     h = res[head.name]
-    peak = PEAK_TFLOPS[head.name]
-    sustained = mfma_sustained(head.name)
+    arith = h["arithmetic"]
+    peak = PEAK_TFLOPS[arith]
+    sustained = mfma_sustained(arith)
     if sustained is not None:
-        log(f"sustained {head.name} MFMA rate (register-only probe): {sustained:.1f} TFLOP/s")
+        log(f"sustained {arith} MFMA rate (register-only probe): {sustained:.1f} TFLOP/s")
 
     cpu = None
     if not args.no_cpu_baseline:

@@ -1075,6 +1075,7 @@ static fh_status adjoint_core_amp(State &s, const void *b_dev, fh_dtype b_dtype,
         return fail(FH_KERNEL, "adjoint kernels: %s", hipGetErrorString(he));
     }
     s.pending.kernel_launches += g.splits > 1 ? 5 : 4;
+    mark(s, 3, stream);  // the reduction phase of the timing: all that follows the pairs
     std::vector<double> res(nocc + nvir);
     st = hip_check(hipMemcpyAsync(res.data(), g.deps, sizeof(double) * res.size(),
                                   hipMemcpyDeviceToHost, stream),
@@ -1083,6 +1084,7 @@ static fh_status adjoint_core_amp(State &s, const void *b_dev, fh_dtype b_dtype,
     st = hip_check(hipStreamSynchronize(stream), "stream sync");
     if (st != FH_OK) return st;
     s.pending.d2h_bytes += sizeof(double) * res.size();
+    finish_timing(s, s.last_timing.items, (int)s.last_timing.tile);
     if (deps) {
         for (size_t k = 0; k < n_eps; ++k) deps[k] = 0.0;
         for (size_t i = 0; i < nocc; ++i) deps[first_occ + i] = res[i];

@@ -58,7 +58,11 @@ typedef enum fh_status {
 
 /* Arithmetic of the (ia|jb) contraction. The orbital-energy denominators and
  * the pair-energy sums are FP64 (compensated) in every mode.
- *   FH_FP64     FP64 MFMA, FP64 accumulation (the plain method)
+ *   FH_FP64     FP64 MFMA, FP64 accumulation (the plain method); energies, pair
+ *               energies, unrestricted blocks and amplitudes of large problems in
+ *               residue arithmetic instead: exact products of B rounded to about
+ *               2^-56 of its row's range, from int8 products under 16 moduli, no
+ *               less accurate
  *   FH_FP32     FP32 operands, FP32 MFMA, FP32 accumulation over the whole Q range
  *   FH_MIXED    FP32 operands (RN from the caller's values), FP32 MFMA over Q
  *               panels of at most 64 rows, each panel's sums added into FP64
@@ -66,7 +70,9 @@ typedef enum fh_status {
  *               (f32 storage, b = 64 f32 panel products, f64 panel sum;
  *               crates/ferric-core/src/gpu/mixed.rs:70,122-180); refused
  *               (FH_RANGE) when max|B| > sqrt(FLT_MAX / 64), as the reference's
- *               check_f32_arithmetic_range with b = 64
+ *               check_f32_arithmetic_range with b = 64. Large problems: residue
+ *               arithmetic under 10 moduli on the same FP32 operands, 2^-32 of
+ *               the row's range, no panel sums
  *   FH_BF16X3   BF16 hi/lo split, hi*hi + hi*lo + lo*hi, FP32 accumulation
  *   FH_FP8_E4M3 OCP E4M3 operands with one power-of-two scale per
  *               (64-row Q block, occupied i), FP32 accumulation
