@@ -27,9 +27,9 @@
 // slabs over the padded (i, a) index space: S (the group's rows, every column
 // from the group on) and St (the transposed blocks of the columns past the
 // group), 2 x R vpg x nocc vpg x 4 bytes (5.5 GB at 100/900/3600 with R = 8,
-// against the 64.8 GB amplitudes the reference holds); then two BF16x3 GEMMs in one launch (bf16x3_nt_kernel, FP32
-// accumulation) add this group's part of Gamma = 4 B T~ into an FP32 gamma,
-// widened to FP64 at the end.
+// against the 64.8 GB amplitudes the reference holds); then two BF16x3 GEMMs in one
+// launch (bf16x3_nt_kernel, FP32 accumulation) add this group's part of
+// Gamma = 4 B T~ into an FP32 gamma, widened to FP64 at the end.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

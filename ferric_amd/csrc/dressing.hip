@@ -70,9 +70,9 @@ fh_status dress_core(State &s, const double *j3, size_t naux, size_t nao, const 
                             (rocblas_stride)(nao * nleft), (int)naux),
                         "dress GEMM 1");
     else
-        st = blas_check(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, (int)nleft,
-                                      (int)(naux * nao), (int)nao, &one, cl, (int)nleft, j3, (int)nao,
-                                      &zero, X, (int)nleft),
+        st = blas_check(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none,
+                                      (int)nleft, (int)(naux * nao), (int)nao, &one, cl,
+                                      (int)nleft, j3, (int)nao, &zero, X, (int)nleft),
                         "dress GEMM 1");
     if (st != FH_OK) return st;
     mark(s, 1, stream);

@@ -23,15 +23,15 @@ enum SlotId {
     kSlotResult,     // energies + row values
     kSlotScalar,     // small scalars (absmax)
     kSlotGamma,      // adjoint: FP64 gamma staging for host calls
-    kSlotT,          // adjoint: per-row T~ block
+    kSlotT,          // adjoint: per-row T~ block, or the whole amplitude matrix
     kSlotDeps,       // adjoint: dE/deps partials
     kSlotBatch,      // batched: descriptors and work list
     kSlotBatchOut,   // batched: per-domain partials
     kSlotDiag,       // BF16: lo^2 row sums
     kSlotStage2,     // adjoint: Q-major padded copy of B
-    kSlotU,          // adjoint: b-major T~ blocks of one row
+    kSlotU,          // adjoint: b-major T~ blocks of one row, or B by Q
     kSlotSplit,      // adjoint: split-K partial tiles of phase B
-    kSlotRed,        // adjoint: per-row reduction partials
+    kSlotRed,        // adjoint: reduction partials of all rows
     kSlotDressX,     // dressing: (Q|nu i) half-transformed rows
     kSlotDressY,     // dressing: undressed MO rows (Q|ia)
     kSlotB2Split,    // INT8X4 adjoint: BF16 hi and lo of the Q-major copy of B
@@ -40,14 +40,14 @@ enum SlotId {
     kSlotPairs,      // pair energies: (e_os, e_ss) per unique pair
     kSlotPnoWork,    // PNO: five nvir x nvir matrices and three vectors per batched pair
     kSlotPnoMeta,    // PNO: pair list, per-pair results, masks, GEMM pointer arrays
-    kSlotFitWork,    // domain fits: padded V_DD and [A_i | A_j] per batched pair
-    kSlotFitMeta,    // domain fits: domain index lists, sizes, pairs, Cholesky info
+    kSlotFitWork,    // domain fits: eliminated rows of [V_DD | A_i | A_j] per batched pair
+    kSlotFitMeta,    // domain fits: aux bits per occupied, pairs, domain lists, pivot info
     kSlotGPairs,     // energies from explicit (ia|jb) blocks: the pair list
     kSlotRexpB,      // INT8X4 opposite spin: row exponents of the beta rows
     kSlotDensAmp,    // MP2 densities: amplitude blocks of every ordered occupied pair
     kSlotDensPart,   // MP2 densities: split-K partial tiles
     kSlotDensOut,    // MP2 densities: P_vv (padded) then P_oo
-    kSlotResidue,    // FP64 in residue arithmetic: the workgroups' residue planes
+    kSlotResidue,    // residue arithmetic: the workgroups' residue planes
     kNumSlots
 };
 

@@ -309,10 +309,10 @@ struct DensArgs {
     int nocc, nvir_pad;
     int mdim;             // M = N: nvir_pad (VV) or nocc (OO)
     int ntile;            // 64-wide output tiles per side
-    int64_t kpanels;      // 16-deep K panels in total
+    int64_t kpanels;      // 8-deep K panels in total
     int splits;           // K slices per output tile
     double cd, ce, scale;
-    double *partial;      // (ntile^2 * splits) tiles of 64 x 64
+    double *partial;      // per slice, the ntile (ntile + 1) / 2 tiles of 64 x 64
     double *out;          // (mdim, mdim) row-major
 };
 hipError_t launch_density(const DensArgs &d, hipStream_t st);

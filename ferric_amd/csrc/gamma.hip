@@ -93,12 +93,12 @@ __global__ __launch_bounds__(256) void gamma_deps_kernel(GammaArgs g) {
 // ---- Gamma ------------------------------------------------------------------
 // 64 Q x 128 (i, a) a workgroup of four waves, 64 x 32 each: v_mfma_f64_16x16x4f64 (64
 // cycles each) bounds it: 61 TFLOP/s at 960 Q and 8569 (i, a), 83 to 89% of the issue
-// slots at the 2.05 GHz that the load leaves of 2.4. 32 of them a wave and 16-deep panel meet 24 KB of operands,
-// so that two workgroups per CU draw 12 B a cycle. The panels come through three LDS
-// stages by direct loads up to three panels ahead; a row's 16-byte chunk c lies at slot
-// c ^ (row & 7), so the 16 rows of a fragment read spread over the banks. Every 16
-// panels the sums move into a second set of accumulators, which keeps the rounding at
-// chains of 64 products instead of K / 4.
+// slots at the 2.05 GHz that the load leaves of 2.4. A wave's 32 products a 16-deep panel
+// meet 24 KB of operands, so two workgroups per CU draw 12 B a cycle. The panels come
+// through three LDS stages by direct loads up to three panels ahead; a row's 16-byte
+// chunk c lies at slot c ^ (row & 7), so the 16 rows of a fragment read spread over the
+// banks. Every 16 panels the sums move into a second set of accumulators, which keeps the
+// rounding at chains of 64 products instead of K / 4.
 constexpr int kGM = 64, kGN = 128, kGK = 16, kGBuf = 3, kFlush = 16;
 constexpr int kGStage = (kGM + kGN) * kGK * 8;
 
