@@ -63,23 +63,25 @@ __global__ __launch_bounds__(256) void pair_k4_kernel(EnergyArgs a) {
 }
 
 // FP64 at tile 64, the energies and the amplitude passes: the items, operands and
-// epilogues of pair_k4_body, with 8-deep panels brought into three LDS stages by direct
-// loads two panels ahead, and a panel's fragments read while the products of the one
-// before it run. v_mfma_f64_16x16x4f64 holds a SIMD 64 cycles, so 16 products a wave and
-// panel cover its 8 KB of LDS reads and the barrier; 48 KB and 143 registers let three
-// workgroups share a CU, whose starts, ends and epilogues the other two fill. Where the
-// last tile of the virtuals holds at most two blocks, the four waves take 16 rows each
-// of it instead of leaving half of them idle (209 virtuals: 3 of 10 items).
-// 41/209/960: 1540 us (53 TFLOP/s of products issued, 70% of the issue slots at the
-// 2.09 GHz that the load leaves of 2.4) against 2330 us for the register-staged body
-// (45%, bank conflicts, an LDS write per operand byte, two workgroups); with 16-deep
-// panels in two stages, two workgroups, 1630 us.
-constexpr int kPK = 8, kPBuf = 3;      // panel depth, stages
+// epilogues of pair_k4_body, with 8-deep panels brought into two LDS stages by direct
+// loads, a panel ahead. v_mfma_f64_16x16x4f64 holds a SIMD 64 cycles, so 16 products a
+// wave and panel, for four waves, outlast a load; 32 KB and 118 registers let four
+// workgroups share a CU, and cover one another's LDS reads, barriers, starts, ends and
+// epilogues. The fragments are read before the next panel's loads are issued: the other
+// order waits for the loads to be taken (1549 us). Where the last tile of the virtuals
+// holds at most two blocks, the four waves take 16 rows each of it instead of leaving
+// half of them idle (209 virtuals: 3 of 10 items).
+// 41/209/960: the call takes 1500 us (54 TFLOP/s of products issued at about 2.1 GHz,
+// what the load leaves of 2.4) against 2386 for the register-staged body (45% of the
+// issue slots, bank conflicts, an LDS write per operand byte, two workgroups). Three
+// stages, three workgroups and the next panel's fragments read ahead 1573; 16-deep panels
+// in two stages, two workgroups 1677.
+constexpr int kPK = 8, kPBuf = 2;      // panel depth, stages
 constexpr int kPS = 64 * kPK * 8;      // one operand's panel
 constexpr int kPStage = 4 * kPS;
 
 template <bool AMP>
-__global__ __launch_bounds__(256, 3) void pair_f64_kernel(EnergyArgs a) {
+__global__ __launch_bounds__(256, 4) void pair_f64_kernel(EnergyArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     constexpr int TILE = 64, NB = 2, kRow = kPK * 8;
     const pair::Item it = decode_item(a);
@@ -128,18 +130,18 @@ __global__ __launch_bounds__(256, 3) void pair_f64_kernel(EnergyArgs a) {
     const uint32_t slot = (uint32_t)(L.g ^ lds_spread(L.r / 4)) * 16;
     const uint32_t ra = (uint32_t)((narrow ? 16 * wid : L.wr * 32) + L.r) * kRow + slot;
     const uint32_t rb = (uint32_t)(L.wc * 32 + L.r) * kRow + slot;
-    v2d f0[2][NB], f1[2][NB], f2[2][NB], f3[2][NB];
+    v2d f0[NB], f1[NB], f2[NB], f3[NB];
     uint32_t cur = 0;
-    auto read = [&](int h) {
+    auto read = [&] {
         const char *s = lds + cur;
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
             // the narrow layout's second row block is not used: any row in the stage
             const uint32_t xa = narrow ? ra : ra + k * 16 * kRow, xb = rb + k * 16 * kRow;
-            f0[h][k] = *(const v2d *)(s + xa);
-            f1[h][k] = *(const v2d *)(s + kPS + xb);
-            f2[h][k] = *(const v2d *)(s + 2 * kPS + xa);
-            f3[h][k] = *(const v2d *)(s + 3 * kPS + xb);
+            f0[k] = *(const v2d *)(s + xa);
+            f1[k] = *(const v2d *)(s + kPS + xb);
+            f2[k] = *(const v2d *)(s + 2 * kPS + xa);
+            f3[k] = *(const v2d *)(s + 3 * kPS + xb);
         }
         cur = cur + kPStage == kPBuf * kPStage ? 0 : cur + kPStage;
         __builtin_amdgcn_sched_barrier(0);
@@ -149,48 +151,35 @@ __global__ __launch_bounds__(256, 3) void pair_f64_kernel(EnergyArgs a) {
     for (int x = 0; x < NB; ++x)
 #pragma unroll
         for (int y = 0; y < NB; ++y) acc1[x][y] = acc2[x][y] = (v4d){0, 0, 0, 0};
-    auto products = [&](int h, auto nx, auto ny) {
+    auto products = [&](auto nx, auto ny) {
 #pragma unroll
         for (int e = 0; e < 2; ++e)
 #pragma unroll
             for (int x = 0; x < decltype(nx)::value; ++x)
 #pragma unroll
                 for (int y = 0; y < decltype(ny)::value; ++y) {
-                    acc1[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(f0[h][x][e], f1[h][y][e],
+                    acc1[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(f0[x][e], f1[y][e],
                                                                       acc1[x][y], 0, 0, 0);
-                    acc2[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(f2[h][x][e], f3[h][y][e],
+                    acc2[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(f2[x][e], f3[y][e],
                                                                       acc2[x][y], 0, 0, 0);
                 }
     };
     auto meet = [&] {  // the next panel is in, the last one is read by every wave
         __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
     auto run = [&](auto nx, auto ny) {
-        int f = 0;
-        for (; f + 2 <= sq.iters; f += 2) {
+        for (int f = 0; f < sq.iters; ++f) {
             meet();
+            read();
             fetch();
-            read(1);
-            products(0, nx, ny);
-            meet();
-            fetch();
-            read(0);
-            products(1, nx, ny);
+            products(nx, ny);
         }
-        if (f < sq.iters) products(0, nx, ny);
     };
     using std::integral_constant;
     const int nx = rv[1] ? 2 : rv[0] ? 1 : 0, ny = cv[1] ? 2 : cv[0] ? 1 : 0;
-#pragma unroll
-    for (int k = 0; k < kPBuf; ++k) {
-        fetch();
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    read(0);
+    fetch();
     // The same barriers on every side.
     if (nx == 2 && ny == 2)
         run(integral_constant<int, 2>{}, integral_constant<int, 2>{});
