@@ -482,7 +482,7 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     ResidueSpace sp;
     fh_status st = reserve_residue(
         s, prec, pl.nitems, pl.ntile > 1 ? 2 : 1, nocc * (size_t)pl.nvir_pad, pl.naux_pad,
-        {{kSlotStage2, sizeof(double) * (size_t)(pl.naux_pad / 64) * nocc * nvir},
+        {{kSlotColMax, sizeof(double) * (size_t)(pl.naux_pad / 64) * nocc * nvir},
          {kSlotEps, sizeof(double) * (nocc + nvir)},
          {kSlotItems, sizeof(double) * 4 * npairs * (size_t)pl.ntp},
          {kSlotRows, sizeof(double) * 4 * nocc},
@@ -515,7 +515,7 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     ord.nocc = ra.ngroup;
     ord.ntp = pl.ntp;
     mark(s, 0, stream);
-    hipError_t he = launch_residue_pack(prec, pa, ord, (double *)s.slots[kSlotStage2].ptr, stream);
+    hipError_t he = launch_residue_pack(prec, pa, ord, (double *)s.slots[kSlotColMax].ptr, stream);
     if (he != hipSuccess) {
         (void)hipGetLastError();
         return fail(FH_KERNEL, "pack kernel: %s", hipGetErrorString(he));

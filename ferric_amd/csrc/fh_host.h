@@ -48,6 +48,8 @@ enum SlotId {
     kSlotDensPart,   // MP2 densities: split-K partial tiles
     kSlotDensOut,    // MP2 densities: P_vv (padded) then P_oo
     kSlotResidue,    // residue arithmetic: the workgroups' residue planes
+    kSlotColMax,     // residue arithmetic: column maxima of B per Q panel (the packer's; no
+                     // entry stages an input here, as some do in kSlotStage and kSlotStage2)
     kNumSlots
 };
 

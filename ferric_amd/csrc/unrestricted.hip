@@ -64,7 +64,7 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
     ResidueSpace sp;
     fh_status st = reserve_residue(
         s, Prec::F64, npairs * ntp, 1, rows_a + rows_b, pa.naux_pad,
-        {{kSlotStage2, sizeof(double) * (size_t)np * (col_a + col_b)},
+        {{kSlotColMax, sizeof(double) * (size_t)np * (col_a + col_b)},
          {kSlotEps, sizeof(double) * neps},
          {kSlotItems, sizeof(double) * 4 * (size_t)(npairs * ntp)},
          {kSlotRows, sizeof(double) * 4 * ca.nocc},
@@ -117,7 +117,7 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
     pk.naux_pad = pa.naux_pad;
     pk.out0 = sp.op;
     const int64_t nrg = (int64_t)(rows_a + rows_b) / 16;
-    double *pmax = (double *)s.slots[kSlotStage2].ptr;
+    double *pmax = (double *)s.slots[kSlotColMax].ptr;
     mark(s, 0, stream);
     pk.b = ba;
     pk.nocc = ra.nocc;
