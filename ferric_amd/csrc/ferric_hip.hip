@@ -452,18 +452,18 @@ double *call_buffer(State &s, size_t nocc, size_t nvir) {
 // they pass through the pinned buffer.
 fh_status upload_eps(State &s, const double *eps, size_t first_occ, size_t nocc, size_t nocc_total,
                      size_t nvir, hipStream_t stream, PackArgs *pack = nullptr) {
-    std::vector<double> own;
     double *e = call_buffer(s, nocc, nvir);
-    if (e) {
+    const bool pinned = e != nullptr;
+    if (pinned) {
         e += 2 + 2 * nocc;
     } else {
-        own.resize(nocc + nvir);
-        e = own.data();
+        s.eps_up.resize(nocc + nvir);
+        e = s.eps_up.data();
     }
     for (size_t i = 0; i < nocc; ++i) e[i] = eps[first_occ + i];
     for (size_t a = 0; a < nvir; ++a) e[nocc + a] = eps[nocc_total + a];
     s.pending.h2d_bytes += sizeof(double) * (nocc + nvir);
-    if (pack && own.empty()) {
+    if (pack && pinned) {
         pack->eps_src = e;
         pack->eps_out = (double *)s.slots[kSlotEps].ptr;
         pack->n_eps = (int)(nocc + nvir);

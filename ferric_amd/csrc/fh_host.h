@@ -90,6 +90,9 @@ struct State {
     // and end with a stream sync, so it serves one at a time; fh_release_workspace
     // frees it.
     double *host = nullptr;
+    // Orbital energies on their way to the device where `host` does not take them: the
+    // copy reads them until the call's stream sync.
+    std::vector<double> eps_up;
     size_t held_bytes() const;
 };
 
