@@ -1055,7 +1055,8 @@ static fh_status adjoint_core_amp(State &s, const void *b_dev, fh_dtype b_dtype,
         s, {{kSlotT, sizeof(double) * nov * ld},
             {kSlotU, sizeof(double) * naux * ld},
             {kSlotDeps, sizeof(double) * (nov * nocc + nocc + nvir)},
-            {kSlotSplit, g.splits > 1 ? sizeof(double) * (size_t)g.splits * naux * nov : 256}});
+            {kSlotSplit, g.splits > 1 ? sizeof(double) * (size_t)g.splits * naux * nov : 256}},
+        true);
     if (st != FH_OK) return st;
     const AmpOut amp{(double *)s.slots[kSlotT].ptr, (int64_t)(nvir * ld), (int64_t)nvir,
                      (int64_t)ld, (int)nvir};
@@ -1104,13 +1105,12 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
         return adjoint_core_i8(s, b_dev, b_dtype, naux, nocc, nvir, eps, n_eps, first_occ,
                                nocc_total, c_os, c_ss, stream, out, gamma_dev, deps);
     if (f64 && nocc * nvir <= kGammaBytes / sizeof(double) / (size_t)gamma_ld(nocc * nvir)) {
-        const uint64_t full = s.stats.fail_pool_full;
+        const Attempt attempt(s);
         const fh_status ast =
             adjoint_core_amp(s, b_dev, b_dtype, naux, nocc, nvir, eps, n_eps, first_occ,
                              nocc_total, c_os, c_ss, stream, out, gamma_dev, deps);
         if (ast != FH_POOL_FULL) return ast;
-        s.stats.fail_pool_full = full;
-        clear_error();
+        attempt.undo();
     }
     const Prec gprec = f64 ? Prec::F64 : Prec::BF16X3;
     EnergyPlan pl = plan_energy(nocc, nvir, naux, prec);

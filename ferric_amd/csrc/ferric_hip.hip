@@ -121,10 +121,32 @@ size_t State::held_bytes() const {
     return t;
 }
 
-// Grow-only named device buffers. All sizes of a call are reserved together,
-// before any transfer; a call whose total would exceed the ceiling is refused
-// without allocating anything.
-fh_status reserve(State &s, const std::vector<std::pair<int, size_t>> &req) {
+// Frees the slots for which pred(k) holds; captured graphs bake in workspace pointers and go
+// with them. Whether there were any.
+template <typename Pred>
+static bool free_slots(State &s, Pred pred) {
+    bool any = false;
+    for (int k = 0; k < kNumSlots; ++k) {
+        if (!s.slots[k].ptr || !pred(k)) continue;
+        if (!any) release_graphs(s);
+        any = true;
+        (void)hipFree(s.slots[k].ptr);
+        s.slots[k] = Slot{};
+    }
+    return any;
+}
+
+// Gives back the spare slots that do not belong to the present call.
+static bool give_back(State &s) {
+    return free_slots(
+        s, [&](int k) { return s.slots[k].spare && !(s.pending.slots >> k & 1); });
+}
+
+// Named device buffers, kept between calls and grown when a call needs more. All sizes of a
+// call are reserved together, before any transfer; a call whose total would exceed the
+// ceiling is refused without allocating anything. Slots that a spare reservation grew are
+// the exception to both: they count only as long as there is room for them.
+fh_status reserve(State &s, const std::vector<std::pair<int, size_t>> &req, bool spare) {
     if (s.arena) {
         // Fixed-arena mode: 256-byte aligned slices in request order, no
         // allocation, no pool accounting.
@@ -144,35 +166,46 @@ fh_status reserve(State &s, const std::vector<std::pair<int, size_t>> &req) {
     size_t limit = 0;
     fh_status st = resolve_pool_limit(s, &limit);
     if (st != FH_OK) return st;
-    size_t total = 0;
-    for (int k = 0; k < kNumSlots; ++k) {
-        size_t want = s.slots[k].bytes;
-        for (const auto &r : req)
-            if (r.first == k) want = std::max(want, r.second);
-        total += want;
-    }
+    auto total_of = [&] {
+        size_t total = 0;
+        for (int k = 0; k < kNumSlots; ++k) {
+            size_t want = s.slots[k].bytes;
+            for (const auto &r : req)
+                if (r.first == k) want = std::max(want, r.second);
+            total += want;
+        }
+        return total;
+    };
+    size_t total = total_of();
+    if (total > limit && give_back(s)) total = total_of();
     if (total > limit)
         return fail(FH_POOL_FULL,
                     "workspace of %.3f GB exceeds the device pool ceiling of %.3f GB",
                     total / 1e9, limit / 1e9);
-    for (const auto &r : req) {
-        Slot &b = s.slots[r.first];
-        if (b.bytes >= r.second) continue;
-        // Captured graphs bake in workspace pointers: drop them on any move.
-        release_graphs(s);
-        if (b.ptr) {
-            (void)hipFree(b.ptr);
-            b.ptr = nullptr;
-            b.bytes = 0;
+    for (bool retry = true;; retry = false) {
+        uint64_t grown = 0;
+        size_t missing = 0;
+        for (const auto &r : req) {
+            Slot &b = s.slots[r.first];
+            if (b.bytes >= r.second) continue;
+            free_slots(s, [&](int k) { return k == r.first; });
+            const size_t n = std::max<size_t>(r.second, 256);
+            if (hipMalloc(&b.ptr, n) != hipSuccess) {
+                b.ptr = nullptr;
+                (void)hipGetLastError();
+                missing = n;
+                break;
+            }
+            b.bytes = n;
+            b.spare = spare;
+            grown |= (uint64_t)1 << r.first;
         }
-        size_t n = std::max<size_t>(r.second, 256);
-        if (hipMalloc(&b.ptr, n) != hipSuccess) {
-            b.ptr = nullptr;
-            (void)hipGetLastError();
-            return fail(FH_POOL_FULL, "hipMalloc of %zu bytes failed", n);
-        }
-        b.bytes = n;
+        if (missing == 0) break;
+        if (spare) free_slots(s, [&](int k) { return grown >> k & 1; });
+        if (!retry || !give_back(s))
+            return fail(FH_POOL_FULL, "hipMalloc of %zu bytes failed", missing);
     }
+    for (const auto &r : req) s.pending.slots |= (uint64_t)1 << r.first;
     s.stats.pool_peak_bytes = std::max<uint64_t>(s.stats.pool_peak_bytes, s.held_bytes());
     return FH_OK;
 }
@@ -180,8 +213,7 @@ fh_status reserve(State &s, const std::vector<std::pair<int, size_t>> &req) {
 void release_all(State &s) {
     for (auto &b : s.slots) {
         if (b.ptr) (void)hipFree(b.ptr);
-        b.ptr = nullptr;
-        b.bytes = 0;
+        b = Slot{};
     }
     if (s.host) (void)hipHostFree(s.host);
     s.host = nullptr;
@@ -357,7 +389,7 @@ fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, siz
     more.push_back({kSlotOp0, rows * (size_t)naux_pad * residue_moduli(prec)});
     more.push_back({kSlotScale, sizeof(int) * rows});
     more.push_back({kSlotResidue, planes + sizeof(int) * ((size_t)words + (size_t)nitems)});
-    const fh_status st = reserve(s, more);
+    const fh_status st = reserve(s, more, true);
     if (st != FH_OK) return st;
     out->op = (int8_t *)s.slots[kSlotOp0].ptr;
     out->rexp = (int *)s.slots[kSlotScale].ptr;
@@ -627,7 +659,7 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
     EnergyPlan rpl;
     if (!signed_k && !(as_noalloc && carved <= (size_t)FH_NOALLOC_SCRATCH_BYTES) &&
         plan_residue(s, nocc, nvir, naux, prec, &rpl)) {
-        const uint64_t full = s.stats.fail_pool_full;
+        const Attempt attempt(s);
         const fh_status rst =
             residue_energy(s, b_dev, in_f32, naux, nocc, nvir, eps, first_occ, nocc_total, kappa,
                            prec, stream, out, row_partials, rpl, amp_out);
@@ -635,8 +667,7 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
         // Its larger workspace may be past the pool ceiling: then the matrix kernel
         // below, which needs half the operand (or less) and no scratch.
         if (rst != FH_POOL_FULL) return rst;
-        s.stats.fail_pool_full = full;
-        clear_error();
+        attempt.undo();
     }
     if (ntp_used) *ntp_used = pl.ntp;
     const bool small = prec == Prec::F64 && !in_f32 && !signed_k && !amp_out &&

@@ -56,11 +56,14 @@ enum SlotId {
 struct Slot {
     void *ptr = nullptr;
     size_t bytes = 0;
+    bool spare = false;  // grown for a route that has another behind it (reserve)
 };
 
 struct Pending {
     uint64_t h2d_bytes = 0, d2h_bytes = 0, kernel_launches = 0;
+    uint64_t slots = 0;  // bit k: slot k belongs to this call
 };
+static_assert(kNumSlots <= 64, "Pending::slots is one word");
 
 struct GraphCache;  // batched.hip
 
@@ -119,7 +122,23 @@ State &state();
 fh_status fail(fh_status st, const char *fmt, ...);
 void clear_error();
 fh_status ensure_device(State &s);
-fh_status reserve(State &s, const std::vector<std::pair<int, size_t>> &req);
+// spare: for a route that has another behind it. What it grows is given back as soon as a
+// later call, or that other route, does not fit beside it, so that no call is refused for
+// the sake of a faster route's workspace.
+fh_status reserve(State &s, const std::vector<std::pair<int, size_t>> &req, bool spare = false);
+// A route with another behind it: undo() after its FH_POOL_FULL, before the other is tried.
+// The failure is not counted, and the slots it reserved no longer belong to the call.
+struct Attempt {
+    State &s;
+    uint64_t full, slots;
+    explicit Attempt(State &st)
+        : s(st), full(st.stats.fail_pool_full), slots(st.pending.slots) {}
+    void undo() const {
+        s.stats.fail_pool_full = full;
+        s.pending.slots = slots;
+        clear_error();
+    }
+};
 void release_all(State &s);
 fh_status hip_check(hipError_t e, const char *what);
 fh_status check_shapes(size_t naux, size_t nocc, size_t nvir, size_t n_eps, size_t first_occ,

@@ -60,7 +60,7 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
     const size_t neps = ca.nocc + ca.nvir + cb.nocc + cb.nvir;
     const int np = pa.naux_pad / 64;
     const size_t col_a = ca.nocc * ca.nvir, col_b = cb.nocc * cb.nvir;
-    const uint64_t full = s.stats.fail_pool_full;
+    const Attempt attempt(s);
     ResidueSpace sp;
     fh_status st = reserve_residue(
         s, Prec::F64, npairs * ntp, 1, rows_a + rows_b, pa.naux_pad,
@@ -71,8 +71,7 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
          {kSlotResult, sizeof(double) * (2 + 2 * ca.nocc)}},
         &sp);
     if (st == FH_POOL_FULL) {  // the matrix kernel needs half of it
-        s.stats.fail_pool_full = full;
-        clear_error();
+        attempt.undo();
         return FH_OK;
     }
     *taken = true;
