@@ -518,14 +518,16 @@ __global__ __launch_bounds__(128 * WN) void bf16x3_nt_kernel(Bf16x3Gemm g0, Bf16
         }
 }
 
-// ---- Energy and dE/deps from the items of every row -----------------------------------
+// ---- Energy and dE/deps from the items of rows r0 .. r1 - 1 ----------------------------
 struct AdjRed {
     int nocc, nvir, tile, ntile, ntp, vec_stride;
+    int r0, r1;
     int jc, nchunks;              // pairs in a chunk of the virtual sums, most chunks of a row
-    const double *item_vec;       // per item, items by pair (i, j >= i) and tile pair
+    const double *item_vec;       // per item, items by pair (i, j >= i) and tile pair, from r0
     const double *item_partials;  // 4 per item
-    double *vpart;                // (nocc, nchunks, nvir, 2) virtual partial sums
+    double *vpart;                // (rows, nchunks, nvir, 2) virtual partial sums
     double *ppart;                // (pairs, 6) per-pair sums
+    double *acc;                  // dE/deps_occ, dE/deps_vir of the rows before r0, compensated
     double *rows;                 // 4 per occupied row
     double *result;               // e_os, e_ss, dE/deps_occ, dE/deps_vir
 };
@@ -564,21 +566,22 @@ __device__ __forceinline__ int64_t pair_index(int i, int j, int nocc) {
     return (int64_t)i * nocc - (int64_t)i * (i - 1) / 2 + (j - i);
 }
 
-// Three launches for all rows, each sum in a fixed order (per row, with one thread to
-// fold the pairs, they took 1.45 ms of the INT8X4 adjoint at 60/450/1800):
-//   adjoint_reduce_kernel, row i = blockIdx.y: blocks [0, nvb nchunks) sum, for 256
+// Two launches for a batch of rows and one at the end, each sum in a fixed order (per row,
+// with one thread to fold the pairs, they took 1.45 ms of the INT8X4 adjoint at 60/450/1800).
+// A batch is every row, or one where the sums of all of them do not fit the pool:
+//   adjoint_reduce_kernel, row i = r0 + blockIdx.y: blocks [0, nvb nchunks) sum, for 256
 //     virtuals each, the t*T~ row and column sums of one chunk of jc pairs (f = 1 for
 //     j = i, else 2) into vpart; the blocks after them take a pair each and sum its
 //     items' energy partials and t*T~ totals into ppart;
 //   adjoint_fold_kernel: blocks [0, nvb) add a virtual's chunks in row and chunk order;
-//     block nvb + k sums the pairs of occupied k (dE/deps_k: -2 sum t T~ of each) and
-//     the energies of its row;
+//     block nvb + k - r0 sums the pairs of occupied k (dE/deps_k: -2 sum t T~ of each)
+//     and the energies of its row;
 //   adjoint_finish_kernel adds the rows in order.
 __global__ __launch_bounds__(256) void adjoint_reduce_kernel(AdjRed r) {
-    const int i = blockIdx.y, npair = r.nocc - i;
+    const int i = r.r0 + blockIdx.y, npair = r.nocc - i;
     const int nvb = (r.nvir + 255) / 256;
     const int b = blockIdx.x;
-    const int64_t p0 = pair_index(i, i, r.nocc);
+    const int64_t p0 = pair_index(i, i, r.nocc) - pair_index(r.r0, r.r0, r.nocc);
     if (b < nvb * r.nchunks) {
         const int ch = b / nvb;
         const int c = (b % nvb) * 256 + threadIdx.x;
@@ -596,7 +599,7 @@ __global__ __launch_bounds__(256) void adjoint_reduce_kernel(AdjRed r) {
                 if (u <= tc) s.add(f * base[(int64_t)tp_of(u, tc) * r.vec_stride + r.tile + off]);
             }
         }
-        double *o = r.vpart + 2 * (((int64_t)i * r.nchunks + ch) * r.nvir + c);
+        double *o = r.vpart + 2 * (((int64_t)blockIdx.y * r.nchunks + ch) * r.nvir + c);
         o[0] = s.s;
         o[1] = s.c;
         return;
@@ -616,23 +619,38 @@ __global__ __launch_bounds__(256) void adjoint_reduce_kernel(AdjRed r) {
 
 __global__ __launch_bounds__(256) void adjoint_fold_kernel(AdjRed r) {
     const int nvb = (r.nvir + 255) / 256;
+    const int64_t p0 = pair_index(r.r0, r.r0, r.nocc);
+    auto before = [&](int k) {  // the sum up to r0
+        KSum s;
+        if (r.r0 > 0) {
+            s.s = r.acc[2 * k];
+            s.c = r.acc[2 * k + 1];
+        }
+        return s;
+    };
+    auto after = [&](int k, const KSum &s) {
+        r.acc[2 * k] = s.s;
+        r.acc[2 * k + 1] = s.c;
+        r.result[2 + k] = s.value();
+    };
     if ((int)blockIdx.x < nvb) {
         const int c = blockIdx.x * 256 + threadIdx.x;
         if (c >= r.nvir) return;
-        KSum s;
-        for (int i = 0; i < r.nocc; ++i) {
-            const double *o = r.vpart + 2 * ((int64_t)i * r.nchunks * r.nvir + c);
+        KSum s = before(r.nocc + c);
+        for (int i = r.r0; i < r.r1; ++i) {
+            const double *o = r.vpart + 2 * ((int64_t)(i - r.r0) * r.nchunks * r.nvir + c);
             const int n = (r.nocc - i + r.jc - 1) / r.jc;
 #pragma unroll 4
             for (int ch = 0; ch < n; ++ch) s.merge(o[2 * ch * r.nvir], o[2 * ch * r.nvir + 1]);
         }
-        r.result[2 + r.nocc + c] = s.value();
+        after(r.nocc + c, s);
         return;
     }
-    const int k = blockIdx.x - nvb;
+    // Pairs (i, j) of the batch's rows i that k is in; rows below r0 have none.
+    const int k = r.r0 + blockIdx.x - nvb;
     KSum eos, ess, dk;
-    for (int j = threadIdx.x; j < r.nocc; j += 256) {
-        const double *o = r.ppart + 6 * pair_index(min(j, k), max(j, k), r.nocc);
+    for (int j = r.r0 + threadIdx.x; j < (k < r.r1 ? r.nocc : r.r1); j += 256) {
+        const double *o = r.ppart + 6 * (pair_index(min(j, k), max(j, k), r.nocc) - p0);
         dk.add(-2.0 * (o[4] + o[5]));
         if (j < k) continue;
         eos.merge(o[0], o[1]);
@@ -640,10 +658,12 @@ __global__ __launch_bounds__(256) void adjoint_fold_kernel(AdjRed r) {
     }
     __shared__ double sums[6];
     block_sums(eos, ess, dk, sums);
-    if (threadIdx.x == 0) {
+    if (threadIdx.x != 0) return;
+    if (k < r.r1)
         for (int q = 0; q < 4; ++q) r.rows[4 * k + q] = sums[q];
-        r.result[2 + k] = sums[4] + sums[5];
-    }
+    KSum s = before(k);
+    s.merge(sums[4], sums[5]);
+    after(k, s);
 }
 
 __global__ __launch_bounds__(256) void adjoint_finish_kernel(AdjRed r) {
@@ -722,16 +742,24 @@ void launch_fill(T *p, int64_t n, T v, hipStream_t st) {
 
 }  // namespace
 
-// Pairs of a chunk of the virtual sums: at most 16 chunks to a row.
-int adjoint_chunk(size_t nocc) { return (int)std::max<size_t>(4, (nocc + 15) / 16); }
+// Pairs of a chunk of the virtual sums: at most 16 chunks to a row, and 512 blocks of 256
+// virtuals.
+int adjoint_chunk(size_t nocc, size_t nvir) {
+    const size_t nvb = (nvir + 255) / 256, most = std::min<size_t>(16, (512 + nvb - 1) / nvb);
+    return (int)std::max<size_t>(4, (nocc + most - 1) / most);
+}
 
-void launch_adjoint_sums(const AdjRed &r, hipStream_t st) {
+// Rows r0 .. r1 - 1; the last batch ends the call's sums.
+void launch_adjoint_sums(AdjRed r, int r0, int r1, hipStream_t st) {
+    r.r0 = r0;
+    r.r1 = r1;
     const int nvb = (r.nvir + 255) / 256;
     hipLaunchKernelGGL(adjoint_reduce_kernel,
-                       dim3((unsigned)(nvb * r.nchunks + r.nocc), (unsigned)r.nocc), dim3(256), 0,
-                       st, r);
-    hipLaunchKernelGGL(adjoint_fold_kernel, dim3((unsigned)(nvb + r.nocc)), dim3(256), 0, st, r);
-    hipLaunchKernelGGL(adjoint_finish_kernel, dim3(1), dim3(256), 0, st, r);
+                       dim3((unsigned)(nvb * r.nchunks + r.nocc - r0), (unsigned)(r1 - r0)),
+                       dim3(256), 0, st, r);
+    hipLaunchKernelGGL(adjoint_fold_kernel, dim3((unsigned)(nvb + r.nocc - r0)), dim3(256), 0, st,
+                       r);
+    if (r1 == r.nocc) hipLaunchKernelGGL(adjoint_finish_kernel, dim3(1), dim3(256), 0, st, r);
 }
 
 // Two products with outputs apart, the deeper one first; an empty second one has N = 0.
@@ -802,6 +830,21 @@ static int i8_adjoint_rows(size_t nocc) {
     return (int)std::min<size_t>(nocc, (size_t)r);
 }
 
+// Reserves `req`, which holds the sums of one row at a time, and `all`, which holds those of
+// every row and so takes two launches instead of two a row, where the pool has room for it.
+// *batch, nocc on entry: the rows at a time.
+static fh_status reserve_sums(State &s, const std::vector<std::pair<int, size_t>> &req,
+                              const std::vector<std::pair<int, size_t>> &all, size_t *batch) {
+    fh_status st = reserve(s, req);
+    if (st != FH_OK) return st;
+    const Attempt attempt(s);
+    st = reserve(s, all, true);
+    if (st != FH_POOL_FULL) return st;
+    attempt.undo();
+    *batch = 1;
+    return reserve(s, req);
+}
+
 static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux,
                                  size_t nocc, size_t nvir, const double *eps, size_t n_eps,
                                  size_t first_occ, size_t nocc_total, double c_os, double c_ss,
@@ -823,8 +866,8 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
     const size_t rows8 = nocc * (size_t)pl.nvir_pad;
     const int vec_stride = 2 * pl.tile + 2;
     const size_t items = (size_t)pl.nitems;
-    const int jc = adjoint_chunk(nocc), nchunks = ((int)nocc + jc - 1) / jc;
-    const size_t vpart = 2 * nocc * (size_t)nchunks * nvir;
+    const int jc = adjoint_chunk(nocc, nvir), nchunks = ((int)nocc + jc - 1) / jc;
+    const size_t vrow = 2 * (size_t)nchunks * nvir;
     std::vector<std::pair<int, size_t>> req = {
         {kSlotOp0, packed_op_bytes(pl, nocc, prec)},
         {kSlotScale, sizeof(int) * rows8},
@@ -838,9 +881,12 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
         {kSlotRows, sizeof(double) * 4 * nocc},
         {kSlotResult, sizeof(double) * (2 + nocc + nvir)},
         {kSlotScalar, 256},
-        {kSlotRed, sizeof(double) * (vpart + 6 * (nocc * (nocc + 1) / 2))},
+        {kSlotAcc, sizeof(double) * 2 * (nocc + nvir)},
+        {kSlotRed, sizeof(double) * (vrow + 6 * nocc)},
     };
-    fh_status st = reserve(s, req);
+    size_t batch = nocc;
+    fh_status st = reserve_sums(
+        s, req, {{kSlotRed, sizeof(double) * (vrow * nocc + 3 * nocc * (nocc + 1))}}, &batch);
     if (st != FH_OK) return st;
     // B enters the GEMMs as FP32 split into BF16: the FP32 range check applies.
     st = range_check(s, b_dev, in_f32, naux * nocc * nvir, naux, stream);
@@ -944,14 +990,13 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
     rd.ntile = pl.ntile;
     rd.ntp = pl.ntp;
     rd.vec_stride = vec_stride;
-    rd.item_vec = ea.item_vec;
-    rd.item_partials = ea.item_partials;
     rd.jc = jc;
     rd.nchunks = nchunks;
     rd.rows = ea.row_partials;
+    rd.acc = (double *)s.slots[kSlotAcc].ptr;
     rd.result = ea.result;
     rd.vpart = (double *)s.slots[kSlotRed].ptr;
-    rd.ppart = rd.vpart + vpart;
+    rd.ppart = rd.vpart + vrow * batch;
     auto first_item = [&](int64_t i) {
         return (i * (int64_t)nocc - i * (i - 1) / 2) * pl.ntp;
     };
@@ -1004,12 +1049,16 @@ static fh_status adjoint_core_i8(State &s, const void *b_dev, fh_dtype b_dtype, 
                            (int)nocc, (int)nvir, vpg, gamma_dev);
     }
     mark(s, 2, stream);
-    launch_adjoint_sums(rd, stream);
+    for (int r0 = 0; r0 < (int)nocc; r0 += (int)batch) {
+        rd.item_vec = ea.item_vec + first_item(r0) * vec_stride;
+        rd.item_partials = ea.item_partials + 4 * first_item(r0);
+        launch_adjoint_sums(rd, r0, std::min((int)nocc, r0 + (int)batch), stream);
+    }
     he = hipGetLastError();
     if (he != hipSuccess) return fail(FH_KERNEL, "adjoint finish: %s", hipGetErrorString(he));
     mark(s, 3, stream);
     const int ngroups = (int)((nocc + R - 1) / R);
-    s.pending.kernel_launches += 2 * ngroups + 9;
+    s.pending.kernel_launches += 2 * ngroups + 7 + 2 * (nocc / batch);
     std::vector<double> res(2 + nocc + nvir);
     st = hip_check(hipMemcpyAsync(res.data(), ea.result, sizeof(double) * res.size(),
                                   hipMemcpyDeviceToHost, stream),
@@ -1148,28 +1197,36 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
     const int64_t k0 = (int64_t)nocc * pl.nvir_pad;
     int splits = (int)std::min<int64_t>((512 + nbB - 1) / nbB, std::max<int64_t>(1, k0 / 256));
     splits = std::max(1, splits);
-    const size_t items = nocc * (nocc + 1) / 2 * (size_t)pl.ntp;
-    const int jc = adjoint_chunk(nocc), nchunks = ((int)nocc + jc - 1) / jc;
-    const size_t vpart = 2 * nocc * (size_t)nchunks * nvir;
+    const size_t row_items = nocc * (size_t)pl.ntp;  // of the first row, the longest
+    const size_t items = (nocc + 1) * row_items / 2;
+    const int jc = adjoint_chunk(nocc, nvir), nchunks = ((int)nocc + jc - 1) / jc;
+    const size_t vrow = 2 * (size_t)nchunks * nvir;
     std::vector<std::pair<int, size_t>> req = {
         {kSlotOp0, op_bytes},
         {kSlotStage2, b2_bytes},
         {kSlotT, t_bytes},
         {kSlotU, u_bytes},
         {kSlotEps, sizeof(double) * (nocc + nvir)},
-        {kSlotItems, sizeof(double) * 4 * items},
-        {kSlotDeps, sizeof(double) * (vec_stride * items)},
+        {kSlotItems, sizeof(double) * 4 * row_items},
+        {kSlotDeps, sizeof(double) * vec_stride * row_items},
         {kSlotRows, sizeof(double) * 4 * nocc},
+        {kSlotAcc, sizeof(double) * 2 * (nocc + nvir)},
         {kSlotResult, sizeof(double) * (2 + nocc + nvir)},
         {kSlotScalar, 256},
         {kSlotSplit, sizeof(double) * (size_t)splits * m_pad * pl.nvir_pad},
-        {kSlotRed, sizeof(double) * (vpart + 6 * (nocc * (nocc + 1) / 2))},
+        {kSlotRed, sizeof(double) * (vrow + 6 * nocc)},
     };
     if (prec == Prec::BF16X3) {
         req.push_back({kSlotOp1, op_bytes});
         req.push_back({kSlotDiag, sizeof(double) * rows});
     }
-    fh_status st = reserve(s, req);
+    size_t batch = nocc;
+    fh_status st =
+        reserve_sums(s, req,
+                     {{kSlotItems, sizeof(double) * 4 * items},
+                      {kSlotDeps, sizeof(double) * vec_stride * items},
+                      {kSlotRed, sizeof(double) * (vrow * nocc + 3 * nocc * (nocc + 1))}},
+                     &batch);
     if (st != FH_OK) return st;
     if (!f64) {
         st = range_check(s, b_dev, in_f32, naux * nocc * nvir, naux, stream);
@@ -1290,9 +1347,10 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
     rd.jc = jc;
     rd.nchunks = nchunks;
     rd.rows = ea.row_partials;
+    rd.acc = (double *)s.slots[kSlotAcc].ptr;
     rd.result = ea.result;
     rd.vpart = (double *)s.slots[kSlotRed].ptr;
-    rd.ppart = rd.vpart + vpart;
+    rd.ppart = rd.vpart + vrow * batch;
 
     int64_t total_items = 0;
     for (size_t i = 0; i < nocc; ++i) {
@@ -1301,8 +1359,12 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
         total_items += ea.nitems;
         he = launch_adjoint_pairs(ea, stream);
         if (he != hipSuccess) return fail(FH_KERNEL, "adjoint pair kernel: %s", hipGetErrorString(he));
-        ea.item_partials += 4 * ea.nitems;
-        ea.item_vec += ea.nitems * vec_stride;
+        if (batch == nocc) {
+            ea.item_partials += 4 * ea.nitems;
+            ea.item_vec += ea.nitems * vec_stride;
+        } else if (i + 1 < nocc) {
+            launch_adjoint_sums(rd, (int)i, (int)i + 1, stream);
+        }
         ga.i = (int)i;
         {
             // Same split count for every row (fixed summation structure); the
@@ -1315,11 +1377,11 @@ static fh_status adjoint_core(State &s, const void *b_dev, fh_dtype b_dtype, siz
         if (he != hipSuccess) return fail(FH_KERNEL, "adjoint GEMM: %s", hipGetErrorString(he));
     }
     mark(s, 2, stream);
-    launch_adjoint_sums(rd, stream);
+    launch_adjoint_sums(rd, (int)(nocc - batch), (int)nocc, stream);
     he = hipGetLastError();
     if (he != hipSuccess) return fail(FH_KERNEL, "adjoint reduction: %s", hipGetErrorString(he));
     mark(s, 3, stream);
-    s.pending.kernel_launches += 3 * nocc + 7;
+    s.pending.kernel_launches += 3 * nocc + 5 + 2 * (nocc / batch);
     std::vector<double> res(2 + nocc + nvir);
     st = hip_check(hipMemcpyAsync(res.data(), ea.result, sizeof(double) * res.size(),
                                   hipMemcpyDeviceToHost, stream),

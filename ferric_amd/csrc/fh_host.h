@@ -27,11 +27,12 @@ enum SlotId {
     kSlotDeps,       // adjoint: dE/deps partials
     kSlotBatch,      // batched: descriptors and work list
     kSlotBatchOut,   // batched: per-domain partials
+    kSlotAcc,        // adjoint: compensated dE/deps sums of the rows so far
     kSlotDiag,       // BF16: lo^2 row sums
     kSlotStage2,     // adjoint: Q-major padded copy of B
     kSlotU,          // adjoint: b-major T~ blocks of one row, or B by Q
     kSlotSplit,      // adjoint: split-K partial tiles of phase B
-    kSlotRed,        // adjoint: reduction partials of all rows
+    kSlotRed,        // adjoint: reduction partials of a batch of rows
     kSlotDressX,     // dressing: (Q|nu i) half-transformed rows
     kSlotDressY,     // dressing: undressed MO rows (Q|ia)
     kSlotB2Split,    // INT8X4 adjoint: BF16 hi and lo of the Q-major copy of B

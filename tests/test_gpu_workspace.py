@@ -78,6 +78,25 @@ def test_ceiling_after_a_residue_call(pool, precision):
     assert _lib.stats()["fail_pool_full"] == 0
 
 
+@pytest.mark.parametrize("precision, ceiling", [(Precision.BF16X3, 15080208),
+                                                (Precision.INT8X4, 40767696),
+                                                (Precision.FP64, 25606928)])
+def test_sums_of_one_row_at_a_time(pool, precision, ceiling):
+    """The bytes of the slots with the sums of one row. The energies and dE/deps are the same
+    compensated sums in another order: 1e-14; Gamma is not touched by it."""
+    if precision == Precision.FP64:
+        assert pool.fh_set_pool_limit(40 << 20) == 0  # the amplitudes alone are 46 MB
+    want = _gradient(precision)
+    assert ceiling < _lib.stats()["pool_peak_bytes"] < 1.2 * ceiling
+    pool.fh_release_workspace()
+    assert pool.fh_set_pool_limit(ceiling) == 0
+    got = _gradient(precision)
+    assert _lib.stats()["fail_pool_full"] == 0
+    assert torch.equal(got[2], want[2])
+    assert abs(got[1] - want[1]) <= 1e-14 * abs(want[1])
+    assert np.max(np.abs(got[3] - want[3])) <= 1e-14 * np.max(np.abs(want[3]))
+
+
 def test_a_call_past_the_ceiling_is_refused_as_before(pool):
     _gradient()
     assert pool.fh_set_pool_limit(8 << 20) == 0  # the row path needs 27 MB
