@@ -220,7 +220,9 @@ __global__ __launch_bounds__(kFitThreads, 4) void fit_pair_kernel(FitArgs g) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const double piv = lane_value(c[i], i);
-                if (piv <= 0.0 && fault == 0) fault = 16 * k + i + 1;
+                // Not positive, NaN, or infinite: a non-finite element of the metric reaches
+                // a pivot as one of them.
+                if (!(piv > 0.0 && piv < INFINITY) && fault == 0) fault = 16 * k + i + 1;
                 c[i] *= 1.0 / sqrt(piv);
 #pragma unroll
                 for (int x = i + 1; x < 16; ++x) c[x] -= lane_value(c[i], x) * c[i];
