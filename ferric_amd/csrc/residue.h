@@ -11,10 +11,13 @@
 // For each modulus m the residues of Y (signed, one byte) are multiplied by
 // v_mfma_i32_16x16x64_i8 with exact int32 sums, and the sum reduced to a signed
 // byte again. The fraction G / P is then sum_k r_k c_k modulo 1 with
-// c_k = ((P / m_k)^-1 mod m_k) / m_k, taken as 72-bit fixed point in nine signed
-// byte layers (v_dot4_i32_i8 over four moduli at a time). The only rounding
+// c_k = ((P / m_k)^-1 mod m_k) / m_k, taken as fixed point in ten (FP64) or nine (MIXED)
+// signed byte layers (v_dot4_i32_i8 over four moduli at a time). The only rounding
 // before the FP64 result is that of Y: half a unit, 2^-(beta + 1) of the row's
-// power-of-two range, and 2^-65 of P from the fixed point.
+// power-of-two range, and about 2^-74 (FP64) or 2^-66 (MIXED) of P from the fixed point.
+// With nine layers that was 2^-53 of the two rows' ranges in FP64 at naux 1000, and the
+// largest error of small products: a pair energy of e^-24 of the largest was off by 1.4e-15
+// of itself. The tenth costs a dword of products per four moduli and element.
 //
 // Why 16 moduli: with 15 a row would keep 52 bits below its largest value and
 // the sums would lose the margin over the FP64 matrix instructions' rounding
@@ -38,7 +41,8 @@ namespace res {
 constexpr int kMaxN = 16;
 constexpr int kMod[kMaxN] = {256, 239, 237, 235, 233, 229, 227, 223,
                              221, 217, 211, 209, 199, 197, 193, 191};
-constexpr int kLayers = 9;  // signed byte layers of c_k: 72 bits
+// Signed byte layers of c_k.
+constexpr int layers_of(int n) { return n == 16 ? 10 : 9; }
 
 typedef unsigned __int128 u128;
 typedef __int128 i128;
@@ -60,8 +64,8 @@ constexpr double kPlo = (double)((i128)product<N>() - (i128)(double)product<N>()
 
 template <int N>
 struct Layers {
-    // v[l][h]: byte l (0 = the highest) of c_k's 72-bit fixed point, k = 4 h .. 4 h + 3.
-    uint32_t v[kLayers][groups_of(N)] = {};
+    // v[l][h]: byte l (0 = the highest) of c_k's fixed point, k = 4 h .. 4 h + 3.
+    uint32_t v[layers_of(N)][groups_of(N)] = {};
 };
 template <int N>
 constexpr Layers<N> make_layers() {
@@ -75,9 +79,9 @@ constexpr Layers<N> make_layers() {
         for (int x = 1; x < m; ++x)
             if (rest * x % m == 1) inv = x;
         if (2 * inv > m) inv -= m;
-        const i128 num = (i128)inv * ((i128)1 << 72);  // c_k = round(inv 2^72 / m)
+        const i128 num = (i128)inv * ((i128)1 << 8 * layers_of(N));
         i128 f = num >= 0 ? (num + m / 2) / m : -((-num + m / 2) / m);
-        for (int l = kLayers - 1; l >= 0; --l) {
+        for (int l = layers_of(N) - 1; l >= 0; --l) {
             const int8_t d = (int8_t)(uint8_t)(f & 0xff);
             f = (f - d) / 256;
             t.v[l][k / 4] |= (uint32_t)(uint8_t)d << (8 * (k % 4));
@@ -140,7 +144,7 @@ __device__ __forceinline__ uint32_t pack_bytes(uint32_t b0, uint32_t b1, uint32_
 // m_k of elements 0..3 in its bytes; frac[e] = G_e / P in [-1/2, 1/2).
 template <int N>
 __device__ __forceinline__ void crt4(const uint32_t (&d)[N], double (&frac)[4]) {
-    constexpr int H = groups_of(N);
+    constexpr int H = groups_of(N), L = layers_of(N);
     uint32_t t[4][H];  // [element][four moduli]
 #pragma unroll
     for (int h = 0; h < H; ++h) {
@@ -159,9 +163,9 @@ __device__ __forceinline__ void crt4(const uint32_t (&d)[N], double (&frac)[4]) 
     }
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
-        int s[kLayers];
+        int s[L];
 #pragma unroll
-        for (int l = 0; l < kLayers; ++l) {
+        for (int l = 0; l < L; ++l) {
             s[l] = 0;
 #pragma unroll
             for (int h = 0; h < H; ++h)
@@ -171,7 +175,9 @@ __device__ __forceinline__ void crt4(const uint32_t (&d)[N], double (&frac)[4]) 
         const uint32_t top = ((uint32_t)s[0] << 24) + ((uint32_t)s[1] << 16) +
                              ((uint32_t)s[2] << 8) + (uint32_t)s[3];
         const int m1 = s[4] * 256 + s[5], m2 = s[6] * 256 + s[7];
-        double f = fma((double)m2, 0x1p-64, (double)s[8] * 0x1p-72);
+        const double m3 = L == 10 ? (double)(s[8] * 256 + s[L - 1]) * 0x1p-80
+                                  : (double)s[8] * 0x1p-72;
+        double f = fma((double)m2, 0x1p-64, m3);
         f = fma((double)m1, 0x1p-48, f);
         frac[x] = fma((double)(int)top, 0x1p-32, f);
     }
