@@ -243,7 +243,8 @@ __global__ __launch_bounds__(256) void pair_bf16x3_kernel(EnergyArgs a) {
 // the library's lock and wait for them.
 __device__ unsigned int rows_done;
 
-__device__ __forceinline__ void fold_rows(const double *rows, int nocc, double *result) {
+__device__ __forceinline__ void fold_rows(const double *rows, int nocc, const int *wide,
+                                          double *result) {
     __shared__ double part[256][4];
     __shared__ unsigned int before;
     if (threadIdx.x == 0) {
@@ -272,11 +273,13 @@ __device__ __forceinline__ void fold_rows(const double *rows, int nocc, double *
         __syncthreads();
     }
     if (folds) result[threadIdx.x / kWave] = sum.value();
+    if (wide && threadIdx.x == 0) result[2 + 2 * (int64_t)nocc] = *wide ? 1.0 : 0.0;
     if (threadIdx.x == 0) rows_done = 0;
 }
 
 __global__ __launch_bounds__(256) void reduce_rows_kernel(const double *__restrict__ ip, int nocc,
-                                                          int ntp, double *rows, double *result) {
+                                                          int ntp, const int *wide, double *rows,
+                                                          double *result) {
     const int i = blockIdx.x;
     const int64_t p0 = (int64_t)i * nocc - (int64_t)i * (i - 1) / 2;
     const int64_t w0 = p0 * ntp, w1 = (p0 + (nocc - i)) * ntp;
@@ -286,13 +289,14 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const double *__restri
         ss.merge(ip[4 * w + 2], ip[4 * w + 3]);
     }
     pair::block_store(os, ss, 1.0, rows + 4 * i);
-    fold_rows(rows, nocc, result);
+    fold_rows(rows, nocc, wide, result);
 }
 
 // Rectangle rows: items [i*per_row, (i+1)*per_row) belong to alpha row i.
 __global__ __launch_bounds__(256) void reduce_rect_rows_kernel(const double *__restrict__ ip,
                                                                int64_t per_row, int nocc,
-                                                               double *rows, double *result) {
+                                                               const int *wide, double *rows,
+                                                               double *result) {
     const int i = blockIdx.x;
     KSum os, ss;
     for (int64_t w = (int64_t)i * per_row + threadIdx.x; w < (int64_t)(i + 1) * per_row;
@@ -301,7 +305,7 @@ __global__ __launch_bounds__(256) void reduce_rect_rows_kernel(const double *__r
         ss.merge(ip[4 * w + 2], ip[4 * w + 3]);
     }
     pair::block_store(os, ss, 1.0, rows + 4 * i);
-    fold_rows(rows, nocc, result);
+    fold_rows(rows, nocc, wide, result);
 }
 
 template <typename K>
@@ -434,13 +438,13 @@ hipError_t launch_energy_rect(const EnergyArgs &a, hipStream_t st) {
 hipError_t launch_rect_reduce(const EnergyArgs &a, hipStream_t st) {
     const int64_t per_row = (int64_t)a.nocc_b * a.ntile * a.ntile_b;
     hipLaunchKernelGGL(reduce_rect_rows_kernel, dim3((unsigned)a.nocc), dim3(256), 0, st,
-                       a.item_partials, per_row, a.nocc, a.row_partials, a.result);
+                       a.item_partials, per_row, a.nocc, a.wide, a.row_partials, a.result);
     return hipGetLastError();
 }
 
 hipError_t launch_energy_reduce(const EnergyArgs &a, hipStream_t st) {
     hipLaunchKernelGGL(reduce_rows_kernel, dim3((unsigned)a.nocc), dim3(256), 0, st,
-                       a.item_partials, a.nocc, a.ntp, a.row_partials, a.result);
+                       a.item_partials, a.nocc, a.ntp, a.wide, a.row_partials, a.result);
     return hipGetLastError();
 }
 

@@ -379,15 +379,16 @@ bool residue_tiles(State &s, size_t nvir, size_t naux, EnergyPlan *pl) {
     return true;
 }
 
-fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, size_t rows,
-                          int naux_pad, std::vector<std::pair<int, size_t>> more,
-                          ResidueSpace *out) {
+fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, size_t nov,
+                          size_t rows, size_t norb, int naux_pad,
+                          std::vector<std::pair<int, size_t>> more, ResidueSpace *out) {
     const int blocks = s.cus / 8 * 8;
     const int words = residue_queue_words(blocks);
     const size_t stride = residue_scratch_stride(prec, products);
     const size_t planes = stride * (size_t)residue_scratch_sets(blocks);
     more.push_back({kSlotOp0, rows * (size_t)naux_pad * residue_moduli(prec)});
     more.push_back({kSlotScale, sizeof(int) * rows});
+    more.push_back({kSlotRange, out->range.bytes(nov, rows / 16, norb, naux_pad)});
     more.push_back({kSlotResidue, planes + sizeof(int) * ((size_t)words + (size_t)nitems)});
     const fh_status st = reserve(s, more, true);
     if (st != FH_OK) return st;
@@ -405,6 +406,9 @@ fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, siz
     ra.scratch_stride = (int64_t)stride;
     ra.queue = (int *)((char *)ra.scratch + planes);
     ra.order = ra.queue + words;
+    out->wide = ra.queue + residue_flag_word(blocks);
+    ra.wide = out->wide;
+    out->range.place(s.slots[kSlotRange].ptr, nov, rows / 16, norb, naux_pad);
     out->order.words = words;
     out->order.queue = ra.queue;
     out->order.order = ra.queue + words;
@@ -449,11 +453,11 @@ bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, En
 }
 
 fh_status fetch_result(State &s, const double *dev, size_t nocc, hipStream_t stream,
-                       fh_spin_components *out, double *row_partials) {
+                       fh_spin_components *out, double *row_partials, bool *wide) {
     std::vector<double> copy;
     const double *res = dev;  // already on the host when it is the pinned buffer
     if (dev != s.host) {
-        copy.resize(2 + 2 * nocc);
+        copy.resize(2 + 2 * nocc + (wide ? 1 : 0));
         const fh_status st = hip_check(hipMemcpyAsync(copy.data(), dev,
                                                       sizeof(double) * copy.size(),
                                                       hipMemcpyDeviceToHost, stream),
@@ -469,15 +473,16 @@ fh_status fetch_result(State &s, const double *dev, size_t nocc, hipStream_t str
     out->e_total = res[0] + res[1];
     if (row_partials)
         for (size_t i = 0; i < 2 * nocc; ++i) row_partials[i] = res[2 + i];
+    if (wide) *wide = res[2 + 2 * nocc] != 0.0;
     return FH_OK;
 }
 
 namespace {
 
-// Where a call's 2 + 2 nocc results go, then its energies: the pinned buffer if it holds
-// both, else null. (Pageable copies of either cost a call about 10 us.)
+// Where a call's 2 + 2 nocc results and a flag go, then its energies: the pinned buffer if it
+// holds both, else null. (Pageable copies of either cost a call about 10 us.)
 double *call_buffer(State &s, size_t nocc, size_t nvir) {
-    return host_buffer(s, 2 + 3 * nocc + nvir);
+    return host_buffer(s, 3 + 3 * nocc + nvir);
 }
 
 // Uploads [eps_occ, eps_vir] of the active orbitals; `pack`: left to that kernel when
@@ -487,7 +492,7 @@ fh_status upload_eps(State &s, const double *eps, size_t first_occ, size_t nocc,
     double *e = call_buffer(s, nocc, nvir);
     const bool pinned = e != nullptr;
     if (pinned) {
-        e += 2 + 2 * nocc;
+        e += 3 + 2 * nocc;
     } else {
         s.eps_up.resize(nocc + nvir);
         e = s.eps_up.data();
@@ -509,16 +514,17 @@ fh_status upload_eps(State &s, const double *eps, size_t first_occ, size_t nocc,
 fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, size_t nocc,
                          size_t nvir, const double *eps, size_t first_occ, size_t nocc_total,
                          double kappa, Prec prec, hipStream_t stream, fh_spin_components *out,
-                         double *row_partials, const EnergyPlan &pl, const AmpOut *amp_out) {
+                         double *row_partials, const EnergyPlan &pl, const AmpOut *amp_out,
+                         bool *wide) {
     const size_t npairs = nocc * (nocc + 1) / 2;
     ResidueSpace sp;
     fh_status st = reserve_residue(
-        s, prec, pl.nitems, pl.ntile > 1 ? 2 : 1, nocc * (size_t)pl.nvir_pad, pl.naux_pad,
-        {{kSlotColMax, sizeof(double) * (size_t)(pl.naux_pad / 64) * nocc * nvir},
-         {kSlotEps, sizeof(double) * (nocc + nvir)},
+        s, prec, pl.nitems, pl.ntile > 1 ? 2 : 1, nocc * nvir, nocc * (size_t)pl.nvir_pad, nocc,
+        pl.naux_pad,
+        {{kSlotEps, sizeof(double) * (nocc + nvir)},
          {kSlotItems, sizeof(double) * 4 * npairs * (size_t)pl.ntp},
          {kSlotRows, sizeof(double) * 4 * nocc},
-         {kSlotResult, sizeof(double) * (2 + 2 * nocc)}},
+         {kSlotResult, sizeof(double) * (3 + 2 * nocc)}},
         &sp);
     if (st != FH_OK) return st;
     if (prec == Prec::MIXED) {
@@ -547,14 +553,15 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     ord.nocc = ra.ngroup;
     ord.ntp = pl.ntp;
     mark(s, 0, stream);
-    hipError_t he = launch_residue_pack(prec, pa, ord, (double *)s.slots[kSlotColMax].ptr, stream);
+    ra.nocc = (int)nocc;
+    ra.nvir = (int)nvir;
+    ra.nvir_pad = pl.nvir_pad;
+    hipError_t he = launch_residue_pack(prec, pa, ord, sp.range, stream);
+    if (he == hipSuccess) he = launch_residue_range(ra, sp.range, sp.wide, stream);
     if (he != hipSuccess) {
         (void)hipGetLastError();
         return fail(FH_KERNEL, "pack kernel: %s", hipGetErrorString(he));
     }
-    ra.nocc = (int)nocc;
-    ra.nvir = (int)nvir;
-    ra.nvir_pad = pl.nvir_pad;
     ra.ntile = pl.ntile;
     ra.ntp = pl.ntp;
     ra.eps_occ = (const double *)s.slots[kSlotEps].ptr;
@@ -567,6 +574,7 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     ea.ntp = ra.ntp;
     ea.item_partials = ra.item_partials;
     ea.row_partials = (double *)s.slots[kSlotRows].ptr;
+    ea.wide = sp.wide;
     ea.result = call_buffer(s, nocc, nvir);
     if (!ea.result) ea.result = (double *)s.slots[kSlotResult].ptr;
     mark(s, 1, stream);
@@ -582,8 +590,8 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
         return fail(FH_KERNEL, "reduction kernels: %s", hipGetErrorString(he));
     }
     mark(s, 3, stream);
-    s.pending.kernel_launches += 4;
-    st = fetch_result(s, ea.result, nocc, stream, out, row_partials);
+    s.pending.kernel_launches += 6;
+    st = fetch_result(s, ea.result, nocc, stream, out, row_partials, wide);
     if (st == FH_OK) finish_timing(s, (uint64_t)pl.nitems, pl.tile);
     return st;
 }
@@ -660,13 +668,14 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
     if (!signed_k && !(as_noalloc && carved <= (size_t)FH_NOALLOC_SCRATCH_BYTES) &&
         plan_residue(s, nocc, nvir, naux, prec, &rpl)) {
         const Attempt attempt(s);
+        bool wide = false;
         const fh_status rst =
             residue_energy(s, b_dev, in_f32, naux, nocc, nvir, eps, first_occ, nocc_total, kappa,
-                           prec, stream, out, row_partials, rpl, amp_out);
+                           prec, stream, out, row_partials, rpl, amp_out, &wide);
         if (ntp_used) *ntp_used = rpl.ntp;
-        // Its larger workspace may be past the pool ceiling: then the matrix kernel
-        // below, which needs half the operand (or less) and no scratch.
-        if (rst != FH_POOL_FULL) return rst;
+        // Its larger workspace may be past the pool ceiling, or the rows past its range: then
+        // the matrix kernel below, which needs half the operand (or less) and no scratch.
+        if (rst != FH_POOL_FULL && !wide) return rst;
         attempt.undo();
     }
     if (ntp_used) *ntp_used = pl.ntp;

@@ -49,8 +49,8 @@ enum SlotId {
     kSlotDensPart,   // MP2 densities: split-K partial tiles
     kSlotDensOut,    // MP2 densities: P_vv (padded) then P_oo
     kSlotResidue,    // residue arithmetic: the workgroups' residue planes
-    kSlotColMax,     // residue arithmetic: column maxima of B per Q panel (the packer's; no
-                     // entry stages an input here, as some do in kSlotStage and kSlotStage2)
+    kSlotRange,      // residue arithmetic: column maxima and sums of B (the packer's; no entry
+                     // stages an input here, as some do in kSlotStage and kSlotStage2)
     kNumSlots
 };
 
@@ -181,15 +181,19 @@ bool residue_tiles(State &s, size_t nvir, size_t naux, EnergyPlan *pl);
 struct ResidueSpace {
     ResidueArgs args;    // prec, np, beta, op, rexp, nitems, blocks, scratch, queue, order
     ResidueOrder order;  // words, queue, order
+    ResidueRange range;
     int8_t *op = nullptr;
     int *rexp = nullptr;
+    int *wide = nullptr;
 };
-fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, size_t rows,
-                          int naux_pad, std::vector<std::pair<int, size_t>> more,
-                          ResidueSpace *out);
-// Copies the device result (energies, then nocc rows' values) back and waits for it.
+// nov: columns of B, rows: packed rows, norb: occupied orbitals (both sides' together).
+fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, size_t nov,
+                          size_t rows, size_t norb, int naux_pad,
+                          std::vector<std::pair<int, size_t>> more, ResidueSpace *out);
+// Copies the device result (energies, then nocc rows' values, then, if asked for, the residue
+// kernel's flag) back and waits for it.
 fh_status fetch_result(State &s, const double *dev, size_t nocc, hipStream_t stream,
-                       fh_spin_components *out, double *row_partials);
+                       fh_spin_components *out, double *row_partials, bool *wide = nullptr);
 bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, EnergyPlan *pl);
 void commit(State &s, Prec prec, bool adjoint, bool batched);
 bool to_prec(int p, Prec *out);

@@ -188,6 +188,8 @@ struct EnergyArgs {
     const double *eps_occ_b = nullptr, *eps_vir_b = nullptr;
     const int *rexp_b = nullptr;  // I8X4: row exponents of the beta rows
     AmpOut amp;  // MP2 densities, FP64 adjoint: store the amplitudes too
+    // Residue arithmetic: its flag, which the reduction stores behind the rows' values.
+    const int *wide = nullptr;
 };
 
 hipError_t launch_energy(const EnergyArgs &a, hipStream_t st);
@@ -214,6 +216,7 @@ struct ResidueArgs {
     void *scratch = nullptr;     // residue_scratch_sets(blocks) x scratch_stride bytes
     int64_t scratch_stride = 0;
     int *queue = nullptr;        // round counter and, per workgroup, parts done: zeroed by the packer
+    const int *wide = nullptr;   // set by launch_residue_range: leave at once
     const int *order = nullptr;  // the items in the order they are taken
 };
 struct ResidueOrder {
@@ -228,11 +231,27 @@ int residue_beta(Prec prec, int naux_pad);
 // or more workgroups to each).
 int residue_scratch_sets(int blocks);
 int residue_queue_words(int blocks);
+int residue_flag_word(int blocks);  // the range test's
 size_t residue_scratch_stride(Prec prec, int products);
-// pmax: (naux_pad / 64) x nocc nvir doubles of scratch. The rows go to row groups rg0
-// on, of nrg in all (0: only these). ord.order null: no order to be made.
-hipError_t launch_residue_pack(Prec prec, const PackArgs &a, const ResidueOrder &ord, double *pmax,
-                               hipStream_t st, int64_t nrg = 0, int64_t rg0 = 0);
+// Scratch of the packer and of the range test, for nov columns and nrg 16-row groups of norb
+// orbitals.
+struct ResidueRange {
+    double *pmax = nullptr;   // column maxima by Q panel
+    double *w = nullptr;      // per orbital and Q: sum over the virtuals of B^2
+    double *s = nullptr;      // per orbital: sum over the virtuals of the rows' squared ranges
+    float *norm = nullptr;    // per row group and Q: sum of B^2, in units of 4^gexp
+    int *gexp = nullptr;      // per row group: the largest exponent
+    size_t bytes(size_t nov, size_t nrg, size_t norb, int naux_pad);
+    void place(void *base, size_t nov, size_t nrg, size_t norb, int naux_pad);
+};
+// The rows go to row groups rg0 on, of nrg in all (0: only these). ord.order null: no order
+// to be made.
+hipError_t launch_residue_pack(Prec prec, const PackArgs &a, const ResidueOrder &ord,
+                               const ResidueRange &rr, hipStream_t st, int64_t nrg = 0,
+                               int64_t rg0 = 0);
+// Sets *wide if some pair's products would lose accuracy (a's sizes and rows; residue.hip).
+hipError_t launch_residue_range(const ResidueArgs &a, const ResidueRange &rr, int *wide,
+                                hipStream_t st);
 hipError_t launch_residue_energy(const ResidueArgs &a, hipStream_t st);
 // Phase A of the adjoint: the pair kernel with the T~ / dE/deps epilogue.
 hipError_t launch_adjoint_pairs(const EnergyArgs &a, hipStream_t st);

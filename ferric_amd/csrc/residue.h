@@ -122,6 +122,13 @@ constexpr Digits make_digits() {
 }
 constexpr Digits kDigit = make_digits();
 
+// The exponent of a row of zeros, below every other.
+constexpr int kZeroRow = -4096;
+
+// Root mean square error of G / P from the fixed point: N residues of up to m / 2 times the
+// rounding of c_k.
+inline double fixed_error(int n) { return 19.0 * sqrt((double)n) * exp2(-8.0 * layers_of(n)); }
+
 // Largest naux the int32 sums and the byte remainders allow (see above).
 constexpr int kMaxNauxPad = 4608;
 

@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
                                                            int naux, int nvir, int nvir_pad,
                                                            int64_t nrows, int np, int beta,
                                                            int64_t nrg, int64_t rg0,
-                                                           const double *__restrict__ pmax,
+                                                           ResidueRange rr,
                                                            int *__restrict__ rexp,
                                                            int8_t *__restrict__ out,
                                                            ResidueOrder ord) {
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
     }
     double m = 0.0;
     if (col >= 0)
-        for (int p = ty; p < np; p += 4) m = fmax(m, pmax[(int64_t)p * nov + col]);
+        for (int p = ty; p < np; p += 4) m = fmax(m, rr.pmax[(int64_t)p * nov + col]);
     part[ty][tx] = m;
     for (int q = ty; q < 64; q += 4) {
         const int qq = q0 + q;
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
     if (ty == 0) {
         double mm = fmax(fmax(part[0][tx], part[1][tx]), fmax(part[2][tx], part[3][tx]));
         if (ROUND32) mm = (double)(float)mm;
-        int e = 0;
+        int e = res::kZeroRow;
         if (mm > 1.7976931348623157e308) {
             e = kI8NonFinite;
         } else if (mm > 0.0) {
@@ -184,13 +184,31 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
         if (blockIdx.y == 0 && r < nrows) rexp[r] = e;
     }
     __syncthreads();
+    // For the range test: a wave to a row group, a lane to a Q. Non-finite rows are not judged.
+    if (r0 + 16 * ty < nrows) {
+        int ge = res::kZeroRow;
+        for (int k = 0; k < 16; ++k) {
+            const int e = exps[16 * ty + k];
+            if (e != kI8NonFinite) ge = max(ge, e);
+        }
+        double sum = 0.0;
+        if (ge > res::kZeroRow)
+            for (int k = 0; k < 16; ++k) {
+                const double v = ldexp(tile[tx][16 * ty + k], -ge);
+                sum += exps[16 * ty + k] != kI8NonFinite ? v * v : 0.0;
+            }
+        const int64_t rg = rg0 + r0 / 16 + ty;
+        // Positive even where it underflows FP32: only a zero has no rounding error.
+        rr.norm[rg * (np * 64) + q0 + tx] = sum > 0.0 ? fmaxf((float)sum, 0x1p-126f) : 0.0f;
+        if (blockIdx.y == 0 && tx == 0) rr.gexp[rg] = ge;
+    }
     // Thread t takes row 16 (t / 64) + t % 16 and the panel's Q = 16 g .. 16 g + 15,
     // g = (t / 16) % 4: lane t % 64 of its row group's kilobyte.
     const int t = threadIdx.x;
-    const int g = (t / 16) % 4, rr = (t / 64) * 16 + t % 16;
-    const int64_t orow = r0 + rr;
+    const int g = (t / 16) % 4, row = (t / 64) * 16 + t % 16;
+    const int64_t orow = r0 + row;
     if (orow >= nrows) return;
-    const int e = exps[rr];
+    const int e = exps[row];
     const bool bad = e == kI8NonFinite;
     const int sh = bad ? 0 : beta - 1 - e;
     uint32_t w[N][4];
@@ -200,7 +218,7 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
         for (int c = 0; c < 4; ++c) w[k][c] = 0u;
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
-        const double y = bad ? 0.0 : rint(ldexp(tile[16 * g + q][rr], sh));
+        const double y = bad ? 0.0 : rint(ldexp(tile[16 * g + q][row], sh));
         // y as 64-bit two's complement: hi = floor(y / 2^32), lo = the rest
         const double h = floor(y * 0x1p-32);
         const uint64_t z =
@@ -227,6 +245,97 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
     for (int k = 0; k < N; ++k)
         *(uint4 *)(o + (int64_t)k * np * nrg * 1024) =
             make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
+}
+
+// ---- Range test ----------------------------------------------------------------
+// One exponent a row makes the rounding of g = (ia|jb) relative to the rows' largest
+// elements, where the matrix kernels' is relative to the products: rows that lie on different
+// aux functions (orbitals far apart) have small products of which few bits would be left. The
+// mean square error of g over a and b is
+//   4^-beta / 12 (s_i sum_Q w_jQ + s_j sum_Q w_iQ) + (fixed point)^2 s_i s_j,
+// s_i the sum over a of the rows' squared ranges 4^(f + 1), w_iQ the sum over a of B^2, the
+// sums over Q where the other orbital is not zero (zeros have no rounding error), and g^2 is
+// sum_Q w_iQ w_jQ for products of random sign. A call with a pair whose error exceeds kBar of
+// that goes to the matrix kernel: the energy kernel leaves at once, and the host sees the flag
+// with the results, so that no wait is added. Pairs by their own size, chain of 24 orbitals
+// decaying as e^-d over 1008 aux functions: 1.9e-10 at d = 21 without the test, and 3.7e-3 in
+// MIXED. What errors the bar admits the sums of the energies average down to their own rounding;
+// the matrix kernels' products are off by 2^-50 (960 aux functions in FP64) and 2^-23 (panels
+// of 64 in FP32) on the same scale. Normal rows, with or without hot aux functions, have
+// 2^-53 to 2^-54, water in cc-pVDZ 2^-54, orbitals that reach three sites 2^-51.
+// What it costs, with the packer's sums and two small kernels (and the tenth layer of the
+// reconstruction): the three blocks of 21/229, 20/230 over 960 aux functions 1396 -> 1439 us,
+// 60/450/1800 in MIXED 9333 -> 9332, 100/200/2400 9513 -> 9571.
+constexpr double bar_of(int n) { return n == 16 ? 0x1p-50 : 0x1p-24; }
+
+// One side's orbitals in the packed rows, and where their sums go.
+struct RangeSide {
+    int norb, nvir, nvir_pad;
+    int64_t rg0;      // first row group
+    const int *rexp;
+    double *w, *s;
+};
+
+// 64 Q of one orbital a workgroup, the row groups dealt to its four waves.
+__global__ __launch_bounds__(256) void residue_norm_kernel(const float *__restrict__ norm,
+                                                           const int *__restrict__ gexp,
+                                                           int naux_pad, RangeSide a,
+                                                           RangeSide b) {
+    const bool second = (int)blockIdx.y >= a.norb;
+    const RangeSide o = second ? b : a;
+    const int i = second ? blockIdx.y - a.norb : blockIdx.y;
+    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave, ng = o.nvir_pad / 16;
+    const int64_t rg = o.rg0 + (int64_t)i * ng;
+    int top = res::kZeroRow;
+    for (int g = lane; g < ng; g += kWave) top = max(top, gexp[rg + g]);
+    for (int m = 1; m < kWave; m *= 2) top = max(top, __shfl_xor(top, m, kWave));
+    const int q = blockIdx.x * 64 + lane;
+    double sum = 0.0;
+#pragma unroll 4
+    for (int g = wid; g < ng; g += 4)
+        sum += ldexp((double)norm[(rg + g) * naux_pad + q], 2 * (gexp[rg + g] - top));
+    __shared__ double part[4][64];
+    part[wid][lane] = sum;
+    __syncthreads();
+    if (wid == 0)
+        o.w[(int64_t)i * naux_pad + q] =
+            (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    if (blockIdx.x != 0 || wid != 1) return;
+    double t = 0.0;
+    for (int v = lane; v < o.nvir; v += kWave) {
+        const int e = o.rexp[(int64_t)i * o.nvir_pad + v];
+        if (e > res::kZeroRow && e != kI8NonFinite) t += ldexp(1.0, 2 * (e + 1 - top));
+    }
+    for (int m = 1; m < kWave; m *= 2) t += __shfl_xor(t, m, kWave);
+    if (lane == 0) o.s[i] = t;
+}
+
+// Orbitals i = blockIdx.y and j, a wave to each j. same: j >= i only.
+__global__ __launch_bounds__(256) void residue_range_kernel(const double *__restrict__ wa,
+                                                            const double *__restrict__ sa,
+                                                            const double *__restrict__ wb,
+                                                            const double *__restrict__ sb, int nb,
+                                                            int naux_pad, bool same, double round2,
+                                                            double fixed2, int *wide) {
+    const int i = blockIdx.y, j = blockIdx.x * 4 + threadIdx.x / kWave;
+    if (j >= nb || (same && j < i)) return;
+    const double *x = wa + (int64_t)i * naux_pad, *y = wb + (int64_t)j * naux_pad;
+    double gg = 0.0, ni = 0.0, nj = 0.0;
+#pragma unroll 4
+    for (int q = threadIdx.x % kWave; q < naux_pad; q += kWave) {
+        const double u = x[q], v = y[q];
+        gg += u * v;
+        ni += v > 0.0 ? u : 0.0;
+        nj += u > 0.0 ? v : 0.0;
+    }
+    for (int m = 1; m < kWave; m *= 2) {
+        gg += __shfl_xor(gg, m, kWave);
+        ni += __shfl_xor(ni, m, kWave);
+        nj += __shfl_xor(nj, m, kWave);
+    }
+    if (threadIdx.x % kWave != 0 || nj == 0.0) return;  // no aux function in common: g = 0
+    const double err = round2 * (sa[i] * nj + sb[j] * ni) + fixed2 * sa[i] * sb[j];
+    if (!(err <= gg)) *wide = 1;
 }
 
 // One product over a run of moduli and every panel: row groups rgA .. rgA + nA against
@@ -636,6 +745,7 @@ template <int N, bool RECT, bool AMP>
 __global__ __launch_bounds__(kThreads) void residue_energy_kernel(ResidueArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     __shared__ int turn;
+    if (*a.wide) return;
     const int tid = threadIdx.x;
     const int wid = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int wr = wid >> 2;
@@ -766,24 +876,24 @@ __global__ __launch_bounds__(kThreads) void residue_energy_kernel(ResidueArgs a)
 }
 
 template <int N, bool ROUND32>  // MIXED: ROUND32
-hipError_t launch_pack_n(const PackArgs &a, const ResidueOrder &ord, double *pmax, int beta,
-                         int64_t nrg, int64_t rg0, hipStream_t st) {
+hipError_t launch_pack_n(const PackArgs &a, const ResidueOrder &ord, const ResidueRange &rr,
+                         int beta, int64_t nrg, int64_t rg0, hipStream_t st) {
     const int64_t nrows = (int64_t)a.nocc * a.nvir_pad, nov = (int64_t)a.nocc * a.nvir;
     const int np = a.naux_pad / 64;
     const dim3 mg((unsigned)((nov + 255) / 256), (unsigned)((a.naux + 63) / 64));
     const dim3 grid((unsigned)((nrows + 63) / 64), (unsigned)np + 1);
     if (a.in_f32) {
         hipLaunchKernelGGL(residue_colmax_kernel<float>, mg, dim3(256), 0, st, (const float *)a.b,
-                           nov, a.naux, pmax);
+                           nov, a.naux, rr.pmax);
         hipLaunchKernelGGL((residue_pack_kernel<N, ROUND32, float>), grid, dim3(256), 0, st,
                            (const float *)a.b, nov, a.naux, a.nvir, a.nvir_pad, nrows, np, beta,
-                           nrg, rg0, (const double *)pmax, a.rexp, (int8_t *)a.out0, ord);
+                           nrg, rg0, rr, a.rexp, (int8_t *)a.out0, ord);
     } else {
         hipLaunchKernelGGL(residue_colmax_kernel<double>, mg, dim3(256), 0, st,
-                           (const double *)a.b, nov, a.naux, pmax);
+                           (const double *)a.b, nov, a.naux, rr.pmax);
         hipLaunchKernelGGL((residue_pack_kernel<N, ROUND32, double>), grid, dim3(256), 0, st,
                            (const double *)a.b, nov, a.naux, a.nvir, a.nvir_pad, nrows, np, beta,
-                           nrg, rg0, (const double *)pmax, a.rexp, (int8_t *)a.out0, ord);
+                           nrg, rg0, rr, a.rexp, (int8_t *)a.out0, ord);
     }
     return hipGetLastError();
 }
@@ -798,24 +908,60 @@ int residue_beta(Prec prec, int naux_pad) {
 
 int residue_scratch_sets(int blocks) { return blocks + blocks / 2; }
 
-int residue_queue_words(int blocks) { return (kQueueStride + blocks + 31) / 32 * 32; }
+int residue_flag_word(int blocks) { return (kQueueStride + blocks + 31) / 32 * 32; }
+
+int residue_queue_words(int blocks) { return residue_flag_word(blocks) + kQueueStride; }
 
 size_t residue_scratch_stride(Prec prec, int products) {
     return (size_t)products * planes_of(residue_moduli(prec));
 }
 
-hipError_t launch_residue_pack(Prec prec, const PackArgs &a, const ResidueOrder &ord, double *pmax,
-                               hipStream_t st, int64_t nrg, int64_t rg0) {
+size_t ResidueRange::bytes(size_t nov, size_t nrg, size_t norb, int naux_pad) {
+    const size_t np = (size_t)naux_pad;
+    return sizeof(double) * (np / 64 * nov + norb * (np + 1)) + (sizeof(float) * np + sizeof(int)) * nrg;
+}
+
+void ResidueRange::place(void *base, size_t nov, size_t nrg, size_t norb, int naux_pad) {
+    const size_t np = (size_t)naux_pad;
+    pmax = (double *)base;
+    w = pmax + np / 64 * nov;
+    s = w + norb * np;
+    norm = (float *)(s + norb);
+    gexp = (int *)(norm + nrg * np);
+}
+
+hipError_t launch_residue_range(const ResidueArgs &a, const ResidueRange &rr, int *wide,
+                                hipStream_t st) {
+    const int naux_pad = a.np * 64, n = residue_moduli(a.prec);
+    const bool rect = a.nocc_b > 0;
+    const RangeSide x{a.nocc, a.nvir, a.nvir_pad, 0, a.rexp, rr.w, rr.s};
+    const RangeSide y{a.nocc_b, a.nvir_b, a.nvir_pad_b, (int64_t)a.nocc * a.nvir_pad / 16, a.rexp_b,
+                      rr.w + (int64_t)a.nocc * naux_pad, rr.s + a.nocc};
+    hipLaunchKernelGGL(residue_norm_kernel,
+                       dim3((unsigned)a.np, (unsigned)(a.nocc + a.nocc_b)), dim3(256), 0, st,
+                       rr.norm, rr.gexp, naux_pad, x, y);
+    const int nb = rect ? a.nocc_b : a.nocc;
+    const double bar = bar_of(n), unit = ldexp(1.0, -2 * a.beta) / (bar * bar);
+    const double fixed = res::fixed_error(n) * (n == 16 ? res::kPhi<16> : res::kPhi<10>);
+    hipLaunchKernelGGL(residue_range_kernel, dim3((unsigned)(nb + 3) / 4, (unsigned)a.nocc),
+                       dim3(256), 0, st, rr.w, rr.s, rect ? y.w : x.w, rect ? y.s : x.s, nb,
+                       naux_pad, !rect, unit / 12.0,
+                       unit * fixed * ldexp(fixed, -2 * a.beta), wide);
+    return hipGetLastError();
+}
+
+hipError_t launch_residue_pack(Prec prec, const PackArgs &a, const ResidueOrder &ord,
+                               const ResidueRange &rr, hipStream_t st, int64_t nrg, int64_t rg0) {
     const int64_t own = (int64_t)a.nocc * a.nvir_pad / 16;
     if (nrg == 0) nrg = own;
     if (rg0 < 0 || rg0 + own > nrg) return hipErrorInvalidValue;
-    if (!a.rexp || !pmax || a.naux_pad % 64 != 0 || a.naux_pad < a.naux ||
+    if (!a.rexp || !rr.pmax || !rr.norm || a.naux_pad % 64 != 0 || a.naux_pad < a.naux ||
         a.naux_pad - a.naux >= 64 || a.naux_pad > res::kMaxNauxPad || a.nvir_pad % 16 != 0)
         return hipErrorInvalidValue;
     const int beta = residue_beta(prec, a.naux_pad);
     switch (prec) {
-    case Prec::F64: return launch_pack_n<16, false>(a, ord, pmax, beta, nrg, rg0, st);
-    case Prec::MIXED: return launch_pack_n<10, true>(a, ord, pmax, beta, nrg, rg0, st);
+    case Prec::F64: return launch_pack_n<16, false>(a, ord, rr, beta, nrg, rg0, st);
+    case Prec::MIXED: return launch_pack_n<10, true>(a, ord, rr, beta, nrg, rg0, st);
     default: return hipErrorInvalidValue;
     }
 }
@@ -824,7 +970,7 @@ hipError_t launch_residue_energy(const ResidueArgs &a, hipStream_t st) {
     const int ng = a.nvir_pad / 16;
     const bool rect = a.nocc_b > 0;
     const int64_t groups = (a.nocc + a.group - 1) / a.group;
-    if (!a.op || !a.rexp || !a.scratch || !a.queue || !a.order || a.blocks <= 0 ||
+    if (!a.op || !a.rexp || !a.scratch || !a.queue || !a.order || !a.wide || a.blocks <= 0 ||
         a.blocks % kXcds != 0 || a.nitems <= 0 || a.nitems > 0x7fffff00LL || a.np <= 0 ||
         a.np * 64 > res::kMaxNauxPad || a.nvir_pad % 16 != 0 || a.ntile * kTB < ng)
         return hipErrorInvalidValue;

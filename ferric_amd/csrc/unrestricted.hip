@@ -58,17 +58,16 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
     if (npairs * ntp > 0x7fffff00LL) return FH_OK;
     const size_t rows_a = ca.nocc * (size_t)pa.nvir_pad, rows_b = cb.nocc * (size_t)pb.nvir_pad;
     const size_t neps = ca.nocc + ca.nvir + cb.nocc + cb.nvir;
-    const int np = pa.naux_pad / 64;
     const size_t col_a = ca.nocc * ca.nvir, col_b = cb.nocc * cb.nvir;
     const Attempt attempt(s);
     ResidueSpace sp;
     fh_status st = reserve_residue(
-        s, Prec::F64, npairs * ntp, 1, rows_a + rows_b, pa.naux_pad,
-        {{kSlotColMax, sizeof(double) * (size_t)np * (col_a + col_b)},
-         {kSlotEps, sizeof(double) * neps},
+        s, Prec::F64, npairs * ntp, 1, col_a + col_b, rows_a + rows_b, ca.nocc + cb.nocc,
+        pa.naux_pad,
+        {{kSlotEps, sizeof(double) * neps},
          {kSlotItems, sizeof(double) * 4 * (size_t)(npairs * ntp)},
          {kSlotRows, sizeof(double) * 4 * ca.nocc},
-         {kSlotResult, sizeof(double) * (2 + 2 * ca.nocc)}},
+         {kSlotResult, sizeof(double) * (3 + 2 * ca.nocc)}},
         &sp);
     if (st == FH_POOL_FULL) {  // the matrix kernel needs half of it
         attempt.undo();
@@ -116,23 +115,25 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
     pk.naux_pad = pa.naux_pad;
     pk.out0 = sp.op;
     const int64_t nrg = (int64_t)(rows_a + rows_b) / 16;
-    double *pmax = (double *)s.slots[kSlotColMax].ptr;
     mark(s, 0, stream);
     pk.b = ba;
     pk.nocc = ra.nocc;
     pk.nvir = ra.nvir;
     pk.nvir_pad = ra.nvir_pad;
     pk.rexp = sp.rexp;
-    hipError_t he = launch_residue_pack(Prec::F64, pk, ord, pmax, stream, nrg, 0);
+    hipError_t he = launch_residue_pack(Prec::F64, pk, ord, sp.range, stream, nrg, 0);
     if (he == hipSuccess) {
         pk.b = bb;
         pk.nocc = ra.nocc_b;
         pk.nvir = ra.nvir_b;
         pk.nvir_pad = ra.nvir_pad_b;
         pk.rexp = sp.rexp + rows_a;
-        he = launch_residue_pack(Prec::F64, pk, ResidueOrder{}, pmax + (size_t)np * col_a, stream,
-                                 nrg, (int64_t)rows_a / 16);
+        ResidueRange beta = sp.range;
+        beta.pmax += (size_t)(pa.naux_pad / 64) * col_a;
+        he = launch_residue_pack(Prec::F64, pk, ResidueOrder{}, beta, stream, nrg,
+                                 (int64_t)rows_a / 16);
     }
+    if (he == hipSuccess) he = launch_residue_range(ra, sp.range, sp.wide, stream);
     if (he != hipSuccess) {
         (void)hipGetLastError();
         return fail(FH_KERNEL, "pack kernel: %s", hipGetErrorString(he));
@@ -152,16 +153,23 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
     ea.item_partials = ra.item_partials;
     ea.row_partials = (double *)s.slots[kSlotRows].ptr;
     ea.result = (double *)s.slots[kSlotResult].ptr;
+    ea.wide = sp.wide;
     he = launch_rect_reduce(ea, stream);
     if (he != hipSuccess) {
         (void)hipGetLastError();
         return fail(FH_KERNEL, "reduction kernels: %s", hipGetErrorString(he));
     }
     mark(s, 3, stream);
-    s.pending.kernel_launches += 6;
+    s.pending.kernel_launches += 8;
     fh_spin_components sc{};
-    st = fetch_result(s, ea.result, 0, stream, &sc, nullptr);
+    bool wide = false;
+    st = fetch_result(s, ea.result, ca.nocc, stream, &sc, nullptr, &wide);
     if (st != FH_OK) return st;
+    if (wide) {  // rows past its range
+        *taken = false;
+        attempt.undo();
+        return FH_OK;
+    }
     finish_timing(s, (uint64_t)(npairs * ntp), pa.tile);
     *energy = sc.e_os;
     return FH_OK;

@@ -60,9 +60,14 @@ typedef enum fh_status {
  * the pair-energy sums are FP64 (compensated) in every mode.
  *   FH_FP64     FP64 MFMA, FP64 accumulation (the plain method); energies, pair
  *               energies, unrestricted blocks and amplitudes of large problems in
- *               residue arithmetic instead: exact products of B rounded to about
- *               2^-56 of its row's range, from int8 products under 16 moduli, no
- *               less accurate
+ *               residue arithmetic instead: exact products, from int8 products under
+ *               16 moduli, of B with every row (i, a) rounded to 2^-(beta + 1) of
+ *               its power-of-two range, beta 55 to 58. A product's error is that
+ *               times the two rows' ranges and 1-norms, not sum_Q |B||B|: elements
+ *               far below their row's largest keep fewer bits than in FP64. A call
+ *               with a pair of occupied orbitals whose products would be off by more
+ *               than 2^-50 of themselves (root mean square over a, b) runs on FP64
+ *               MFMA, which the device decides
  *   FH_FP32     FP32 operands, FP32 MFMA, FP32 accumulation over the whole Q range
  *   FH_MIXED    FP32 operands (RN from the caller's values), FP32 MFMA over Q
  *               panels of at most 64 rows, each panel's sums added into FP64
@@ -71,8 +76,9 @@ typedef enum fh_status {
  *               crates/ferric-core/src/gpu/mixed.rs:70,122-180); refused
  *               (FH_RANGE) when max|B| > sqrt(FLT_MAX / 64), as the reference's
  *               check_f32_arithmetic_range with b = 64. Large problems: residue
- *               arithmetic under 10 moduli on the same FP32 operands, 2^-32 of
- *               the row's range, no panel sums
+ *               arithmetic under 10 moduli on the same FP32 operands, rounded to
+ *               2^-33 of the row's range, no panel sums; with the same test as in
+ *               FP64, at 2^-24
  *   FH_BF16X3   BF16 hi/lo split, hi*hi + hi*lo + lo*hi, FP32 accumulation
  *   FH_FP8_E4M3 OCP E4M3 operands with one power-of-two scale per
  *               (64-row Q block, occupied i), FP32 accumulation
