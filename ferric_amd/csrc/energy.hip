@@ -314,12 +314,16 @@ hipError_t launch_items(K kern, const EnergyArgs &a, hipStream_t st, int threads
     return hipGetLastError();
 }
 
-template <typename K>
-hipError_t launch_f64(K kern, const EnergyArgs &a, hipStream_t st) {
-    if (a.naux_pad < 16 || a.naux_pad % 16 != 0 || a.nvir_pad % 16 != 0 ||
-        64LL * a.naux_pad * 8 > 0xffffffffLL)  // row offsets inside a tile are 32-bit
+// pair_f64_kernel's row offsets inside a tile are 32-bit: past 8388607 aux functions the
+// register-staged body, whose offsets are not.
+template <bool AMP>
+hipError_t launch_f64(const EnergyArgs &a, hipStream_t st) {
+    if (64LL * a.naux_pad * 8 > 0xffffffffLL)
+        return launch_items(pair_k4_kernel<double, 64, 16, false, false, false, AMP>, a, st);
+    if (a.naux_pad < 16 || a.naux_pad % 16 != 0 || a.nvir_pad % 16 != 0)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kern, dim3((unsigned)a.nitems), dim3(256), kPBuf * kPStage, st, a);
+    hipLaunchKernelGGL(pair_f64_kernel<AMP>, dim3((unsigned)a.nitems), dim3(256),
+                       kPBuf * kPStage, st, a);
     return hipGetLastError();
 }
 
@@ -331,7 +335,7 @@ hipError_t launch_energy(const EnergyArgs &a, hipStream_t st) {
     if (a.amp.base) {  // FP64 energy that also stores the amplitudes
         if (a.prec != Prec::F64 || a.q_neg < a.naux_pad) return hipErrorInvalidValue;
         if (a.tile == 128) e = launch_items(pair_k4_kernel<double, 128, 16, false, false, false, true>, a, st);
-        else if (a.tile == 64) e = launch_f64(pair_f64_kernel<true>, a, st);
+        else if (a.tile == 64) e = launch_f64<true>(a, st);
         else if (a.tile == 32) e = launch_items(pair_k4_kernel<double, 32, 16, false, false, false, true>, a, st);
         return e;
     }
@@ -350,7 +354,7 @@ hipError_t launch_energy(const EnergyArgs &a, hipStream_t st) {
     switch (a.prec) {
     case Prec::F64:
         if (a.tile == 128) e = launch_items(pair_k4_kernel<double, 128, 16, false>, a, st);
-        else if (a.tile == 64) e = launch_f64(pair_f64_kernel<false>, a, st);
+        else if (a.tile == 64) e = launch_f64<false>(a, st);
         else if (a.tile == 32) e = launch_items(pair_k4_kernel<double, 32, 16, false>, a, st);
         break;
     case Prec::F32:
