@@ -83,6 +83,8 @@ static fh_status init_locked(State &s, int device) {
                     prop.gcnArchName);
     if (hipSetDevice(device) != hipSuccess) return fail(FH_DEVICE, "hipSetDevice(%d)", device);
     s.device = device;
+    s.cus = 0;  // asked anew
+    s.wall_khz = -1;
     s.initialised = true;
     return FH_OK;
 }
