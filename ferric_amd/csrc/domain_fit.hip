@@ -4,8 +4,8 @@
 //   J_ij = A_{i,D}^T V_DD^{-1} A_{j,D},   D = the aux functions within `radius`
 //                                          of the centre of i or of j,
 //
-// with A the unwhitened (P|ia) and V the aux metric: one workgroup per pair gathers,
-// factors, solves and multiplies.
+// with A the unwhitened (P|ia) and V the aux metric: one workgroup per pair, or several
+// for large domains, gathers, factors, solves and multiplies.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -47,6 +47,7 @@ struct FitArgs {
     int cap;               // rows of a slot, a multiple of 16
     int32_t *dom;          // cap per pair
     double *u;             // cap (cap + 32 nv) per pair
+    int32_t *size;         // split rows: the domain's size per pair
     int32_t *info;
     double *j;
 };
@@ -61,19 +62,11 @@ __device__ __forceinline__ double lane_value(double x, int lane) {
     return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
-__global__ __launch_bounds__(kFitThreads, 4) void fit_pair_kernel(FitArgs g) {
-    __shared__ double diag[16][17];
-    __shared__ double linv[16][17];
+// The domain: the aux functions near i or j, in aux order. Its size.
+__device__ __forceinline__ int fit_domain(const FitArgs &g, int oi, int oj, int32_t *dom) {
     __shared__ int wsum[kFitWaves];
-    __shared__ int bad;
     const int tid = threadIdx.x, lane = tid % kWave;
     const int wid = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int r = lane % 16, gg = lane / 16;
-    const int64_t p = blockIdx.x;
-    const int oi = g.pairs[2 * p], oj = g.pairs[2 * p + 1];
-    int32_t *dom = g.dom + p * g.cap;
-
-    // The domain: the aux functions near i or j, in aux order.
     int d = 0;
     for (int w0 = 0; w0 < g.words; w0 += kFitThreads) {
         const int w = w0 + tid;
@@ -97,160 +90,175 @@ __global__ __launch_bounds__(kFitThreads, 4) void fit_pair_kernel(FitArgs g) {
         d += total;
         __syncthreads();
     }
-    if (tid == 0) bad = 0;
-    d = __builtin_amdgcn_readfirstlane(d);
+    return __builtin_amdgcn_readfirstlane(d);
+}
+
+// Block row k of a pair's elimination: the diagonal block and the columns past it, c of C
+// workgroups taking every C-th turn of kFitHeld blocks a wave (SPLIT), or all. Each of them
+// factors the diagonal block for itself. The first bad pivot, from 1, or 0.
+template <bool SPLIT>
+__device__ __forceinline__ int fit_row(const FitArgs &g, int oi, int oj, const int32_t *dom, int d,
+                                       double *u, int k, int c, int C) {
+    __shared__ double diag[16][17];
+    __shared__ double linv[16][17];
+    __shared__ int bad;
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int wid = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int r = lane % 16, gg = lane / 16;
     const int nd = (d + 15) / 16;
     const int64_t ldu = (int64_t)(nd + 2 * g.nv) * 16;
-    double *u = g.u + p * g.cap * (int64_t)(g.cap + 32 * g.nv);
     const uint32_t off = (uint32_t)(gg * (int)ldu + r);
-
-    for (int k = 0; k < nd; ++k) {
-        const int nblk = nd - k + 2 * g.nv;  // block t: columns 16 (k + t) .. + 16
-        int row[4];
+    const int nblk = nd - k + 2 * g.nv;  // block t: columns 16 (k + t) .. + 16
+    int row[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) row[v] = dom[min(16 * k + 4 * v + gg, d - 1)];
-        // Blocks t = t0 + wid, t0 + wid + 4, ..., H of them (one past the last stands for
-        // it and is not stored), as they stand before any elimination (the lower triangle
-        // of V, the identity past the domain, A past V), less the products with the rows
-        // above. All loads of a step are issued before the products of the last one.
-        v4d acc[kFitHeld];
-        auto update = [&](auto held, int t0) {
-            constexpr int H = decltype(held)::value;
-            int32_t first[H];  // of the column: V's row, A's column
+    for (int v = 0; v < 4; ++v) row[v] = dom[min(16 * k + 4 * v + gg, d - 1)];
+    // Blocks t = t0 + wid, t0 + wid + 4, ..., H of them (one past the last stands for
+    // it and is not stored), as they stand before any elimination (the lower triangle
+    // of V, the identity past the domain, A past V), less the products with the rows
+    // above. All loads of a step are issued before the products of the last one.
+    v4d acc[kFitHeld];
+    auto update = [&](auto held, int t0) {
+        constexpr int H = decltype(held)::value;
+        int32_t first[H];  // of the column: V's row, A's column
 #pragma unroll
-            for (int q = 0; q < H; ++q) {
-                const int t = min(t0 + wid + q * kFitWaves, nblk - 1), x = t - (nd - k);
-                first[q] = x < 0 ? dom[min(16 * (k + t) + r, d - 1)]
-                                 : min((x < g.nv ? x : x - g.nv) * 16 + r, g.nvir - 1);
-            }
+        for (int q = 0; q < H; ++q) {
+            const int t = min(t0 + wid + q * kFitWaves, nblk - 1), x = t - (nd - k);
+            first[q] = x < 0 ? dom[min(16 * (k + t) + r, d - 1)]
+                             : min((x < g.nv ? x : x - g.nv) * 16 + r, g.nvir - 1);
+        }
 #pragma unroll
-            for (int q = 0; q < H; ++q) {
-                const int t = min(t0 + wid + q * kFitWaves, nblk - 1), x = t - (nd - k);
-                const double *base = x < 0 ? g.v : g.a + (int64_t)(x < g.nv ? oi : oj) * g.nvir;
-                const int64_t sr = x < 0 ? 1 : g.nov, sc = x < 0 ? g.naux : 1;
+        for (int q = 0; q < H; ++q) {
+            const int t = min(t0 + wid + q * kFitWaves, nblk - 1), x = t - (nd - k);
+            const double *base = x < 0 ? g.v : g.a + (int64_t)(x < g.nv ? oi : oj) * g.nvir;
+            const int64_t sr = x < 0 ? 1 : g.nov, sc = x < 0 ? g.naux : 1;
 #pragma unroll
-                for (int v = 0; v < 4; ++v) acc[q][v] = base[row[v] * sr + first[q] * sc];
+            for (int v = 0; v < 4; ++v) acc[q][v] = base[row[v] * sr + first[q] * sc];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const double *um = u + 16 * k, *ut = um + 16 * (t0 + wid);
+        const int last = 16 * (min(t0 + wid + (H - 1) * kFitWaves, nblk - 1) - t0 - wid);
+        double fa[2][2], fb[2][2][H];
+        auto fetch = [&](int h) {  // half of the 16 rows at um
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int64_t at = 4 * (2 * h + s) * ldu;
+                fa[h][s] = (um + at)[off];
+#pragma unroll
+                for (int q = 0; q < H; ++q)
+                    fb[h][s][q] = (ut + at + (q + 1 < H ? 16 * kFitWaves * q : last))[off];
             }
             __builtin_amdgcn_sched_barrier(0);
-            const double *um = u + 16 * k, *ut = um + 16 * (t0 + wid);
-            const int last = 16 * (min(t0 + wid + (H - 1) * kFitWaves, nblk - 1) - t0 - wid);
-            double fa[2][2], fb[2][2][H];
-            auto fetch = [&](int h) {  // half of the 16 rows at um
-#pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    const int64_t at = 4 * (2 * h + s) * ldu;
-                    fa[h][s] = (um + at)[off];
-#pragma unroll
-                    for (int q = 0; q < H; ++q)
-                        fb[h][s][q] = (ut + at + (q + 1 < H ? 16 * kFitWaves * q : last))[off];
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            auto products = [&](int h) {
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-#pragma unroll
-                    for (int q = 0; q < H; ++q)
-                        acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(-fa[h][s], fb[h][s][q],
-                                                                      acc[q], 0, 0, 0);
-            };
-            if (k > 0) fetch(0);
-#pragma unroll
-            for (int q = 0; q < H; ++q) {
-                const int t = min(t0 + wid + q * kFitWaves, nblk - 1), x = t - (nd - k);
-                const int C = 16 * (k + t) + r, lim = (x < g.nv ? g.nvir : g.nvir + 16 * g.nv);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int R = 16 * k + 4 * v + gg;
-                    const bool in = R < d && (x < 0 ? C < d : 16 * x + r < lim);
-                    acc[q][v] = in ? acc[q][v] : (R == C ? 1.0 : 0.0);
-                }
-            }
-            for (int m = 0; m < k; ++m) {
-                fetch(1);
-                products(0);
-                if (m + 1 < k) {
-                    um += 16 * ldu;
-                    ut += 16 * ldu;
-                }
-                fetch(0);
-                products(1);
-            }
         };
-        auto finish = [&](auto held, int t0) {
-            constexpr int H = decltype(held)::value;
-            double fa[4];
+        auto products = [&](int h) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) fa[s] = linv[r][4 * s + gg];
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int q = 0; q < H; ++q) {
-                const int t = t0 + wid + q * kFitWaves;
-                v4d o = {0, 0, 0, 0};
+                for (int q = 0; q < H; ++q)
+                    acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(-fa[h][s], fb[h][s][q],
+                                                                  acc[q], 0, 0, 0);
+        };
+        if (k > 0) fetch(0);
 #pragma unroll
-                for (int s = 0; s < 4; ++s)
-                    o = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s], acc[q][s], o, 0, 0, 0);
-                if (t >= nblk || t == 0) continue;
+        for (int q = 0; q < H; ++q) {
+            const int t = min(t0 + wid + q * kFitWaves, nblk - 1), x = t - (nd - k);
+            const int C = 16 * (k + t) + r, lim = (x < g.nv ? g.nvir : g.nvir + 16 * g.nv);
 #pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    (u + (16 * k + 4 * v) * ldu + 16 * (k + t))[off] = o[v];
+            for (int v = 0; v < 4; ++v) {
+                const int R = 16 * k + 4 * v + gg;
+                const bool in = R < d && (x < 0 ? C < d : 16 * x + r < lim);
+                acc[q][v] = in ? acc[q][v] : (R == C ? 1.0 : 0.0);
             }
-        };
-        auto with_held = [&](int t0, auto f) {
-            const int n = (nblk - t0 + kFitWaves - 1) / kFitWaves;
-            if (n >= kFitHeld) f(std::integral_constant<int, kFitHeld>{});
-            else if (n == 5) f(std::integral_constant<int, 5>{});
-            else if (n == 4) f(std::integral_constant<int, 4>{});
-            else if (n == 3) f(std::integral_constant<int, 3>{});
-            else if (n == 2) f(std::integral_constant<int, 2>{});
-            else f(std::integral_constant<int, 1>{});
-        };
+        }
+        for (int m = 0; m < k; ++m) {
+            fetch(1);
+            products(0);
+            if (m + 1 < k) {
+                um += 16 * ldu;
+                ut += 16 * ldu;
+            }
+            fetch(0);
+            products(1);
+        }
+    };
+    auto finish = [&](auto held, int t0) {
+        constexpr int H = decltype(held)::value;
+        double fa[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) fa[s] = linv[r][4 * s + gg];
+#pragma unroll
+        for (int q = 0; q < H; ++q) {
+            const int t = t0 + wid + q * kFitWaves;
+            v4d o = {0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                o = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s], acc[q][s], o, 0, 0, 0);
+            if (t >= nblk || t == 0) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                (u + (16 * k + 4 * v) * ldu + 16 * (k + t))[off] = o[v];
+        }
+    };
+    auto with_held = [&](int t0, auto f) {
+        const int n = (nblk - t0 + kFitWaves - 1) / kFitWaves;
+        if (n >= kFitHeld) f(std::integral_constant<int, kFitHeld>{});
+        else if (n == 4) f(std::integral_constant<int, 4>{});
+        else if (n == 3) f(std::integral_constant<int, 3>{});
+        else if (n == 2) f(std::integral_constant<int, 2>{});
+        else f(std::integral_constant<int, 1>{});
+    };
+    if (!SPLIT || c == 0)
         with_held(0, [&](auto h) { update(h, 0); });
-        if (wid == 0)
+    else
+        update(std::integral_constant<int, 1>{}, 0);
+    if (wid == 0)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) diag[4 * v + gg][r] = acc[0][v];
-        __syncthreads();
-        if (wid == 0) {
-            // Lanes 0 .. 15 hold the block's columns, 16 .. 31 the identity's; rows below
-            // the diagonal of a column are never read by another lane.
-            double c[16];
+        for (int v = 0; v < 4; ++v) diag[4 * v + gg][r] = acc[0][v];
+    __syncthreads();
+    if (wid == 0) {
+        // Lanes 0 .. 15 hold the block's columns, 16 .. 31 the identity's; rows below
+        // the diagonal of a column are never read by another lane.
+        double c[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
-                c[i] = lane < 16 ? diag[i][r] : (lane < 32 && i == r ? 1.0 : 0.0);
-            int fault = 0;
+        for (int i = 0; i < 16; ++i)
+            c[i] = lane < 16 ? diag[i][r] : (lane < 32 && i == r ? 1.0 : 0.0);
+        int fault = 0;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const double piv = lane_value(c[i], i);
-                // Not positive, NaN, or infinite: a non-finite element of the metric reaches
-                // a pivot as one of them.
-                if (!(piv > 0.0 && piv < INFINITY) && fault == 0) fault = 16 * k + i + 1;
-                c[i] *= 1.0 / sqrt(piv);
+        for (int i = 0; i < 16; ++i) {
+            const double piv = lane_value(c[i], i);
+            // Not positive, NaN, or infinite: a non-finite element of the metric reaches
+            // a pivot as one of them.
+            if (!(piv > 0.0 && piv < INFINITY) && fault == 0) fault = 16 * k + i + 1;
+            c[i] *= 1.0 / sqrt(piv);
 #pragma unroll
-                for (int x = i + 1; x < 16; ++x) c[x] -= lane_value(c[i], x) * c[i];
-            }
-            if (lane >= 16 && lane < 32)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) linv[i][r] = c[i];
-            if (lane == 0) bad = fault;
+            for (int x = i + 1; x < 16; ++x) c[x] -= lane_value(c[i], x) * c[i];
         }
-        __syncthreads();
-        if (bad) {
-            if (tid == 0) g.info[p] = bad;
-            return;
-        }
-        with_held(0, [&](auto h) { finish(h, 0); });
-        for (int t0 = kFitHeld * kFitWaves; t0 < nblk; t0 += kFitHeld * kFitWaves) {
-            with_held(t0, [&](auto h) { update(h, t0); });
-            with_held(t0, [&](auto h) { finish(h, t0); });
-        }
-        __syncthreads();
+        if (lane >= 16 && lane < 32)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) linv[i][r] = c[i];
+        if (lane == 0) bad = fault;
     }
-    if (tid == 0) g.info[p] = 0;
+    __syncthreads();
+    if (bad) return bad;
+    if (!SPLIT || c == 0) with_held(0, [&](auto h) { finish(h, 0); });
+    const int turn = kFitHeld * kFitWaves;
+    for (int t0 = (!SPLIT ? 1 : c == 0 ? C : c) * turn; t0 < nblk; t0 += (SPLIT ? C : 1) * turn) {
+        with_held(t0, [&](auto h) { update(h, t0); });
+        with_held(t0, [&](auto h) { finish(h, t0); });
+    }
+    __syncthreads();
+    return 0;
+}
 
-    // J = Y_i^T Y_j, 32 x 64 a wave and turn.
+// Turns first, first + step, ... of J = Y_i^T Y_j, 32 x 64 a wave and turn.
+__device__ __forceinline__ void fit_product(const FitArgs &g, int d, const double *u, double *jp,
+                                            int first, int step) {
+    const int lane = threadIdx.x % kWave, r = lane % 16, gg = lane / 16;
+    const int nd = (d + 15) / 16;
+    const int64_t ldu = (int64_t)(nd + 2 * g.nv) * 16;
+    const uint32_t off = (uint32_t)(gg * (int)ldu + r);
     const int na = (g.nv + 1) / 2, nb = (g.nv + 3) / 4;
     const double *yi = u + 16 * nd, *yj = yi + 16 * g.nv;
-    double *jp = g.j + p * (int64_t)g.nvir * g.nvir;
-    for (int t = wid; t < na * nb; t += kFitWaves) {
+    for (int t = first; t < na * nb; t += step) {
         const int a0 = t / nb * 2, b0 = t % nb * 4;
         int ca[2], cb[4];  // blocks past the end repeat the last one
 #pragma unroll
@@ -308,6 +316,83 @@ __global__ __launch_bounds__(kFitThreads, 4) void fit_pair_kernel(FitArgs g) {
     }
 }
 
+__device__ __forceinline__ double *fit_slot(const FitArgs &g, int64_t p) {
+    return g.u + p * g.cap * (int64_t)(g.cap + 32 * g.nv);
+}
+
+__global__ __launch_bounds__(kFitThreads, 4) void fit_pair_kernel(FitArgs g) {
+    const int64_t p = blockIdx.x;
+    const int oi = g.pairs[2 * p], oj = g.pairs[2 * p + 1];
+    int32_t *dom = g.dom + p * g.cap;
+    const int d = fit_domain(g, oi, oj, dom);
+    double *u = fit_slot(g, p);
+    for (int k = 0; k < (d + 15) / 16; ++k)
+        if (const int bad = fit_row<false>(g, oi, oj, dom, d, u, k, 0, 1)) {
+            if (threadIdx.x == 0) g.info[p] = bad;
+            return;
+        }
+    if (threadIdx.x == 0) g.info[p] = 0;
+    fit_product(g, d, u, g.j + p * (int64_t)g.nvir * g.nvir,
+                __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), kFitWaves);
+}
+
+// ---- Several workgroups per pair -----------------------------------------------
+// The same operations in the same order, a launch to a block row, for large domains: one
+// workgroup takes d^3 (359 ms for a domain of 6000, and the rest of the chip idles).
+__global__ __launch_bounds__(kFitThreads) void fit_domain_kernel(FitArgs g) {
+    const int64_t p = blockIdx.x;
+    const int d = fit_domain(g, g.pairs[2 * p], g.pairs[2 * p + 1], g.dom + p * g.cap);
+    if (threadIdx.x == 0) {
+        g.size[p] = d;
+        g.info[p] = 0;
+    }
+}
+
+__global__ __launch_bounds__(kFitThreads, 2) void fit_row_kernel(FitArgs g, int k) {
+    const int64_t p = blockIdx.x;
+    const int d = g.size[p], nblk = (d + 15) / 16 - k + 2 * g.nv;
+    // A pair whose bad pivot was found is of no more interest.
+    if (16 * k >= d || (int)blockIdx.y * kFitHeld * kFitWaves >= nblk || g.info[p]) return;
+    const int bad = fit_row<true>(g, g.pairs[2 * p], g.pairs[2 * p + 1], g.dom + p * g.cap, d,
+                                  fit_slot(g, p), k, blockIdx.y, gridDim.y);
+    if (bad && blockIdx.y == 0 && threadIdx.x == 0) g.info[p] = bad;
+}
+
+__global__ __launch_bounds__(kFitThreads, 2) void fit_product_kernel(FitArgs g) {
+    const int64_t p = blockIdx.x;
+    if (g.info[p]) return;
+    fit_product(g, g.size[p], fit_slot(g, p), g.j + p * (int64_t)g.nvir * g.nvir,
+                __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) + kFitWaves * blockIdx.y,
+                kFitWaves * gridDim.y);
+}
+
+// Where n pairs of up to dmax aux functions take several workgroups each. ms, one / several, at
+// 100 virtuals: 16 pairs of 300 0.44 / 0.40, 16 of 400 0.64 / 0.58 (36 at 20 virtuals 0.48 /
+// 0.50), 64 of 480 0.99 / 0.79, 136 of 480 1.02 / 1.08, 820 of 480 4.75 / 5.10, 1 of 1000 3.6 /
+// 2.4, 400 of 1000 14.05 / 14.00, 300 of 1500 34.5 / 31.2, 1 of 2000 18.9 / 8.8, 400 of 2000
+// 124 / 88, 4 of 3000 54 / 20, 1 of 6000 360 / 76 (100 with rocSOLVER and rocBLAS).
+bool split_rows(size_t dmax, size_t n) { return dmax >= 1000 || (dmax >= 400 && n <= 64); }
+
+hipError_t launch_fit(const FitArgs &g, size_t n, bool split, hipStream_t st, uint64_t *launches) {
+    if (!split) {
+        hipLaunchKernelGGL(fit_pair_kernel, dim3((unsigned)n), dim3(kFitThreads), 0, st, g);
+        *launches += 1;
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(fit_domain_kernel, dim3((unsigned)n), dim3(kFitThreads), 0, st, g);
+    auto grid = [&](int blocks, int per) {
+        return dim3((unsigned)n, (unsigned)((blocks + per - 1) / per));
+    };
+    for (int k = 0; k < g.cap / 16; ++k)
+        hipLaunchKernelGGL(fit_row_kernel,
+                           grid(g.cap / 16 - k + 2 * g.nv, kFitHeld * kFitWaves),
+                           dim3(kFitThreads), 0, st, g, k);
+    hipLaunchKernelGGL(fit_product_kernel, grid((g.nv + 1) / 2 * ((g.nv + 3) / 4), kFitWaves),
+                       dim3(kFitThreads), 0, st, g);
+    *launches += (uint64_t)g.cap / 16 + 2;
+    return hipGetLastError();
+}
+
 // Pairs of one batch, of `per` bytes each: 4 GiB of them.
 size_t fit_batch(size_t npairs, size_t per) {
     size_t nb = 0;
@@ -334,14 +419,15 @@ fh_status fit_pairs(State &s, const double *a, const double *v, size_t naux, siz
     const size_t near_bytes = sizeof(uint64_t) * near.size();
     fh_status st = reserve(s, {{kSlotFitWork, sizeof(double) * nb * slot},
                                {kSlotFitMeta, near_bytes + sizeof(int32_t) * (npairs * 2 +
-                                                                              nb * (cap + 1))}});
+                                                                              nb * (cap + 2))}});
     if (st != FH_OK) return st;
     g.u = (double *)s.slots[kSlotFitWork].ptr;
     uint64_t *dnear = (uint64_t *)s.slots[kSlotFitMeta].ptr;
     int32_t *dpairs = (int32_t *)(dnear + near.size());
     g.near = dnear;
     g.dom = dpairs + 2 * npairs;
-    g.info = g.dom + nb * cap;
+    g.size = g.dom + nb * cap;
+    g.info = g.size + nb;
     st = hip_check(hipMemcpyAsync(dnear, near.data(), near_bytes, hipMemcpyHostToDevice, stream),
                    "H2D domains");
     if (st != FH_OK) return st;
@@ -357,10 +443,9 @@ fh_status fit_pairs(State &s, const double *a, const double *v, size_t naux, siz
         const size_t n = std::min(nb, npairs - p0);
         g.pairs = dpairs + 2 * p0;
         g.j = j_out + p0 * nvir * nvir;
-        hipLaunchKernelGGL(fit_pair_kernel, dim3((unsigned)n), dim3(kFitThreads), 0, stream, g);
-        st = hip_check(hipGetLastError(), "domain fit kernel");
+        st = hip_check(launch_fit(g, n, split_rows(dmax, n), stream, &s.pending.kernel_launches),
+                       "domain fit kernel");
         if (st != FH_OK) return st;
-        s.pending.kernel_launches += 1;
         st = hip_check(hipMemcpyAsync(info.data(), g.info, sizeof(int32_t) * n,
                                       hipMemcpyDeviceToHost, stream),
                        "D2H Cholesky info");
