@@ -417,39 +417,56 @@ fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, siz
     return FH_OK;
 }
 
-// Which calls run in residue arithmetic (residue.hip), and on what tiles. Measured
-// against the matrix kernel of the same precision (its time / residue time):
-// FP64    the chip is full and the rebuild of a product (16 moduli, the same at any aux
-//         count) is small beside it: 24/208/742 1.15, 70/208/889 1.4, 100/200/2400 1.9,
-//         60/450/1800 1.8, 100/900/3600 1.8. Small work: 20/150/529 1.13, 12/160/1100
-//         1.0, 11/250/500 0.8; few pairs: 10/250/1500 1.3, 8/256/1059 below 1. With 65 to
-//         128 virtuals two orbitals share a tile: 60/66/627 1.1, 60/80/420 1.0, 40/112/486
-//         1.1, 20/128/726 0.8. Two tiles: 16/400/919 1.1, 9/400/1600 1.0, and up to 362
-//         virtuals, where a third of the tiles' area is used: 16/300/1633 1.07 but
-//         24/300/900 0.94, 30/280/700 0.9. Fewer than 65 virtuals: below 1.
-// MIXED   24/208/742 1.35, 70/208/889 2.0, 60/450/1800 1.8, 24/160/588 1.15, 40/112/486
-//         1.2, 24/112/435 0.9.
+// Which calls run in residue arithmetic (residue.hip): those whose pass is estimated at less
+// than 0.93 of that of the matrix kernel of the same precision, 64-wide, for which the 1500
+// calls of residue_estimate gave the constants below (off by 7% in FP64, 4% in MIXED, 6%
+// opposite spin). Residues need a full chip (rounds of a workgroup per CU) and a rebuild of
+// the products, the same at any aux count, that is small beside them. matrix / residue, us:
+// FP64 15/215/4073 1325 / 604, 51/109/4278 2799 / 1510, but 46/200/60 and 25/153/503 (264 / 295)
+// the other way; MIXED 36/221/2347 2633 / 1167, but 23/491/177 574 / 781. Over 900 other calls
+// of the same ranges 453 went to the residues: 7 of 180 in FP64 by more than 2% slower so (at
+// most 5%), none of 137 in MIXED, 4 of 136 in opposite spin (at most 7%).
+// Fewer than 65 virtuals leave three quarters of a tile empty: never faster.
 // INT8X4 stays with its digit slices: ten moduli against their thirteen products gave
-//         70/208/889 1.2, but 70/340/1312 0.95 and 100/900/3600 0.98.
+// 70/208/889 1.2, but 70/340/1312 0.95 and 100/900/3600 0.98.
+// FERRIC_HIP_TILE=256 takes the residues wherever they can run.
+bool residue_pays(const ResidueShape &p, double flops, double items, double naux) {
+    if (forced_residue()) return true;
+    // Products of the padded virtuals, and of whole 64 x 64 tiles (which the opposite-spin
+    // kernel multiplies), in FLOP; tiles, and the depth of one.
+    const double tiles = items * 4096.0 * (p.rect ? 2.0 : 4.0) * naux;
+    const double matrix =
+        p.rect ? 67 + flops * 2.9e-9 + tiles * 16e-9 + items * 12.8e-3 + naux * 30e-3
+        : p.prec == Prec::F64
+            ? 75 + flops * 15.1e-9 + tiles * 1.2e-9 + items * 7.8e-3 + naux * 37e-3
+            : 138 + flops * 6.3e-9 + tiles * 4.9e-9 + items * 14.7e-3 + naux * 45e-3;
+    return residue_estimate(p) < 0.93 * matrix;
+}
+
 bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, EnergyPlan *pl) {
     EnergyPlan p;
-    if (!residue_tiles(s, nvir, naux, &p)) return false;
+    if ((prec != Prec::F64 && prec != Prec::MIXED) || nvir <= 64 ||
+        !residue_tiles(s, nvir, naux, &p))
+        return false;
     p.group = nvir <= 128 ? 2 : 1;
-    const double work = (double)nocc * (nocc + 1) * (double)nvir * nvir * (double)naux;
-    if (nvir <= 64) return false;
-    switch (prec) {
-    case Prec::F64:
-        if (work < (nvir <= 128 || nocc < 11 ? 1e10 : nvir <= 256 ? 5e9 : 3e10)) return false;
-        if (nvir > 256 && nvir <= 362 && naux < 1500) return false;
-        break;
-    case Prec::MIXED:
-        if (work < 5e9) return false;
-        break;
-    default: return false;
-    }
     const int64_t ngroup = ((int64_t)nocc + p.group - 1) / p.group;
-    p.nitems = ngroup * (ngroup + 1) / 2 * p.ntp;
+    const int64_t pairs = ngroup * (ngroup + 1) / 2;
+    p.nitems = pairs * p.ntp;
     if (p.nitems > 0x7fffff00LL) return false;
+    ResidueShape r;
+    r.prec = prec;
+    r.pairs = pairs;
+    r.ntile = p.ntile;
+    r.ntp = p.ntp;
+    r.wA = r.wB = p.group * ((p.nvir_pad / 16 + p.ntile - 1) / p.ntile);
+    r.np = p.naux_pad / 64;
+    r.cus = s.cus;
+    r.elements = (double)naux * (double)(nocc * nvir);
+    const double unique = 0.5 * (double)nocc * (double)(nocc + 1), vp = p.nvir_pad;
+    const double t = (p.nvir_pad + 63) / 64;
+    if (!residue_pays(r, 2.0 * unique * vp * vp * (double)naux, unique * t * (t + 1) / 2,
+                      (double)naux))
+        return false;
     *pl = p;
     return true;
 }

@@ -150,6 +150,8 @@ fh_status range_check(State &s, const void *b, bool in_f32, size_t n, size_t dep
 EnergyPlan plan_energy(size_t nocc, size_t nvir, size_t naux, Prec prec);
 // FERRIC_HIP_TILE's tile side, or 0 when it is unset.
 int forced_tile();
+// FERRIC_HIP_TILE=256: residue arithmetic wherever it can run.
+bool forced_residue();
 // Tile side of n batched domains: FERRIC_HIP_TILE's if set, else the first
 // tile-table entry whose bounds hold the domain, else 0 (one environment
 // read, one lock).
@@ -178,6 +180,8 @@ int compute_units(State &s);  // of the device, asked once; at least 1
 // run at all (aux count, forced tiles, fixed arena); whether an energy of this
 // shape is faster so, and its plan; and the workspace of a launch.
 bool residue_tiles(State &s, size_t nvir, size_t naux, EnergyPlan *pl);
+// Whether it is faster: FLOP and 64 x 64 items of the padded problem on the matrix kernel.
+bool residue_pays(const ResidueShape &p, double flops, double items, double naux);
 struct ResidueSpace {
     ResidueArgs args;    // prec, np, beta, op, rexp, nitems, blocks, scratch, queue, order
     ResidueOrder order;  // words, queue, order

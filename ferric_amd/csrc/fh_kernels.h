@@ -225,6 +225,15 @@ struct ResidueOrder {
     int words = 0;           // of the queue
     int *queue = nullptr, *order = nullptr;
 };
+// A pass as its kernel will run it: tiles of wA x wB blocks, products of two where rect is not.
+struct ResidueShape {
+    Prec prec = Prec::F64;
+    int64_t pairs = 0;     // of orbital groups
+    int ntile = 0, ntp = 0, wA = 0, wB = 0, np = 0, cus = 0;
+    bool rect = false;
+    double elements = 0;   // of B
+};
+double residue_estimate(const ResidueShape &p);  // us of a call
 int residue_moduli(Prec prec);
 int residue_beta(Prec prec, int naux_pad);
 // Plane sets of a launch: one per workgroup, and one per item of a split round (two

@@ -37,6 +37,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "fh_device.h"
 #include "fh_kernels.h"
 #include "pair_body.h"
@@ -132,7 +134,8 @@ __device__ void order_items(const ResidueOrder &o) {
 
 // One 64 x 64 tile (64 packed rows, one Q panel) to residues. The exponent f of a row
 // is that of the INT8X4 format: the least with max |x| <= (1 - 2^-7) 2^(f + 1); Y =
-// RN(x 2^(beta - 1 - f)). The rows go to row groups rg0 on, of nrg in all. ROUND32: x is first rounded to FP32 (MIXED).
+// RN(x 2^(beta - 1 - f)). The rows go to row groups rg0 on, of nrg in all. ROUND32: x is
+// first rounded to FP32 (MIXED).
 template <int N, bool ROUND32, typename Tin>
 __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict__ b, int64_t nov,
                                                            int naux, int nvir, int nvir_pad,
@@ -900,6 +903,37 @@ hipError_t launch_pack_n(const PackArgs &a, const ResidueOrder &ord, const Resid
 
 }  // namespace
 
+// The longest XCD's rounds (the last by the moduli that its split workgroups take each), in
+// steps of a panel and modulus whose cost follows the blocks that the waves multiply, and in
+// rebuilds; packing; launches and the wait. Fitted to 1500 calls of 65 to 560 virtuals, 4 to
+// 90 occupied and 60 to 4608 aux functions (0.15 to 20 ms): off by 9% in FP64 and 6% in MIXED.
+double residue_estimate(const ResidueShape &p) {
+    const int n = residue_moduli(p.prec), wide = p.cus / kXcds;
+    double steps = 0.0, ends = 0.0;
+    for (int x = 0; x < kXcds; ++x) {
+        const int64_t items = (p.pairs * (x + 1) / kXcds - p.pairs * x / kXcds) * p.ntp;
+        const int64_t full = items / wide;
+        const int rest = (int)(items % wide), split = rest ? std::min(wide / rest, kMaxSplit) : 1;
+        const double part = rest ? (double)((n + split - 1) / split) / n : 0.0;
+        steps = std::max(steps, (double)full + part);
+        ends = std::max(ends, (double)full + (rest ? 1 : 0));
+    }
+    // Off-diagonal tile pairs take two products; a single round is as long as its longest item.
+    const double products =
+        p.rect ? 1.0 : ends <= 1.0 && p.ntile > 1 ? 2.0 : 2.0 * p.ntile / (p.ntile + 1);
+    const int rows = (p.wA + 1) / 2, blocks = p.wA + p.wB;  // run_rows' choice
+    const int nx = rows <= 4 && blocks <= 16   ? 4
+                   : rows <= 6 && blocks <= 24 ? 6
+                   : rows <= 7                 ? 7
+                                               : 8;
+    const int ny = std::max(2, (p.wB + 3) / 4);
+    const bool f64 = p.prec == Prec::F64;
+    const double step = f64 ? 0.30 + 0.43 * nx * ny / 32.0 : 0.34 + 0.24 * nx * ny / 32.0;
+    return (f64 ? 100.0 : 150.0) + steps * products * n * p.np * step +
+           ends * products * n * (p.wA * p.wB / 256.0) * (f64 ? 7.5 : 10.4) +
+           p.elements * (f64 ? 1.0e-6 : 9.0e-6);
+}
+
 int residue_moduli(Prec prec) { return prec == Prec::F64 ? 16 : 10; }
 
 int residue_beta(Prec prec, int naux_pad) {
@@ -918,7 +952,8 @@ size_t residue_scratch_stride(Prec prec, int products) {
 
 size_t ResidueRange::bytes(size_t nov, size_t nrg, size_t norb, int naux_pad) {
     const size_t np = (size_t)naux_pad;
-    return sizeof(double) * (np / 64 * nov + norb * (np + 1)) + (sizeof(float) * np + sizeof(int)) * nrg;
+    return sizeof(double) * (np / 64 * nov + norb * (np + 1)) +
+           (sizeof(float) * np + sizeof(int)) * nrg;
 }
 
 void ResidueRange::place(void *base, size_t nov, size_t nrg, size_t norb, int naux_pad) {

@@ -34,6 +34,11 @@ int forced_tile() {
     return 0;
 }
 
+bool forced_residue() {
+    const char *env = getenv("FERRIC_HIP_TILE");
+    return env && *env && atoi(env) == 256;
+}
+
 static int table_tile(Prec prec, size_t nvir, size_t naux) {
     // First entry (in installation order) whose bucket holds the shape.
     for (const auto &e : g_table)

@@ -39,23 +39,33 @@ fh_status check_channel(const fh_spin_channel *ch, size_t naux, bool *empty) {
 
 // The FP64 opposite-spin block in residue arithmetic (residue.hip): alpha and beta
 // rows behind one another in one operand. *taken is false where the matrix kernel
-// is used instead. Sizes as for the closed shell (plan_residue): all three blocks of
-// 21/229, 20/230 over 960 aux 1.92 -> 1.43 ms; under 144 virtuals a side's tiles stay
-// half empty (one orbital a tile here).
+// is used instead (residue_pays; one orbital a tile here): all three blocks of 21/229, 20/230
+// over 960 aux 1.92 -> 1.43 ms.
 fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_channel &cb,
                            const void *ba, const void *bb, bool in_f32, size_t naux,
                            hipStream_t stream, double *energy, bool *taken) {
     *taken = false;
-    const double work =
-        2.0 * ca.nocc * cb.nocc * (double)ca.nvir * (double)cb.nvir * (double)naux;
-    if (std::min(ca.nvir, cb.nvir) < 144 || work < (ca.nocc * cb.nocc >= 64 ? 2.5e9 : 8e9))
-        return FH_OK;
     EnergyPlan pa, pb;
-    if (!residue_tiles(s, ca.nvir, naux, &pa) || !residue_tiles(s, cb.nvir, naux, &pb))
+    if (std::min(ca.nvir, cb.nvir) <= 64 || !residue_tiles(s, ca.nvir, naux, &pa) ||
+        !residue_tiles(s, cb.nvir, naux, &pb))
         return FH_OK;
     const int64_t npairs = (int64_t)ca.nocc * (int64_t)cb.nocc;
     const int ntp = pa.ntile * pb.ntile;
     if (npairs * ntp > 0x7fffff00LL) return FH_OK;
+    ResidueShape r;
+    r.pairs = npairs;
+    r.ntile = pa.ntile;
+    r.ntp = ntp;
+    r.wA = (pa.nvir_pad / 16 + pa.ntile - 1) / pa.ntile;
+    r.wB = (pb.nvir_pad / 16 + pb.ntile - 1) / pb.ntile;
+    r.np = pa.naux_pad / 64;
+    r.cus = s.cus;
+    r.rect = true;
+    r.elements = (double)naux * (double)(ca.nocc * ca.nvir + cb.nocc * cb.nvir);
+    const double ta = (pa.nvir_pad + 63) / 64, tb = (pb.nvir_pad + 63) / 64;
+    if (!residue_pays(r, 2.0 * (double)npairs * pa.nvir_pad * pb.nvir_pad * (double)naux,
+                      (double)npairs * ta * tb, (double)naux))
+        return FH_OK;
     const size_t rows_a = ca.nocc * (size_t)pa.nvir_pad, rows_b = cb.nocc * (size_t)pb.nvir_pad;
     const size_t neps = ca.nocc + ca.nvir + cb.nocc + cb.nvir;
     const size_t col_a = ca.nocc * ca.nvir, col_b = cb.nocc * cb.nvir;

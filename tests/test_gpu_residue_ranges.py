@@ -1,7 +1,7 @@
 """Residue arithmetic on rows that span a wide range over the aux functions (run with -m gpu).
 
 Pair energies, each judged by its own size against the matrix kernel of the same precision
-(FERRIC_HIP_TILE selects it), whose error follows sum |B||B| of the pair itself. The rows of
+(FERRIC_HIP_TILE selects either), whose error follows sum |B||B| of the pair itself. The rows of
 an occupied orbital lie on the aux functions of its site and decay from there, so that a
 pair's products are small beside the rows' largest elements.
 
@@ -23,6 +23,11 @@ from ferric_amd.dlpno import estimate_pair_energies_from_b_ov  # noqa: E402
 
 NOCC, NVIR = 24, 160
 BAR = {Precision.FP64: 1e-15, Precision.MIXED: 8e-8}
+
+
+@pytest.fixture(autouse=True)
+def residue_route(monkeypatch):
+    monkeypatch.setenv("FERRIC_HIP_TILE", "256")  # whatever is faster at these sizes
 
 
 @pytest.fixture
