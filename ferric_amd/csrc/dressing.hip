@@ -61,8 +61,11 @@ fh_status dress_core(State &s, const double *j3, size_t naux, size_t nao, const 
     // As one product, rocBLAS takes 128-wide tiles and multiplies the rows past nleft too;
     // as naux products of one Q each, narrower ones. us, one / many: 250 x 20 x 900 (nao,
     // nleft, naux) 371/218, 300 x 60 x 1200 692/629, 510 x 60 x 1800 2207/1465, 1000 x 60 x
-    // 1200 4793/2941, but 510 x 65 x 1800 2448/2904, 1000 x 100 x 1200 5136/5482.
-    if (nleft <= 64)
+    // 1200 4793/2941, but 510 x 65 x 1800 2448/2904, 1000 x 100 x 1200 5136/5482; and with few
+    // Q the chip is not full (a call's us): 357 x 38 x 7 58/74, 327 x 7 x 18 69/79, 599 x 45 x 4
+    // 84/95, but 291 x 25 x 27 76/73, 432 x 45 x 48 133/104. One column: 210 x 1 x 2619 520/778,
+    // 247 x 1 x 423 130/180.
+    if (nleft > 1 && nleft <= 64 && naux >= 24)
         st = blas_check(rocblas_dgemm_strided_batched(
                             h, rocblas_operation_none, rocblas_operation_none, (int)nleft,
                             (int)nao, (int)nao, &one, cl, (int)nleft, 0, j3, (int)nao,
