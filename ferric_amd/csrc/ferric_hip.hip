@@ -316,17 +316,19 @@ size_t packed_op_bytes(const EnergyPlan &pl, size_t nocc, Prec prec) {
 // the Q rows of one FP32 accumulation (the whole naux for the FP32-accumulating
 // modes, the 64-row panel for MIXED, as the reference's b).
 fh_status range_check(State &s, const void *b, bool in_f32, size_t n, size_t depth,
-                      hipStream_t stream) {
+                      hipStream_t stream, bool *wide) {
     unsigned int *dbits = (unsigned int *)s.slots[kSlotScalar].ptr;
     fh_status st = hip_check(launch_absmax(b, in_f32, (int64_t)n, dbits, stream), "absmax");
     if (st != FH_OK) return st;
-    unsigned int bits = 0;
-    st = hip_check(hipMemcpyAsync(&bits, dbits, 4, hipMemcpyDeviceToHost, stream), "D2H absmax");
+    unsigned int bits[2] = {0, 0};
+    st = hip_check(hipMemcpyAsync(bits, dbits, wide ? 8 : 4, hipMemcpyDeviceToHost, stream),
+                   "D2H absmax");
     if (st != FH_OK) return st;
     st = hip_check(hipStreamSynchronize(stream), "sync absmax");
     if (st != FH_OK) return st;
+    if (wide) *wide = bits[1] != 0;
     float m;
-    memcpy(&m, &bits, 4);
+    memcpy(&m, bits, 4);
     const double limit = std::sqrt((double)std::numeric_limits<float>::max() / (double)depth);
     if ((double)m > limit)
         return fail(FH_RANGE,
@@ -382,7 +384,7 @@ bool residue_tiles(State &s, size_t nvir, size_t naux, EnergyPlan *pl) {
 }
 
 fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, size_t nov,
-                          size_t rows, size_t norb, int naux_pad,
+                          size_t rows, size_t norb, size_t nvir, int naux_pad,
                           std::vector<std::pair<int, size_t>> more, ResidueSpace *out) {
     const int blocks = s.cus / 8 * 8;
     const int words = residue_queue_words(blocks);
@@ -390,8 +392,9 @@ fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, siz
     const size_t planes = stride * (size_t)residue_scratch_sets(blocks);
     more.push_back({kSlotOp0, rows * (size_t)naux_pad * residue_moduli(prec)});
     more.push_back({kSlotScale, sizeof(int) * rows});
-    more.push_back({kSlotRange, out->range.bytes(nov, rows / 16, norb, naux_pad)});
+    more.push_back({kSlotRange, out->range.bytes(nov, norb, nvir, naux_pad)});
     more.push_back({kSlotResidue, planes + sizeof(int) * ((size_t)words + (size_t)nitems)});
+    more.push_back({kSlotScalar, 256});
     const fh_status st = reserve(s, more, true);
     if (st != FH_OK) return st;
     out->op = (int8_t *)s.slots[kSlotOp0].ptr;
@@ -408,9 +411,9 @@ fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, siz
     ra.scratch_stride = (int64_t)stride;
     ra.queue = (int *)((char *)ra.scratch + planes);
     ra.order = ra.queue + words;
-    out->wide = ra.queue + residue_flag_word(blocks);
+    out->wide = (int *)s.slots[kSlotScalar].ptr + 1;
     ra.wide = out->wide;
-    out->range.place(s.slots[kSlotRange].ptr, nov, rows / 16, norb, naux_pad);
+    out->range.place(s.slots[kSlotRange].ptr, nov, norb, nvir, naux_pad);
     out->order.words = words;
     out->order.queue = ra.queue;
     out->order.order = ra.queue + words;
@@ -539,21 +542,12 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     ResidueSpace sp;
     fh_status st = reserve_residue(
         s, prec, pl.nitems, pl.ntile > 1 ? 2 : 1, nocc * nvir, nocc * (size_t)pl.nvir_pad, nocc,
-        pl.naux_pad,
+        nvir, pl.naux_pad,
         {{kSlotEps, sizeof(double) * (nocc + nvir)},
          {kSlotItems, sizeof(double) * 4 * npairs * (size_t)pl.ntp},
          {kSlotRows, sizeof(double) * 4 * nocc},
          {kSlotResult, sizeof(double) * (3 + 2 * nocc)}},
         &sp);
-    if (st != FH_OK) return st;
-    if (prec == Prec::MIXED) {
-        st = reserve(s, {{kSlotScalar, 256}});
-        if (st == FH_OK)
-            st = range_check(s, b_dev, in_f32, naux * nocc * nvir,
-                             std::min(naux, (size_t)kMixedPanel), stream);
-        if (st != FH_OK) return st;
-    }
-    st = upload_eps(s, eps, first_occ, nocc, nocc_total, nvir, stream);
     if (st != FH_OK) return st;
     PackArgs pa{};
     pa.b = b_dev;
@@ -566,17 +560,30 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
     pa.out0 = sp.op;
     pa.rexp = sp.rexp;
     ResidueArgs ra = sp.args;
+    ra.nocc = (int)nocc;
+    ra.nvir = (int)nvir;
+    ra.nvir_pad = pl.nvir_pad;
     ra.group = pl.group;
     ra.ngroup = ((int)nocc + pl.group - 1) / pl.group;
     ResidueOrder ord = sp.order;
     ord.nocc = ra.ngroup;
     ord.ntp = pl.ntp;
     mark(s, 0, stream);
-    ra.nocc = (int)nocc;
-    ra.nvir = (int)nvir;
-    ra.nvir_pad = pl.nvir_pad;
-    hipError_t he = launch_residue_pack(prec, pa, ord, sp.range, stream);
+    hipError_t he = launch_residue_scan(prec, pa, sp.range, sp.wide, stream);
     if (he == hipSuccess) he = launch_residue_range(ra, sp.range, sp.wide, stream);
+    if (he != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(FH_KERNEL, "scan kernels: %s", hipGetErrorString(he));
+    }
+    s.pending.kernel_launches += 3;
+    if (prec == Prec::MIXED) {
+        st = range_check(s, b_dev, in_f32, naux * nocc * nvir, std::min(naux, (size_t)kMixedPanel),
+                         stream, wide);
+        if (st != FH_OK || *wide) return st;
+    }
+    st = upload_eps(s, eps, first_occ, nocc, nocc_total, nvir, stream);
+    if (st != FH_OK) return st;
+    he = launch_residue_pack(prec, pa, ord, sp.wide, stream);
     if (he != hipSuccess) {
         (void)hipGetLastError();
         return fail(FH_KERNEL, "pack kernel: %s", hipGetErrorString(he));
@@ -609,7 +616,7 @@ fh_status residue_energy(State &s, const void *b_dev, bool in_f32, size_t naux, 
         return fail(FH_KERNEL, "reduction kernels: %s", hipGetErrorString(he));
     }
     mark(s, 3, stream);
-    s.pending.kernel_launches += 6;
+    s.pending.kernel_launches += 3;
     st = fetch_result(s, ea.result, nocc, stream, out, row_partials, wide);
     if (st == FH_OK) finish_timing(s, (uint64_t)pl.nitems, pl.tile);
     return st;
@@ -684,6 +691,7 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
     size_t carved = 0;
     for (const auto &r : req) carved = (carved + 255) / 256 * 256 + r.second;
     EnergyPlan rpl;
+    bool checked = false;  // the range of B
     if (!signed_k && !(as_noalloc && carved <= (size_t)FH_NOALLOC_SCRATCH_BYTES) &&
         plan_residue(s, nocc, nvir, naux, prec, &rpl)) {
         const Attempt attempt(s);
@@ -694,7 +702,8 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
         if (ntp_used) *ntp_used = rpl.ntp;
         // Its larger workspace may be past the pool ceiling, or the rows past its range: then
         // the matrix kernel below, which needs half the operand (or less) and no scratch.
-        if (rst != FH_POOL_FULL && !wide) return rst;
+        if (rst != FH_POOL_FULL && !(rst == FH_OK && wide)) return rst;
+        checked = rst == FH_OK;
         attempt.undo();
     }
     if (ntp_used) *ntp_used = pl.ntp;
@@ -705,7 +714,7 @@ fh_status energy_core(State &s, const void *b_dev, fh_dtype b_dtype, size_t naux
 
     // INT8 slices carry their own power-of-two scale per row: any finite
     // value is in range.
-    if (prec != Prec::F64 && prec != Prec::I8X4) {
+    if (prec != Prec::F64 && prec != Prec::I8X4 && !checked) {
         const size_t depth = prec == Prec::MIXED ? std::min(naux, (size_t)kMixedPanel)
                                                  : naux + (signed_k ? naux_neg : 0);
         st = range_check(s, b_dev, in_f32, naux * nov, depth, stream);

@@ -49,8 +49,8 @@ enum SlotId {
     kSlotDensPart,   // MP2 densities: split-K partial tiles
     kSlotDensOut,    // MP2 densities: P_vv (padded) then P_oo
     kSlotResidue,    // residue arithmetic: the workgroups' residue planes
-    kSlotRange,      // residue arithmetic: column maxima and sums of B (the packer's; no entry
-                     // stages an input here, as some do in kSlotStage and kSlotStage2)
+    kSlotRange,      // residue arithmetic: column maxima and sums of B (no entry stages an
+                     // input here, as some do in kSlotStage and kSlotStage2)
     kNumSlots
 };
 
@@ -145,8 +145,9 @@ fh_status hip_check(hipError_t e, const char *what);
 fh_status check_shapes(size_t naux, size_t nocc, size_t nvir, size_t n_eps, size_t first_occ,
                        size_t nocc_total, bool *empty);
 fh_status check_kappa(double kappa, bool *has);
+// wide: also the flag of the residue range test, the second word of kSlotScalar.
 fh_status range_check(State &s, const void *b, bool in_f32, size_t n, size_t depth,
-                      hipStream_t stream);
+                      hipStream_t stream, bool *wide = nullptr);
 EnergyPlan plan_energy(size_t nocc, size_t nvir, size_t naux, Prec prec);
 // FERRIC_HIP_TILE's tile side, or 0 when it is unset.
 int forced_tile();
@@ -190,9 +191,10 @@ struct ResidueSpace {
     int *rexp = nullptr;
     int *wide = nullptr;
 };
-// nov: columns of B, rows: packed rows, norb: occupied orbitals (both sides' together).
+// nov: columns of B, rows: packed rows, norb: occupied orbitals (both sides' together), nvir:
+// the larger side's.
 fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, size_t nov,
-                          size_t rows, size_t norb, int naux_pad,
+                          size_t rows, size_t norb, size_t nvir, int naux_pad,
                           std::vector<std::pair<int, size_t>> more, ResidueSpace *out);
 // Copies the device result (energies, then nocc rows' values, then, if asked for, the residue
 // kernel's flag) back and waits for it.

@@ -240,27 +240,27 @@ int residue_beta(Prec prec, int naux_pad);
 // or more workgroups to each).
 int residue_scratch_sets(int blocks);
 int residue_queue_words(int blocks);
-int residue_flag_word(int blocks);  // the range test's
 size_t residue_scratch_stride(Prec prec, int products);
-// Scratch of the packer and of the range test, for nov columns and nrg 16-row groups of norb
-// orbitals.
+// Scratch of the scan, for nov columns of norb orbitals of up to nvir virtuals.
 struct ResidueRange {
     double *pmax = nullptr;   // column maxima by Q panel
     double *w = nullptr;      // per orbital and Q: sum over the virtuals of B^2
-    double *s = nullptr;      // per orbital: sum over the virtuals of the rows' squared ranges
-    float *norm = nullptr;    // per row group and Q: sum of B^2, in units of 4^gexp
-    int *gexp = nullptr;      // per row group: the largest exponent
-    size_t bytes(size_t nov, size_t nrg, size_t norb, int naux_pad);
-    void place(void *base, size_t nov, size_t nrg, size_t norb, int naux_pad);
+    double *s = nullptr;      // per orbital and 64 virtuals: sum of the rows' squared ranges
+    int chunks = 0;           // of 64 virtuals, of s
+    size_t bytes(size_t nov, size_t norb, size_t nvir, int naux_pad);
+    void place(void *base, size_t nov, size_t norb, size_t nvir, int naux_pad);
 };
+// The rows' exponents (a.rexp) and the sums of the range test; *wide to 0 unless it is null.
+hipError_t launch_residue_scan(Prec prec, const PackArgs &a, const ResidueRange &rr, int *wide,
+                               hipStream_t st);
+// Sets *wide if some pair's products would lose accuracy (a's sizes; residue.hip); the packer
+// and the energy kernel then leave at once.
+hipError_t launch_residue_range(const ResidueArgs &a, const ResidueRange &rr, int *wide,
+                                hipStream_t st);
 // The rows go to row groups rg0 on, of nrg in all (0: only these). ord.order null: no order
 // to be made.
 hipError_t launch_residue_pack(Prec prec, const PackArgs &a, const ResidueOrder &ord,
-                               const ResidueRange &rr, hipStream_t st, int64_t nrg = 0,
-                               int64_t rg0 = 0);
-// Sets *wide if some pair's products would lose accuracy (a's sizes and rows; residue.hip).
-hipError_t launch_residue_range(const ResidueArgs &a, const ResidueRange &rr, int *wide,
-                                hipStream_t st);
+                               const int *wide, hipStream_t st, int64_t nrg = 0, int64_t rg0 = 0);
 hipError_t launch_residue_energy(const ResidueArgs &a, hipStream_t st);
 // Phase A of the adjoint: the pair kernel with the T~ / dE/deps epilogue.
 hipError_t launch_adjoint_pairs(const EnergyArgs &a, hipStream_t st);

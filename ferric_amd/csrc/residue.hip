@@ -68,30 +68,79 @@ constexpr Recip recip() {
 }
 __constant__ const Recip kRecip = recip();
 
-// Largest |B| of every column over one 64-deep Q panel (256 columns a block; a
-// NaN counts as an infinity). The packer folds the panels: together they read B
-// once more than the packing itself, at the memory's rate (one pass with a thread
-// per column, as the INT8X4 packer's, took 105 us at 41/209/960 and 215 us at
-// 60/450/1800 on the latency of its few loads in flight).
+// One orbital and one 64-deep Q panel: the largest |B| of every column (a NaN counts as an
+// infinity) and, for the range test, the sum over the virtuals of B^2 at every Q. One read of
+// B at the memory's rate; 16 rows of 64 columns in flight a wave.
 template <typename Tin>
-__global__ __launch_bounds__(256) void residue_colmax_kernel(const Tin *__restrict__ b, int64_t nov,
-                                                             int naux, double *__restrict__ pmax) {
-    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (c >= nov) return;
-    const int q0 = blockIdx.y * 64, n = min(64, naux - q0);
-    const Tin *p = b + (int64_t)q0 * nov + c;
-    double m = 0.0;
-    auto take = [&](double v) { m = v <= 1.7976931348623157e308 ? fmax(m, v) : INFINITY; };
-    int q = 0;
-    for (; q + 16 <= n; q += 16) {
-        double v[16];
+__global__ __launch_bounds__(256) void residue_scan_kernel(const Tin *__restrict__ b, int64_t nov,
+                                                           int naux, int nvir, ResidueRange rr,
+                                                           int *wide) {
+    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+    const int i = blockIdx.y, q0 = blockIdx.x * 64 + 16 * wid, n = min(16, naux - q0);
+    if (wide && blockIdx.x == 0 && i == 0 && threadIdx.x == 0) *wide = 0;
+    const Tin *p = b + (int64_t)q0 * nov + (int64_t)i * nvir;
+    __shared__ double part[2][4][64];
+    double sum[16];
 #pragma unroll
-        for (int t = 0; t < 16; ++t) v[t] = fabs((double)p[(int64_t)(q + t) * nov]);
+    for (int t = 0; t < 16; ++t) sum[t] = 0.0;
+    for (int a0 = 0; a0 < nvir; a0 += 64) {
+        const int a = a0 + lane;
+        double v[16], m = 0.0;
 #pragma unroll
-        for (int t = 0; t < 16; ++t) take(v[t]);
+        for (int t = 0; t < 16; ++t) v[t] = t < n && a < nvir ? (double)p[t * nov + a] : 0.0;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            const double x = fabs(v[t]);
+            const bool finite = x <= 1.7976931348623157e308;
+            m = finite ? fmax(m, x) : INFINITY;
+            sum[t] += finite ? x * x : 0.0;
+        }
+        double(*out)[64] = part[a0 / 64 % 2];
+        out[wid][lane] = m;
+        __syncthreads();
+        if (wid == 0 && a < nvir)
+            rr.pmax[(int64_t)blockIdx.x * nov + (int64_t)i * nvir + a] =
+                fmax(fmax(out[0][lane], out[1][lane]), fmax(out[2][lane], out[3][lane]));
     }
-    for (; q < n; ++q) take(fabs((double)p[(int64_t)q * nov]));
-    pmax[(int64_t)blockIdx.y * nov + c] = m;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+        for (int m = 1; m < kWave; m *= 2) sum[t] += __shfl_xor(sum[t], m, kWave);
+        if (lane == t) rr.w[((int64_t)i * gridDim.x + blockIdx.x) * 64 + 16 * wid + t] = sum[t];
+    }
+}
+
+// 64 rows of an orbital: the exponent f of each is that of the INT8X4 format, the least with
+// max |x| <= (1 - 2^-7) 2^(f + 1); the sum of 4^(f + 1), non-finite rows left out.
+template <bool ROUND32>  // x is first rounded to FP32 (MIXED)
+__global__ __launch_bounds__(256) void residue_rows_kernel(ResidueRange rr, int64_t nov, int np,
+                                                           int nvir, int nvir_pad,
+                                                           int *__restrict__ rexp) {
+    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+    const int i = blockIdx.y, a = blockIdx.x * 64 + lane;
+    double m = 0.0;
+    if (a < nvir) {
+        const double *p = rr.pmax + (int64_t)i * nvir + a;
+#pragma unroll 4
+        for (int k = wid; k < np; k += 4) m = fmax(m, p[k * nov]);
+    }
+    __shared__ double part[4][64];
+    part[wid][lane] = m;
+    __syncthreads();
+    if (wid != 0) return;
+    double mm = fmax(fmax(part[0][lane], part[1][lane]), fmax(part[2][lane], part[3][lane]));
+    if (ROUND32) mm = (double)(float)mm;
+    int e = res::kZeroRow;
+    double s = 0.0;
+    if (mm > 1.7976931348623157e308) {
+        e = kI8NonFinite;
+    } else if (mm > 0.0) {
+        (void)frexp(mm, &e);
+        if (mm <= ldexp(1.0 - 0x1p-7, e)) e -= 1;
+        s = ldexp(1.0, 2 * (e + 1));
+    }
+    if (a < nvir_pad) rexp[(int64_t)i * nvir_pad + a] = e;
+    for (int k = 1; k < kWave; k *= 2) s += __shfl_xor(s, k, kWave);
+    if (lane == 0) rr.s[(int64_t)i * rr.chunks + blockIdx.x] = s;
 }
 
 // Item order: the pair triangle in blocks of 4 x 8 pairs, cut into one run of pairs
@@ -132,22 +181,19 @@ __device__ void order_items(const ResidueOrder &o) {
     }
 }
 
-// One 64 x 64 tile (64 packed rows, one Q panel) to residues. The exponent f of a row
-// is that of the INT8X4 format: the least with max |x| <= (1 - 2^-7) 2^(f + 1); Y =
-// RN(x 2^(beta - 1 - f)). The rows go to row groups rg0 on, of nrg in all. ROUND32: x is
-// first rounded to FP32 (MIXED).
+// One 64 x 64 tile (64 packed rows, one Q panel) to residues. Y = RN(x 2^(beta - 1 - f)).
+// The rows go to row groups rg0 on, of nrg in all. ROUND32: x is first rounded to FP32
+// (MIXED).
 template <int N, bool ROUND32, typename Tin>
 __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict__ b, int64_t nov,
                                                            int naux, int nvir, int nvir_pad,
                                                            int64_t nrows, int np, int beta,
                                                            int64_t nrg, int64_t rg0,
-                                                           ResidueRange rr,
-                                                           int *__restrict__ rexp,
+                                                           const int *__restrict__ rexp,
                                                            int8_t *__restrict__ out,
-                                                           ResidueOrder ord) {
+                                                           ResidueOrder ord, const int *wide) {
     __shared__ double tile[64][65];
-    __shared__ double part[4][64];
-    __shared__ int exps[64];
+    if (*wide) return;
     if ((int)blockIdx.y == np) {  // one more row of blocks: the item order and the queue words
         if (ord.order) order_items(ord);
         return;
@@ -162,10 +208,6 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
         const int a = (int)(r % nvir_pad);
         if (a < nvir) col = i * nvir + a;
     }
-    double m = 0.0;
-    if (col >= 0)
-        for (int p = ty; p < np; p += 4) m = fmax(m, rr.pmax[(int64_t)p * nov + col]);
-    part[ty][tx] = m;
     for (int q = ty; q < 64; q += 4) {
         const int qq = q0 + q;
         double v = 0.0;
@@ -173,45 +215,13 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
         tile[q][tx] = ROUND32 ? (double)(float)v : v;
     }
     __syncthreads();
-    if (ty == 0) {
-        double mm = fmax(fmax(part[0][tx], part[1][tx]), fmax(part[2][tx], part[3][tx]));
-        if (ROUND32) mm = (double)(float)mm;
-        int e = res::kZeroRow;
-        if (mm > 1.7976931348623157e308) {
-            e = kI8NonFinite;
-        } else if (mm > 0.0) {
-            (void)frexp(mm, &e);
-            if (mm <= ldexp(1.0 - 0x1p-7, e)) e -= 1;
-        }
-        exps[tx] = e;
-        if (blockIdx.y == 0 && r < nrows) rexp[r] = e;
-    }
-    __syncthreads();
-    // For the range test: a wave to a row group, a lane to a Q. Non-finite rows are not judged.
-    if (r0 + 16 * ty < nrows) {
-        int ge = res::kZeroRow;
-        for (int k = 0; k < 16; ++k) {
-            const int e = exps[16 * ty + k];
-            if (e != kI8NonFinite) ge = max(ge, e);
-        }
-        double sum = 0.0;
-        if (ge > res::kZeroRow)
-            for (int k = 0; k < 16; ++k) {
-                const double v = ldexp(tile[tx][16 * ty + k], -ge);
-                sum += exps[16 * ty + k] != kI8NonFinite ? v * v : 0.0;
-            }
-        const int64_t rg = rg0 + r0 / 16 + ty;
-        // Positive even where it underflows FP32: only a zero has no rounding error.
-        rr.norm[rg * (np * 64) + q0 + tx] = sum > 0.0 ? fmaxf((float)sum, 0x1p-126f) : 0.0f;
-        if (blockIdx.y == 0 && tx == 0) rr.gexp[rg] = ge;
-    }
     // Thread t takes row 16 (t / 64) + t % 16 and the panel's Q = 16 g .. 16 g + 15,
     // g = (t / 16) % 4: lane t % 64 of its row group's kilobyte.
     const int t = threadIdx.x;
     const int g = (t / 16) % 4, row = (t / 64) * 16 + t % 16;
     const int64_t orow = r0 + row;
     if (orow >= nrows) return;
-    const int e = exps[row];
+    const int e = rexp[orow];
     const bool bad = e == kI8NonFinite;
     const int sh = bad ? 0 : beta - 1 - e;
     uint32_t w[N][4];
@@ -258,87 +268,55 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const Tin *__restrict
 //   4^-beta / 12 (s_i sum_Q w_jQ + s_j sum_Q w_iQ) + (fixed point)^2 s_i s_j,
 // s_i the sum over a of the rows' squared ranges 4^(f + 1), w_iQ the sum over a of B^2, the
 // sums over Q where the other orbital is not zero (zeros have no rounding error), and g^2 is
-// sum_Q w_iQ w_jQ for products of random sign. A call with a pair whose error exceeds kBar of
-// that goes to the matrix kernel: the energy kernel leaves at once, and the host sees the flag
-// with the results, so that no wait is added. Pairs by their own size, chain of 24 orbitals
+// sum_Q w_iQ w_jQ for products of random sign. A call with a pair whose error exceeds bar_of
+// of that goes to the matrix kernel: the packer and the energy kernel leave at once, and the
+// host sees the flag with the results, so that no wait is added (in MIXED with the range check
+// of B, whose wait comes first anyway). Pairs by their own size, chain of 24 orbitals
 // decaying as e^-d over 1008 aux functions: 1.9e-10 at d = 21 without the test, and 3.7e-3 in
 // MIXED. What errors the bar admits the sums of the energies average down to their own rounding;
 // the matrix kernels' products are off by 2^-50 (960 aux functions in FP64) and 2^-23 (panels
 // of 64 in FP32) on the same scale. Normal rows, with or without hot aux functions, have
 // 2^-53 to 2^-54, water in cc-pVDZ 2^-54, orbitals that reach three sites 2^-51.
-// What it costs, with the packer's sums and two small kernels (and the tenth layer of the
-// reconstruction): the three blocks of 21/229, 20/230 over 960 aux functions 1396 -> 1439 us,
-// 60/450/1800 in MIXED 9333 -> 9332, 100/200/2400 9513 -> 9571.
+// What it costs (with the tenth layer of the reconstruction): the three blocks of 21/229,
+// 20/230 over 960 aux functions 1396 -> 1439 us, 60/450/1800 in MIXED 9391 -> 9328, 100/200/2400
+// 9501 -> 9505; and a call that ends on the matrix kernel, over that kernel alone: 24/160/1008 in
+// MIXED 497 -> 542, opposite spin 953 -> 1063, 60/450/1800 19.9 -> 20.1 and 64.2 -> 64.8 ms.
 constexpr double bar_of(int n) { return n == 16 ? 0x1p-50 : 0x1p-24; }
 
-// One side's orbitals in the packed rows, and where their sums go.
-struct RangeSide {
-    int norb, nvir, nvir_pad;
-    int64_t rg0;      // first row group
-    const int *rexp;
-    double *w, *s;
-};
-
-// 64 Q of one orbital a workgroup, the row groups dealt to its four waves.
-__global__ __launch_bounds__(256) void residue_norm_kernel(const float *__restrict__ norm,
-                                                           const int *__restrict__ gexp,
-                                                           int naux_pad, RangeSide a,
-                                                           RangeSide b) {
-    const bool second = (int)blockIdx.y >= a.norb;
-    const RangeSide o = second ? b : a;
-    const int i = second ? blockIdx.y - a.norb : blockIdx.y;
-    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave, ng = o.nvir_pad / 16;
-    const int64_t rg = o.rg0 + (int64_t)i * ng;
-    int top = res::kZeroRow;
-    for (int g = lane; g < ng; g += kWave) top = max(top, gexp[rg + g]);
-    for (int m = 1; m < kWave; m *= 2) top = max(top, __shfl_xor(top, m, kWave));
-    const int q = blockIdx.x * 64 + lane;
-    double sum = 0.0;
-#pragma unroll 4
-    for (int g = wid; g < ng; g += 4)
-        sum += ldexp((double)norm[(rg + g) * naux_pad + q], 2 * (gexp[rg + g] - top));
-    __shared__ double part[4][64];
-    part[wid][lane] = sum;
-    __syncthreads();
-    if (wid == 0)
-        o.w[(int64_t)i * naux_pad + q] =
-            (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
-    if (blockIdx.x != 0 || wid != 1) return;
-    double t = 0.0;
-    for (int v = lane; v < o.nvir; v += kWave) {
-        const int e = o.rexp[(int64_t)i * o.nvir_pad + v];
-        if (e > res::kZeroRow && e != kI8NonFinite) t += ldexp(1.0, 2 * (e + 1 - top));
-    }
-    for (int m = 1; m < kWave; m *= 2) t += __shfl_xor(t, m, kWave);
-    if (lane == 0) o.s[i] = t;
-}
-
-// Orbitals i = blockIdx.y and j, a wave to each j. same: j >= i only.
+// Orbitals i = blockIdx.y and j, a wave to each j. same: j >= i only. Sums out of the range of
+// FP64's squares count as past the bar.
 __global__ __launch_bounds__(256) void residue_range_kernel(const double *__restrict__ wa,
                                                             const double *__restrict__ sa,
                                                             const double *__restrict__ wb,
                                                             const double *__restrict__ sb, int nb,
-                                                            int naux_pad, bool same, double round2,
-                                                            double fixed2, int *wide) {
-    const int i = blockIdx.y, j = blockIdx.x * 4 + threadIdx.x / kWave;
+                                                            int chunks, int naux_pad, bool same,
+                                                            double round2, double fixed2,
+                                                            int *wide) {
+    const int i = blockIdx.y, j = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x % kWave;
     if (j >= nb || (same && j < i)) return;
     const double *x = wa + (int64_t)i * naux_pad, *y = wb + (int64_t)j * naux_pad;
-    double gg = 0.0, ni = 0.0, nj = 0.0;
+    double gg = 0.0, ni = 0.0, nj = 0.0, si = 0.0, sj = 0.0;
 #pragma unroll 4
-    for (int q = threadIdx.x % kWave; q < naux_pad; q += kWave) {
+    for (int q = lane; q < naux_pad; q += kWave) {
         const double u = x[q], v = y[q];
         gg += u * v;
         ni += v > 0.0 ? u : 0.0;
         nj += u > 0.0 ? v : 0.0;
     }
+    for (int c = lane; c < chunks; c += kWave) {
+        si += sa[(int64_t)i * chunks + c];
+        sj += sb[(int64_t)j * chunks + c];
+    }
     for (int m = 1; m < kWave; m *= 2) {
         gg += __shfl_xor(gg, m, kWave);
         ni += __shfl_xor(ni, m, kWave);
         nj += __shfl_xor(nj, m, kWave);
+        si += __shfl_xor(si, m, kWave);
+        sj += __shfl_xor(sj, m, kWave);
     }
-    if (threadIdx.x % kWave != 0 || nj == 0.0) return;  // no aux function in common: g = 0
-    const double err = round2 * (sa[i] * nj + sb[j] * ni) + fixed2 * sa[i] * sb[j];
-    if (!(err <= gg)) *wide = 1;
+    if (lane != 0 || nj == 0.0) return;  // no aux function in common: g = 0
+    const double err = round2 * (si * nj + sj * ni) + fixed2 * si * sj;
+    if (!(err <= gg && gg > 1e-280 && gg < 1e280)) *wide = 1;
 }
 
 // One product over a run of moduli and every panel: row groups rgA .. rgA + nA against
@@ -879,26 +857,26 @@ __global__ __launch_bounds__(kThreads) void residue_energy_kernel(ResidueArgs a)
 }
 
 template <int N, bool ROUND32>  // MIXED: ROUND32
-hipError_t launch_pack_n(const PackArgs &a, const ResidueOrder &ord, const ResidueRange &rr,
-                         int beta, int64_t nrg, int64_t rg0, hipStream_t st) {
+hipError_t launch_pack_n(const PackArgs &a, const ResidueOrder &ord, const int *wide, int beta,
+                         int64_t nrg, int64_t rg0, hipStream_t st) {
     const int64_t nrows = (int64_t)a.nocc * a.nvir_pad, nov = (int64_t)a.nocc * a.nvir;
     const int np = a.naux_pad / 64;
-    const dim3 mg((unsigned)((nov + 255) / 256), (unsigned)((a.naux + 63) / 64));
     const dim3 grid((unsigned)((nrows + 63) / 64), (unsigned)np + 1);
-    if (a.in_f32) {
-        hipLaunchKernelGGL(residue_colmax_kernel<float>, mg, dim3(256), 0, st, (const float *)a.b,
-                           nov, a.naux, rr.pmax);
+    if (a.in_f32)
         hipLaunchKernelGGL((residue_pack_kernel<N, ROUND32, float>), grid, dim3(256), 0, st,
                            (const float *)a.b, nov, a.naux, a.nvir, a.nvir_pad, nrows, np, beta,
-                           nrg, rg0, rr, a.rexp, (int8_t *)a.out0, ord);
-    } else {
-        hipLaunchKernelGGL(residue_colmax_kernel<double>, mg, dim3(256), 0, st,
-                           (const double *)a.b, nov, a.naux, rr.pmax);
+                           nrg, rg0, (const int *)a.rexp, (int8_t *)a.out0, ord, wide);
+    else
         hipLaunchKernelGGL((residue_pack_kernel<N, ROUND32, double>), grid, dim3(256), 0, st,
                            (const double *)a.b, nov, a.naux, a.nvir, a.nvir_pad, nrows, np, beta,
-                           nrg, rg0, rr, a.rexp, (int8_t *)a.out0, ord);
-    }
+                           nrg, rg0, (const int *)a.rexp, (int8_t *)a.out0, ord, wide);
     return hipGetLastError();
+}
+
+bool pack_sizes(const PackArgs &a) {
+    return a.rexp && a.nocc > 0 && a.nvir > 0 && a.naux_pad % 64 == 0 && a.naux_pad >= a.naux &&
+           a.naux_pad - a.naux < 64 && a.naux_pad <= res::kMaxNauxPad && a.nvir_pad % 16 == 0 &&
+           a.nvir_pad >= a.nvir;
 }
 
 }  // namespace
@@ -942,61 +920,65 @@ int residue_beta(Prec prec, int naux_pad) {
 
 int residue_scratch_sets(int blocks) { return blocks + blocks / 2; }
 
-int residue_flag_word(int blocks) { return (kQueueStride + blocks + 31) / 32 * 32; }
-
-int residue_queue_words(int blocks) { return residue_flag_word(blocks) + kQueueStride; }
+int residue_queue_words(int blocks) { return (kQueueStride + blocks + 31) / 32 * 32; }
 
 size_t residue_scratch_stride(Prec prec, int products) {
     return (size_t)products * planes_of(residue_moduli(prec));
 }
 
-size_t ResidueRange::bytes(size_t nov, size_t nrg, size_t norb, int naux_pad) {
+size_t ResidueRange::bytes(size_t nov, size_t norb, size_t nvir, int naux_pad) {
     const size_t np = (size_t)naux_pad;
-    return sizeof(double) * (np / 64 * nov + norb * (np + 1)) +
-           (sizeof(float) * np + sizeof(int)) * nrg;
+    return sizeof(double) * (np / 64 * nov + norb * (np + (nvir + 63) / 64));
 }
 
-void ResidueRange::place(void *base, size_t nov, size_t nrg, size_t norb, int naux_pad) {
-    const size_t np = (size_t)naux_pad;
+void ResidueRange::place(void *base, size_t nov, size_t norb, size_t nvir, int naux_pad) {
     pmax = (double *)base;
-    w = pmax + np / 64 * nov;
-    s = w + norb * np;
-    norm = (float *)(s + norb);
-    gexp = (int *)(norm + nrg * np);
+    w = pmax + (size_t)naux_pad / 64 * nov;
+    s = w + norb * (size_t)naux_pad;
+    chunks = (int)((nvir + 63) / 64);
+}
+
+hipError_t launch_residue_scan(Prec prec, const PackArgs &a, const ResidueRange &rr, int *wide,
+                               hipStream_t st) {
+    if (!pack_sizes(a) || !rr.pmax || rr.chunks * 64 < a.nvir) return hipErrorInvalidValue;
+    const int64_t nov = (int64_t)a.nocc * a.nvir;
+    const unsigned np = (unsigned)a.naux_pad / 64;
+    const dim3 grid(np, (unsigned)a.nocc), rows((unsigned)rr.chunks, (unsigned)a.nocc);
+    if (a.in_f32)
+        hipLaunchKernelGGL(residue_scan_kernel<float>, grid, dim3(256), 0, st, (const float *)a.b,
+                           nov, a.naux, a.nvir, rr, wide);
+    else
+        hipLaunchKernelGGL(residue_scan_kernel<double>, grid, dim3(256), 0, st,
+                           (const double *)a.b, nov, a.naux, a.nvir, rr, wide);
+    hipLaunchKernelGGL(prec == Prec::MIXED ? residue_rows_kernel<true> : residue_rows_kernel<false>,
+                       rows, dim3(256), 0, st, rr, nov, (int)np, a.nvir, a.nvir_pad, a.rexp);
+    return hipGetLastError();
 }
 
 hipError_t launch_residue_range(const ResidueArgs &a, const ResidueRange &rr, int *wide,
                                 hipStream_t st) {
     const int naux_pad = a.np * 64, n = residue_moduli(a.prec);
     const bool rect = a.nocc_b > 0;
-    const RangeSide x{a.nocc, a.nvir, a.nvir_pad, 0, a.rexp, rr.w, rr.s};
-    const RangeSide y{a.nocc_b, a.nvir_b, a.nvir_pad_b, (int64_t)a.nocc * a.nvir_pad / 16, a.rexp_b,
-                      rr.w + (int64_t)a.nocc * naux_pad, rr.s + a.nocc};
-    hipLaunchKernelGGL(residue_norm_kernel,
-                       dim3((unsigned)a.np, (unsigned)(a.nocc + a.nocc_b)), dim3(256), 0, st,
-                       rr.norm, rr.gexp, naux_pad, x, y);
     const int nb = rect ? a.nocc_b : a.nocc;
+    const double *wb = rr.w + (rect ? (int64_t)a.nocc * naux_pad : 0);
+    const double *sb = rr.s + (rect ? (int64_t)a.nocc * rr.chunks : 0);
     const double bar = bar_of(n), unit = ldexp(1.0, -2 * a.beta) / (bar * bar);
     const double fixed = res::fixed_error(n) * (n == 16 ? res::kPhi<16> : res::kPhi<10>);
     hipLaunchKernelGGL(residue_range_kernel, dim3((unsigned)(nb + 3) / 4, (unsigned)a.nocc),
-                       dim3(256), 0, st, rr.w, rr.s, rect ? y.w : x.w, rect ? y.s : x.s, nb,
-                       naux_pad, !rect, unit / 12.0,
-                       unit * fixed * ldexp(fixed, -2 * a.beta), wide);
+                       dim3(256), 0, st, rr.w, rr.s, wb, sb, nb, rr.chunks, naux_pad, !rect,
+                       unit / 12.0, unit * fixed * ldexp(fixed, -2 * a.beta), wide);
     return hipGetLastError();
 }
 
 hipError_t launch_residue_pack(Prec prec, const PackArgs &a, const ResidueOrder &ord,
-                               const ResidueRange &rr, hipStream_t st, int64_t nrg, int64_t rg0) {
+                               const int *wide, hipStream_t st, int64_t nrg, int64_t rg0) {
     const int64_t own = (int64_t)a.nocc * a.nvir_pad / 16;
     if (nrg == 0) nrg = own;
-    if (rg0 < 0 || rg0 + own > nrg) return hipErrorInvalidValue;
-    if (!a.rexp || !rr.pmax || !rr.norm || a.naux_pad % 64 != 0 || a.naux_pad < a.naux ||
-        a.naux_pad - a.naux >= 64 || a.naux_pad > res::kMaxNauxPad || a.nvir_pad % 16 != 0)
-        return hipErrorInvalidValue;
+    if (rg0 < 0 || rg0 + own > nrg || !wide || !pack_sizes(a)) return hipErrorInvalidValue;
     const int beta = residue_beta(prec, a.naux_pad);
     switch (prec) {
-    case Prec::F64: return launch_pack_n<16, false>(a, ord, rr, beta, nrg, rg0, st);
-    case Prec::MIXED: return launch_pack_n<10, true>(a, ord, rr, beta, nrg, rg0, st);
+    case Prec::F64: return launch_pack_n<16, false>(a, ord, wide, beta, nrg, rg0, st);
+    case Prec::MIXED: return launch_pack_n<10, true>(a, ord, wide, beta, nrg, rg0, st);
     default: return hipErrorInvalidValue;
     }
 }

@@ -73,7 +73,7 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
     ResidueSpace sp;
     fh_status st = reserve_residue(
         s, Prec::F64, npairs * ntp, 1, col_a + col_b, rows_a + rows_b, ca.nocc + cb.nocc,
-        pa.naux_pad,
+        std::max(ca.nvir, cb.nvir), pa.naux_pad,
         {{kSlotEps, sizeof(double) * neps},
          {kSlotItems, sizeof(double) * 4 * (size_t)(npairs * ntp)},
          {kSlotRows, sizeof(double) * 4 * ca.nocc},
@@ -131,19 +131,23 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
     pk.nvir = ra.nvir;
     pk.nvir_pad = ra.nvir_pad;
     pk.rexp = sp.rexp;
-    hipError_t he = launch_residue_pack(Prec::F64, pk, ord, sp.range, stream, nrg, 0);
-    if (he == hipSuccess) {
-        pk.b = bb;
-        pk.nocc = ra.nocc_b;
-        pk.nvir = ra.nvir_b;
-        pk.nvir_pad = ra.nvir_pad_b;
-        pk.rexp = sp.rexp + rows_a;
-        ResidueRange beta = sp.range;
-        beta.pmax += (size_t)(pa.naux_pad / 64) * col_a;
-        he = launch_residue_pack(Prec::F64, pk, ResidueOrder{}, beta, stream, nrg,
-                                 (int64_t)rows_a / 16);
-    }
+    PackArgs pkb = pk;
+    pkb.b = bb;
+    pkb.nocc = ra.nocc_b;
+    pkb.nvir = ra.nvir_b;
+    pkb.nvir_pad = ra.nvir_pad_b;
+    pkb.rexp = sp.rexp + rows_a;
+    ResidueRange beta = sp.range;
+    beta.pmax += (size_t)(pa.naux_pad / 64) * col_a;
+    beta.w += ca.nocc * (size_t)pa.naux_pad;
+    beta.s += ca.nocc * (size_t)beta.chunks;
+    hipError_t he = launch_residue_scan(Prec::F64, pk, sp.range, sp.wide, stream);
+    if (he == hipSuccess) he = launch_residue_scan(Prec::F64, pkb, beta, nullptr, stream);
     if (he == hipSuccess) he = launch_residue_range(ra, sp.range, sp.wide, stream);
+    if (he == hipSuccess) he = launch_residue_pack(Prec::F64, pk, ord, sp.wide, stream, nrg, 0);
+    if (he == hipSuccess)
+        he = launch_residue_pack(Prec::F64, pkb, ResidueOrder{}, sp.wide, stream, nrg,
+                                 (int64_t)rows_a / 16);
     if (he != hipSuccess) {
         (void)hipGetLastError();
         return fail(FH_KERNEL, "pack kernel: %s", hipGetErrorString(he));
@@ -170,7 +174,7 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
         return fail(FH_KERNEL, "reduction kernels: %s", hipGetErrorString(he));
     }
     mark(s, 3, stream);
-    s.pending.kernel_launches += 8;
+    s.pending.kernel_launches += 9;
     fh_spin_components sc{};
     bool wide = false;
     st = fetch_result(s, ea.result, ca.nocc, stream, &sc, nullptr, &wide);
