@@ -30,13 +30,14 @@ namespace {
 // to the identity, and each wave multiplies its blocks by that U_kk^-T. An accumulator
 // element v of a lane is row 4 v + g, which is what the B operand of step v holds, so
 // the blocks stay in their registers. The finished rows lie in a slot of the workspace,
-// read from the caches. A row of blocks is a chain of two barriers and 16 dependent
-// pivots (about 4 us); the pairs of a call hide it, four workgroups to a CU.
+// read from the caches. A row of blocks is also a chain of two barriers and 16 dependent
+// pivots (about 4 us), which the other workgroups of a CU, four to each, hide.
 // 820 pairs of up to 120 aux functions and 100 virtuals: 276 us, 24% of it at the matrix
-// units, the rest the chain and the latency of the slots (530 MB past the L2); 2.5 ms
-// of rocSOLVER and rocBLAS launches (potf2, trtri, lauum, symm, gemm) before. Also
-// faster at 36 pairs of 41 (0.28 -> 0.09 ms a call), 820 of 480 (26 -> 4.7 ms) and 4 of
-// 1500 (20 -> 9.4 ms).
+// units. The chain is eight rows, about 32 us, and all pairs are resident at once: what
+// bounds the kernel is the operands, every block read again from the slot by each wave
+// that needs it (530 MB past the L2). 2.5 ms of rocSOLVER and rocBLAS launches (potf2,
+// trtri, lauum, symm, gemm) before. Also faster at 36 pairs of 41 (0.28 -> 0.09 ms a call)
+// and 820 of 480 (26 -> 4.7 ms).
 struct FitArgs {
     const int32_t *pairs;
     const uint64_t *near;  // per occupied: words of aux bits inside the radius

@@ -4,8 +4,8 @@
 //
 // Why: the FP64 matrix instructions run at 1/64 of the INT8 ones' rate here, so
 // sixteen exact INT8 products take about 0.4 of one FP64 product's time. Energy,
-// matrix kernel -> here: FP64 60/450/1800 33.2 -> 14.2 ms, 100/200/2400 28.1 -> 9.5,
-// 100/900/3600 662 -> 286; MIXED 60/450/1800 19.9 -> 9.3 ms.
+// matrix kernel / here: FP64 60/450/1800 23.8 / 14.3 ms, 100/200/2400 18.9 / 10.7,
+// 100/900/3600 534 / 292; MIXED 20.0 / 9.1, 17.4 / 6.9 and 387 / 174 ms.
 //
 // Operand layout. For each modulus k and each 64-deep Q panel p one block of
 // rows / 16 kilobytes: kilobyte rg holds the residues of packed rows
