@@ -178,7 +178,9 @@ fh_status fh_init(int device);
 const char *fh_last_error(void);
 
 /* Pool ceiling in bytes for the library's device workspace (0 restores the
- * default: FERRIC_GPU_MEM_GB if set, else 80% of free device memory). */
+ * default: FERRIC_GPU_MEM_GB if set, else 80% of free device memory). Some
+ * calls take a faster route with a larger workspace where it fits; what such
+ * a route grew is given back when a later call needs the room. */
 fh_status fh_set_pool_limit(size_t bytes);
 fh_status fh_get_pool_limit(size_t *bytes);
 

@@ -149,3 +149,33 @@ def test_other_entries(tail, monkeypatch, timing):
     monkeypatch.setenv("FERRIC_HIP_TILE", "64")
     want, _ = results()
     assert all(np.array_equal(x, y) for x, y in zip(got, want))
+
+
+@pytest.mark.parametrize("weight", [lambda d: np.exp(-d), lambda d: np.ones_like(d)],
+                         ids=["wide", "ordinary"])
+def test_mixed_out_of_range_is_refused_on_either_route(weight):
+    """max|B| past sqrt(FLT_MAX / 64) = 2.3e18."""
+    print("residue ranges, refused", flush=True)
+    b, eps = _chain(weight, 42)
+    with pytest.raises(_lib.RangeError):
+        estimate_pair_energies_from_b_ov(torch.from_numpy(b * 1e21).cuda(), eps, NOCC, NVIR,
+                                         precision=Precision.MIXED)
+
+
+@pytest.mark.parametrize("scale", [1e-120, 1e-30, 1e30, 1e120])
+def test_scaled_rows(scale, monkeypatch, timing):
+    """A scale of B by itself moves no digits; where the squares leave the range of the test, or
+    come near its ends, the matrix kernel's bits (at 1e120 the energies themselves overflow)."""
+    print("residue ranges, scale", scale, flush=True)
+    b, eps = _chain(lambda d: np.ones_like(d), 42)
+    t = torch.from_numpy(b * scale).cuda()
+    pe = estimate_pair_energies_from_b_ov(t, eps, NOCC, NVIR)
+    if 1e-60 < scale < 1e60:
+        assert _tile() == 256
+        _against_matrix(b * scale, eps, Precision.FP64, monkeypatch)
+        return
+    assert _tile() == 64
+    monkeypatch.setenv("FERRIC_HIP_TILE", "64")
+    pm = estimate_pair_energies_from_b_ov(t, eps, NOCC, NVIR)
+    assert np.array_equal(pe.e_os, pm.e_os, equal_nan=True)
+    assert np.array_equal(pe.e_ss, pm.e_ss, equal_nan=True)

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-from ferric_amd import Precision, _lib, rimp2, synthetic  # noqa: E402
+from ferric_amd import Precision, _lib, batched, rimp2, synthetic  # noqa: E402
 from ferric_amd.dlpno import estimate_pair_energies_from_b_ov  # noqa: E402
 from tests.test_gpu_adjoint_amplitudes import _host, _problem  # noqa: E402
 
@@ -103,3 +103,35 @@ def test_a_call_past_the_ceiling_is_refused_as_before(pool):
     with pytest.raises(_lib.PoolFullError):
         _gradient()
     assert _lib.stats()["fail_pool_full"] == 1
+
+
+def test_batched_graph_after_slots_were_given_back(pool):
+    """The captured graphs hold workspace pointers: a residue call grows the operand slot that
+    they read, a ceiling makes the next call free it, and the domains' energies stay the same
+    bit for bit."""
+    rng = np.random.default_rng(2)
+    nocc, nvir, naux = np.array([3, 5, 8]), np.array([40, 90, 130]), np.array([100, 200, 333])
+    size = nocc * nvir * naux
+    b = torch.from_numpy(rng.standard_normal(int(size.sum())) * 0.02).cuda()
+    eps = torch.from_numpy(np.concatenate(
+        [np.concatenate([np.linspace(-1.2, -0.4, o), np.linspace(0.2, 4.0, v)])
+         for o, v in zip(nocc, nvir)])).cuda()
+    offs = np.concatenate([[0], np.cumsum(size)[:-1]])
+    eoff = np.concatenate([[0], np.cumsum(nocc + nvir)[:-1]])
+
+    def run():
+        return batched.domain_energies(b, eps, nocc, nvir, naux, offs, eoff,
+                                       precision=Precision.BF16X3)
+
+    want = run()
+    assert all(np.array_equal(x, y) for x, y in zip(want, run()))
+    small = _lib.stats()["pool_peak_bytes"]
+    p = synthetic.decane_scale()
+    t = torch.from_numpy(p.b_ov).cuda()
+    for _ in range(2):
+        estimate_pair_energies_from_b_ov(t, p.eps, p.nocc, p.nvir)
+        assert all(np.array_equal(x, y) for x, y in zip(want, run()))
+        assert pool.fh_set_pool_limit(small + (64 << 20)) == 0
+        _gradient(Precision.BF16X3)
+        assert all(np.array_equal(x, y) for x, y in zip(want, run()))
+        assert pool.fh_set_pool_limit(0) == 0
