@@ -41,7 +41,8 @@ def test_diagonal(at, bad):
     print("fit diagonal", at, bad, flush=True)
     v = _metric()
     v[at, at] = bad
-    with pytest.raises(_lib.KernelError, match=rf"not positive definite \(Cholesky info {at + 1}\)"):
+    with pytest.raises(_lib.KernelError,
+                       match=rf"not positive definite \(Cholesky info {at + 1}\)"):
         _fit(v)
 
 
