@@ -420,30 +420,49 @@ fh_status reserve_residue(State &s, Prec prec, int64_t nitems, int products, siz
     return FH_OK;
 }
 
+// Estimated us of a call of the matrix kernels, 64-wide, off by 6% in FP64, 5% in MIXED and
+// 7% opposite spin at the calls of residue_estimate: a call, the depth of an item, items, and
+// 1000 aux functions of 1000 items. FP64 counts items of full tiles with the two products of
+// i < j off the diagonal, with one, and those with a last tile that is spread over the waves
+// (at most 32 virtuals; 1.6 of them where it has more than 16); without two products anywhere
+// an item is half as deep. The others take whole tiles, so items and their padded FLOP do.
+double matrix_estimate(const ResidueShape &p, double nocc, int ng, double nocc_b, int ng_b,
+                       double naux) {
+    const int t = (ng + 3) / 4, t_b = (ng_b + 3) / 4;
+    const double depth = naux * 1e-3;
+    if (p.rect || p.prec != Prec::F64) {
+        const double pairs = p.rect ? nocc * nocc_b : 0.5 * nocc * (nocc + 1);
+        const double items = pairs * (p.rect ? t * t_b : 0.5 * t * (t + 1)) * 1e-3;
+        const double full = pairs * ng * ng_b / 16 * 1e-3;  // tiles without their padding
+        return p.rect ? 74 + depth * (25 + 126 * items + 31.8 * full) + 11.1 * items
+                      : 137 + depth * (49 + 72.2 * items + 55.8 * full) + 17.9 * items;
+    }
+    const double off = 0.5 * nocc * (nocc - 1) * 1e-3, diag = nocc * 1e-3;
+    const int last = ng - 4 * (t - 1), f = last <= 2 ? t - 1 : t;
+    const double two = off * (0.5 * f * (f - 1)), one = off * f + diag * (0.5 * f * (f + 1));
+    double narrow = 0.0;
+    if (f < t) narrow = ((off + 0.5 * diag) * f + 0.5 * (off + diag)) * (last == 1 ? 1.0 : 1.6);
+    return 75 + depth * ((f > 1 ? 54 : 29) + 273 * two + 94 * one + 110 * narrow) +
+           9.1 * (off + diag) * (0.5 * t * (t + 1));
+}
+
 // Which calls run in residue arithmetic (residue.hip): those whose pass is estimated at less
-// than 0.93 of that of the matrix kernel of the same precision, 64-wide, for which the 1500
-// calls of residue_estimate gave the constants below (off by 7% in FP64, 4% in MIXED, 6%
-// opposite spin). Residues need a full chip (rounds of a workgroup per CU) and a rebuild of
-// the products, the same at any aux count, that is small beside them. matrix / residue, us:
+// than that of the matrix kernel of the same precision, 64-wide. Residues need a full chip
+// (rounds of a workgroup per CU) and a rebuild of the products, the same at any aux count, that
+// is small beside them. matrix / residue, us:
 // FP64 15/215/4073 1325 / 604, 51/109/4278 2799 / 1510, but 46/200/60 and 25/153/503 (264 / 295)
-// the other way; MIXED 36/221/2347 2633 / 1167, but 23/491/177 574 / 781. Over 900 other calls
-// of the same ranges 453 went to the residues: 7 of 180 in FP64 by more than 2% slower so (at
-// most 5%), none of 137 in MIXED, 4 of 136 in opposite spin (at most 7%).
+// the other way; MIXED 36/221/2347 2633 / 1167, but 23/491/177 574 / 781. Over 1300 other calls
+// of the same ranges the route taken was the slower one by more than 2% for 63 of 814 in FP64
+// (at most 20%), 12 of 236 in MIXED (9%) and 10 of 250 in opposite spin (9%).
 // Fewer than 65 virtuals leave three quarters of a tile empty: never faster.
 // INT8X4 stays with its digit slices: ten moduli against their thirteen products gave
 // 70/208/889 1.2, but 70/340/1312 0.95 and 100/900/3600 0.98.
 // FERRIC_HIP_TILE=256 takes the residues wherever they can run.
-bool residue_pays(const ResidueShape &p, double flops, double items, double naux) {
+bool residue_pays(const ResidueShape &p, size_t nocc, int nvir_pad, size_t nocc_b, int nvir_pad_b,
+                  size_t naux) {
     if (forced_residue()) return true;
-    // Products of the padded virtuals, and of whole 64 x 64 tiles (which the opposite-spin
-    // kernel multiplies), in FLOP; tiles, and the depth of one.
-    const double tiles = items * 4096.0 * (p.rect ? 2.0 : 4.0) * naux;
-    const double matrix =
-        p.rect ? 67 + flops * 2.9e-9 + tiles * 16e-9 + items * 12.8e-3 + naux * 30e-3
-        : p.prec == Prec::F64
-            ? 75 + flops * 15.1e-9 + tiles * 1.2e-9 + items * 7.8e-3 + naux * 37e-3
-            : 138 + flops * 6.3e-9 + tiles * 4.9e-9 + items * 14.7e-3 + naux * 45e-3;
-    return residue_estimate(p) < 0.93 * matrix;
+    return residue_estimate(p) < matrix_estimate(p, (double)nocc, nvir_pad / 16, (double)nocc_b,
+                                                 nvir_pad_b / 16, (double)naux);
 }
 
 bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, EnergyPlan *pl) {
@@ -465,11 +484,7 @@ bool plan_residue(State &s, size_t nocc, size_t nvir, size_t naux, Prec prec, En
     r.np = p.naux_pad / 64;
     r.cus = s.cus;
     r.elements = (double)naux * (double)(nocc * nvir);
-    const double unique = 0.5 * (double)nocc * (double)(nocc + 1), vp = p.nvir_pad;
-    const double t = (p.nvir_pad + 63) / 64;
-    if (!residue_pays(r, 2.0 * unique * vp * vp * (double)naux, unique * t * (t + 1) / 2,
-                      (double)naux))
-        return false;
+    if (!residue_pays(r, nocc, p.nvir_pad, nocc, p.nvir_pad, naux)) return false;
     *pl = p;
     return true;
 }

@@ -182,7 +182,8 @@ int compute_units(State &s);  // of the device, asked once; at least 1
 // shape is faster so, and its plan; and the workspace of a launch.
 bool residue_tiles(State &s, size_t nvir, size_t naux, EnergyPlan *pl);
 // Whether it is faster: FLOP and 64 x 64 items of the padded problem on the matrix kernel.
-bool residue_pays(const ResidueShape &p, double flops, double items, double naux);
+bool residue_pays(const ResidueShape &p, size_t nocc, int nvir_pad, size_t nocc_b, int nvir_pad_b,
+                  size_t naux);
 struct ResidueSpace {
     ResidueArgs args;    // prec, np, beta, op, rexp, nitems, blocks, scratch, queue, order
     ResidueOrder order;  // words, queue, order

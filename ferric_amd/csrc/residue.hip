@@ -883,8 +883,10 @@ bool pack_sizes(const PackArgs &a) {
 
 // The longest XCD's rounds (the last by the moduli that its split workgroups take each), in
 // steps of a panel and modulus whose cost follows the blocks that the waves multiply, and in
-// rebuilds; packing; launches and the wait. Fitted to 1500 calls of 65 to 560 virtuals, 4 to
-// 90 occupied and 60 to 4608 aux functions (0.15 to 20 ms): off by 9% in FP64 and 6% in MIXED.
+// rebuilds, both cheaper while the chip has one round; packing; launches and the wait. Fitted
+// to the 1800 of 2600 calls (65 to 560 virtuals, 4 to 90 occupied, 60 to 4608 aux functions,
+// 0.15 to 20 ms) whose two routes are within 1.7 of each other: off by 5% in FP64, 4% in MIXED
+// and 3% opposite spin.
 double residue_estimate(const ResidueShape &p) {
     const int n = residue_moduli(p.prec), wide = p.cus / kXcds;
     double steps = 0.0, ends = 0.0;
@@ -905,11 +907,17 @@ double residue_estimate(const ResidueShape &p) {
                    : rows <= 7                 ? 7
                                                : 8;
     const int ny = std::max(2, (p.wB + 3) / 4);
-    const bool f64 = p.prec == Prec::F64;
-    const double step = f64 ? 0.30 + 0.43 * nx * ny / 32.0 : 0.34 + 0.24 * nx * ny / 32.0;
-    return (f64 ? 100.0 : 150.0) + steps * products * n * p.np * step +
-           ends * products * n * (p.wA * p.wB / 256.0) * (f64 ? 7.5 : 10.4) +
-           p.elements * (f64 ? 1.0e-6 : 9.0e-6);
+    // A call, then us of a step at 32 blocks, a step, a rebuilt tile of 16 x 16 blocks and
+    // modulus with one round, the same with more, a modulus's pass, and 1e6 elements of B.
+    static const double kCost[3][9] = {
+        {130.5, 0.509, 0.162, 4.80, 0.480, 0.221, 8.90, -0.557, 5.86},   // FP64
+        {180.0, 0.444, 0.176, 5.92, 0.279, 0.269, 10.87, 0.083, 8.46},   // MIXED
+        {103.1, 0.464, 0.195, 5.36, 0.493, 0.177, 6.20, 1.119, 7.69}};   // opposite spin
+    const double *k = kCost[p.rect ? 2 : p.prec == Prec::F64 ? 0 : 1];
+    const double *c = ends <= 1.0 ? k + 1 : k + 4;
+    const double passes = ends * products * n;
+    return k[0] + steps * products * n * p.np * (c[0] * nx * ny / 32.0 + c[1]) +
+           passes * (c[2] * p.wA * p.wB / 256.0 + k[7]) + p.elements * 1e-6 * k[8];
 }
 
 int residue_moduli(Prec prec) { return prec == Prec::F64 ? 16 : 10; }

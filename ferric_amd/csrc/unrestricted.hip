@@ -62,9 +62,7 @@ fh_status opposite_residue(State &s, const fh_spin_channel &ca, const fh_spin_ch
     r.cus = s.cus;
     r.rect = true;
     r.elements = (double)naux * (double)(ca.nocc * ca.nvir + cb.nocc * cb.nvir);
-    const double ta = (pa.nvir_pad + 63) / 64, tb = (pb.nvir_pad + 63) / 64;
-    if (!residue_pays(r, 2.0 * (double)npairs * pa.nvir_pad * pb.nvir_pad * (double)naux,
-                      (double)npairs * ta * tb, (double)naux))
+    if (!residue_pays(r, ca.nocc, pa.nvir_pad, cb.nocc, pb.nvir_pad, naux))
         return FH_OK;
     const size_t rows_a = ca.nocc * (size_t)pa.nvir_pad, rows_b = cb.nocc * (size_t)pb.nvir_pad;
     const size_t neps = ca.nocc + ca.nvir + cb.nocc + cb.nvir;
